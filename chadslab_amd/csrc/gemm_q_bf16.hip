@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "chadq_common.h"
+#include "gemm_tile_q.h"
 
 #ifndef CHADQ_GEMM_ABLATE
 #define CHADQ_GEMM_ABLATE 0  // measurement builds only: 1 = the dequantisation compiled out (packed words go to the matrix core as they are)
@@ -429,21 +430,35 @@ static int launch_gemm(const uint16_t *x, const void *wq, const typename F::scal
     return launch_gemm_g<F, 2, false, OUTF32>(x, wq, sc, y, M, N, K, groups, ngroups, st);
 }
 
-bool gemm_big_i4g32_ok(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, int M, int N, int K);
-int gemm_big_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, hipStream_t st);
+// Which tile.  A tile alone on a compute unit takes about as long as one on each of them, so a launch lasts as many rounds
+// of 256 tiles as it has, the last one 1/2 + fill/2 of a full one (measured: 0.65 at a quarter, 0.7-0.75 at a half).  A
+// full round of the 128 x 64 tile of this file takes 24 us per 4096 k (int8: 28), one of the 128 x 128 tile of
+// gemm_tile_q.hip 38, one of its 256 x 256 tile 114: the larger the tile, the less is fetched and dequantised per
+// product.  The rule takes the shortest and was the right one at every shape tried, e.g. at 4096 columns and k:
+// 512 rows 24 us (128 x 128: 27), 1024 rows 38 (128 x 64: 47), 2048 rows 74 (256 x 256: 78), 4096 rows 113 (144).
+enum GemmTile { TILE_128x64, TILE_128, TILE_256 };
+static GemmTile pick_tile(int M, int N, int K, bool int4) {
+    auto cost = [&](int bm, int bn, double full) {
+        const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn), rounds = (tiles + 255) / 256;
+        const double fill = (double)(tiles - (rounds - 1) * 256) / 256.0;
+        return full * ((double)(rounds - 1) + 0.5 + 0.5 * fill);
+    };
+    const double c64 = cost(128, 64, int4 ? 24.0 : 28.0), c128 = cost(128, 128, 38.0), c256 = cost(256, 256, 114.0);
+    if (!gemm_tile_q_ok(K) || (c64 <= c128 && c64 <= c256)) return TILE_128x64;
+    return c128 <= c256 ? TILE_128 : TILE_256;
+}
 
 int gemm_i4g32_bf16_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N,
                              int K, hipStream_t st) {
-    // many rows: the 256 x 256 tile, which dequantises a weight once per 256 rows, as soon as its tiles cover most of
-    // the chip (a tile alone on a compute unit takes about as long as all of them together: at 4096 columns the small
-    // tile is still ahead at 2048 rows, 101 against 115 us)
-    const int64_t big_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-    if (big_tiles >= 176 && gemm_big_i4g32_ok(x, wp, sc, M, N, K)) return gemm_big_i4g32_launch(x, wp, sc, y, M, N, K, st);
+    const GemmTile t = pick_tile(M, N, K, true);
+    if (t != TILE_128x64) return gemm_tile_i4g32_launch(x, wp, sc, y, M, N, K, t == TILE_256, st);
     return launch_gemm<FmtI4G32, false>(x, wp, sc, y, M, N, K, nullptr, 0, st);
 }
 
 int gemm_i8row_bf16_dispatch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K,
                              hipStream_t st) {
+    const GemmTile t = pick_tile(M, N, K, false);
+    if (t != TILE_128x64) return gemm_tile_i8row_launch(x, w8, sc, y, M, N, K, t == TILE_256, st);
     return launch_gemm<FmtI8Row, false>(x, w8, sc, y, M, N, K, nullptr, 0, st);
 }
 

@@ -442,6 +442,26 @@ def test_gemm_int4_many_rows_tile(ops, m, n, k):
     assert O.rel_l2(y, O.qgemm_int4g32_f64(xb, packed, s)) <= TOL_BF16
 
 
+@pytest.mark.parametrize("m,n,k", [(385, 8200, 64), (641, 4100, 96), (1025, 4095, 32), (1024, 4096, 384), (897, 4223, 1312),  # 128 x 128 tiles
+                                   (3841, 3847, 32), (4096, 4097, 288), (3840, 4096, 256)])                               # 256 x 256
+@pytest.mark.parametrize("weight", ["int4", "int8"])
+def test_gemm_eight_wave_tiles_every_row_and_column(ops, weight, m, n, k):
+    """The tiles of gemm_tile_q.hip at ragged ends of rows, columns and k (k of one, two and three steps, no multiple of a
+    step or of a 256-k block of scales).  Every row and every column of the result is held to the bf16 bound by itself, so
+    that one wrong row at the edge of a tile cannot hide in the norm of the whole."""
+    if weight == "int4":
+        packed, s, xb, qw = i4_case(620 + m + k, m, n, k)
+        ref = O.qgemm_int4g32_f64(xb, packed, s)
+    else:
+        x, w, s, qw = i8_case(620 + m + k, m, n, k)
+        xb = O.f32_to_bf16(x)
+        ref = O.qgemm_int8_f64(xb, w, s)
+    y = O.bf16_to_f32(bits(ops.qgemm(bf16_tensor(xb), qw)))
+    err = (y - ref) ** 2
+    for axis in (0, 1):
+        assert np.sqrt(err.sum(axis=axis) / (ref ** 2).sum(axis=axis)).max() <= TOL_BF16
+
+
 def test_gemm_int4_many_rows_full_k_and_integer_exact(ops):
     from chadslab_amd import QWeightInt4G32
 

@@ -157,6 +157,23 @@ __device__ __forceinline__ bf16x8 dequant8_i4(uint32_t w, float s, float s16, fl
     return o;
 }
 
+// Eight fp32 values as two MFMA operands of eight bf16 each: `hi` holds the values cut off after 16 bits (exact), `lo`
+// what is left, cut off the same way, so hi + lo carries 16 mantissa bits of every value - more than the bf16 K and V
+// rows they are multiplied with.  Element e sits in half-word e.
+__device__ __forceinline__ void split_bf16x8(const f32x4 a, const f32x4 b, bf16x8 &hi, bf16x8 &lo) {
+    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t u0 = __float_as_uint(v[2 * e]), u1 = __float_as_uint(v[2 * e + 1]);
+        h[e] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // the two high half-words
+        const float r0 = v[2 * e] - __uint_as_float(u0 & 0xFFFF0000u), r1 = v[2 * e + 1] - __uint_as_float(u1 & 0xFFFF0000u);
+        l[e] = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), 0x07060302u);
+    }
+    __builtin_memcpy(&hi, h, 16);
+    __builtin_memcpy(&lo, l, 16);
+}
+
 // A constant the optimiser must keep in a vector register.
 __device__ __forceinline__ uint32_t vgpr_const(uint32_t v) {
     uint32_t r;

@@ -341,23 +341,6 @@ __global__ __launch_bounds__(256) void rope_table_kernel(float *__restrict__ tab
     table[2 * i + 1] = sn;
 }
 
-// Eight fp32 values as two MFMA operands of eight bf16 each: `hi` holds the values cut off after 16 bits (exact), `lo`
-// what is left, cut off the same way, so hi + lo carries 16 mantissa bits of every value - more than the bf16 K and V
-// rows they are multiplied with.  Element e sits in half-word e.
-__device__ __forceinline__ void split_bf16x8(const f32x4 a, const f32x4 b, bf16x8 &hi, bf16x8 &lo) {
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    uint32_t h[4], l[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const uint32_t u0 = __float_as_uint(v[2 * e]), u1 = __float_as_uint(v[2 * e + 1]);
-        h[e] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // the two high half-words
-        const float r0 = v[2 * e] - __uint_as_float(u0 & 0xFFFF0000u), r1 = v[2 * e + 1] - __uint_as_float(u1 & 0xFFFF0000u);
-        l[e] = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), 0x07060302u);
-    }
-    __builtin_memcpy(&hi, h, 16);
-    __builtin_memcpy(&lo, l, 16);
-}
-
 // Workgroup b: positions [32b, 32b+32).  qkv fp32 = [hq*dh | dh | dh] straight from the projection.  Every
 // workgroup rotates q itself (table lookup): thread (head, 8-column piece) rotates its piece once and the rotated q
 // goes through LDS.  The workgroup that owns position pos also rotates k, writes row pos of both caches and puts the
@@ -486,7 +469,7 @@ __global__ __launch_bounds__(256) void attn_mqa_fused_kernel(const float *__rest
     for (int j = 0; j < 4; ++j) {
         const int ch = tid + 256 * j, row = ch / lpr, vcc = ch % lpr;
         if (row < ATT_CS && !(own && p0 + row == p))
-            *reinterpret_cast<u32x4 *>(&s_v[row][vcc * 8]) = (!FULL || p0 + row < ctx) ? vld[j] : u32x4{0, 0, 0, 0};
+            *reinterpret_cast<u32x4 *>(&s_v[row][vcc * 8]) = p0 + row < ctx ? vld[j] : u32x4{0, 0, 0, 0};
     }
     if (own) {
         if (tid < half) {

@@ -61,6 +61,9 @@ SIGNATURES = {
     "chadq_gemv_i4g32_argmax_scratch_bytes": (c_size_t, [c_int, c_int]),
     "chadq_gemv_i4g32_argmax": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int,
                                         c_void_p, c_void_p]),
+    "chadq_prompt_i4g32_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "chadq_prompt_i4g32": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
+                                   c_int, c_float, c_void_p, c_void_p, c_size_t, c_void_p]),
     "chadq_sample_topk_f32": (c_int, [c_void_p, c_int, c_int, c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
 }
 
@@ -68,6 +71,12 @@ SIGNATURES = {
 class MoeExpertI4G32(ctypes.Structure):
     """Mirror of chadq_moe_expert_i4g32: six device pointers."""
     _fields_ = [(n, c_void_p) for n in ("wg", "sg", "wu", "su", "wd", "sd")]
+
+
+class PromptLayerI4G32(ctypes.Structure):
+    """Mirror of chadq_prompt_layer_i4g32: the device pointers of one layer."""
+    _fields_ = [(n, c_void_p) for n in ("ln1", "wqkv", "sqkv", "wo", "so", "ln2", "wgu", "sgu", "wd", "sd", "kcache", "vcache")]
+
 
 _STATUS_EXC = {-1: ValueError, -2: ValueError, -3: ValueError, -4: ValueError, -5: RuntimeError, -6: RuntimeError}
 

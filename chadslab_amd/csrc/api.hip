@@ -95,6 +95,10 @@ int argmax_embed_launch(const float *, bool, float *, int32_t *, int, int, int32
 bool gemv_i4g32_argmax_ok(const uint16_t *, int, int);
 int gemv_i4g32_argmax_launch(const uint16_t *, const uint8_t *, const uint16_t *, float *, int, int, float *, int32_t *, int *,
                              hipStream_t);
+bool prompt_i4g32_ok(int, int, int, int);
+size_t prompt_i4g32_workspace_bytes(int, int, int, int, int);
+int prompt_i4g32_launch(const chadq_prompt_layer_i4g32 *, int, const int32_t *, const uint8_t *, const uint16_t *, int, const float *, int, int,
+                        int, int, int, int, float, float *, void *, hipStream_t);
 int sample_topk_launch(const float *, int, int, float, const float *, float *, int32_t *, int32_t *, int32_t *, int, hipStream_t);
 
 }  // namespace chadq
@@ -509,6 +513,37 @@ int chadq_sample_topk_f32(const float *v, int n, int k, float temperature, const
     float *cv = reinterpret_cast<float *>(workspace);
     int32_t *ci = reinterpret_cast<int32_t *>(cv + 96 * 64);
     return sample_topk_launch(v, n, k, temperature, u, cv, ci, token, pos, advance, st);
+}
+
+size_t chadq_prompt_i4g32_workspace_bytes(int T, int d, int hq, int dh, int ffn) {
+    if (T < 1 || !prompt_i4g32_ok(d, hq, dh, ffn)) return 0;
+    return prompt_i4g32_workspace_bytes(T, d, hq, dh, ffn);
+}
+
+int chadq_prompt_i4g32(const chadq_prompt_layer_i4g32 *layers, int n_layers, const int32_t *tokens, const uint8_t *emb,
+                       const uint16_t *semb, int V, const float *rope_table, int T, int pos, int d, int hq, int dh, int ffn,
+                       int max_ctx, float eps, float *x_last, void *workspace, size_t workspace_bytes, void *stream) {
+    ENTER();
+    CHADQ_REQUIRE(T >= 1 && n_layers >= 1 && V >= 1 && prompt_i4g32_ok(d, hq, dh, ffn), CHADQ_ERR_SHAPE,
+                  "chadq_prompt_i4g32: T=%d n_layers=%d V=%d d=%d hq=%d dh=%d ffn=%d (d, hq*dh, ffn multiples of 256, d <= 2048, "
+                  "dh 64, 128 or 256)", T, n_layers, V, d, hq, dh, ffn);
+    CHADQ_REQUIRE(pos >= 0 && pos <= max_ctx - T, CHADQ_ERR_SHAPE, "chadq_prompt_i4g32: positions %d..%d do not fit %d cache rows", pos,
+                  pos + T - 1, max_ctx);
+    CHADQ_REQUIRE(layers && tokens && emb && semb && rope_table && x_last, CHADQ_ERR_NULL, "chadq_prompt_i4g32: null pointer");
+    for (int i = 0; i < n_layers; ++i) {
+        const chadq_prompt_layer_i4g32 &l = layers[i];
+        CHADQ_REQUIRE(l.ln1 && l.wqkv && l.sqkv && l.wo && l.so && l.ln2 && l.wgu && l.sgu && l.wd && l.sd && l.kcache && l.vcache,
+                      CHADQ_ERR_NULL, "chadq_prompt_i4g32: layer %d has a null pointer", i);
+        CHADQ_REQUIRE(aligned16(l.ln1) && aligned16(l.wqkv) && aligned16(l.sqkv) && aligned16(l.wo) && aligned16(l.so) && aligned16(l.ln2) &&
+                          aligned16(l.wgu) && aligned16(l.sgu) && aligned16(l.wd) && aligned16(l.sd) && aligned16(l.kcache) && aligned16(l.vcache),
+                      CHADQ_ERR_ALIGN, "chadq_prompt_i4g32: layer %d: every array must be 16-byte aligned", i);
+    }
+    CHADQ_REQUIRE(aligned16(emb) && aligned16(x_last) && aligned16(workspace), CHADQ_ERR_ALIGN,
+                  "chadq_prompt_i4g32: emb, x_last and workspace must be 16-byte aligned");
+    const size_t need = prompt_i4g32_workspace_bytes(T, d, hq, dh, ffn);
+    CHADQ_REQUIRE(workspace && workspace_bytes >= need, CHADQ_ERR_WORKSPACE, "chadq_prompt_i4g32: workspace of %zu bytes needed, %zu given",
+                  need, workspace ? workspace_bytes : (size_t)0);
+    return prompt_i4g32_launch(layers, n_layers, tokens, emb, semb, V, rope_table, T, pos, d, hq, dh, ffn, eps, x_last, workspace, st);
 }
 
 }  // extern "C"

@@ -11,5 +11,13 @@ bool gemm_tile_q_ok(int K);
 // y bf16 [M,N]; big: 256 x 256 tiles, else 128 x 128
 int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, bool big, hipStream_t st);
 int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, bool big, hipStream_t st);
+// int4 weights taken exactly (nothing rounded before the fp32 sums); K % 256 == 0, x, wp and sc 16-byte aligned
+constexpr int kExactMaxSplits = 8;
+int gemm_exact_splits(int M, int N, int K);  // K splits to use for gemm_exact_f32_launch
+// y_parts fp32 [ksplit][M,N]
+int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
+                          hipStream_t st);
+// weight rows in (gate, up) pairs: h[m,i] = bf16(gelu_tanh(y[m,2i]) * y[m,2i+1]), [M, N/2]
+int gemm_exact_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st);
 
 }  // namespace chadq

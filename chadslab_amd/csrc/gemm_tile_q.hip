@@ -464,4 +464,40 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
     return K % 128 ? tileq::launch<false, 4, 2, 4, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 4, 2, 4, false>(x, w, sc, y, M, N, K, 1, st);
 }
 
+// ---- exact weights (HILO), K % 256 == 0: the projections of a prompt, whose tokens must come out as the decode step's do.
+// Tiles of 32, 64 or 128 rows x 128 weight rows; with few rows the weight stream decides, not the padding.
+template <int EPI>
+static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st) {
+    if (M <= 32) return tileq::launch<true, 4, 2, 1, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    if (M <= 64) return tileq::launch<true, 4, 2, 2, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    return tileq::launch<true, 4, 2, 4, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+}
+
+// K splits that make the launch shortest: rounds of 256 workgroups times the k of each (and what a workgroup costs
+// besides, about 256 k worth).  At most kMaxSplits parts, each a multiple of 256 k.
+int gemm_exact_splits(int M, int N, int K) {
+    const int bm = M <= 32 ? 32 : M <= 64 ? 64 : 128;
+    const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + 127) / 128);
+    int best = 1;
+    int64_t best_cost = 0;
+    for (int s = 1; s <= kExactMaxSplits; s *= 2) {
+        if (K % (s * 256) != 0) break;
+        const int64_t cost = (tiles * s + 255) / 256 * (K / s + 256);
+        if (s == 1 || cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
+                          hipStream_t st) {
+    return launch_exact<tileq::EPI_F32>(x, wp, sc, y_parts, M, N, K, ksplit, st);
+}
+
+int gemm_exact_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st) {
+    return launch_exact<tileq::EPI_GEGLU>(x, wp, sc, h, M, N, K, 1, st);
+}
+
 }  // namespace chadq

@@ -17,6 +17,10 @@ from . import _lib
 from .formats import QWeightInt4G32, quantize_int4_g32
 
 
+PROMPT_CHUNK = 256  # tokens that go through a layer together
+PROMPT_MIN = 3      # shorter sequences are quicker token by token
+
+
 @dataclass
 class DecoderConfig:
     n_layers: int = 18
@@ -138,6 +142,19 @@ class QuantDecoder:
         self.graph_steps = 1        # tokens per replay of the captured graph
         self.ring = None            # the tokens between the steps of one replay (capture(steps > 1))
 
+    def _describe_layers(self):
+        """The layers' device pointers as chadq_prompt_i4g32 takes them; None where it does not cover the model's sizes."""
+        c = self.cfg
+        if not (self.fused_geglu and self.fused_attn) or self.lib.chadq_prompt_i4g32_workspace_bytes(1, c.d, c.hq, c.dh, c.ffn) == 0:
+            return None
+        arr = (_lib.PromptLayerI4G32 * c.n_layers)()
+        for li, L in enumerate(self.w["layers"]):
+            wqkv, wo, wd, wgu = L["wqkv"], L["wo"], L["wd"], self.wgu_il[li]
+            arr[li] = _lib.PromptLayerI4G32(*(t.data_ptr() for t in (
+                L["ln1"], wqkv.packed, wqkv.scale, wo.packed, wo.scale, L["ln2"], wgu.packed, wgu.scale, wd.packed, wd.scale,
+                self.kcache[li], self.vcache[li])))
+        return arr if all(p % 16 == 0 for a in arr for p in (getattr(a, n) for n, _ in a._fields_)) else None
+
     # ---- single launches -------------------------------------------------------------------------------
     def _s(self):
         return torch.cuda.current_stream().cuda_stream
@@ -245,13 +262,24 @@ class QuantDecoder:
         self._norm(pending, self.w["lnf"])
         if trace is not None:
             trace.append(self.x.clone())
+        self._choose(token_out, u, x_start)
+        if self.x is not x_start:  # an odd number of exchanges: the next step starts from the same buffer as this one
+            self.x, self.x2 = x_start, self.x
+
+    def _output(self, token_out, u, next_x) -> None:
+        """Final norm and output table for the residual vector in self.x, and the choice of the next token."""
+        self._norm(None, self.w["lnf"])
+        self._choose(token_out, u, next_x)
+
+    def _choose(self, token_out, u, next_x) -> None:
+        c, lib, s = self.cfg, self.lib, self._s()
         if self.sampling is None:
             # the output table's GEMV leaves per-workgroup argmax candidates; the kernel that picks the winner also writes
             # the winner's table row where the next step starts from
             emb = self.w["emb"]
             _lib.check(lib.chadq_gemv_i4g32_argmax(self.xn.data_ptr(), emb.packed.data_ptr(), emb.scale.data_ptr(),
                                                    self.logits.data_ptr(), emb.N, emb.K, self.scratch.data_ptr(),
-                                                   token_out.data_ptr(), self.pos.data_ptr(), 1, x_start.data_ptr(), s),
+                                                   token_out.data_ptr(), self.pos.data_ptr(), 1, next_x.data_ptr(), s),
                        "chadq_gemv_i4g32_argmax")
         else:
             self._gemv(self.xn, self.w["emb"], self.logits)
@@ -259,8 +287,6 @@ class QuantDecoder:
             _lib.check(lib.chadq_sample_topk_f32(self.logits.data_ptr(), c.vocab, k, temperature, u.data_ptr(),
                                                  self.sample_ws.data_ptr(), token_out.data_ptr(), self.pos.data_ptr(), 1, s),
                        "chadq_sample_topk_f32")
-        if self.x is not x_start:  # an odd number of exchanges: the next step starts from the same buffer as this one
-            self.x, self.x2 = x_start, self.x
 
     def set_sampling(self, top_k: int = 0, temperature: float = 1.0, seed: int = 0) -> None:
         """top_k = 0: greedy (argmax).  Otherwise the next token is drawn from the top_k most likely ones at the given
@@ -323,11 +349,16 @@ class QuantDecoder:
                 raise ValueError("token %d is outside the vocabulary [0, %d)" % (int(t), self.cfg.vocab))
 
     def feed(self, tokens, pos: int = 0) -> int:
-        """Runs the step over a given token sequence starting at position `pos` (the prompt, one token at a time: there
-        is no batched prefill here), filling the caches; returns the token the model proposes after the last one.
-        Raises ValueError if the sequence would run past max_ctx or holds a token outside the vocabulary."""
+        """Reads a given token sequence starting at position `pos` (a prompt) into the caches and returns the token the
+        model proposes after the last one.  Where the prompt kernels cover the model's sizes, whole chunks of the sequence
+        go through a layer at once (chadq_prompt_i4g32: every weight is read once per chunk instead of once per token, and
+        only the last token meets the output table); else, and for a sequence of one or two tokens, the step runs token by
+        token.  Raises ValueError if the sequence would run past max_ctx or holds a token outside the vocabulary."""
         tokens = list(tokens)
         self._check_range(pos, len(tokens), tokens)
+        layers = self._describe_layers() if len(tokens) >= PROMPT_MIN else None
+        if layers is not None:
+            return self._feed_chunks(layers, tokens, pos)
         self.pos.fill_(pos)
         for t in tokens:
             self.token.fill_(int(t))  # overrides the token the previous step proposed
@@ -339,6 +370,27 @@ class QuantDecoder:
                 self.graph.replay()
             else:
                 self.step()
+        return int(self.token.item())
+
+    def _feed_chunks(self, layers, tokens: List[int], pos: int) -> int:
+        c, lib, s = self.cfg, self.lib, self._s()
+        ids = torch.tensor(tokens, dtype=torch.int32).to(self.dev)
+        emb = self.w["emb"]
+        ws = torch.empty(lib.chadq_prompt_i4g32_workspace_bytes(min(len(tokens), PROMPT_CHUNK), c.d, c.hq, c.dh, c.ffn),
+                         dtype=torch.uint8, device=self.dev)
+        for t0 in range(0, len(tokens), PROMPT_CHUNK):
+            n = min(PROMPT_CHUNK, len(tokens) - t0)
+            _lib.check(lib.chadq_prompt_i4g32(layers, c.n_layers, ids.data_ptr() + 4 * t0, emb.packed.data_ptr(),
+                                              emb.scale.data_ptr(), c.vocab, self.rope.data_ptr(), n, pos + t0, c.d, c.hq, c.dh, c.ffn,
+                                              c.max_ctx, c.eps, self.x.data_ptr(), ws.data_ptr(), ws.numel(), s), "chadq_prompt_i4g32")
+        self.pos.fill_(pos + len(tokens) - 1)  # the output kernels advance it
+        if self.sampling is not None:
+            # the draw the last token would have got had every token drawn one: a draw moves the generator on by a fixed amount
+            before = self.rng.get_offset()
+            self.u.uniform_(0.0, 1.0, generator=self.rng)
+            self.rng.set_offset(before + (self.rng.get_offset() - before) * (len(tokens) - 1))
+            self.u.uniform_(0.0, 1.0, generator=self.rng)
+        self._output(self.token, self.u[:1], self.x)
         return int(self.token.item())
 
     def generate(self, first_token: int, pos: int, n: int) -> List[int]:

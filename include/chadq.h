@@ -337,6 +337,39 @@ int chadq_gemv_i4g32_argmax(const uint16_t *x_bf16, const uint8_t *wp, const uin
 int chadq_sample_topk_f32(const float *v, int n, int k, float temperature, const float *u, void *workspace, int32_t *token,
                           int32_t *pos, int advance, void *stream);
 
+/* ---- a prompt through the same decoder ----------------------------------------------------- */
+/* Device pointers of one layer.  wqkv [(hq+2)*dh, d], wo [d, hq*dh], wd [d, ffn] int4 group-32; wgu [2*ffn, d] with the
+ * gate row and the up row of a feature next to each other; ln1, ln2 fp32 [d]; caches bf16 [max_ctx, dh]. */
+typedef struct chadq_prompt_layer_i4g32 {
+    const float *ln1;
+    const uint8_t *wqkv;
+    const uint16_t *sqkv;
+    const uint8_t *wo;
+    const uint16_t *so;
+    const float *ln2;
+    const uint8_t *wgu;
+    const uint16_t *sgu;
+    const uint8_t *wd;
+    const uint16_t *sd;
+    uint16_t *kcache;
+    uint16_t *vcache;
+} chadq_prompt_layer_i4g32;
+
+/* Bytes of device workspace chadq_prompt_i4g32 needs (0 if it does not cover the sizes: d, hq*dh and ffn multiples of 256,
+ * d <= 2048, dh one of 64, 128, 256, T >= 1). */
+size_t chadq_prompt_i4g32_workspace_bytes(int T, int d, int hq, int dh, int ffn);
+
+/*
+ * T tokens (device, int32 [T], clamped into the table) at positions pos .. pos+T-1 through n_layers layers (HOST array of
+ * structs): rows pos .. pos+T-1 of every cache, and x_last fp32 [d] = the residual vector of the last token in front of the
+ * final norm, as T decode steps would leave them (activations rounded to bf16 in the same places, weights taken exactly;
+ * sums in another order).  rope_table from chadq_rope_table for at least pos+T rows; emb/semb the int4 table [V, d].
+ * pos + T <= max_ctx is checked.  Everything 16-byte aligned.  Nothing is allocated, nothing waits for the host.
+ */
+int chadq_prompt_i4g32(const chadq_prompt_layer_i4g32 *layers, int n_layers, const int32_t *tokens, const uint8_t *emb,
+                       const uint16_t *semb, int V, const float *rope_table, int T, int pos, int d, int hq, int dh, int ffn,
+                       int max_ctx, float eps, float *x_last, void *workspace, size_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

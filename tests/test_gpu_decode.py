@@ -727,6 +727,67 @@ def test_decoder_feed_then_generate_continues_the_same_sequence():
     assert b.generate(nxt, 7, 5) == seq[7:12]
 
 
+@pytest.mark.parametrize("t,pos,layers,d,hq,dh,ffn", [(3, 0, 2, 512, 4, 64, 1024), (32, 7, 2, 512, 4, 64, 1024), (33, 31, 1, 256, 2, 128, 768),
+                                                      (64, 0, 1, 1024, 8, 128, 1280), (65, 200, 3, 768, 3, 256, 2304), (128, 33, 2, 2048, 8, 256, 4096),
+                                                      (257, 100, 1, 512, 8, 64, 512), (300, 0, 2, 1024, 4, 256, 2048)])
+def test_decoder_prompt_in_chunks_equals_the_step_token_by_token(t, pos, layers, d, hq, dh, ffn):
+    """feed() of a whole prompt (chadq_prompt_i4g32) against the decode step over the same tokens, at the edges of its row
+    tiles (32, 64, 128), of a chunk (256) and of the attention's blocks.  The step rounds in the same places and takes the
+    weights exactly, so the first layer's cache rows may differ by single roundings of a sum in another order only (were
+    the weights rounded to bf16 they would be 2e-3 off); deeper down a rounding that falls the other way grows, by the
+    5e-3 per layer that the layer-by-layer test of the full model allows.  Cache rows the prompt may not see hold NaN."""
+    import chadslab_amd.decoder as D
+
+    cfg = D.DecoderConfig(n_layers=layers, d=d, hq=hq, dh=dh, ffn=ffn, vocab=1003, max_ctx=600)
+    w = D.random_weights(cfg, 60 + t, DEV)
+    a, b = D.QuantDecoder(cfg, w, DEV), D.QuantDecoder(cfg, w, DEV)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(t)
+    for name in ("kcache", "vcache"):
+        for ca, cb in zip(getattr(a, name), getattr(b, name)):
+            ca[:pos * dh] = torch.randn(pos * dh, device=DEV, generator=g).to(torch.bfloat16)
+            cb.copy_(ca)
+            cb[pos * dh:] = float("nan")
+    toks = torch.randint(0, cfg.vocab, (t,), device=DEV, generator=g).tolist()
+    for i, tok in enumerate(toks):
+        a.set_state(tok, pos + i)
+        a.step()
+    nxt = b.feed(toks, pos)
+    assert nxt == int(b.token.item()) and int(b.pos.item()) == pos + t
+
+    def rel(x, y):
+        return float((x.double() - y.double()).norm() / y.double().norm())
+
+    end = (pos + t) * dh
+    for name in ("kcache", "vcache"):
+        for li, (ca, cb) in enumerate(zip(getattr(a, name), getattr(b, name))):
+            assert torch.equal(cb[:pos * dh], ca[:pos * dh]) and bool(torch.isnan(cb[end:]).all())
+            assert rel(cb[pos * dh:end], ca[pos * dh:end]) <= (3e-4 if li == 0 else 5e-3 * li)
+    assert rel(b.logits, a.logits) <= 5e-3 * layers
+    top = b.logits.max()
+    assert float(b.logits[nxt]) == float(top)
+    # what feed() leaves behind is what the next step starts from
+    b.step(embed=False)
+    a.set_state(nxt, pos + t)
+    a.step()
+    assert rel(b.logits, a.logits) <= 5e-3 * layers
+
+
+def test_decoder_prompt_in_chunks_draws_what_single_tokens_would_have_drawn():
+    import chadslab_amd.decoder as D
+
+    cfg = D.DecoderConfig(n_layers=1, d=256, hq=4, dh=64, ffn=512, vocab=300, max_ctx=64)
+    w = D.random_weights(cfg, 77, DEV)
+    a, b = D.QuantDecoder(cfg, w, DEV), D.QuantDecoder(cfg, w, DEV)
+    for dec in (a, b):
+        dec.set_sampling(top_k=20, temperature=1.0, seed=5)
+    toks = list(range(3, 24))
+    for i in range(0, len(toks)):
+        a.feed(toks[i:i + 1], i)
+    b.feed(toks, 0)
+    assert torch.equal(a.u, b.u) and a.rng.get_offset() == b.rng.get_offset()
+
+
 @pytest.mark.parametrize("layers,steps", [(2, 4), (3, 3), (2, 1)])
 def test_decoder_graph_of_several_steps_produces_the_same_tokens(layers, steps):
     """A graph that holds several consecutive steps (tokens handed on through a ring in device memory) against the same

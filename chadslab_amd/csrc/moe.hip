@@ -5,7 +5,7 @@
 // Everything runs on the caller's stream without a host round trip: the router kernel also sorts the
 // (token, slot) pairs by expert (stable: by pair index inside an expert) and writes the per-expert descriptors
 // of the grouped GEMM launches and the list of token tiles that exist, so row counts never leave the GPU.
-// Gate/up/down run on the skinny grouped kernel (gate and up fused with the SiLU gate and reading the activations
+// Gate/up/down of at most 16 tokens run on the weight-streaming kernel of moe_few_i4g32.hip; else on the skinny grouped kernel (gate and up fused with the SiLU gate and reading the activations
 // through the sorted token list, down split over K) when H and F are multiples of 256, else on the prefill
 // dequant-GEMM kernel in grouped mode on a gathered copy of the activations with a separate SiLU kernel; the small
 // kernels here are the router, the gather, the SiLU gate and the weighted combine.
@@ -62,6 +62,14 @@ int gemm_expert_gateup(const GemmGroup *groups, const int32_t *tiles, const int3
 int gemm_expert_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int E, int H, int F, const uint16_t *ha,
                      const float *rs, const uint16_t *ghi, const uint16_t *glo, float *yp, int ksplit, size_t ysplit_stride,
                      hipStream_t st);
+// at most 16 tokens, either weight order (moe_few_i4g32.hip)
+bool moe_few_ok(int T, int H, int F, int E, int top_k, bool tiled);
+int moe_few_tile_rows();
+int moe_few_down_splits(int F);
+int moe_few_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int E, int F, int H, bool tiled,
+                   hipStream_t st);
+int moe_few_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int E, int H, int F, int nsplit, size_t split_stride, bool tiled,
+                 hipStream_t st);
 
 // Workgroup 0.  Phase 1: softmax + top-k per token.  Phase 2: stable counting sort of the pairs by expert.
 // Phase 3: descriptors.  idx/w may be the caller's arrays (chadq_moe_route) with everything else null.
@@ -345,20 +353,23 @@ int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe
     }
     const int P = T * top_k;
     const int m_max = P < T ? P : T;  // an expert gets a token at most once
-    const int tile_rows = tiled ? gemm_expert_tile_rows() : gemm_skinny_tile_rows();
-    const int ntiles = E + P / tile_rows;  // sum over experts of ceil(rows / tile_rows) <= this
     int nsplit = 1;
     bool aligned = true;  // the expert kernels load scales 16 bytes at a time
     for (int e = 0; e < E; ++e)
         aligned = aligned && aligned16(experts[e].wg) && aligned16(experts[e].sg) && aligned16(experts[e].wu) &&
                   aligned16(experts[e].su) && aligned16(experts[e].wd) && aligned16(experts[e].sd);
-    const bool skinny = aligned && (tiled ? gemm_expert_ok(H, F) : gemm_skinny_ok(H, F)) && tile_rows <= 128;
+    const bool expert_ok = aligned && (tiled ? gemm_expert_ok(H, F) : gemm_skinny_ok(H, F));
+    const bool few = expert_ok && moe_few_ok(T, H, F, E, top_k, tiled);
+    const int tile_rows = few ? moe_few_tile_rows() : tiled ? gemm_expert_tile_rows() : gemm_skinny_tile_rows();
+    const int ntiles = few ? E : E + P / tile_rows;  // sum over experts of ceil(rows / tile_rows) <= this
+    const bool skinny = expert_ok && tile_rows <= 128;
     if (tiled && !skinny) return fail(CHADQ_ERR_ALIGN, "moe_ffn (tiled): weights and scales must be 16-byte aligned, H and F multiples of 256");
     const int route_threads = P <= 256 ? 256 : P <= 512 ? 512 : 1024;
     int rc;
     if (skinny) {  // the router also lists the token tiles; gate/up read the activations through tok
-        hipLaunchKernelGGL(moe_route_kernel, dim3(tiled ? 1 + T : 1), dim3(route_threads), 0, st, logits, ws.idx, ws.w, T, E, top_k, renorm,
-                           ws, ex, H, F, x, tile_rows, ntiles, tiled ? x : nullptr);
+        const bool prep = tiled && !few;
+        hipLaunchKernelGGL(moe_route_kernel, dim3(prep ? 1 + T : 1), dim3(route_threads), 0, st, logits, ws.idx, ws.w, T, E, top_k, renorm,
+                           ws, ex, H, F, x, tile_rows, ntiles, prep ? x : nullptr);
         rc = hip_check(hipGetLastError(), "moe route launch");
     } else {
         hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(route_threads), 0, st, logits, ws.idx, ws.w, T, E, top_k, renorm, ws, ex,
@@ -367,7 +378,14 @@ int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe
         rc = hip_check(hipGetLastError(), "moe route/gather launch");
     }
     if (rc) return rc;
-    if (tiled) {
+    if (few) {
+        rc = moe_few_gateup(ws.groups, ws.tiles, ws.tok, ntiles, E, F, H, tiled, st);
+        if (rc) return rc;
+        nsplit = moe_few_down_splits(F);
+        static_assert(MOE_KSPLIT >= 4, "parts of the down product");
+        rc = moe_few_down(ws.groups, ws.tiles, ntiles, E, H, F, nsplit, (size_t)P * H, tiled, st);
+        if (rc) return rc;
+    } else if (tiled) {
         // (the router's launch also made the fp16 form of the activations) gate/up with the SiLU gate, h to fp16, down split over K
         rc = gemm_expert_gateup(ws.groups, ws.tiles, ws.tok, ntiles, E, F, H, ws.xs, ws.rsx, ws.gxh, ws.gxl, ws.h, ws.rowmax, st);
         if (rc) return rc;

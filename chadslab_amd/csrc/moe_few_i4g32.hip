@@ -1,0 +1,291 @@
+// Expert products of a mixture of experts for at most 16 rows per expert (a few decoding tokens): a stream of the weights.
+//
+// What bounds it: the weight stream.  A 4096 x 14336 expert holds 99 MB of packed weights and scales for one to sixteen
+// rows of activations.  The many-row kernel (gemm_skinny_i4g32.hip) takes 256 weight rows per workgroup: with few experts
+// hit that is one and a fraction rounds of the chip, the last one nearly empty.  Here:
+//   * An item of work is 32 weight rows (MODE 1: 16 features of gate and up; MODE 0: 32 rows of down) times K, or times a
+//     K split.  Three workgroups per compute unit walk the items at a stride of the grid, and the loads of the next item
+//     are requested while the present one is summed, so a workgroup's stream has no gap between items.
+//   * The four waves of a workgroup take the item's blocks of 256 k in turn; their sums meet in LDS once per item.
+//   * Everything goes straight to registers, one block ahead: 4 KiB of weights, the scales and the activation operands
+//     (which the caches serve).  Three waves per SIMD with one block ahead measured 4-8 % faster than two with two ahead.
+//   * In row order a load takes whole 128-byte lines of 8 rows, not 64 bytes of 16 (gate/up 97 -> 87 us); two DPP moves
+//     per register pair put the halves in place.
+// Gate/up | down in us, 8 experts of 4096 x 14336, top 2, the skinny kernel in brackets: 4 tokens 87 | 50 (130 | 72),
+// 16 tokens 145 | 81 (191 | 85); 16 experts of 2048 x 4096, top 4, 16 tokens 46 | 27 (47 | 24); 1 token of 1024 x 2048
+// 5.2 | 4.5 (12.8 | 7.0).
+// Arithmetic: v_mfma_f32_16x16x32_bf16 on unscaled weights.  A lane holds a whole scale group of its weight row (16
+// bytes); the lanes' words are exchanged (v_permlane16_swap, v_permlane32_swap) so that one MFMA holds one scale group;
+// nibbles become the bf16 value 128 + u, another MFMA of the same activations with the constant -136 takes the 136 off
+// beforehand for both of the item's row blocks, and one fp32 FMA per value applies the scale: weights are exact.
+// Blocks past the end and rows without a token are requested beyond the buffer's range and arrive as zeros.
+#include "chadq_common.h"
+
+namespace chadq {
+
+constexpr int FEW_ROWS = 16;     // activation rows of an expert
+constexpr int FEW_ENTRIES = 16;  // experts (one entry of the tile list each, as every expert has at most FEW_ROWS rows)
+constexpr int RB = 2;            // blocks of 16 weight rows per item
+constexpr uint32_t kBeyond = 0x80000000u;
+constexpr int kRange = 0x7FFFFFFF;
+
+template <int MODE, bool TILED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void moe_few_i4g32_kernel(
+    const GemmGroup *__restrict__ groups, const int32_t *__restrict__ tiles, const int32_t *__restrict__ tok, int ntiles, int E, int N,
+    int K, int nsplit, size_t split_stride) {
+    struct Entry {
+        const void *w[2], *s[2], *x;
+        void *y;
+        int rows, pad;
+    };
+    __shared__ Entry s_ent[FEW_ENTRIES];
+    __shared__ uint32_t s_xoff[FEW_ENTRIES][FEW_ROWS];
+    __shared__ __attribute__((aligned(16))) f32x4 s_red[2][4][RB][64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, j = lane >> 4;
+
+    {   // thread (entry, row)
+        const int n = tid >> 4, m = tid & 15;
+        const int tile = n < ntiles ? tiles[n] : -1;
+        int rows = 0;
+        if (tile >= 0) {
+            const int e = tile & 0xFFFF;
+            const GemmGroup a = groups[MODE == 1 ? e : 2 * E + e];
+            rows = a.M < FEW_ROWS ? a.M : FEW_ROWS;
+            uint32_t row = m;
+            if (MODE == 1) row = m < rows ? (uint32_t)tok[a.pad + m] : 0u;
+            s_xoff[n][m] = m < rows ? row * (uint32_t)K * 2u : kBeyond;
+            if (m == 0) {
+                const GemmGroup b = groups[MODE == 1 ? E + e : 2 * E + e], d = groups[2 * E + e];
+                s_ent[n] = Entry{{a.w, b.w}, {a.sc, b.sc}, a.x, MODE == 1 ? const_cast<uint16_t *>(d.x) : a.y, rows, 0};
+            }
+        } else if (m == 0) {
+            s_ent[n].rows = 0;
+        }
+    }
+    __syncthreads();
+    int entries = 0;  // the list holds them in front
+    while (entries < ntiles && s_ent[entries].rows > 0) ++entries;
+    entries = __builtin_amdgcn_readfirstlane(entries);
+    const int ntn = MODE == 1 ? N / 16 : N / 32, per = MODE == 1 ? ntn : ntn * nsplit;
+    const int total = entries * per, stride = gridDim.x, nb = K >> 8;
+    auto first_block = [&](int split) { return MODE == 1 ? split * nb : split * nb / nsplit; };
+    auto blocks_of = [&](int item) {  // of each wave
+        const int split = MODE == 1 ? 0 : item % per / ntn;
+        return (first_block(split + 1) - first_block(split) + 3) >> 2;
+    };
+
+    struct Block {  // 256 k = eight scale groups
+        u32x4 x[8], w[RB][2], s[RB];
+    };
+    // ---- the request side
+    int l_item = blockIdx.x, l_i = 0, l_n = 0, l_kb = 0, l_end = 0;
+    __amdgpu_buffer_rsrc_t wr[RB], sr[RB], xr;
+    uint32_t woff = 0, soff = 0, xoff = 0;  // of the lane, in the first row block
+    // the second row block: the same rows of the up matrix, or the next 16 rows
+    const uint32_t wblk = MODE == 1 ? 0u : TILED ? 256u : 8u * K, sblk = MODE == 1 ? 0u : TILED ? 128u : (uint32_t)K;
+    auto uniform = [](const void *p) {
+        const uint64_t v = reinterpret_cast<uint64_t>(p);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+        return reinterpret_cast<void *>(((uint64_t)hi << 32) | lo);
+    };
+    auto open = [&]() {
+        const int en = l_item / per, rem = l_item % per, nt = rem % ntn, split = rem / ntn;
+        l_kb = first_block(split) + wave;
+        l_end = first_block(split + 1);
+        l_n = blocks_of(l_item);
+        l_i = 0;
+        xr = __builtin_amdgcn_make_buffer_rsrc(uniform(s_ent[en].x), 0, kRange, 0x00020000);
+        xoff = s_xoff[en][r] + 16u * j;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            wr[b] = __builtin_amdgcn_make_buffer_rsrc(uniform(s_ent[en].w[b]), 0, kRange, 0x00020000);
+            sr[b] = __builtin_amdgcn_make_buffer_rsrc(uniform(s_ent[en].s[b]), 0, kRange, 0x00020000);
+        }
+        const uint32_t n = (MODE == 1 ? nt * 16 : nt * 32) + r;
+        if (TILED) {  // units of 32 rows x 256 k: [8 groups][32 rows][16 B]; scales [even, odd groups][32 rows][4]
+            woff = (n >> 5) * (uint32_t)nb * 4096u + j * 512u + (n & 31u) * 16u;
+            soff = (n >> 5) * (uint32_t)nb * 512u + (n & 31u) * 8u;
+        } else {  // a load takes 8 rows x 128 bytes, whole lines: the lanes of rows 8..15 take groups 4..7 of rows 0..7
+            woff = (n & ~8u) * (uint32_t)(K >> 1) + j * 16u + (r >> 3) * 64u;
+            soff = n * (uint32_t)(K >> 4);
+        }
+    };
+    auto request = [&](Block &q) {
+        if (l_item >= total) return;
+        const uint32_t kb = l_kb, beyond = l_kb < l_end ? 0u : kBeyond, wv = woff | beyond, sv = soff | beyond, xv = xoff | beyond;
+#pragma unroll
+        for (int b = 0; b < RB; ++b) {
+            if (TILED) {
+                const uint32_t sk = kb * 512u + b * sblk;
+                const u32x2 ev = __builtin_amdgcn_raw_buffer_load_b64(sr[b], sv, sk, 0), od = __builtin_amdgcn_raw_buffer_load_b64(sr[b], sv + 256u, sk, 0);
+                q.s[b] = u32x4{ev.x, ev.y, od.x, od.y};
+            } else {
+                q.s[b] = __builtin_amdgcn_raw_buffer_load_b128(sr[b], sv, kb * 16u + b * sblk, 0);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)  // tile order: non-temporal (5 % faster at 4 tokens; in row order the same)
+                q.w[b][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[b], wv, kb * (TILED ? 4096u : 128u) + b * wblk + h * (TILED ? 2048u : 4u * K), TILED ? 2 : 0);
+        }
+#pragma unroll
+        for (int g = 0; g < 8; ++g) q.x[g] = __builtin_amdgcn_raw_buffer_load_b128(xr, xv + 64u * g, kb * 512u, 0);
+        l_kb += 4;
+        if (++l_i == l_n) {
+            l_item += stride;
+            if (l_item < total) open();
+        }
+    };
+
+    const uint32_t mask_r = vgpr_const(0x000F000Fu), magic_r = vgpr_const(kBf16Magic);
+    bf16x8 bias;
+    {
+        const u32x4 v = {0xC308C308u, 0xC308C308u, 0xC308C308u, 0xC308C308u};  // -136
+        __builtin_memcpy(&bias, &v, 16);
+    }
+    static_assert(kMagicBias == 136.f, "the constant above");
+    // ---- the summing side
+    int c_item = blockIdx.x, c_i = 0, c_n = 0, par = 0;
+    f32x4 acc[RB];
+#pragma unroll
+    for (int b = 0; b < RB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto finish = [&]() {
+#pragma unroll
+        for (int b = 0; b < RB; ++b) {
+            s_red[par][wave][b][lane] = acc[b];
+            acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        // the bare barrier instruction: __syncthreads() would also wait for every load in flight.  Two buffers: the next
+        // item's sums go to the other one, and nobody writes to this one again before the barrier of that item.
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int en = c_item / per, rem = c_item % per, nt = rem % ntn, split = rem / ntn;
+        const int m = tid >> 4, n = tid & 15, src = 16 * (m >> 2) + n;
+        float v[RB];
+#pragma unroll
+        for (int b = 0; b < RB; ++b) {
+            v[b] = 0.f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) v[b] += reinterpret_cast<const float *>(&s_red[par][w][b][src])[m & 3];
+        }
+        if (m < s_ent[en].rows) {
+            if (MODE == 1) {
+                uint16_t *const y = reinterpret_cast<uint16_t *>(s_ent[en].y) + (size_t)m * N + nt * 16 + n;
+                *y = (uint16_t)f32_to_bf16_bits(v[0] / (1.f + __expf(-v[0])) * v[1]);
+            } else {
+                float *const y = reinterpret_cast<float *>(s_ent[en].y) + split * split_stride + (size_t)m * N + nt * 32 + n;
+#pragma unroll
+                for (int b = 0; b < RB; ++b) y[16 * b] = v[b];
+            }
+        }
+        par ^= 1;
+    };
+    auto consume = [&](Block &q) {  // false after the workgroup's last item
+        if (!TILED) {  // the two loads trade halves: [h] then holds groups 4h .. 4h+3 of rows 0..15
+#pragma unroll
+            for (int b = 0; b < RB; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int lo = (int)q.w[b][0][e], hi = (int)q.w[b][1][e];
+                    q.w[b][0][e] = (uint32_t)__builtin_amdgcn_update_dpp(lo, hi, 0x128, 0xF, 0xC, false);  // row_ror 8 into lanes 8..15
+                    q.w[b][1][e] = (uint32_t)__builtin_amdgcn_update_dpp(hi, lo, 0x128, 0xF, 0x3, false);  // ... into lanes 0..7
+                }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            uint32_t word[RB][4];  // [row block][group]
+#pragma unroll
+            for (int b = 0; b < RB; ++b) {
+                const u32x4 w = q.w[b][h];
+                const u32x2 lo = __builtin_amdgcn_permlane16_swap(w.x, w.y, false, false);
+                const u32x2 hi = __builtin_amdgcn_permlane16_swap(w.z, w.w, false, false);
+                const u32x2 g02 = __builtin_amdgcn_permlane32_swap(lo.x, hi.x, false, false);
+                const u32x2 g13 = __builtin_amdgcn_permlane32_swap(lo.y, hi.y, false, false);
+                word[b][0] = g02.x;
+                word[b][1] = g13.x;
+                word[b][2] = g02.y;
+                word[b][3] = g13.y;
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const u32x4 xv = q.x[4 * h + t];
+                const uint32_t a[4] = {xv.x, xv.y, xv.z, xv.w};
+                uint32_t o[4];
+                pair_x8(a, o);
+                bf16x8 av;
+                __builtin_memcpy(&av, o, 16);
+                const f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bias, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < RB; ++b) {
+                    uint32_t p[4];
+                    unpack8_magic_r(word[b][t], mask_r, magic_r, p);
+                    bf16x8 bv;
+                    __builtin_memcpy(&bv, p, 16);
+                    const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, d0, 0, 0, 0);
+                    const uint32_t sw = q.s[b][TILED ? 2 * (t & 1) + h : 2 * h + (t >> 1)];  // group 4h + t
+                    acc[b] += d * f16_bits_to_f32((uint16_t)((TILED ? t >> 1 : t & 1) ? sw >> 16 : sw & 0xFFFFu));
+                }
+            }
+        }
+        if (++c_i == c_n) {
+            finish();
+            c_i = 0;
+            c_item += stride;
+            if (c_item >= total) return false;
+            c_n = blocks_of(c_item);
+        }
+        return true;
+    };
+    if (l_item >= total) return;
+    open();
+    c_n = l_n;
+    Block q0, q1;
+    request(q0);
+    for (;;) {
+        request(q1);
+        if (!consume(q0)) break;
+        request(q0);
+        if (!consume(q1)) break;
+    }
+}
+
+// T <= 16: no expert gets more than one tile of rows.  32-bit byte offsets into a matrix.  Row order: always (figures
+// above).  In tile order the many-row kernel streams large experts better (16 tokens, 8 experts of 4096 x 14336: 164 us
+// for the whole call against 195; 16 experts of 2048 x 4096, top 4: 67 against 77) but has a launch more and coarser
+// tiles, which is what a few small experts take (one token, top 2 of 1024 x 2048: 31 against 18): few bytes only.
+bool moe_few_ok(int T, int H, int F, int E, int top_k, bool tiled) {
+    if (T > FEW_ROWS || E > FEW_ENTRIES || H % 256 != 0 || F % 256 != 0 || (int64_t)H * F / 2 >= (int64_t)kRange) return false;
+    const int64_t hit = T * top_k < E ? T * top_k : E;
+    return !tiled || hit * H * F * 27 / 16 <= (int64_t)64 << 20;  // three matrices of 9/16 byte per weight
+}
+
+int moe_few_tile_rows() { return FEW_ROWS; }
+
+// K splits of the down product: items of at least four blocks of 256 k
+int moe_few_down_splits(int F) { return F >= 4096 ? 4 : F >= 2048 ? 2 : 1; }
+
+template <int MODE, bool TILED>
+static int few_launch(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int E, int N, int K, int nsplit,
+                      size_t split_stride, hipStream_t st) {
+    const int64_t most = (int64_t)ntiles * (MODE == 1 ? N / 16 : N / 32 * nsplit);
+    hipLaunchKernelGGL((moe_few_i4g32_kernel<MODE, TILED>), dim3(most < 768 ? (int)most : 768), dim3(256), 0, st, groups, tiles, tok, ntiles,
+                       E, N, K, nsplit, split_stride);
+    return hip_check(hipGetLastError(), "moe_few launch");
+}
+
+// gate/up with the SiLU gate: h bf16 [P,F] through the down descriptors' x pointers
+int moe_few_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int E, int F, int H, bool tiled,
+                   hipStream_t st) {
+    return tiled ? few_launch<1, true>(groups, tiles, tok, ntiles, E, F, H, 1, 0, st) : few_launch<1, false>(groups, tiles, tok, ntiles, E, F, H, 1, 0, st);
+}
+
+// down: fp32 parts [nsplit][P,H]
+int moe_few_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int E, int H, int F, int nsplit, size_t split_stride, bool tiled,
+                 hipStream_t st) {
+    return tiled ? few_launch<0, true>(groups, tiles, nullptr, ntiles, E, H, F, nsplit, split_stride, st)
+                 : few_launch<0, false>(groups, tiles, nullptr, ntiles, E, H, F, nsplit, split_stride, st);
+}
+
+}  // namespace chadq

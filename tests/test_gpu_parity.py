@@ -737,6 +737,28 @@ def test_moe_ffn_tiled_agrees_with_row_major_and_oracle(ops, t, h, f, e, top_k):
     assert np.array_equal(yp, yt[perm])
 
 
+@pytest.mark.parametrize("t,h,f,e,top_k", [(1, 256, 256, 1, 1), (4, 1024, 2048, 8, 2), (16, 768, 4352, 16, 4), (16, 2304, 1280, 4, 1), (17, 512, 2048, 4, 2), (8, 2048, 4096, 8, 2)])
+def test_moe_ffn_few_tokens(ops, t, h, f, e, top_k):
+    """Up to 16 tokens stream the weights exactly (17: the many-row kernels), both orders with the same sums: one and
+    several blocks of 256 k per wave, block counts that four waves and the K splits do not divide, an expert with all
+    tokens beside empty ones."""
+    host, dev = _experts(9400 + t + h, e, h, f)
+    r = rng(9401 + t + h)
+    xb = O.f32_to_bf16(r.standard_normal((t, h)).astype(np.float32))
+    logits = r.standard_normal((t, e)).astype(np.float32)
+    logits[:, e - 1] += 20.0  # every token takes the last expert
+    x, z = bf16_tensor(xb), torch.from_numpy(logits).to(DEV)
+    tiled = [tuple(ops.to_tiles(m) for m in tr) for tr in dev]
+    ref = O.bf16_to_f32(O.moe_qffn(xb, logits, host, top_k, True))
+    y, yt = (bits(ops.moe_ffn(x, z, ex, top_k=top_k, renorm=True)) for ex in (dev, tiled))
+    small = min(e, t * top_k) * h * f * 27 // 16 <= 64 << 20  # what the tile order sends to the same kernel
+    if t <= 16 and small:
+        # bf16 roundings of h (some flip one ulp against the oracle's float64) and of the result, weights exact
+        assert np.array_equal(y, yt) and O.rel_l2(O.bf16_to_f32(y), ref) <= 2.0 ** -8
+    for v in (y, yt):
+        assert O.rel_l2(O.bf16_to_f32(v), ref) <= TOL_BF16
+
+
 def test_moe_ffn_tiled_wide_ranges_of_activations_and_scales(ops):
     """The tile-order kernels carry activations and dequantised weights as fp16: rows are scaled by a power of two first,
     so activations far outside fp16's range (and rows of very different magnitude side by side) must come out as the

@@ -53,9 +53,9 @@ int unpack_i4_launch(const uint8_t *, int8_t *, int64_t, hipStream_t);
 int pack_i4_launch(const int8_t *, uint8_t *, int64_t, hipStream_t);
 int dequant_i4g32_launch(const uint8_t *, const uint16_t *, float *, int, int, hipStream_t);
 int dequant_i8row_launch(const int8_t *, const float *, float *, int, int, hipStream_t);
-int gemv_i4g32_dispatch(const uint16_t *, const uint8_t *, const uint16_t *, float *, int, int, int, hipStream_t);
-int gemv_i4g32_mfma_dispatch(const uint16_t *, const uint8_t *, const uint16_t *, float *, int, int, int, hipStream_t);
-int gemv_i8row_dispatch(const float *, const int8_t *, const float *, float *, int, int, int, bool, hipStream_t);
+// bf16_out: y is bf16, the sums rounded once
+int gemv_i4g32_mfma_dispatch(const uint16_t *, const uint8_t *, const uint16_t *, float *, int, int, int, bool bf16_out, hipStream_t);
+int gemv_i8row_dispatch(const float *, const int8_t *, const float *, float *, int, int, int, bool fp32_only, bool bf16_out, hipStream_t);
 int gemm_i4g32_bf16_dispatch(const uint16_t *, const uint8_t *, const uint16_t *, uint16_t *, int, int, int,
                              hipStream_t);
 int gemm_i8row_bf16_dispatch(const uint16_t *, const int8_t *, const float *, uint16_t *, int, int, int,
@@ -154,15 +154,26 @@ int chadq_dequant_i8row(const int8_t *w8, const float *scale, float *w, int N, i
     return dequant_i8row_launch(w8, scale, w, N, K, st);
 }
 
+static int gemv_i4g32_entry(const char *name, const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, float *y, int M, int N,
+                            int K, bool bf16_out, hipStream_t st) {
+    CHADQ_REQUIRE(M >= 1 && M <= 16, CHADQ_ERR_SHAPE, "%s: M=%d outside [1,16] (use chadq_gemm_i4g32_bf16)", name, M);
+    CHADQ_REQUIRE(N >= 0 && K >= 32 && K % 32 == 0, CHADQ_ERR_SHAPE, "%s: N=%d K=%d (K must be a positive multiple of 32)", name, N, K);
+    if (N == 0) return 0;
+    CHADQ_REQUIRE(x_bf16 && wp && scale_f16 && y, CHADQ_ERR_NULL, "%s: null pointer", name);
+    CHADQ_REQUIRE(aligned16(x_bf16) && aligned16(wp), CHADQ_ERR_ALIGN, "%s: x and wp must be 16-byte aligned", name);
+    return gemv_i4g32_mfma_dispatch(x_bf16, wp, scale_f16, y, M, N, K, bf16_out, st);
+}
+
 int chadq_gemv_i4g32(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, float *y, int M, int N,
                      int K, void *stream) {
     ENTER();
-    CHADQ_REQUIRE(M >= 1 && M <= 16, CHADQ_ERR_SHAPE, "chadq_gemv_i4g32: M=%d outside [1,16] (use chadq_gemm_i4g32_bf16)", M);
-    CHADQ_REQUIRE(N >= 0 && K >= 32 && K % 32 == 0, CHADQ_ERR_SHAPE, "chadq_gemv_i4g32: N=%d K=%d (K must be a positive multiple of 32)", N, K);
-    if (N == 0) return 0;
-    CHADQ_REQUIRE(x_bf16 && wp && scale_f16 && y, CHADQ_ERR_NULL, "chadq_gemv_i4g32: null pointer");
-    CHADQ_REQUIRE(aligned16(x_bf16) && aligned16(wp), CHADQ_ERR_ALIGN, "chadq_gemv_i4g32: x and wp must be 16-byte aligned");
-    return gemv_i4g32_mfma_dispatch(x_bf16, wp, scale_f16, y, M, N, K, st);
+    return gemv_i4g32_entry("chadq_gemv_i4g32", x_bf16, wp, scale_f16, y, M, N, K, false, st);
+}
+
+int chadq_gemv_i4g32_bf16(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, uint16_t *y_bf16, int M, int N,
+                          int K, void *stream) {
+    ENTER();
+    return gemv_i4g32_entry("chadq_gemv_i4g32_bf16", x_bf16, wp, scale_f16, reinterpret_cast<float *>(y_bf16), M, N, K, true, st);
 }
 
 int chadq_gemv_i4g32_splitk(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, float *y_parts, int N,
@@ -226,25 +237,31 @@ int chadq_gemv_i4g32_addnorm_geglu(const float *res, const float *delta, int n_d
 }
 
 static int gemv_i8row_entry(const char *name, bool fp32_only, const float *x, const int8_t *w8, const float *scale, float *y, int M,
-                           int N, int K, hipStream_t st) {
+                           int N, int K, bool bf16_out, hipStream_t st) {
     CHADQ_REQUIRE(M >= 1 && M <= 16, CHADQ_ERR_SHAPE, "%s: M=%d outside [1,16]", name, M);
     CHADQ_REQUIRE(N >= 0 && K >= 16 && K % 16 == 0, CHADQ_ERR_SHAPE, "%s: N=%d K=%d (K must be a positive multiple of 16)", name, N, K);
     if (N == 0) return 0;
     CHADQ_REQUIRE(x && w8 && scale && y, CHADQ_ERR_NULL, "%s: null pointer", name);
     CHADQ_REQUIRE(aligned16(x) && aligned16(w8), CHADQ_ERR_ALIGN, "%s: x and w8 must be 16-byte aligned", name);
-    return gemv_i8row_dispatch(x, w8, scale, y, M, N, K, fp32_only, st);
+    return gemv_i8row_dispatch(x, w8, scale, y, M, N, K, fp32_only, bf16_out, st);
 }
 
 int chadq_gemv_i8row(const float *x, const int8_t *w8, const float *scale, float *y, int M, int N, int K,
                      void *stream) {
     ENTER();
-    return gemv_i8row_entry("chadq_gemv_i8row", false, x, w8, scale, y, M, N, K, st);
+    return gemv_i8row_entry("chadq_gemv_i8row", false, x, w8, scale, y, M, N, K, false, st);
+}
+
+int chadq_gemv_i8row_bf16(const float *x, const int8_t *w8, const float *scale, uint16_t *y_bf16, int M, int N, int K,
+                          void *stream) {
+    ENTER();
+    return gemv_i8row_entry("chadq_gemv_i8row_bf16", false, x, w8, scale, reinterpret_cast<float *>(y_bf16), M, N, K, true, st);
 }
 
 int chadq_gemv_i8row_fp32(const float *x, const int8_t *w8, const float *scale, float *y, int M, int N, int K,
                           void *stream) {
     ENTER();
-    return gemv_i8row_entry("chadq_gemv_i8row_fp32", true, x, w8, scale, y, M, N, K, st);
+    return gemv_i8row_entry("chadq_gemv_i8row_fp32", true, x, w8, scale, y, M, N, K, false, st);
 }
 
 int chadq_gemm_i4g32_bf16(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, uint16_t *y_bf16,
@@ -498,7 +515,7 @@ int chadq_gemv_i4g32_argmax(const uint16_t *x_bf16, const uint8_t *wp, const uin
         if (rc != 0) return rc;
         return argmax_embed_launch(y, false, pv, pi, n_cand, N, token, pos, advance, wp, scale_f16, next_x, K, st);
     }
-    const int rc = gemv_i4g32_mfma_dispatch(x_bf16, wp, scale_f16, y, 1, N, K, st);
+    const int rc = gemv_i4g32_mfma_dispatch(x_bf16, wp, scale_f16, y, 1, N, K, false, st);
     if (rc != 0) return rc;
     return argmax_embed_launch(y, true, pv, pi, 256, N, token, pos, advance, wp, scale_f16, next_x, K, st);
 }

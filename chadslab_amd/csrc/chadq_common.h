@@ -67,6 +67,16 @@ __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
     return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
 }
 
+// element i of a result matrix that is fp32, or (bf16_out) the same sums rounded once to bf16
+__device__ __forceinline__ void store_sum(float *y, size_t i, float v, bool bf16_out) {
+    if (bf16_out) reinterpret_cast<uint16_t *>(y)[i] = (uint16_t)f32_to_bf16_bits(v);
+    else y[i] = v;
+}
+// the same matrix from element `off` on (host)
+inline float *sum_at(float *y, size_t off, bool bf16_out) {
+    return bf16_out ? reinterpret_cast<float *>(reinterpret_cast<uint16_t *>(y) + off) : y + off;
+}
+
 __device__ __forceinline__ bf16x2 as_bf16x2(uint32_t v) {
     bf16x2 r;
     __builtin_memcpy(&r, &v, 4);

@@ -20,7 +20,7 @@ template <int CH, int R, int MB>
 __global__ __launch_bounds__(256) void gemv_i4g32_rows_kernel(const uint16_t *__restrict__ x,
                                                               const uint8_t *__restrict__ wp,
                                                               const uint16_t *__restrict__ sc,
-                                                              float *__restrict__ y, int N, int K) {
+                                                              float *__restrict__ y, int N, int K, int bf16_out) {
     const int lane = threadIdx.x & 63;
     const int gw = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int row0 = gw * R;
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void gemv_i4g32_rows_kernel(const uint16_t *__
 #pragma unroll
         for (int m = 0; m < MB; ++m) {
             const float t = wave_sum_to_lane63(acc[m]);
-            if (lane == 63 && row0 + r < N) y[(size_t)m * N + row0 + r] = t;
+            if (lane == 63 && row0 + r < N) store_sum(y, (size_t)m * N + row0 + r, t, bf16_out);
         }
     }
 }
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) void gemv_i4g32_rows_kernel(const uint16_t *__
 __global__ __launch_bounds__(256) void gemv_i4g32_generic_kernel(const uint16_t *__restrict__ x,
                                                                  const uint8_t *__restrict__ wp,
                                                                  const uint16_t *__restrict__ sc,
-                                                                 float *__restrict__ y, int M, int N, int K) {
+                                                                 float *__restrict__ y, int M, int N, int K, int bf16_out) {
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= N) return;
@@ -144,38 +144,39 @@ __global__ __launch_bounds__(256) void gemv_i4g32_generic_kernel(const uint16_t 
             acc = __builtin_fmaf(s, g - kMagicBias * sum, acc);
         }
         const float t = wave_sum_to_lane63(acc);
-        if (lane == 63) y[(size_t)m * N + row] = t;
+        if (lane == 63) store_sum(y, (size_t)m * N + row, t, bf16_out);
     }
 }
 
 template <int CH, int R, int MB>
-static void launch_rows(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int N, int K,
+static void launch_rows(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int N, int K, bool bf16_out,
                         hipStream_t st) {
     const int waves = (N + R - 1) / R;
-    hipLaunchKernelGGL((gemv_i4g32_rows_kernel<CH, R, MB>), dim3((waves + 3) / 4), dim3(256), 0, st, x, wp, sc, y, N, K);
+    hipLaunchKernelGGL((gemv_i4g32_rows_kernel<CH, R, MB>), dim3((waves + 3) / 4), dim3(256), 0, st, x, wp, sc, y, N, K,
+                       (int)bf16_out);
 }
 
 int gemv_i4g32_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K,
-                        hipStream_t st) {
+                        bool bf16_out, hipStream_t st) {
     if (K <= 4096) {
         // rows per wave: enough waves to fill 256 CUs several times over, few enough to keep loads deep
         const bool big = N >= 8192;
         int m0 = 0;
         while (m0 < M) {
             const uint16_t *xm = x + (size_t)m0 * K;
-            float *ym = y + (size_t)m0 * N;
+            float *ym = sum_at(y, (size_t)m0 * N, bf16_out);
             const int mb = (M - m0 >= 2) ? 2 : 1;
             if (K <= 2048) {
-                if (mb == 2) big ? launch_rows<1, 8, 2>(xm, wp, sc, ym, N, K, st) : launch_rows<1, 2, 2>(xm, wp, sc, ym, N, K, st);
-                else big ? launch_rows<1, 8, 1>(xm, wp, sc, ym, N, K, st) : launch_rows<1, 2, 1>(xm, wp, sc, ym, N, K, st);
+                if (mb == 2) big ? launch_rows<1, 8, 2>(xm, wp, sc, ym, N, K, bf16_out, st) : launch_rows<1, 2, 2>(xm, wp, sc, ym, N, K, bf16_out, st);
+                else big ? launch_rows<1, 8, 1>(xm, wp, sc, ym, N, K, bf16_out, st) : launch_rows<1, 2, 1>(xm, wp, sc, ym, N, K, bf16_out, st);
             } else {
-                if (mb == 2) big ? launch_rows<2, 4, 2>(xm, wp, sc, ym, N, K, st) : launch_rows<2, 1, 2>(xm, wp, sc, ym, N, K, st);
-                else big ? launch_rows<2, 4, 1>(xm, wp, sc, ym, N, K, st) : launch_rows<2, 1, 1>(xm, wp, sc, ym, N, K, st);
+                if (mb == 2) big ? launch_rows<2, 4, 2>(xm, wp, sc, ym, N, K, bf16_out, st) : launch_rows<2, 1, 2>(xm, wp, sc, ym, N, K, bf16_out, st);
+                else big ? launch_rows<2, 4, 1>(xm, wp, sc, ym, N, K, bf16_out, st) : launch_rows<2, 1, 1>(xm, wp, sc, ym, N, K, bf16_out, st);
             }
             m0 += mb;
         }
     } else {
-        hipLaunchKernelGGL(gemv_i4g32_generic_kernel, dim3((N + 3) / 4), dim3(256), 0, st, x, wp, sc, y, M, N, K);
+        hipLaunchKernelGGL(gemv_i4g32_generic_kernel, dim3((N + 3) / 4), dim3(256), 0, st, x, wp, sc, y, M, N, K, (int)bf16_out);
     }
     return hip_check(hipGetLastError(), "gemv_i4g32 launch");
 }

@@ -39,6 +39,7 @@
 namespace chadq {
 
 constexpr int ZERO_BYTES = 1024;
+constexpr int kPvBf16Out = 1 << 16;  // beside the tile rows in a kernel argument: y is bf16, not fp32
 
 // KC = k per chunk (4096, or 2048 for short rows)
 template <int MT, int HP, int S, int RBW, int KC>
@@ -98,6 +99,7 @@ __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(4))) 
     const float *__restrict__ a2, int N, int K, int pvn, int kspan, float *__restrict__ y, float *__restrict__ res_out, float eps) {
     const uint16_t *__restrict__ x = reinterpret_cast<const uint16_t *>(a0);
     const int pv = pvn & 0xFF;
+    const bool bf16_out = XM == 0 && YM == 0 && (pvn & kPvBf16Out);  // y bf16 (no pre.n in this mode)
     const GemvPre pre{reinterpret_cast<const float *>(a0), a1, a2, res_out, pvn >> 8, eps};
     constexpr bool XG = (XM == 1), XN = (XM == 2);
     typedef GemvCfg<MT, HP, S, RBW, KC> C;
@@ -399,7 +401,7 @@ __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(4))) 
                 reinterpret_cast<int32_t *>(const_cast<float *>(a2))[blockIdx.x] = bb;
             }
         } else {
-            if (lane < P && lane < pv && nn < N) y[nn] = t;
+            if (lane < P && lane < pv && nn < N) store_sum(y, nn, t, bf16_out);
         }
         return;
     }
@@ -437,7 +439,7 @@ __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(4))) 
             if (!(rr & 1) && rr + 1 < pv && nn + 1 < N && mm < M)  // mm: the padding rows of a two-row pass write nothing
                 reinterpret_cast<uint16_t *>(y)[nn >> 1] = (uint16_t)f32_to_bf16_bits(gelu_tanh_dev(t) * up);
         } else {
-            if (rr < pv && nn < N && mm < M) y[(size_t)mm * N + nn] = t;
+            if (rr < pv && nn < N && mm < M) store_sum(y, (size_t)mm * N + nn, t, bf16_out);
         }
     }
 }
@@ -487,7 +489,9 @@ struct GemvPairCfg {
 template <int MT, int S, int RBW, int D, int KC>
 __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(S == 16 ? 2 : 4))) void gemv_i4g32_mfma_pair_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wp, const uint16_t *__restrict__ sc,
-    float *__restrict__ y, int N, int K, int pv) {
+    float *__restrict__ y, int N, int K, int pvf) {
+    const int pv = pvf & 0xFF;
+    const bool bf16_out = pvf & kPvBf16Out;
     typedef GemvPairCfg<S, RBW, KC> C;
     constexpr int M = MT, P = C::P, MR = C::MR, KS = C::KS, T = C::T, XI = C::XI;
     static_assert(M >= 1 && M <= MR, "eight rows of A per scale group");
@@ -655,7 +659,7 @@ __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(S == 
                 t += reinterpret_cast<const float *>(red)[(wsrc * 64 + lsrc) * 4 + (m & 3)];
             }
         const int nn = ((blockIdx.x * RBW + un) * (4 / KS) + rb) * pv + rr;
-        if (rr < pv && nn < N && m < M) y[(size_t)m * N + nn] = t;
+        if (rr < pv && nn < N && m < M) store_sum(y, (size_t)m * N + nn, t, bf16_out);
     }
 }
 
@@ -694,7 +698,9 @@ template <int S, int RBW, int D, int KC>
 // (two waves per SIMD at most: a workgroup's operands take 68 KB or more of LDS, so a wave may use 256 registers)
 __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(2))) void gemv_i4g32_mfma_rows16_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wp, const uint16_t *__restrict__ sc,
-    float *__restrict__ y, int M, int N, int K, int pv) {
+    float *__restrict__ y, int M, int N, int K, int pvf) {
+    const int pv = pvf & 0xFF;
+    const bool bf16_out = pvf & kPvBf16Out;
     typedef GemvRows16Cfg<S, RBW, KC> C;
     constexpr int P = C::P, KS = C::KS, T = C::T, XI = C::XI;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -842,11 +848,11 @@ __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(2))) 
             t += reinterpret_cast<const float *>(red)[(wsrc * 64 + lsrc) * 4 + (m & 3)];
         }
         const int nn = ((blockIdx.x * RBW + un) * (4 / KS) + rb) * pv + rr;
-        if (rr < pv && nn < N && m < M) y[(size_t)m * N + nn] = t;
+        if (rr < pv && nn < N && m < M) store_sum(y, (size_t)m * N + nn, t, bf16_out);
     }
 }
 
-int gemv_i4g32_dispatch(const uint16_t *, const uint8_t *, const uint16_t *, float *, int, int, int, hipStream_t);
+int gemv_i4g32_dispatch(const uint16_t *, const uint8_t *, const uint16_t *, float *, int, int, int, bool, hipStream_t);
 
 // Rows of a P-row tile to use.  All workgroups of these grids are resident at once, so the launch lasts as long as
 // the compute unit with the most workgroups: ceil(workgroups / CUs) of them.  Using a few rows less per tile can turn
@@ -880,7 +886,7 @@ static int pick_tile_rows(int N, int P, int tiles_per_wg, int ksplit) {
 
 template <int MT, int HP, int S, int RBW, int D, int KC = 4096, int XM = 0, int YM = 0, int D0 = D>
 static int launch_mfma(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int N, int K,
-                       hipStream_t st, int ksplit = 1, GemvPre pre = GemvPre{}, int *workgroups = nullptr) {
+                       hipStream_t st, int ksplit = 1, GemvPre pre = GemvPre{}, int *workgroups = nullptr, bool bf16_out = false) {
     typedef GemvCfg<MT, HP, S, RBW, KC> C;
     static std::atomic<bool> attr_set{false};  // setting it twice from two threads is harmless
     if (!attr_set.load(std::memory_order_acquire)) {
@@ -896,13 +902,13 @@ static int launch_mfma(const uint16_t *x, const uint8_t *wp, const uint16_t *sc,
     if (workgroups) *workgroups = (tiles + tiles_per_wg - 1) / tiles_per_wg;
     if (workgroups && !wp) return 0;  // asked for the grid only
     hipLaunchKernelGGL((gemv_i4g32_mfma_kernel<MT, HP, S, RBW, D, KC, XM, YM, D0>), dim3((tiles + tiles_per_wg - 1) / tiles_per_wg, ksplit),
-                       dim3(256 * RBW), C::TOTAL, st, wp, sc, a0, pre.delta, pre.w, N, K, pv | (pre.n << 8), K / ksplit, y, pre.res_out,
+                       dim3(256 * RBW), C::TOTAL, st, wp, sc, a0, pre.delta, pre.w, N, K, pv | (pre.n << 8) | (bf16_out ? kPvBf16Out : 0), K / ksplit, y, pre.res_out,
                        pre.eps);
     return hip_check(hipGetLastError(), "gemv_i4g32_mfma launch");
 }
 
 template <int MT, int S, int RBW, int D, int KC = 4096>
-static int launch_pair(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int N, int K, hipStream_t st) {
+static int launch_pair(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int N, int K, hipStream_t st, bool bf16_out) {
     typedef GemvPairCfg<S, RBW, KC> C;
     static std::atomic<bool> attr_set{false};
     if (!attr_set.load(std::memory_order_acquire)) {
@@ -914,12 +920,13 @@ static int launch_pair(const uint16_t *x, const uint8_t *wp, const uint16_t *sc,
     const int pv = pick_tile_rows(N, C::P, tiles_per_wg, 1);
     const int tiles = (N + pv - 1) / pv;
     hipLaunchKernelGGL((gemv_i4g32_mfma_pair_kernel<MT, S, RBW, D, KC>), dim3((tiles + tiles_per_wg - 1) / tiles_per_wg), dim3(256 * RBW),
-                       C::TOTAL, st, x, wp, sc, y, N, K, pv);
+                       C::TOTAL, st, x, wp, sc, y, N, K, pv | (bf16_out ? kPvBf16Out : 0));
     return hip_check(hipGetLastError(), "gemv_i4g32_mfma_pair launch");
 }
 
 template <int S, int RBW, int D, int KC = 2048>
-static int launch_rows16(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, hipStream_t st) {
+static int launch_rows16(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, hipStream_t st,
+                         bool bf16_out) {
     typedef GemvRows16Cfg<S, RBW, KC> C;
     static std::atomic<bool> attr_set{false};
     if (!attr_set.load(std::memory_order_acquire)) {
@@ -931,23 +938,23 @@ static int launch_rows16(const uint16_t *x, const uint8_t *wp, const uint16_t *s
     const int pv = pick_tile_rows(N, C::P, tiles_per_wg, 1);
     const int tiles = (N + pv - 1) / pv;
     hipLaunchKernelGGL((gemv_i4g32_mfma_rows16_kernel<S, RBW, D, KC>), dim3((tiles + tiles_per_wg - 1) / tiles_per_wg), dim3(256 * RBW),
-                       C::TOTAL, st, x, wp, sc, y, M, N, K, pv);
+                       C::TOTAL, st, x, wp, sc, y, M, N, K, pv | (bf16_out ? kPvBf16Out : 0));
     return hip_check(hipGetLastError(), "gemv_i4g32_mfma_rows16 launch");
 }
 
 int gemv_i4g32_mfma_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K,
-                             hipStream_t st) {
+                             bool bf16_out, hipStream_t st) {
     // the matrix-core kernel wants 16-byte aligned scale rows (K % 256 == 0) and 32-bit byte offsets
     if ((K & 255) != 0 || (int64_t)N * (K / 2) >= ((int64_t)1 << 31) || (reinterpret_cast<uintptr_t>(sc) & 15u) != 0)
-        return gemv_i4g32_dispatch(x, wp, sc, y, M, N, K, st);
+        return gemv_i4g32_dispatch(x, wp, sc, y, M, N, K, bf16_out, st);
     // 9 to 16 activation rows: the 16-row form reads the weights once
     if (M > 8 && M <= 16)
-        return N >= 8192 ? launch_rows16<8, 2, 4>(x, wp, sc, y, M, N, K, st) : launch_rows16<4, 1, 4>(x, wp, sc, y, M, N, K, st);
+        return N >= 8192 ? launch_rows16<8, 2, 4>(x, wp, sc, y, M, N, K, st, bf16_out) : launch_rows16<4, 1, 4>(x, wp, sc, y, M, N, K, st, bf16_out);
     // up to 8 activation rows per launch (more than 16 rows: the kernels run on 8 rows at a time)
     for (int m0 = 0; m0 < M; m0 += 8) {
         const int mm = (M - m0) < 8 ? (M - m0) : 8;
         const uint16_t *xm = x + (size_t)m0 * K;
-        float *ym = y + (size_t)m0 * N;
+        float *ym = sum_at(y, (size_t)m0 * N, bf16_out);
         int rc = 0;
         // <rows, K-parts, steps per wave, 4-wave groups per workgroup, prefetch distance>, picked by measurement
         // Matrices with many rows run with 32 (M <= 4) or 64-row workgroups whose waves walk 16 steps of a chunk:
@@ -957,31 +964,31 @@ int gemv_i4g32_mfma_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_
         switch (mm) {
             case 1:
                 if (K <= 2048)  // rows of at most 2048 k: 2048-wide chunks (no loads past the row)
-                    rc = tall ? launch_mfma<1, 2, 8, 1, 4, 2048>(xm, wp, sc, ym, N, K, st)
-                              : launch_mfma<1, 4, 4, 1, 4, 2048>(xm, wp, sc, ym, N, K, st);
+                    rc = tall ? launch_mfma<1, 2, 8, 1, 4, 2048>(xm, wp, sc, ym, N, K, st, 1, GemvPre{}, nullptr, bf16_out)
+                              : launch_mfma<1, 4, 4, 1, 4, 2048>(xm, wp, sc, ym, N, K, st, 1, GemvPre{}, nullptr, bf16_out);
                 else
-                    rc = tall ? launch_mfma<1, 2, 16, 1, 4>(xm, wp, sc, ym, N, K, st) : launch_mfma<1, 4, 8, 1, 3>(xm, wp, sc, ym, N, K, st);
+                    rc = tall ? launch_mfma<1, 2, 16, 1, 4>(xm, wp, sc, ym, N, K, st, 1, GemvPre{}, nullptr, bf16_out) : launch_mfma<1, 4, 8, 1, 3>(xm, wp, sc, ym, N, K, st, 1, GemvPre{}, nullptr, bf16_out);
                 break;
             case 2:
-                rc = tall ? launch_mfma<2, 2, 16, 1, 3>(xm, wp, sc, ym, N, K, st) : launch_mfma<2, 2, 8, 1, 2>(xm, wp, sc, ym, N, K, st);
+                rc = tall ? launch_mfma<2, 2, 16, 1, 3>(xm, wp, sc, ym, N, K, st, 1, GemvPre{}, nullptr, bf16_out) : launch_mfma<2, 2, 8, 1, 2>(xm, wp, sc, ym, N, K, st, 1, GemvPre{}, nullptr, bf16_out);
                 break;
             case 3:
-                rc = tall ? launch_mfma<3, 1, 16, 1, 4>(xm, wp, sc, ym, N, K, st) : launch_mfma<3, 1, 8, 1, 8>(xm, wp, sc, ym, N, K, st);
+                rc = tall ? launch_mfma<3, 1, 16, 1, 4>(xm, wp, sc, ym, N, K, st, 1, GemvPre{}, nullptr, bf16_out) : launch_mfma<3, 1, 8, 1, 8>(xm, wp, sc, ym, N, K, st, 1, GemvPre{}, nullptr, bf16_out);
                 break;
             case 4:
-                rc = tall ? launch_mfma<4, 1, 16, 1, 4>(xm, wp, sc, ym, N, K, st) : launch_mfma<4, 1, 8, 1, 8>(xm, wp, sc, ym, N, K, st);
+                rc = tall ? launch_mfma<4, 1, 16, 1, 4>(xm, wp, sc, ym, N, K, st, 1, GemvPre{}, nullptr, bf16_out) : launch_mfma<4, 1, 8, 1, 8>(xm, wp, sc, ym, N, K, st, 1, GemvPre{}, nullptr, bf16_out);
                 break;
             case 5:
-                rc = tall ? launch_pair<5, 16, 2, 4>(xm, wp, sc, ym, N, K, st) : launch_pair<5, 8, 2, 3>(xm, wp, sc, ym, N, K, st);
+                rc = tall ? launch_pair<5, 16, 2, 4>(xm, wp, sc, ym, N, K, st, bf16_out) : launch_pair<5, 8, 2, 3>(xm, wp, sc, ym, N, K, st, bf16_out);
                 break;
             case 6:
-                rc = tall ? launch_pair<6, 16, 2, 4>(xm, wp, sc, ym, N, K, st) : launch_pair<6, 8, 2, 3>(xm, wp, sc, ym, N, K, st);
+                rc = tall ? launch_pair<6, 16, 2, 4>(xm, wp, sc, ym, N, K, st, bf16_out) : launch_pair<6, 8, 2, 3>(xm, wp, sc, ym, N, K, st, bf16_out);
                 break;
             case 7:
-                rc = tall ? launch_pair<7, 16, 2, 4>(xm, wp, sc, ym, N, K, st) : launch_pair<7, 8, 2, 3>(xm, wp, sc, ym, N, K, st);
+                rc = tall ? launch_pair<7, 16, 2, 4>(xm, wp, sc, ym, N, K, st, bf16_out) : launch_pair<7, 8, 2, 3>(xm, wp, sc, ym, N, K, st, bf16_out);
                 break;
             default:
-                rc = tall ? launch_pair<8, 16, 2, 4>(xm, wp, sc, ym, N, K, st) : launch_pair<8, 8, 2, 3>(xm, wp, sc, ym, N, K, st);
+                rc = tall ? launch_pair<8, 16, 2, 4>(xm, wp, sc, ym, N, K, st, bf16_out) : launch_pair<8, 8, 2, 3>(xm, wp, sc, ym, N, K, st, bf16_out);
                 break;
         }
         if (rc != 0) return rc;

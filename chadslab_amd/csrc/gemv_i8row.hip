@@ -16,7 +16,7 @@ template <int CH, int R, int MB, int WPB>
 __global__ __launch_bounds__(64 * WPB) void gemv_i8row_rows_kernel(const float *__restrict__ x,
                                                               const int8_t *__restrict__ w8,
                                                               const float *__restrict__ sc, float *__restrict__ y,
-                                                              int N, int K) {
+                                                              int N, int K, int bf16_out) {
     const int lane = threadIdx.x & 63;
     const int gw = blockIdx.x * WPB + (threadIdx.x >> 6);
     const int row0 = gw * R;  // waves past the last row run on clamped rows and store nothing (no return before the barrier)
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(64 * WPB) void gemv_i8row_rows_kernel(const float *
 #pragma unroll
         for (int m = 0; m < MB; ++m) {
             const float t = wave_sum_to_lane63(acc[m]);
-            if (lane == 63 && row < N) y[(size_t)m * N + row] = t * s;
+            if (lane == 63 && row < N) store_sum(y, (size_t)m * N + row, t * s, bf16_out);
         }
     }
 }
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(64 * WPB) void gemv_i8row_rows_kernel(const float *
 __global__ __launch_bounds__(256) void gemv_i8row_generic_kernel(const float *__restrict__ x,
                                                                  const int8_t *__restrict__ w8,
                                                                  const float *__restrict__ sc,
-                                                                 float *__restrict__ y, int M, int N, int K) {
+                                                                 float *__restrict__ y, int M, int N, int K, int bf16_out) {
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= N) return;
@@ -128,52 +128,52 @@ __global__ __launch_bounds__(256) void gemv_i8row_generic_kernel(const float *__
             }
         }
         const float t = wave_sum_to_lane63(acc);
-        if (lane == 63) y[(size_t)m * N + row] = t * s;
+        if (lane == 63) store_sum(y, (size_t)m * N + row, t * s, bf16_out);
     }
 }
 
 template <int CH, int R, int MB, int WPB>
-static void launch_rows8(const float *x, const int8_t *w8, const float *sc, float *y, int N, int K, hipStream_t st) {
+static void launch_rows8(const float *x, const int8_t *w8, const float *sc, float *y, int N, int K, bool bf16_out, hipStream_t st) {
     const int waves = (N + R - 1) / R;
     hipLaunchKernelGGL((gemv_i8row_rows_kernel<CH, R, MB, WPB>), dim3((waves + WPB - 1) / WPB), dim3(64 * WPB), 0, st, x, w8, sc, y,
-                       N, K);
+                       N, K, (int)bf16_out);
 }
 
 bool gemv_i8row_mfma_ok(int M, int K);
-int gemv_i8row_mfma_launch(const float *, const int8_t *, const float *, float *, int, int, int, hipStream_t);
+int gemv_i8row_mfma_launch(const float *, const int8_t *, const float *, float *, int, int, int, bool, hipStream_t);
 
 // fp32_only: the fp32 kernels for every K (chadq_gemv_i8row_fp32)
 int gemv_i8row_dispatch(const float *x, const int8_t *w8, const float *sc, float *y, int M, int N, int K, bool fp32_only,
-                        hipStream_t st) {
+                        bool bf16_out, hipStream_t st) {
     // K a multiple of 128: the int8 matrix core, one pass over W for all M (gemv_i8row_mfma.hip); the fp32 kernels
     // below keep the other row lengths
-    if (!fp32_only && N > 0 && gemv_i8row_mfma_ok(M, K)) return gemv_i8row_mfma_launch(x, w8, sc, y, M, N, K, st);
+    if (!fp32_only && N > 0 && gemv_i8row_mfma_ok(M, K)) return gemv_i8row_mfma_launch(x, w8, sc, y, M, N, K, bf16_out, st);
     // <1024-wide chunks per row, rows per wave, activation rows, waves per workgroup>, picked by measurement: eight
     // waves share one copy of the activations; matrices with many rows give a wave 2 or 4 rows
     if (K <= 2048) {
         const bool big = N >= 8192;
         for (int m0 = 0; m0 < M;) {
             const float *xm = x + (size_t)m0 * K;
-            float *ym = y + (size_t)m0 * N;
+            float *ym = sum_at(y, (size_t)m0 * N, bf16_out);
             const int mb = (M - m0 >= 2) ? 2 : 1;
             if (K <= 1024) {
-                if (mb == 2) big ? launch_rows8<1, 4, 2, 8>(xm, w8, sc, ym, N, K, st) : launch_rows8<1, 2, 2, 8>(xm, w8, sc, ym, N, K, st);
-                else big ? launch_rows8<1, 4, 1, 8>(xm, w8, sc, ym, N, K, st) : launch_rows8<1, 2, 1, 8>(xm, w8, sc, ym, N, K, st);
+                if (mb == 2) big ? launch_rows8<1, 4, 2, 8>(xm, w8, sc, ym, N, K, bf16_out, st) : launch_rows8<1, 2, 2, 8>(xm, w8, sc, ym, N, K, bf16_out, st);
+                else big ? launch_rows8<1, 4, 1, 8>(xm, w8, sc, ym, N, K, bf16_out, st) : launch_rows8<1, 2, 1, 8>(xm, w8, sc, ym, N, K, bf16_out, st);
             } else {
-                if (mb == 2) big ? launch_rows8<2, 2, 2, 8>(xm, w8, sc, ym, N, K, st) : launch_rows8<2, 1, 2, 8>(xm, w8, sc, ym, N, K, st);
-                else big ? launch_rows8<2, 2, 1, 8>(xm, w8, sc, ym, N, K, st) : launch_rows8<2, 1, 1, 8>(xm, w8, sc, ym, N, K, st);
+                if (mb == 2) big ? launch_rows8<2, 2, 2, 8>(xm, w8, sc, ym, N, K, bf16_out, st) : launch_rows8<2, 1, 2, 8>(xm, w8, sc, ym, N, K, bf16_out, st);
+                else big ? launch_rows8<2, 2, 1, 8>(xm, w8, sc, ym, N, K, bf16_out, st) : launch_rows8<2, 1, 1, 8>(xm, w8, sc, ym, N, K, bf16_out, st);
             }
             m0 += mb;
         }
     } else if (K <= 8192) {  // rows of up to 4096 / 8192 k: the same kernel with 4 or 8 chunks per row, one activation row at a time
         for (int m0 = 0; m0 < M; ++m0) {
             const float *xm = x + (size_t)m0 * K;
-            float *ym = y + (size_t)m0 * N;
-            if (K <= 4096) N >= 4096 ? launch_rows8<4, 2, 1, 8>(xm, w8, sc, ym, N, K, st) : launch_rows8<4, 1, 1, 8>(xm, w8, sc, ym, N, K, st);
-            else launch_rows8<8, 1, 1, 8>(xm, w8, sc, ym, N, K, st);
+            float *ym = sum_at(y, (size_t)m0 * N, bf16_out);
+            if (K <= 4096) N >= 4096 ? launch_rows8<4, 2, 1, 8>(xm, w8, sc, ym, N, K, bf16_out, st) : launch_rows8<4, 1, 1, 8>(xm, w8, sc, ym, N, K, bf16_out, st);
+            else launch_rows8<8, 1, 1, 8>(xm, w8, sc, ym, N, K, bf16_out, st);
         }
     } else {
-        hipLaunchKernelGGL(gemv_i8row_generic_kernel, dim3((N + 3) / 4), dim3(256), 0, st, x, w8, sc, y, M, N, K);
+        hipLaunchKernelGGL(gemv_i8row_generic_kernel, dim3((N + 3) / 4), dim3(256), 0, st, x, w8, sc, y, M, N, K, (int)bf16_out);
     }
     return hip_check(hipGetLastError(), "gemv_i8row launch");
 }

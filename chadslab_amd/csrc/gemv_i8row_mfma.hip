@@ -60,7 +60,7 @@ __device__ __forceinline__ int half_row_merge(uint32_t old, uint32_t src) {
 template <int SETS>
 __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__restrict__ x, const int8_t *w8,
                                                               const float *sc, float *__restrict__ y, int M, int N,
-                                                              int K) {
+                                                              int K, int bf16_out) {
     using C = GemvI8Cfg<SETS>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint32_t *amax = reinterpret_cast<uint32_t *>(smem + C::AMAX_OFF);
@@ -276,14 +276,14 @@ __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__res
 #pragma unroll
     for (int r = 0; r < C::RES; ++r) {
         const int m = (SETS == 3) ? 4 * g + r : 4 * r + g;
-        if (m < M && n < N) y[(size_t)m * N + n] = (yacc[r] + other[r]) * scale;
+        if (m < M && n < N) store_sum(y, (size_t)m * N + n, (yacc[r] + other[r]) * scale, bf16_out);
     }
 }
 
 bool gemv_i8row_mfma_ok(int M, int K) { return M >= 1 && M <= 16 && K % 128 == 0; }
 
 template <int SETS>
-static int launch_i8_mfma(const float *x, const int8_t *w8, const float *sc, float *y, int M, int N, int K, hipStream_t st) {
+static int launch_i8_mfma(const float *x, const int8_t *w8, const float *sc, float *y, int M, int N, int K, bool bf16_out, hipStream_t st) {
     using C = GemvI8Cfg<SETS>;
     static std::atomic<bool> attr_set{false};  // setting it twice from two threads is harmless
     if (!attr_set.load(std::memory_order_acquire)) {
@@ -291,16 +291,16 @@ static int launch_i8_mfma(const float *x, const int8_t *w8, const float *sc, flo
                                       hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS));
         attr_set.store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL(gemv_i8row_mfma_kernel<SETS>, dim3((N + 63) / 64), dim3(512), C::LDS, st, x, w8, sc, y, M, N, K);
+    hipLaunchKernelGGL(gemv_i8row_mfma_kernel<SETS>, dim3((N + 63) / 64), dim3(512), C::LDS, st, x, w8, sc, y, M, N, K, (int)bf16_out);
     return hip_check(hipGetLastError(), "gemv_i8row_mfma launch");
 }
 
 // 1..16 activation rows, K a multiple of 128 (x and w8 16-byte aligned as for every int8 GEMV)
 int gemv_i8row_mfma_launch(const float *x, const int8_t *w8, const float *sc, float *y, int M, int N, int K,
-                           hipStream_t st) {
-    if (M <= 4) return launch_i8_mfma<1>(x, w8, sc, y, M, N, K, st);
-    if (M <= 8) return launch_i8_mfma<2>(x, w8, sc, y, M, N, K, st);
-    return launch_i8_mfma<3>(x, w8, sc, y, M, N, K, st);
+                           bool bf16_out, hipStream_t st) {
+    if (M <= 4) return launch_i8_mfma<1>(x, w8, sc, y, M, N, K, bf16_out, st);
+    if (M <= 8) return launch_i8_mfma<2>(x, w8, sc, y, M, N, K, bf16_out, st);
+    return launch_i8_mfma<3>(x, w8, sc, y, M, N, K, bf16_out, st);
 }
 
 }  // namespace chadq

@@ -82,7 +82,13 @@ def qgemv(x: torch.Tensor, qw: QWeight, out: Optional[torch.Tensor] = None, *, f
     fp32_elements (int8 weights only): fp32 arithmetic on every activation (chadq_gemv_i8row_fp32) instead of the
     matrix-core kernel's per-block fixed point, whose error on a small activation grows with the largest one of its
     2048-k block; the weights are then streamed once per pair of activation rows."""
+    return _gemv(x, qw, out, fp32_elements, False)
+
+
+def _gemv(x: torch.Tensor, qw: QWeight, out: Optional[torch.Tensor], fp32_elements: bool, bf16_out: bool) -> torch.Tensor:
+    """qgemv with the sums as fp32 or, bf16_out, rounded to bf16 by the kernel that forms them."""
     lib = _lib.load()
+    y_dtype = torch.bfloat16 if bf16_out else torch.float32
     if x.dim() != 2 or x.shape[1] != qw.K:
         raise ValueError("x must be [M,%d], got %s" % (qw.K, tuple(x.shape)))
     m = x.shape[0]
@@ -91,16 +97,16 @@ def qgemv(x: torch.Tensor, qw: QWeight, out: Optional[torch.Tensor] = None, *, f
     if isinstance(qw, QWeightInt4G32):
         x = _dev(x, "x", torch.bfloat16)
         p, s = _dev(qw.packed, "packed", torch.uint8), _dev(qw.scale, "scale", torch.float16)
-        y = _out(out, (m, qw.N), torch.float32, x.device)
-        _lib.check(lib.chadq_gemv_i4g32(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, qw.N, qw.K,
-                                        _stream()), "chadq_gemv_i4g32")
+        y = _out(out, (m, qw.N), y_dtype, x.device)
+        name = "chadq_gemv_i4g32_bf16" if bf16_out else "chadq_gemv_i4g32"
+        _lib.check(getattr(lib, name)(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, qw.N, qw.K, _stream()), name)
         return y
     if isinstance(qw, QWeightInt8):
         x = _dev(x, "x", torch.float32)
         w, s = _dev(qw.w, "w", torch.int8), _dev(qw.scale, "scale", torch.float32)
-        y = _out(out, (m, qw.N), torch.float32, x.device)
-        fn, name = (lib.chadq_gemv_i8row_fp32, "chadq_gemv_i8row_fp32") if fp32_elements else (lib.chadq_gemv_i8row, "chadq_gemv_i8row")
-        _lib.check(fn(x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, qw.N, qw.K, _stream()), name)
+        y = _out(out, (m, qw.N), y_dtype, x.device)
+        name = "chadq_gemv_i8row_fp32" if fp32_elements else "chadq_gemv_i8row_bf16" if bf16_out else "chadq_gemv_i8row"
+        _lib.check(getattr(lib, name)(x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, qw.N, qw.K, _stream()), name)
         return y
     raise TypeError("unknown weight container %r" % type(qw))
 
@@ -130,7 +136,8 @@ def qlinear(x: torch.Tensor, qw: QWeight, *, out_dtype: Optional[torch.dtype] = 
     """y = x @ dequant(W).T over the last axis of x.
 
     Up to 16 rows go to the bandwidth-bound GEMV (fp32 result); more rows go to the MFMA GEMM (bf16 result).
-    out_dtype picks the result type; asking for the other type than the kernel's native one casts.
+    out_dtype picks the result type.  The GEMV writes bf16 itself if that is asked for (the same sums rounded once); any
+    other type than the kernel's native one is a cast.
     """
     lead, k = x.shape[:-1], x.shape[-1]
     x2 = x.reshape(-1, k)
@@ -138,7 +145,7 @@ def qlinear(x: torch.Tensor, qw: QWeight, *, out_dtype: Optional[torch.dtype] = 
     use_gemv = m <= GEMV_MAX_M and not (isinstance(qw, QWeightInt8) and x2.dtype == torch.bfloat16)
     if isinstance(qw, QWeightInt8) and x2.dtype == torch.float32 and not use_gemv:
         raise ValueError("int8 weights with fp32 activations are served for at most %d rows" % GEMV_MAX_M)
-    y = qgemv(x2, qw) if use_gemv else qgemm(x2, qw)
+    y = _gemv(x2, qw, None, False, out_dtype == torch.bfloat16) if use_gemv else qgemm(x2, qw)
     if out_dtype is not None and y.dtype != out_dtype:
         y = y.to(out_dtype)
     return y.reshape(*lead, qw.N)

@@ -82,6 +82,10 @@ int chadq_dequant_i8row(const int8_t *w8, const float *scale, float *w, int N, i
 int chadq_gemv_i4g32(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, float *y, int M, int N,
                      int K, void *stream);
 
+/* The same sums, rounded to bf16 (nearest even) as they are stored. */
+int chadq_gemv_i4g32_bf16(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, uint16_t *y_bf16, int M, int N,
+                          int K, void *stream);
+
 /*
  * Split-K form of the M = 1 product for matrices with few rows and long K (a down projection): y_parts fp32
  * [ksplit, N], part s = the sum over k in [s*K/ksplit, (s+1)*K/ksplit); the caller adds the parts
@@ -131,6 +135,10 @@ int chadq_gemv_i4g32_addnorm_geglu(const float *res, const float *delta, int n_d
  */
 int chadq_gemv_i8row(const float *x, const int8_t *w8, const float *scale, float *y, int M, int N, int K,
                      void *stream);
+
+/* The same results, rounded to bf16 (nearest even) as they are stored. */
+int chadq_gemv_i8row_bf16(const float *x, const int8_t *w8, const float *scale, uint16_t *y_bf16, int M, int N, int K,
+                          void *stream);
 
 /*
  * The same product with fp32 arithmetic on every element, whatever K: x[m,k] * float(W[n,k]) accumulated in fp32, the

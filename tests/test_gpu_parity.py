@@ -592,6 +592,23 @@ def _experts(seed, e, h, f):
     return host, dev
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(1000, 2048), (8197, 512), (515, 4352), (300, 96), (301, 4128)])
+def test_qlinear_bf16_result_is_the_fp32_one_rounded(ops, m, n, k):
+    """Every GEMV kernel (tall and short matrices, K % 256 != 0, K beyond the row kernels) with the bf16 store."""
+    from chadslab_amd import QWeightInt4G32, QWeightInt8
+
+    r = rng(6100 + m + n)
+    x = torch.from_numpy(r.standard_normal((m, k)).astype(np.float32)).to(DEV)
+    p = torch.from_numpy(r.integers(0, 256, (n, k // 2), dtype=np.uint8)).to(DEV)
+    s = torch.from_numpy(r.lognormal(-5, 0.5, (n, k // 32)).astype(np.float16)).to(DEV)
+    w8 = torch.from_numpy(r.integers(-127, 128, (n, k), dtype=np.int8)).to(DEV)
+    s8 = torch.from_numpy(r.lognormal(-8, 0.5, n).astype(np.float32)).to(DEV)
+    for xv, qw in ((x.to(torch.bfloat16), QWeightInt4G32(p, s)), (x, QWeightInt8(w8, s8))):
+        y = ops.qlinear(xv, qw, out_dtype=torch.bfloat16)
+        assert y.dtype == torch.bfloat16 and torch.equal(y, ops.qlinear(xv, qw).to(torch.bfloat16))
+
+
 def test_moe_route_matches_oracle(ops):
     r = rng(70)
     logits = r.standard_normal((300, 8)).astype(np.float32)

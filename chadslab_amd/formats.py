@@ -37,11 +37,11 @@ class QWeightInt8:
 
     @property
     def N(self) -> int:
-        return self.w.shape[0]
+        return self.w.size(0)
 
     @property
     def K(self) -> int:
-        return self.w.shape[1]
+        return self.w.size(1)
 
     def to(self, device) -> "QWeightInt8":
         return QWeightInt8(self.w.to(device).contiguous(), self.scale.to(device).contiguous())
@@ -63,11 +63,11 @@ class QWeightInt4G32:
 
     @property
     def N(self) -> int:
-        return self.packed.shape[0]
+        return self.packed.size(0)
 
     @property
     def K(self) -> int:
-        return self.packed.shape[1] * 2
+        return self.packed.size(1) * 2
 
     def to(self, device) -> "QWeightInt4G32":
         return QWeightInt4G32(self.packed.to(device).contiguous(), self.scale.to(device).contiguous())
@@ -89,11 +89,11 @@ class QWeightInt4G32Tiles:
 
     @property
     def N(self) -> int:
-        return self.packed.shape[0]
+        return self.packed.size(0)
 
     @property
     def K(self) -> int:
-        return self.packed.shape[1] * 2
+        return self.packed.size(1) * 2
 
 
 def pack_int4(q: torch.Tensor) -> torch.Tensor:

@@ -450,6 +450,8 @@ static GemmTile pick_tile(int M, int N, int K, bool int4) {
 
 int gemm_i4g32_bf16_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N,
                              int K, hipStream_t st) {
+    // at most 64 rows: 12 to 60 % faster than the 128 x 64 kernel at every shape tried (gemm_tile_q.hip)
+    if (M <= 64 && gemm_tile_q_ok(K)) return gemm_tile_few_i4g32_launch(x, wp, sc, y, M, N, K, st);
     const GemmTile t = pick_tile(M, N, K, true);
     if (t != TILE_128x64) return gemm_tile_i4g32_launch(x, wp, sc, y, M, N, K, t == TILE_256, st);
     return launch_gemm<FmtI4G32, false>(x, wp, sc, y, M, N, K, nullptr, 0, st);
@@ -457,6 +459,7 @@ int gemm_i4g32_bf16_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_
 
 int gemm_i8row_bf16_dispatch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K,
                              hipStream_t st) {
+    if (M <= 64 && gemm_tile_q_ok(K)) return gemm_tile_few_i8row_launch(x, w8, sc, y, M, N, K, st);
     const GemmTile t = pick_tile(M, N, K, false);
     if (t != TILE_128x64) return gemm_tile_i8row_launch(x, w8, sc, y, M, N, K, t == TILE_256, st);
     return launch_gemm<FmtI8Row, false>(x, w8, sc, y, M, N, K, nullptr, 0, st);

@@ -56,7 +56,7 @@ struct Cfg {
     static constexpr int S_BUF = !I4 ? 0 : GUARD ? 256 : 1024, S_WAVE = 2 * S_BUF;
     static constexpr int SPB = 4 / WK;                               // steps per 256 k
     static constexpr int EP_PITCH = BN * 2 + 16;                     // result tile in LDS: bf16 rows, padded
-    static constexpr int OPER = S_OFF + NW * S_WAVE, EPI = BM * EP_PITCH, RED = WK > 1 ? BM * BN * 4 : 0;
+    static constexpr int OPER = S_OFF + NW * S_WAVE, EPI = BM * EP_PITCH, RED = WK == 4 ? BM * BN * 16 : WK > 1 ? BM * BN * 4 : 0;
     static constexpr int LDS0 = OPER > EPI ? OPER : EPI, LDS = LDS0 > RED ? LDS0 : RED;
     static constexpr int AHEAD = WMB > 4 ? 1 : 2;  // slices between a fragment's request and its MFMAs (what the registers allow)
     static_assert(LDS <= 163840, "one workgroup per compute unit");
@@ -144,8 +144,10 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(wq) + (size_t)n0 * wrow, 0, nrows * wrow, 0x00020000);
     constexpr uint32_t kOut = 0x80000000u;
     uint32_t aoff[C::A_DMA], boff[C::B_DMA];
-    int apc[C::A_DMA];
+    int apc[C::A_DMA], bpc[C::B_DMA];
     constexpr int BPR = BB / 16;  // 16-byte pieces per weight row and step
+    // WK = 4: a row's 128 or 256 bytes span half or all of the banks, so its pieces are XOR-swizzled by the row as A's are
+    auto bkey = [](int r) { return WK < 4 ? 0 : BPR == 8 ? (r >> 1) & 7 : r & 15; };
 #pragma unroll
     for (int q = 0; q < C::A_DMA; ++q) {  // 8 row segments of 128 B per instruction, [k half][row][128 B]
         const int e = (q * C::NW + wave) * 8 + (lane >> 3), r = e % BM;
@@ -155,7 +157,8 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
     for (int q = 0; q < C::B_DMA; ++q) {  // 64 / BPR rows per instruction
         const int r = (q * C::NW + wave) * (64 / BPR) + lane / BPR;
-        boff[q] = r < nrows ? (uint32_t)r * (uint32_t)wrow + 16u * (lane % BPR) : kOut;
+        bpc[q] = 16 * ((lane % BPR) ^ bkey(r));
+        boff[q] = r < nrows ? (uint32_t)r * (uint32_t)wrow + (uint32_t)bpc[q] : kOut;
     }
     const uint16_t *srow = nullptr;
     if constexpr (I4) {
@@ -180,7 +183,7 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
         for (int q = 0; q < C::B_DMA; ++q) {
             const int soff = (I4 ? kbeg >> 1 : kbeg) + step * BB;
-            dma(brsrc, GUARD && soff + 16 * (lane % BPR) >= wrow ? kOut : boff[q], soff, stage + C::A_STAGE + (q * C::NW + wave) * 1024);
+            dma(brsrc, GUARD && soff + bpc[q] >= wrow ? kOut : boff[q], soff, stage + C::A_STAGE + (q * C::NW + wave) * 1024);
         }
     };
     auto issue_s = [&](int blk) {  // blk: 256-k block, or (GUARD) step
@@ -196,7 +199,10 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
     uint32_t foff[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) foff[t] = (uint32_t)(wk * BM * 128 + nl * 128 + (((4 * kq + t) ^ ((nl >> 1) & 7)) << 4));
-    const uint32_t woff = (uint32_t)(C::A_STAGE + (wn * 32 + nl) * BB + (2 * wk + kq) * (BB / (2 * WK)));
+    constexpr int BQ = I4 ? 1 : 2;  // 16-byte pieces of a lane's 32 k
+    uint32_t woff[BQ];
+#pragma unroll
+    for (int e = 0; e < BQ; ++e) woff[e] = (uint32_t)(C::A_STAGE + (wn * 32 + nl) * BB + 16 * (((2 * wk + kq) * BQ + e) ^ bkey(wn * 32 + nl)));
 
     const uint32_t c_mlo = vgpr_const(0x000F000Fu), c_mhi = vgpr_const(0x00F000F0u), c_magic = vgpr_const(0x64006400u);
 
@@ -206,13 +212,12 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[a][v] = 0.f;
 
-    constexpr int BQ = I4 ? 1 : 2;
     u32x4 bq[BQ];  // the lane's packed weights of a step: 32 k
     uint16_t sraw = 0;
     float cs[4];
     auto fetch = [&](int step, const uint8_t *stage) {
 #pragma unroll
-        for (int e = 0; e < BQ; ++e) bq[e] = *reinterpret_cast<const u32x4 *>(stage + woff + e * 16);
+        for (int e = 0; e < BQ; ++e) bq[e] = *reinterpret_cast<const u32x4 *>(stage + woff[e]);
         if constexpr (I4) {
             if (GUARD) sraw = *reinterpret_cast<const uint16_t *>(slds + (step & 1) * C::S_BUF + lane * 4);
             else sraw = *reinterpret_cast<const uint16_t *>(slds + (step / C::SPB & 1) * C::S_BUF + nl * 16 + (((step * WK + wk) & 3) * 2 + kq) * 2);
@@ -242,7 +247,7 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
     // ---- prologue: two stages and the scales they need
     uint8_t *cur = lds, *nxt = lds + C::STAGE, *far = lds + 2 * C::STAGE;
     issue_s(0);
-    if (GUARD ? steps > 1 : C::SPB == 2 && steps > 2) issue_s(1);
+    if (GUARD || C::SPB == 1 ? steps > 1 : C::SPB == 2 && steps > 2) issue_s(1);
     issue_b(0, cur);
     issue_a(0, 0, C::A_DMA, cur);
     if (steps > 1) {
@@ -293,7 +298,7 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
                 else wait_vmcnt<0>();
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this stage has been read
                 wg_barrier();
-                if (GUARD) {
+                if (GUARD || C::SPB == 1) {
                     if (more2) issue_s(i + 2);
                 } else if (I4 && (i + 3) % C::SPB == 0 && i + 3 < steps) {
                     issue_s((i + 3) / C::SPB);
@@ -332,8 +337,9 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
     wg_barrier();  // every wave is done with the stages, which everything below reuses
     // WK = 2: the two waves that hold the k halves of one result exchange halves of it through LDS and each finishes one:
     // lower row blocks by the first, upper ones by the second.  (A tile of one row block: its upper eight values.)
-    constexpr int PARTS = WMB == 1 ? 2 : WMB;                  // units of exchange: row blocks, or halves of the only one
-    constexpr int UV = WMB == 1 ? 8 : 16, PE = PARTS / WK;     // values per unit, units a wave finishes
+    // WK = 4: every wave leaves all of its values and finishes a quarter of the sums, added in the order of the k.
+    constexpr int PARTS = WK == 4 ? 4 : WMB == 1 ? 2 : WMB;    // units of exchange: row blocks, halves of the only one, quarters
+    constexpr int UV = WK == 4 ? WMB * 4 : WMB == 1 ? 8 : 16, PE = PARTS / WK;  // values per unit, units a wave finishes
     auto val = [&](int u, int v) { return WMB == 1 ? acc[0][u * 8 + v] : acc[WMB == 1 ? 0 : u][v]; };
     float res[PE][UV];
     if constexpr (WK == 2) {
@@ -357,6 +363,23 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
                 for (int e = 0; e < 4; ++e) res[u][4 * q + e] = (wk ? val(PE + u, 4 * q + e) : val(u, 4 * q + e)) + o[e];
             }
         __syncthreads();
+    } else if constexpr (WK == 4) {
+        float *const red = reinterpret_cast<float *>(lds) + lane * 4;
+#pragma unroll
+        for (int q = 0; q < WMB * 4; ++q) {
+            const f32x4 o = {acc[q / 4][q % 4 * 4], acc[q / 4][q % 4 * 4 + 1], acc[q / 4][q % 4 * 4 + 2], acc[q / 4][q % 4 * 4 + 3]};
+            *reinterpret_cast<f32x4 *>(red + (wave * WMB * 4 + q) * 256) = o;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < UV / 4; ++q) {
+            f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < WK; ++w) o += *reinterpret_cast<const f32x4 *>(red + ((w * WN + wn) * WMB * 4 + wk * (UV / 4) + q) * 256);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) res[0][4 * q + e] = o[e];
+        }
+        __syncthreads();
     } else {
 #pragma unroll
         for (int u = 0; u < PE; ++u)
@@ -365,6 +388,10 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
     }
     const int u0 = wk * PE;  // the wave's first unit
     auto row_of = [&](int u, int v) {
+        if (WK == 4) {
+            const int f = u0 * UV + v, vv = f & 15;
+            return (f >> 4) * 32 + 8 * (vv >> 2) + 4 * kq + (vv & 3);
+        }
         const int vv = WMB == 1 ? (u0 + u) * 8 + v : v;
         return (WMB == 1 ? 0 : (u0 + u) * 32) + 8 * (vv >> 2) + 4 * kq + (vv & 3);
     };
@@ -462,6 +489,25 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
     if (big)
         return K % 64 ? tileq::launch<false, 8, 1, 8, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 8, 1, 8, false>(x, w, sc, y, M, N, K, 1, st);
     return K % 128 ? tileq::launch<false, 4, 2, 4, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 4, 2, 4, false>(x, w, sc, y, M, N, K, 1, st);
+}
+
+// At most 64 rows: 32 or 64 rows x 64 weight rows, the eight waves two side by side and four along K (256 k per step).
+// What bounds it is the weight stream and the latency of a step: as many weight rows per workgroup as the 128 x 64 kernel
+// has (one round of the chip up to 16384 of them), but twice the waves, a quarter of the steps and no padding to 128 rows.
+// us (the 128 x 64 kernel in brackets): int4 48 x 14336 x 4096 14.8 (23.0), 17 x 4096 x 4096 9.5 (18.5), 64 x 4096 x 14336
+// 36 (53), 64 x 32768 x 4096 31 (44), 64 x 1024 x 1024 5.3 (8.3); int8 48 x 14336 x 4096 13.6 (22.5).
+int gemm_tile_few_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, hipStream_t st) {
+    const bool guard = K % 256 != 0 || !aligned16(sc);
+    if (M <= 32)
+        return guard ? tileq::launch<true, 2, 4, 1, true>(x, wp, sc, y, M, N, K, 1, st) : tileq::launch<true, 2, 4, 1, false>(x, wp, sc, y, M, N, K, 1, st);
+    return guard ? tileq::launch<true, 2, 4, 2, true>(x, wp, sc, y, M, N, K, 1, st) : tileq::launch<true, 2, 4, 2, false>(x, wp, sc, y, M, N, K, 1, st);
+}
+
+int gemm_tile_few_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, hipStream_t st) {
+    const uint8_t *w = reinterpret_cast<const uint8_t *>(w8);
+    if (M <= 32)
+        return K % 256 ? tileq::launch<false, 2, 4, 1, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 2, 4, 1, false>(x, w, sc, y, M, N, K, 1, st);
+    return K % 256 ? tileq::launch<false, 2, 4, 2, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 2, 4, 2, false>(x, w, sc, y, M, N, K, 1, st);
 }
 
 // ---- exact weights (HILO), K % 256 == 0: the projections of a prompt, whose tokens must come out as the decode step's do.

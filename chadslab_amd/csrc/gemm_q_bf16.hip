@@ -448,10 +448,19 @@ static GemmTile pick_tile(int M, int N, int K, bool int4) {
     return c128 <= c256 ? TILE_128 : TILE_256;
 }
 
+// Whether the 64 x 64 tile (32 x 64 for at most 32 rows) of gemm_tile_q.hip takes the product: up to 64 rows, or a launch
+// whose 64 x 64 tiles all run at once.  The larger tiles then leave compute units idle and each lasts longer.  us, that
+// tile against what pick_tile gives: int4 128 x 4096 x 4096 (128 tiles) 12.9 / 19.6, 256 x 4096 x 4096 (256 tiles)
+// 15.9 / 20.3, 256 x 1024 x 1024 5.5 / 9.0, 512 x 2048 x 14336 46 / 61, 1000 x 1024 x 4096 15.0 / 20.3; int8 200 x 4096 x
+// 4096 15.2 / 23.1.  With a second round it is the slower one: 384 x 4096 x 4096 (384 tiles) 27.4 / 22.2.
+static bool takes_small_tile(int M, int N, int K) {
+    const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+    return gemm_tile_q_ok(K) && (M <= 64 || tiles <= 256);
+}
+
 int gemm_i4g32_bf16_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N,
                              int K, hipStream_t st) {
-    // at most 64 rows: 12 to 60 % faster than the 128 x 64 kernel at every shape tried (gemm_tile_q.hip)
-    if (M <= 64 && gemm_tile_q_ok(K)) return gemm_tile_few_i4g32_launch(x, wp, sc, y, M, N, K, st);
+    if (takes_small_tile(M, N, K)) return gemm_tile_small_i4g32_launch(x, wp, sc, y, M, N, K, st);
     const GemmTile t = pick_tile(M, N, K, true);
     if (t != TILE_128x64) return gemm_tile_i4g32_launch(x, wp, sc, y, M, N, K, t == TILE_256, st);
     return launch_gemm<FmtI4G32, false>(x, wp, sc, y, M, N, K, nullptr, 0, st);
@@ -459,7 +468,7 @@ int gemm_i4g32_bf16_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_
 
 int gemm_i8row_bf16_dispatch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K,
                              hipStream_t st) {
-    if (M <= 64 && gemm_tile_q_ok(K)) return gemm_tile_few_i8row_launch(x, w8, sc, y, M, N, K, st);
+    if (takes_small_tile(M, N, K)) return gemm_tile_small_i8row_launch(x, w8, sc, y, M, N, K, st);
     const GemmTile t = pick_tile(M, N, K, false);
     if (t != TILE_128x64) return gemm_tile_i8row_launch(x, w8, sc, y, M, N, K, t == TILE_256, st);
     return launch_gemm<FmtI8Row, false>(x, w8, sc, y, M, N, K, nullptr, 0, st);

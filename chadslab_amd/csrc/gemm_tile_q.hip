@@ -491,19 +491,20 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
     return K % 128 ? tileq::launch<false, 4, 2, 4, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 4, 2, 4, false>(x, w, sc, y, M, N, K, 1, st);
 }
 
-// At most 64 rows: 32 or 64 rows x 64 weight rows, the eight waves two side by side and four along K (256 k per step).
+// At most 64 rows, or few enough tiles for one round: 32 or 64 rows x 64 weight rows, the eight waves two side by side and
+// four along K (256 k per step).
 // What bounds it is the weight stream and the latency of a step: as many weight rows per workgroup as the 128 x 64 kernel
 // has (one round of the chip up to 16384 of them), but twice the waves, a quarter of the steps and no padding to 128 rows.
 // us (the 128 x 64 kernel in brackets): int4 48 x 14336 x 4096 14.8 (23.0), 17 x 4096 x 4096 9.5 (18.5), 64 x 4096 x 14336
 // 36 (53), 64 x 32768 x 4096 31 (44), 64 x 1024 x 1024 5.3 (8.3); int8 48 x 14336 x 4096 13.6 (22.5).
-int gemm_tile_few_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, hipStream_t st) {
+int gemm_tile_small_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, hipStream_t st) {
     const bool guard = K % 256 != 0 || !aligned16(sc);
     if (M <= 32)
         return guard ? tileq::launch<true, 2, 4, 1, true>(x, wp, sc, y, M, N, K, 1, st) : tileq::launch<true, 2, 4, 1, false>(x, wp, sc, y, M, N, K, 1, st);
     return guard ? tileq::launch<true, 2, 4, 2, true>(x, wp, sc, y, M, N, K, 1, st) : tileq::launch<true, 2, 4, 2, false>(x, wp, sc, y, M, N, K, 1, st);
 }
 
-int gemm_tile_few_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, hipStream_t st) {
+int gemm_tile_small_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, hipStream_t st) {
     const uint8_t *w = reinterpret_cast<const uint8_t *>(w8);
     if (M <= 32)
         return K % 256 ? tileq::launch<false, 2, 4, 1, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 2, 4, 1, false>(x, w, sc, y, M, N, K, 1, st);

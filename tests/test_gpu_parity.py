@@ -444,7 +444,8 @@ def test_gemm_int4_many_rows_tile(ops, m, n, k):
 
 @pytest.mark.parametrize("m,n,k", [(385, 8200, 64), (641, 4100, 96), (1025, 4095, 32), (1024, 4096, 384), (897, 4223, 1312),  # 128 x 128 tiles
                                    (3841, 3847, 32), (4096, 4097, 288), (3840, 4096, 256),                                # 256 x 256
-                                   (17, 100, 32), (32, 515, 512), (33, 1000, 4352), (64, 64, 256), (63, 4097, 1056)])     # at most 64 rows
+                                   (17, 100, 32), (32, 515, 512), (33, 1000, 4352), (64, 64, 256), (63, 4097, 1056),      # 64 x 64, at most 64 rows
+                                   (65, 100, 32), (128, 8192, 64), (129, 5440, 1056), (1000, 1000, 288), (2049, 447, 512)])   # and in one round
 @pytest.mark.parametrize("weight", ["int4", "int8"])
 def test_gemm_eight_wave_tiles_every_row_and_column(ops, weight, m, n, k):
     """The tiles of gemm_tile_q.hip at ragged ends of rows, columns and k (k of one, two and three steps, no multiple of a

@@ -144,6 +144,9 @@ __global__ __launch_bounds__(128) void prompt_rope_kernel(const float *__restric
 //           positions x 8 columns, transposes them with 32 byte permutes and leaves 16-byte operands in LDS
 //           ([g][column]; the place of a column inside its group of eight is XORed with the group, so that neither the
 //           stores, one column of many groups, nor the loads, 16 columns, meet in the same banks).
+// The rows of a workgroup belong to one to sixteen tokens and share the V operands: a position that the later ones see and
+// the earlier ones must not goes in like any other while its V row is finite (its probability is 0 for those), and apart,
+// row by row, if it is not.
 template <int DH>
 __global__ __launch_bounds__(256) void prompt_attn_kernel(const float *__restrict__ q, const uint16_t *__restrict__ kc,
                                                           const uint16_t *__restrict__ vc, uint16_t *__restrict__ out, int T,
@@ -158,6 +161,7 @@ __global__ __launch_bounds__(256) void prompt_attn_kernel(const float *__restric
     const int r0 = blockIdx.x * 16, total = T * hq;
     const int t_last = min(r0 + 15, total - 1) / hq;
     const int nctx = pos + t_last + 1, nblk = (nctx + 31) >> 5;
+    const int seen = pos + r0 / hq + 1;  // every row of the workgroup sees the positions below, only some those from here on
 
     int lim[4];  // first position row 4g+e may not see
 #pragma unroll
@@ -205,12 +209,27 @@ __global__ __launch_bounds__(256) void prompt_attn_kernel(const float *__restric
     }
     for (int b = wave; b < nblk; b += 4) {
         const int p0 = b * 32;
+        // Positions only some of the rows see in a block with a V row that is not finite: the others' probability 0 times it
+        // would be NaN.  (Packed maxima of the magnitudes: two instructions per word, of the wave with the last block only.)
+        bool apart = false;
+        if (p0 + 32 > seen) {
+            u16x2 top[4] = {};
+#pragma unroll
+            for (int it = 0; it < NT; ++it)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) top[k] = __builtin_elementwise_max(top[k], __builtin_bit_cast(u16x2, vr[it][e][k] & 0x7FFF7FFFu));
+            top[0] = __builtin_elementwise_max(__builtin_elementwise_max(top[0], top[1]), __builtin_elementwise_max(top[2], top[3]));
+            apart = __any(top[0].x >= 0x7F80 || top[0].y >= 0x7F80);
+        }
+        const int pz = apart ? seen : nctx;  // rows from here on (past the context, or to be added apart) become zeros
 #pragma unroll
         for (int it = 0; it < NT; ++it) {
             const int task = it * 64 + lane, gq = task / CG, cg = task % CG;
 #pragma unroll
-            for (int e = 0; e < 8; ++e)  // rows past the context become zeros
-                if (p0 + 8 * gq + e >= nctx) vr[it][e] = u32x4{0, 0, 0, 0};
+            for (int e = 0; e < 8; ++e)
+                if (p0 + 8 * gq + e >= pz) vr[it][e] = u32x4{0, 0, 0, 0};
             if (vlive) {
 #pragma unroll
                 for (int c = 0; c < 8; ++c) {
@@ -268,6 +287,20 @@ __global__ __launch_bounds__(256) void prompt_attn_kernel(const float *__restric
             for (int e = 0; e < 4; ++e) o[c][e] *= alpha[e];
             o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, vb, o[c], 0, 0, 0);
             o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vb, o[c], 0, 0, 0);
+        }
+        if (__builtin_expect(apart, false)) {  // to the rows that see them, one position after the other
+            for (int p = max(seen, p0); p < min(nctx, p0 + 32); ++p) {
+                float pr[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) pr[e] = sp[(4 * g + e) * PP + p - p0];
+#pragma unroll
+                for (int c = 0; c < CB; ++c) {
+                    const float v = bf16_bits_to_f32(vc[(size_t)p * DH + 16 * c + li]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (p < lim[e]) o[c][e] = __builtin_fmaf(pr[e], v, o[c][e]);
+                }
+            }
         }
         __builtin_amdgcn_wave_barrier();
     }

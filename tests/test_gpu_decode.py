@@ -773,6 +773,38 @@ def test_decoder_prompt_in_chunks_equals_the_step_token_by_token(t, pos, layers,
     assert rel(b.logits, a.logits) <= 5e-3 * layers
 
 
+@pytest.mark.parametrize("t,bad,pos,d,hq,dh,ffn", [(16, (9,), 5, 512, 8, 64, 512), (21, (6, 13), 0, 256, 2, 128, 512), (40, (33, 39), 30, 256, 1, 256, 512),
+                                                   (33, (0, 17, 31), 3, 768, 3, 256, 768), (300, (260, 270), 0, 256, 4, 64, 512)])
+def test_decoder_prompt_a_token_that_is_not_finite_reaches_no_earlier_token(t, bad, pos, d, hq, dh, ffn):
+    """Tokens whose table rows are NaN, at several places of the attention's blocks of 16 rows and 32 positions: the cache
+    rows of every layer are NaN exactly where the decode step, which never reads a later position, has them NaN (probability
+    0 times a V row that is not finite would be NaN), and the others agree with the step's."""
+    import chadslab_amd.decoder as D
+
+    cfg = D.DecoderConfig(n_layers=3, d=d, hq=hq, dh=dh, ffn=ffn, vocab=500, max_ctx=400)
+    w = D.random_weights(cfg, 90 + t, DEV)
+    w["emb"].scale[7] = float("nan")
+    toks = [7 if i in bad else 8 + (i * 31) % 490 for i in range(t)]
+    a, b = D.QuantDecoder(cfg, w, DEV), D.QuantDecoder(cfg, w, DEV)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(t)
+    for name in ("kcache", "vcache"):
+        for ca, cb in zip(getattr(a, name), getattr(b, name)):
+            ca[:pos * dh] = torch.randn(pos * dh, device=DEV, generator=g).to(torch.bfloat16)
+            cb.copy_(ca)
+    for i, tok in enumerate(toks):
+        a.set_state(tok, pos + i)
+        a.step()
+    b.feed(toks, pos)
+    end = (pos + t) * dh
+    for name in ("kcache", "vcache"):
+        for li, (ca, cb) in enumerate(zip(getattr(a, name), getattr(b, name))):
+            ca, cb = ca[:end].float(), cb[:end].float()
+            assert torch.equal(torch.isnan(cb), torch.isnan(ca)), (name, li)
+            ca, cb = torch.nan_to_num(ca), torch.nan_to_num(cb)
+            assert float((cb - ca).norm() / ca.norm()) <= (3e-4 if li == 0 else 5e-3 * li), (name, li)
+
+
 def test_decoder_prompt_in_chunks_draws_what_single_tokens_would_have_drawn():
     import chadslab_amd.decoder as D
 

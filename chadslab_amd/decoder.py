@@ -8,6 +8,7 @@ embedding / output table without embedding scaling or logit soft-capping.
 """
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
 from typing import Dict, List, Optional
 
@@ -18,7 +19,19 @@ from .formats import QWeightInt4G32, quantize_int4_g32
 
 
 PROMPT_CHUNK = 256  # tokens that go through a layer together
-PROMPT_MIN = 3      # shorter sequences are quicker token by token
+
+
+def prompt_min(pos: int, dh: int) -> int:
+    """Tokens from which on the prompt kernels are quicker than the decode step, for a sequence that starts at `pos`.
+
+    For a few tokens their time is the weights' and then the walk of a few workgroups over the whole context (a workgroup
+    takes 16 rows of the attention and does not share their context with others, as the step's does), which hardly
+    depends on the number of tokens.  Measured, in decode steps at the same position (8 heads of 256 and 4 heads of 256;
+    8 heads of 128; 8 heads of 64; 3 to 32 tokens): at 0: 2.3, 2.4; 2.0; 2.3.  1000: 3.0, 3.0; 2.3; 2.6.  4000: 4.6, 4.4;
+    2.8; 3.1.  8000: 6.2, 5.8; 3.0; 3.2.  16000: 8.4, 7.7; 3.2; 3.3.  32000: 10.9, 10.8; 3.3; 3.4.  65000: 12.7, 15.5;
+    3.4; 3.4.  The quotient below follows the larger ones, rounded up: the step is left only for what is quicker."""
+    grow = 3.0e-5 if dh > 128 else 1.65e-4  # the step's attention, per position
+    return max(3, math.ceil((2.4 + 6.7e-4 * pos) / (1.0 + grow * pos)))
 
 
 @dataclass
@@ -352,11 +365,11 @@ class QuantDecoder:
         """Reads a given token sequence starting at position `pos` (a prompt) into the caches and returns the token the
         model proposes after the last one.  Where the prompt kernels cover the model's sizes, whole chunks of the sequence
         go through a layer at once (chadq_prompt_i4g32: every weight is read once per chunk instead of once per token, and
-        only the last token meets the output table); else, and for a sequence of one or two tokens, the step runs token by
-        token.  Raises ValueError if the sequence would run past max_ctx or holds a token outside the vocabulary."""
+        only the last token meets the output table); else, and for sequences too short for that to pay (prompt_min()), the
+        step runs token by token.  Raises ValueError if the sequence would run past max_ctx or holds a token outside the vocabulary."""
         tokens = list(tokens)
         self._check_range(pos, len(tokens), tokens)
-        layers = self._describe_layers() if len(tokens) >= PROMPT_MIN else None
+        layers = self._describe_layers() if len(tokens) >= prompt_min(pos, self.cfg.dh) else None
         if layers is not None:
             return self._feed_chunks(layers, tokens, pos)
         self.pos.fill_(pos)

@@ -805,6 +805,29 @@ def test_decoder_prompt_a_token_that_is_not_finite_reaches_no_earlier_token(t, b
             assert float((cb - ca).norm() / ca.norm()) <= (3e-4 if li == 0 else 5e-3 * li), (name, li)
 
 
+@pytest.mark.parametrize("dh,pos,few,enough", [(256, 0, 2, 3), (256, 4000, 4, 5), (256, 16000, 8, 9), (64, 0, 2, 3), (64, 16000, 3, 4)])
+def test_decoder_feed_of_few_tokens_at_a_long_context_runs_the_step(monkeypatch, dh, pos, few, enough):
+    """The prompt kernels walk the whole context in a few workgroups: below the measured number of tokens the step, which
+    spreads it over the chip, is quicker and has to be what runs (bit for bit), from there on the prompt kernels."""
+    import chadslab_amd.decoder as D
+
+    cfg = D.DecoderConfig(n_layers=1, d=256, hq=4, dh=dh, ffn=512, vocab=300, max_ctx=16384)
+    dec = D.QuantDecoder(cfg, D.random_weights(cfg, 79, DEV), DEV)
+    dec.kcache[0].normal_()
+    dec.vcache[0].normal_()
+    chunked, real = [], dec._feed_chunks
+    monkeypatch.setattr(dec, "_feed_chunks", lambda layers, toks, p: chunked.append(len(toks)) or real(layers, toks, p))
+    toks = list(range(20, 20 + enough))
+    dec.feed(toks, pos)
+    assert chunked == [enough]
+    nxt, k = dec.feed(toks[:few], pos), dec.kcache[0].clone()
+    assert chunked == [enough]
+    for i, t in enumerate(toks[:few]):
+        dec.set_state(t, pos + i)
+        dec.step()
+    assert nxt == int(dec.token.item()) and torch.equal(dec.kcache[0], k)
+
+
 def test_decoder_prompt_in_chunks_draws_what_single_tokens_would_have_drawn():
     import chadslab_amd.decoder as D
 

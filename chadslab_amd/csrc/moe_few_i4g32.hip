@@ -16,8 +16,14 @@
 // 5.2 | 4.5 (12.8 | 7.0).
 // Arithmetic: v_mfma_f32_16x16x32_bf16 on unscaled weights.  A lane holds a whole scale group of its weight row (16
 // bytes); the lanes' words are exchanged (v_permlane16_swap, v_permlane32_swap) so that one MFMA holds one scale group;
-// nibbles become the bf16 value 128 + u, another MFMA of the same activations with the constant -136 takes the 136 off
-// beforehand for both of the item's row blocks, and one fp32 FMA per value applies the scale: weights are exact.
+// nibbles become the bf16 value u / 2^9 (unpack8_fp8), another MFMA of the same activations with the constant -8 / 2^9 takes
+// the 8 off beforehand for both of the item's row blocks, one fp32 FMA per value applies the scale and the finished sum is
+// multiplied by 2^9: weights are exact.  32 x 15 < 2^9, so every group's sum is finite for all finite activations, and it
+// errs by 8 / 2^24 of its largest activation at most where the weight there is 0.  (With 128 + u, the magic number of the
+// GEMVs, sums overflowed to NaN from activations of 1e35 on and the error was 17 times this: 512 x 512, one activation 1e5
+// or 1e6 times the others and all weights there 0, 8.9e-3 or 0.21 off, now 2.4e-3 or 4.4e-3, of which 2.3e-3 is the
+// rounding of h and y.  Signed operands, v_cvt_off_f32_i4 and no second MFMA, would leave no error and take 4 % more time;
+// this form takes 0.3 % more than 128 + u.)  An infinite activation gives NaN, as in the GEMVs.
 // Blocks past the end and rows without a token are requested beyond the buffer's range and arrive as zeros.
 #include "chadq_common.h"
 
@@ -28,6 +34,23 @@ constexpr int FEW_ENTRIES = 16;  // experts (one entry of the tile list each, as
 constexpr int RB = 2;            // blocks of 16 weight rows per item
 constexpr uint32_t kBeyond = 0x80000000u;
 constexpr int kRange = 0x7FFFFFFF;
+
+// 8 nibbles u -> 8 bf16 u / 2^9, exact: a nibble in a byte of its own is the e4m3 number u / 2^9 (its low eight values are
+// the subnormals, the others the next binade, with the same spacing).  Order: (u0, u2) (u4, u6) (u1, u3) (u5, u7).
+__device__ __forceinline__ void unpack8_fp8(uint32_t w, uint32_t p[4]) {
+    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+    p[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.f, false));
+    p[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.f, true));
+    p[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, false));
+    p[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, true));
+}
+// 8 bf16 activations in the same order
+__device__ __forceinline__ void order_x8(const uint32_t a[4], uint32_t o[4]) {
+    o[0] = __builtin_amdgcn_perm(a[1], a[0], 0x05040100u);
+    o[1] = __builtin_amdgcn_perm(a[3], a[2], 0x05040100u);
+    o[2] = __builtin_amdgcn_perm(a[1], a[0], 0x07060302u);
+    o[3] = __builtin_amdgcn_perm(a[3], a[2], 0x07060302u);
+}
 
 template <int MODE, bool TILED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void moe_few_i4g32_kernel(
@@ -137,13 +160,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         }
     };
 
-    const uint32_t mask_r = vgpr_const(0x000F000Fu), magic_r = vgpr_const(kBf16Magic);
     bf16x8 bias;
     {
-        const u32x4 v = {0xC308C308u, 0xC308C308u, 0xC308C308u, 0xC308C308u};  // -136
+        const u32x4 v = {0xBC80BC80u, 0xBC80BC80u, 0xBC80BC80u, 0xBC80BC80u};  // -8 / 2^9
         __builtin_memcpy(&bias, &v, 16);
     }
-    static_assert(kMagicBias == 136.f, "the constant above");
     // ---- the summing side
     int c_item = blockIdx.x, c_i = 0, c_n = 0, par = 0;
     f32x4 acc[RB];
@@ -169,6 +190,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             v[b] = 0.f;
 #pragma unroll
             for (int w = 0; w < 4; ++w) v[b] += reinterpret_cast<const float *>(&s_red[par][w][b][src])[m & 3];
+            v[b] *= 512.f;  // 2^9
         }
         if (m < s_ent[en].rows) {
             if (MODE == 1) {
@@ -213,14 +235,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
                 const u32x4 xv = q.x[4 * h + t];
                 const uint32_t a[4] = {xv.x, xv.y, xv.z, xv.w};
                 uint32_t o[4];
-                pair_x8(a, o);
+                order_x8(a, o);
                 bf16x8 av;
                 __builtin_memcpy(&av, o, 16);
                 const f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bias, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
                 for (int b = 0; b < RB; ++b) {
                     uint32_t p[4];
-                    unpack8_magic_r(word[b][t], mask_r, magic_r, p);
+                    unpack8_fp8(word[b][t], p);
                     bf16x8 bv;
                     __builtin_memcpy(&bv, p, 16);
                     const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, d0, 0, 0, 0);

@@ -778,6 +778,58 @@ def test_moe_ffn_few_tokens(ops, t, h, f, e, top_k):
         assert O.rel_l2(O.bf16_to_f32(v), ref) <= TOL_BF16
 
 
+@pytest.mark.parametrize("big", [0.0, 3e37, -2.9e38])
+def test_moe_ffn_few_tokens_large_activations(ops, big):
+    """One activation near the top of bf16's range in some tokens (its gate weights have the scale 0, so that the gate stays
+    moderate), h as large: every sum of the exact result is finite, so the result must be, in both orders, and rows of
+    ordinary size beside such rows keep their accuracy."""
+    from chadslab_amd import QWeightInt4G32
+
+    t, h, f, e = 6, 512, 768, 2
+    host, _ = _experts(9700, e, h, f)
+    for gp, gs, up, us, dp, ds in host:
+        gs[:, 3] = 0
+        us[:] = us.astype(np.float32) * 2.0 ** -6 if big else us
+        ds[:] = ds.astype(np.float32) * 2.0 ** -6 if big else ds
+    dev = [tuple(QWeightInt4G32(torch.from_numpy(tr[2 * i]).to(DEV), torch.from_numpy(tr[2 * i + 1]).to(DEV)) for i in range(3)) for tr in host]
+    r = rng(9701)
+    x = r.standard_normal((t, h)).astype(np.float32)
+    if big:
+        x[::2, 3 * 32 + 5] = big
+    xb = O.f32_to_bf16(x)
+    logits = r.standard_normal((t, e)).astype(np.float32)
+    ref = O.bf16_to_f32(O.moe_qffn(xb, logits, host, 2, True)).astype(np.float64)
+    assert np.isfinite(ref).all()
+    for ex in (dev, [tuple(ops.to_tiles(m) for m in tr) for tr in dev]):
+        y = O.bf16_to_f32(bits(ops.moe_ffn(bf16_tensor(xb), torch.from_numpy(logits).to(DEV), ex, top_k=2, renorm=True))).astype(np.float64)
+        for row in range(t):
+            assert np.linalg.norm(y[row] - ref[row]) <= 2.0 ** -8 * np.linalg.norm(ref[row]), row
+
+
+@pytest.mark.parametrize("outlier", [1e3, -1e5])
+def test_moe_ffn_few_tokens_beside_an_outlier_of_zero_weight(ops, outlier):
+    """One activation far larger than the others of its scale group, all gate and up weights at it 0: the others count as
+    ever.  The group's zero-point term, 8 times the outlier, is added and taken off in fp32: 1e5 * 8 * 2^-24 = 0.05 against a
+    gate of some 16 groups of sqrt(32) * 4.6 = 100, 5e-4, beside the two bf16 roundings."""
+    from chadslab_amd import QWeightInt4G32
+
+    t, h, f, e = 4, 512, 768, 2
+    host, _ = _experts(9750, e, h, f)
+    for gp, gs, up, us, dp, ds in host:
+        for p in (gp, up):
+            p[:, 50] = (p[:, 50] & 0xF0) | 8
+    dev = [tuple(QWeightInt4G32(torch.from_numpy(tr[2 * i]).to(DEV), torch.from_numpy(tr[2 * i + 1]).to(DEV)) for i in range(3)) for tr in host]
+    r = rng(9751)
+    x = r.standard_normal((t, h)).astype(np.float32)
+    x[:, 100] = outlier
+    xb = O.f32_to_bf16(x)
+    logits = r.standard_normal((t, e)).astype(np.float32)
+    ref = O.bf16_to_f32(O.moe_qffn(np.where(np.arange(h) == 100, 0, xb).astype(xb.dtype), logits, host, 2, True))
+    for ex in (dev, [tuple(ops.to_tiles(m) for m in tr) for tr in dev]):
+        y = O.bf16_to_f32(bits(ops.moe_ffn(bf16_tensor(xb), torch.from_numpy(logits).to(DEV), ex, top_k=2, renorm=True)))
+        assert O.rel_l2(y, ref) <= 2.0 ** -8
+
+
 def test_moe_ffn_tiled_wide_ranges_of_activations_and_scales(ops):
     """The tile-order kernels carry activations and dequantised weights as fp16: rows are scaled by a power of two first,
     so activations far outside fp16's range (and rows of very different magnitude side by side) must come out as the

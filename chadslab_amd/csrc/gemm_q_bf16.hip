@@ -417,11 +417,17 @@ static int launch_gemm_g(const uint16_t *x, const void *wq, const typename F::sc
 
 // NB = 2 (128 x 64 tiles).  The kernel is written for any NB; NB = 4 halves the traffic on the activation panel
 // but needs 256 accumulator registers plus two sets of dequantised operands and spills, so it is not instantiated.
+static int activations_ok(int M, int K) {
+    CHADQ_REQUIRE((int64_t)M * K * 2 < ((int64_t)1 << 32), CHADQ_ERR_SHAPE,
+                  "gemm: activations of %d x %d exceed the 4 GiB the kernel's 32-bit offsets cover", M, K);
+    return 0;
+}
+
 template <typename F, bool OUTF32>
 static int launch_gemm(const uint16_t *x, const void *wq, const typename F::scale_t *sc, void *y, int M, int N, int K,
                        const GemmGroup *groups, int ngroups, hipStream_t st) {
-    CHADQ_REQUIRE((int64_t)M * K * 2 < ((int64_t)1 << 32), CHADQ_ERR_SHAPE,
-                  "gemm: activations of %d x %d exceed the 4 GiB the kernel's 32-bit offsets cover", M, K);
+    const int rc = activations_ok(M, K);
+    if (rc != 0) return rc;
     // the unguarded int4 form fetches scale rows 16 bytes at a time: it needs 16-byte aligned scale rows, which only a
     // plain launch can check here (a grouped launch's pointers live in device memory)
     const bool scale_rows_ok = Tile<F, 2>::KL != 32 || (!groups && (reinterpret_cast<uintptr_t>(sc) & 15u) == 0);
@@ -460,6 +466,8 @@ static bool takes_small_tile(int M, int N, int K) {
 
 int gemm_i4g32_bf16_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N,
                              int K, hipStream_t st) {
+    const int rc = activations_ok(M, K);  // the limit of the 128 x 64 tile, whichever tile is picked
+    if (rc != 0) return rc;
     if (takes_small_tile(M, N, K)) return gemm_tile_small_i4g32_launch(x, wp, sc, y, M, N, K, st);
     const GemmTile t = pick_tile(M, N, K, true);
     if (t != TILE_128x64) return gemm_tile_i4g32_launch(x, wp, sc, y, M, N, K, t == TILE_256, st);
@@ -468,6 +476,8 @@ int gemm_i4g32_bf16_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_
 
 int gemm_i8row_bf16_dispatch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K,
                              hipStream_t st) {
+    const int rc = activations_ok(M, K);
+    if (rc != 0) return rc;
     if (takes_small_tile(M, N, K)) return gemm_tile_small_i8row_launch(x, w8, sc, y, M, N, K, st);
     const GemmTile t = pick_tile(M, N, K, false);
     if (t != TILE_128x64) return gemm_tile_i8row_launch(x, w8, sc, y, M, N, K, t == TILE_256, st);

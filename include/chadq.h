@@ -153,7 +153,7 @@ int chadq_gemv_i8row_fp32(const float *x, const int8_t *w8, const float *scale, 
 
 /*
  * y[m,n] = bf16_rne( sum_k x[m,k] * w[n,k] ), w as in chadq_dequant_i4g32 rounded to bf16
- * for the MFMA, fp32 accumulate.  x bf16 [M,K], y bf16 [M,N].  K % 32 == 0, any M >= 1.
+ * for the MFMA, fp32 accumulate.  x bf16 [M,K], y bf16 [M,N].  K % 32 == 0, any M >= 1 with M * K * 2 bytes of x below 4 GiB.
  */
 int chadq_gemm_i4g32_bf16(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, uint16_t *y_bf16,
                           int M, int N, int K, void *stream);

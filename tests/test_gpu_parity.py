@@ -464,6 +464,27 @@ def test_gemm_eight_wave_tiles_every_row_and_column(ops, weight, m, n, k):
         assert np.sqrt(err.sum(axis=axis) / (ref ** 2).sum(axis=axis)).max() <= TOL_BF16
 
 
+@pytest.mark.parametrize("n", [64, 128, 512])
+def test_gemm_refuses_4_gib_of_activations_for_every_tile(ops, n):
+    """One row below the limit is served and right in its last rows; at the limit the call is refused, whichever tile N picks."""
+    from chadslab_amd import QWeightInt4G32, QWeightInt8
+
+    m, k = 65536, 32768
+    r = rng(640 + n)
+    x = torch.zeros(m, k, dtype=torch.bfloat16, device=DEV)
+    xb = O.f32_to_bf16(r.standard_normal((3, k)).astype(np.float32))
+    x[-4:-1] = bf16_tensor(xb)
+    packed = r.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    s = r.lognormal(-5, 0.5, (n, k // 32)).astype(np.float16)
+    qw = QWeightInt4G32(torch.from_numpy(packed).to(DEV), torch.from_numpy(s).to(DEV))
+    with pytest.raises(ValueError, match="4 GiB"):
+        ops.qgemm(x, qw)
+    with pytest.raises(ValueError, match="4 GiB"):
+        ops.qgemm(x, QWeightInt8(torch.zeros(n, k, dtype=torch.int8, device=DEV), torch.ones(n, device=DEV)))
+    y = ops.qgemm(x[:-1], qw)
+    assert not bool(y[:-3].any()) and O.rel_l2(O.bf16_to_f32(bits(y[-3:])), O.qgemm_int4g32_f64(xb, packed, s)) <= TOL_BF16
+
+
 def test_gemm_int4_many_rows_full_k_and_integer_exact(ops):
     from chadslab_amd import QWeightInt4G32
 

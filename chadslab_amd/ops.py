@@ -164,9 +164,6 @@ def moe_route(logits: torch.Tensor, top_k: int = 2, renorm: bool = True):
     return idx, w
 
 
-_moe_ws = {}  # (device, stream, bytes) -> workspace tensor, reused between calls on that stream
-
-
 def _repack(w, to_tiles: bool):
     lib = _lib.load()
     p, s = _dev(w.packed, "packed", torch.uint8), _dev(w.scale, "scale", torch.float16)
@@ -222,14 +219,11 @@ def moe_ffn(x: torch.Tensor, logits: torch.Tensor, experts, *, top_k: int = 2, r
     need = lib.chadq_moe_ffn_i4g32_workspace_bytes(t, h, f, e, top_k)
     if need == 0:
         raise ValueError("unsupported MoE sizes T=%d H=%d F=%d E=%d top_k=%d" % (t, h, f, e, top_k))
-    # The workspace holds the router's output and every intermediate of the call, so two calls in flight at once must
-    # not share one: calls on one stream are ordered and reuse theirs, another stream gets its own.  A graph captured
-    # on a stream keeps using that stream's workspace on every replay: do not run eager calls of the same sizes on the
-    # capture stream while a replay is in flight.
-    key = (x.device, _stream(), need)
-    ws = _moe_ws.get(key)
-    if ws is None:
-        ws = _moe_ws[key] = torch.empty(need, dtype=torch.uint8, device=x.device)
+    # The workspace holds the router's output and every intermediate of the call.  A fresh one each time, from torch's
+    # allocator: calls in flight on other streams have their own, a later call on this stream may reuse the memory, a
+    # captured graph's stays with the graph, and none is kept for a number of tokens that does not come again (480 MiB
+    # at 512 tokens, top 4, 4096 x 14336).
+    ws = x.new_empty(need, dtype=torch.uint8)
     y = torch.empty(t, h, dtype=torch.bfloat16, device=x.device)
     fn = lib.chadq_moe_ffn_i4g32_tiled if tiled else lib.chadq_moe_ffn_i4g32
     _lib.check(fn(x.data_ptr(), z.data_ptr(), arr, y.data_ptr(), t, h, f, e, top_k, int(renorm), ws.data_ptr(), need, _stream()),

@@ -851,6 +851,19 @@ def test_moe_ffn_few_tokens_beside_an_outlier_of_zero_weight(ops, outlier):
         assert O.rel_l2(y, ref) <= 2.0 ** -8
 
 
+def test_moe_ffn_keeps_no_memory_per_size(ops):
+    """A server whose batch varies: what a call has used is free again when the next one of another size begins."""
+    _, dev = _experts(9900, 2, 256, 512)
+    r = rng(9901)
+    z = torch.from_numpy(r.standard_normal((80, 2)).astype(np.float32)).to(DEV)
+    x = bf16_tensor(O.f32_to_bf16(r.standard_normal((80, 256)).astype(np.float32)))
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    for t in range(1, 81):
+        ops.moe_ffn(x[:t], z[:t], dev, top_k=2)
+        assert torch.cuda.memory_allocated() == before, t
+
+
 def test_moe_ffn_tiled_wide_ranges_of_activations_and_scales(ops):
     """The tile-order kernels carry activations and dequantised weights as fp16: rows are scaled by a power of two first,
     so activations far outside fp16's range (and rows of very different magnitude side by side) must come out as the

@@ -367,7 +367,7 @@ class QuantDecoder:
         go through a layer at once (chadq_prompt_i4g32: every weight is read once per chunk instead of once per token, and
         only the last token meets the output table); else, and for sequences too short for that to pay (prompt_min()), the
         step runs token by token.  Raises ValueError if the sequence would run past max_ctx or holds a token outside the vocabulary."""
-        tokens = list(tokens)
+        tokens = [int(t) for t in tokens]
         self._check_range(pos, len(tokens), tokens)
         layers = self._describe_layers() if len(tokens) >= prompt_min(pos, self.cfg.dh) else None
         if layers is not None:

@@ -828,6 +828,20 @@ def test_decoder_feed_of_few_tokens_at_a_long_context_runs_the_step(monkeypatch,
     assert nxt == int(dec.token.item()) and torch.equal(dec.kcache[0], k)
 
 
+def test_decoder_feed_takes_whatever_int_takes():
+    """The tokens of a prompt may be any objects that int() converts, chunked or not."""
+    from fractions import Fraction
+
+    import chadslab_amd.decoder as D
+
+    cfg = D.DecoderConfig(n_layers=1, d=256, hq=4, dh=64, ffn=512, vocab=300, max_ctx=64)
+    dec = D.QuantDecoder(cfg, D.random_weights(cfg, 78, DEV), DEV)
+    want = dec.feed([3, 4, 5, 6], 0)
+    k = dec.kcache[0].clone()
+    for toks in (np.array([3, 4, 5, 6]), torch.tensor([3, 4, 5, 6], device=DEV), [np.array(3), 4, 5, 6], ["3", 4, Fraction(5), 6.0]):
+        assert dec.feed(toks, 0) == want and torch.equal(dec.kcache[0], k)
+
+
 def test_decoder_prompt_in_chunks_draws_what_single_tokens_would_have_drawn():
     import chadslab_amd.decoder as D
 

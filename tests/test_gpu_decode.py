@@ -842,6 +842,55 @@ def test_decoder_feed_takes_whatever_int_takes():
         assert dec.feed(toks, 0) == want and torch.equal(dec.kcache[0], k)
 
 
+def test_prompt_entry_point_refuses_what_it_cannot_serve(lib):
+    """chadq_prompt_i4g32 by itself: every rule of the header is checked on the host, with its own status and message, and a
+    refused call leaves caches and result alone."""
+    import ctypes
+
+    import chadslab_amd.decoder as D
+    from chadslab_amd import _lib
+
+    c = D.DecoderConfig(n_layers=2, d=256, hq=4, dh=64, ffn=512, vocab=300, max_ctx=64)
+    dec = D.QuantDecoder(c, D.random_weights(c, 81, DEV), DEV)
+    emb, ids = dec.w["emb"], torch.arange(8, dtype=torch.int32, device=DEV)
+    x = torch.full((c.d + 4,), 5.0, device=DEV)
+    need = lib.chadq_prompt_i4g32_workspace_bytes(8, c.d, c.hq, c.dh, c.ffn)
+    ws = torch.empty(need + 16, dtype=torch.uint8, device=DEV)
+    good = dict(layers=dec._describe_layers(), n_layers=2, tokens=ids.data_ptr(), emb=emb.packed.data_ptr(), semb=emb.scale.data_ptr(), V=300,
+                rope=dec.rope.data_ptr(), T=8, pos=0, d=256, hq=4, dh=64, ffn=512, max_ctx=64, eps=1e-6, x=x.data_ptr(), ws=ws.data_ptr(), bytes=need,
+                stream=stream())
+
+    def call(**change):
+        return lib.chadq_prompt_i4g32(*dict(good, **change).values())
+
+    def layer(name, value):
+        arr = (_lib.PromptLayerI4G32 * 2)()
+        ctypes.memmove(arr, good["layers"], ctypes.sizeof(arr))
+        setattr(arr[1], name, value)
+        return arr
+
+    SHAPE, NULL, ALIGN, WORKSPACE = -2, -1, -3, -4
+    for rc, message, change in [
+            (SHAPE, b"T=0", dict(T=0)), (SHAPE, b"n_layers=0", dict(n_layers=0)), (SHAPE, b"V=0", dict(V=0)), (SHAPE, b"d=128", dict(d=128)),
+            (SHAPE, b"d=2304", dict(d=2304)), (SHAPE, b"dh=32", dict(dh=32)), (SHAPE, b"hq=3", dict(hq=3)), (SHAPE, b"hq=0", dict(hq=0)),
+            (SHAPE, b"ffn=500", dict(ffn=500)), (SHAPE, b"-1..6", dict(pos=-1)), (SHAPE, b"57..64", dict(pos=57)),
+            (SHAPE, b"do not fit", dict(pos=2 ** 31 - 1)), (NULL, b"null", dict(layers=None)), (NULL, b"null", dict(tokens=None)),
+            (NULL, b"null", dict(emb=None)), (NULL, b"null", dict(semb=None)), (NULL, b"null", dict(rope=None)), (NULL, b"null", dict(x=None)),
+            (ALIGN, b"aligned", dict(emb=good["emb"] + 8)), (ALIGN, b"aligned", dict(x=good["x"] + 8)), (ALIGN, b"aligned", dict(ws=good["ws"] + 8)),
+            (WORKSPACE, b"workspace", dict(bytes=need - 1)), (WORKSPACE, b"workspace", dict(ws=None))]:
+        assert call(**change) == rc and message in lib.chadq_last_error(), (change, lib.chadq_last_error())
+    for name, _ in _lib.PromptLayerI4G32._fields_:
+        assert call(layers=layer(name, None)) == NULL and b"layer 1" in lib.chadq_last_error(), name
+        assert call(layers=layer(name, getattr(good["layers"][1], name) + 2)) == ALIGN and b"layer 1" in lib.chadq_last_error(), name
+    for sizes in ((0, 256, 4, 64, 512), (8, 2304, 4, 64, 512), (8, 256, 4, 32, 512), (8, 256, 3, 64, 512), (8, 256, 4, 64, 500)):
+        assert lib.chadq_prompt_i4g32_workspace_bytes(*sizes) == 0
+    torch.cuda.synchronize()
+    assert bool((x == 5).all()) and not any(bool(t.any()) for t in dec.kcache + dec.vcache)
+    assert call() == 0 and call(pos=56) == 0  # the last position that fits
+    torch.cuda.synchronize()
+    assert bool((x[:256] != 5).any()) and bool((x[256:] == 5).all()) and bool(dec.kcache[1][63 * 64:].any())
+
+
 def test_decoder_prompt_in_chunks_draws_what_single_tokens_would_have_drawn():
     import chadslab_amd.decoder as D
 

@@ -458,7 +458,11 @@ static GemmTile pick_tile(int M, int N, int K, bool int4) {
 // whose 64 x 64 tiles all run at once.  The larger tiles then leave compute units idle and each lasts longer.  us, that
 // tile against what pick_tile gives: int4 128 x 4096 x 4096 (128 tiles) 12.9 / 19.6, 256 x 4096 x 4096 (256 tiles)
 // 15.9 / 20.3, 256 x 1024 x 1024 5.5 / 9.0, 512 x 2048 x 14336 46 / 61, 1000 x 1024 x 4096 15.0 / 20.3; int8 200 x 4096 x
-// 4096 15.2 / 23.1.  With a second round it is the slower one: 384 x 4096 x 4096 (384 tiles) 27.4 / 22.2.
+// 4096 15.2 / 23.1.  With a second round it is the slower one: 384 x 4096 x 4096 (384 tiles) 27.4 / 22.2.  Up to 64 rows it
+// wins in any number of rounds, because the other tiles are padded to 128 rows there and every round of theirs carries the
+// same weights: 33 x 20000 x 2048 (313 tiles) 15.4 / 23.7, 64 x 20000 x 2048 16.1 / 24.4, 48 x 32768 x 4096 (512) 27.5 / 41.6,
+// 64 x 256000 x 2048 (4000) 151 / 299, 64 x 16384 x 16384 (256) 63 / 87; int8 64 x 20000 x 2048 15.6 / 25.0, 64 x 256000 x
+// 2048 161 / 235.  Few weight rows leave most of the chip idle on either tile: 48 x 512 x 16384 (8 tiles) 36.3 / 56.5.
 static bool takes_small_tile(int M, int N, int K) {
     const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
     return gemm_tile_q_ok(K) && (M <= 64 || tiles <= 256);

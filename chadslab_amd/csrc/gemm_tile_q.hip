@@ -10,6 +10,9 @@
 //                    256 activation rows.
 //   128 x 128 tile   four waves side by side, twice (WN = 4, WK = 2): the two halves of the workgroup take alternate
 //                    64-k blocks and meet in LDS at the end.  For grids that would leave the chip empty with the large one.
+//   64 x 64 tile     two waves side by side, four times (WN = 2, WK = 4); 32 x 64 for at most 32 rows.  For few rows and for
+//                    grids of one round (gemm_q_bf16.hip: takes_small_tile).
+//   exact weights    (HILO) 128, 64 or 32 rows x 128 weight rows, WN = 4, WK = 2, K possibly split over workgroups.
 //
 //   * A (activations): global -> LDS by DMA, three stages of 64 * WK k, read back as fragments one or two slices (16 k)
 //     ahead of their MFMAs.  16-byte pieces of a 128-byte row segment are XOR-swizzled by row / 2: LDS has 64 banks, two
@@ -493,10 +496,12 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
 
 // At most 64 rows, or few enough tiles for one round: 32 or 64 rows x 64 weight rows, the eight waves two side by side and
 // four along K (256 k per step).
-// What bounds it is the weight stream and the latency of a step: as many weight rows per workgroup as the 128 x 64 kernel
-// has (one round of the chip up to 16384 of them), but twice the waves, a quarter of the steps and no padding to 128 rows.
-// us (the 128 x 64 kernel in brackets): int4 48 x 14336 x 4096 14.8 (23.0), 17 x 4096 x 4096 9.5 (18.5), 64 x 4096 x 14336
-// 36 (53), 64 x 32768 x 4096 31 (44), 64 x 1024 x 1024 5.3 (8.3); int8 48 x 14336 x 4096 13.6 (22.5).
+// What bounds it is the operands' way into the compute unit: at 48 x 14336 x 4096 a workgroup pulls 393 KB of activations and
+// 147 KB of weights and scales, and these requests alone, nothing computed, take 10.1 of its 13.5 us in a queue of launches
+// (2.2 of them the launch; the weights alone 6.2).  As many weight rows per workgroup as the 128 x 64 kernel has (one
+// round of the chip up to 16384 of them), but twice the waves, a quarter of the steps and no padding to 128 rows.
+// us (the 128 x 64 kernel in brackets): int4 48 x 14336 x 4096 13.5 (21.0), 17 x 4096 x 4096 9.7 (18.1), 64 x 2048 x 14336
+// 36 (52), 64 x 32768 x 4096 28 (42), 64 x 1024 x 1024 5.5 (8.6); int8 48 x 14336 x 4096 13.6 (21.7).
 int gemm_tile_small_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, hipStream_t st) {
     const bool guard = K % 256 != 0 || !aligned16(sc);
     if (M <= 32)
@@ -521,7 +526,7 @@ static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc
 }
 
 // K splits that make the launch shortest: rounds of 256 workgroups times the k of each (and what a workgroup costs
-// besides, about 256 k worth).  At most kMaxSplits parts, each a multiple of 256 k.
+// besides, about 256 k worth).  At most kExactMaxSplits parts, each a multiple of 256 k.
 int gemm_exact_splits(int M, int N, int K) {
     const int bm = M <= 32 ? 32 : M <= 64 ? 64 : 128;
     const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + 127) / 128);

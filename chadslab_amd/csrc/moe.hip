@@ -5,10 +5,12 @@
 // Everything runs on the caller's stream without a host round trip: the router kernel also sorts the
 // (token, slot) pairs by expert (stable: by pair index inside an expert) and writes the per-expert descriptors
 // of the grouped GEMM launches and the list of token tiles that exist, so row counts never leave the GPU.
-// Gate/up/down of at most 16 tokens run on the weight-streaming kernel of moe_few_i4g32.hip; else on the skinny grouped kernel (gate and up fused with the SiLU gate and reading the activations
-// through the sorted token list, down split over K) when H and F are multiples of 256, else on the prefill
-// dequant-GEMM kernel in grouped mode on a gathered copy of the activations with a separate SiLU kernel; the small
-// kernels here are the router, the gather, the SiLU gate and the weighted combine.
+// Gate/up/down run on one of three kernels (moe_few_ok() and the alignment decide).  At most 16 tokens, in row order always,
+// in tile order if the experts hit are small: the weight-streaming kernel of moe_few_i4g32.hip.  Else, with H and F
+// multiples of 256: the grouped kernel of the weight order (gate and up fused with the SiLU gate and reading the activations
+// through the sorted token list, down split over K).  Else (row order only): the prefill dequant-GEMM kernel in grouped mode
+// on a gathered copy of the activations with a separate SiLU kernel.  The small kernels here are the router, the gather,
+// the SiLU gate and the weighted combine.
 #include "chadq_common.h"
 #include "expert_prep.h"
 

@@ -12,7 +12,8 @@
 //   * In row order a load takes whole 128-byte lines of 8 rows, not 64 bytes of 16 (gate/up 97 -> 87 us); two DPP moves
 //     per register pair put the halves in place.
 // Gate/up | down in us, 8 experts of 4096 x 14336, top 2, the skinny kernel in brackets: 4 tokens 87 | 50 (130 | 72),
-// 16 tokens 145 | 81 (191 | 85); 16 experts of 2048 x 4096, top 4, 16 tokens 46 | 27 (47 | 24); 1 token of 1024 x 2048
+// 16 tokens 145 | 81 (191 | 85); 16 experts of 2048 x 4096, top 4, 16 tokens 46 | 27 (47 | 24: the one shape found whose
+// down product is slower here; the whole call is the quicker one all the same, 84.6 against 88.5); 1 token of 1024 x 2048
 // 5.2 | 4.5 (12.8 | 7.0).
 // Arithmetic: v_mfma_f32_16x16x32_bf16 on unscaled weights.  A lane holds a whole scale group of its weight row (16
 // bytes); the lanes' words are exchanged (v_permlane16_swap, v_permlane32_swap) so that one MFMA holds one scale group;
@@ -273,10 +274,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
 }
 
-// T <= 16: no expert gets more than one tile of rows.  32-bit byte offsets into a matrix.  Row order: always (figures
-// above).  In tile order the many-row kernel streams large experts better (16 tokens, 8 experts of 4096 x 14336: 164 us
-// for the whole call against 195; 16 experts of 2048 x 4096, top 4: 67 against 77) but has a launch more and coarser
-// tiles, which is what a few small experts take (one token, top 2 of 1024 x 2048: 31 against 18): few bytes only.
+// T <= 16: no expert gets more than one tile of rows.  32-bit byte offsets into a matrix.  Row order: always (whole calls
+// of 1 to 16 tokens on thirteen expert layers, 7 to 1500 MB: 1.01 to 2.6 times as fast as on the many-row kernel).
+// In tile order the many-row kernel streams large experts better but has a launch more and coarser tiles, which is what few
+// bytes take.  Whole calls there, many-row / this kernel in us, by the experts' bytes hit (at most) and the tokens:
+//     7 MB  1 token  29.3 / 17.5    27 MB  1  40.8 / 24.2    27 MB 16  31.4 / 23.5    54 MB  1  49.8 / 31.1    54 MB  4  38.2 / 30.6
+//   108 MB  1 token  60.7 / 42.2   108 MB  2  50.7 / 36.5   108 MB  4  42.0 / 37.7   108 MB 16  43.5 / 44.3
+//   189 MB  1 token  76.2 / 63.1   216 MB  4  56.3 / 60.4   216 MB 16  65.2 / 75.6   378 MB 16  86.2 / 75.4   378 MB  1 103.8 / 107.7
+//   756 MB  4 tokens 116.7 / 120.3  756 MB 16 153.0 / 185.5  1512 MB 16 280 / 352
+// Up to 64 MB this kernel is ahead at every number of tokens; beyond 100 MB it depends on the tokens and the shape.
 bool moe_few_ok(int T, int H, int F, int E, int top_k, bool tiled) {
     if (T > FEW_ROWS || E > FEW_ENTRIES || H % 256 != 0 || F % 256 != 0 || (int64_t)H * F / 2 >= (int64_t)kRange) return false;
     const int64_t hit = T * top_k < E ? T * top_k : E;

@@ -366,7 +366,10 @@ class QuantDecoder:
         model proposes after the last one.  Where the prompt kernels cover the model's sizes, whole chunks of the sequence
         go through a layer at once (chadq_prompt_i4g32: every weight is read once per chunk instead of once per token, and
         only the last token meets the output table); else, and for sequences too short for that to pay (prompt_min()), the
-        step runs token by token.  Raises ValueError if the sequence would run past max_ctx or holds a token outside the vocabulary."""
+        step runs token by token.  Both round in the same places and take the weights exactly, but a product's sums over K are
+        added in an order that follows the number of tokens read together: the same tokens fed in one call or in several agree
+        within rounding, not bit for bit, and two nearly equal logits may change places.  Raises ValueError if the sequence
+        would run past max_ctx or holds a token outside the vocabulary."""
         tokens = [int(t) for t in tokens]
         self._check_range(pos, len(tokens), tokens)
         layers = self._describe_layers() if len(tokens) >= prompt_min(pos, self.cfg.dh) else None

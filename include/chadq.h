@@ -186,6 +186,8 @@ size_t chadq_moe_ffn_i4g32_workspace_bytes(int T, int H, int F, int E, int top_k
 
 /*
  * y[t] = bf16( sum_j w[t,j] * Wd_e ( bf16( silu(Wg_e x_t) * (Wu_e x_t) ) ) ),  e = idx[t,j] from chadq_moe_route.
+ * H and F multiples of 256 and 16-byte aligned arrays: at most 16 tokens take the weights exactly (an infinite activation
+ * then gives NaN); otherwise dequantised weights are rounded to bf16.
  * x bf16 [T,H], logits fp32 [T,E], y bf16 [T,H].  `experts` is a HOST array of E structs holding device pointers.
  * H % 32 == 0, F % 32 == 0.  Runs entirely on `stream`; no host synchronisation, nothing allocated.
  */
@@ -216,6 +218,8 @@ int chadq_unrepack_i4g32_tiles(const uint8_t *wp_tiles, const uint16_t *scale_ti
  * the matrix core as fp16(u * scale), the zero point as a separate exact term per scale group.  The results agree with
  * chadq_moe_ffn_i4g32 within rounding (they are the closer of the two to a float64 evaluation: fp16 keeps 3 more bits
  * of the dequantised weight than bf16), not bit for bit.  About 20 % faster at 256 tokens x 8 experts of 14336 x 4096.
+ * At most 16 tokens whose experts (top_k * T of them at most) hold at most 64 MB run on the kernel that chadq_moe_ffn_i4g32
+ * uses for them: the same bits, exact weights.
  * H % 256 == 0 and F % 256 == 0; scales must be below 64 in magnitude (1024 * scale has to be a finite fp16);
  * T * top_k * max(H, F) < 2^30.
  */

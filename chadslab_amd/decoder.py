@@ -351,15 +351,18 @@ class QuantDecoder:
         torch.cuda.synchronize()
         self.graph = g
 
-    def _check_range(self, pos: int, n: int, tokens=()) -> None:
-        """The kernels clamp a position to the cache and a token to the table so that nothing is addressed out of
-        bounds, but a clamped step is a wrong step (it overwrites the last cache row and rotates by the wrong angle):
-        refuse on the host what would run past the cache or name a token outside the vocabulary."""
+    def _check_range(self, pos: int, n: int, tokens=()) -> List[int]:
+        """The tokens as ints, once they and the positions are known to be in range.  The kernels clamp a position to the cache
+        and a token to the table so that nothing is addressed out of bounds, but a clamped step is a wrong step (it overwrites
+        the last cache row and rotates by the wrong angle): refuse on the host what would run past the cache or name a token
+        outside the vocabulary."""
         if pos < 0 or n < 0 or pos + n > self.cfg.max_ctx:
             raise ValueError("positions %d..%d do not fit the cache of %d rows" % (pos, pos + n - 1, self.cfg.max_ctx))
-        for t in tokens:
-            if not 0 <= int(t) < self.cfg.vocab:
-                raise ValueError("token %d is outside the vocabulary [0, %d)" % (int(t), self.cfg.vocab))
+        tokens = [t if type(t) is int else int(t) for t in tokens]
+        if tokens and (min(tokens) < 0 or max(tokens) >= self.cfg.vocab):
+            bad = next(t for t in tokens if not 0 <= t < self.cfg.vocab)
+            raise ValueError("token %d is outside the vocabulary [0, %d)" % (bad, self.cfg.vocab))
+        return tokens
 
     def feed(self, tokens, pos: int = 0) -> int:
         """Reads a given token sequence starting at position `pos` (a prompt) into the caches and returns the token the
@@ -370,14 +373,14 @@ class QuantDecoder:
         added in an order that follows the number of tokens read together: the same tokens fed in one call or in several agree
         within rounding, not bit for bit, and two nearly equal logits may change places.  Raises ValueError if the sequence
         would run past max_ctx or holds a token outside the vocabulary."""
-        tokens = [int(t) for t in tokens]
-        self._check_range(pos, len(tokens), tokens)
+        tokens = list(tokens)
+        tokens = self._check_range(pos, len(tokens), tokens)
         layers = self._describe_layers() if len(tokens) >= prompt_min(pos, self.cfg.dh) else None
         if layers is not None:
             return self._feed_chunks(layers, tokens, pos)
         self.pos.fill_(pos)
         for t in tokens:
-            self.token.fill_(int(t))  # overrides the token the previous step proposed
+            self.token.fill_(t)  # overrides the token the previous step proposed
             if self.sampling is not None:
                 self.u.uniform_(0.0, 1.0, generator=self.rng)
             if self.graph is not None and self.graph_steps == 1:

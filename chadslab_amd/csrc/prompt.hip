@@ -211,8 +211,8 @@ __global__ __launch_bounds__(256) void prompt_attn_kernel(const float *__restric
         const int p0 = b * 32;
         // Positions only some of the rows see in a block, one of them with a V row that is not finite: the others' probability 0
         // times it would be NaN.  (Packed maxima of the magnitudes, two instructions per word, of the words e that can hold
-        // such a position: with 8 heads there is one position, an eighth of the block, and the check does not show in the
-        // kernel's time; over whole blocks it was 0.8 us per layer.)
+        // such a position: with 8 heads there is one position, an eighth of the block.  It does not show in the time of a call:
+        // 256 tokens through 18 layers, 2881 us with and 2882 without.)
         bool apart = false;
         if (p0 + 32 > seen) {
             const int lo = max(seen - p0, 0), hi = min(nctx - p0, 32);

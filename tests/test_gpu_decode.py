@@ -805,6 +805,41 @@ def test_decoder_prompt_a_token_that_is_not_finite_reaches_no_earlier_token(t, b
             assert float((cb - ca).norm() / ca.norm()) <= (3e-4 if li == 0 else 5e-3 * li), (name, li)
 
 
+def test_decoder_prompt_an_infinite_v_row_reaches_no_earlier_token():
+    """One token has a feature no other token has, whose norm weight and value weights take its V row of the first layer to
+    infinity (q and k do not read the feature): finite cache rows exactly where the step has them, and the earlier tokens'
+    equal to the step's."""
+    import chadslab_amd.decoder as D
+
+    t, bad, feature, dh = 21, 13, 37, 128
+    cfg = D.DecoderConfig(n_layers=3, d=256, hq=2, dh=dh, ffn=512, vocab=500, max_ctx=64)
+    w = D.random_weights(cfg, 97, DEV)
+    byte, odd = feature // 2, feature % 2
+
+    def set_nibble(packed, rows, value):
+        col = packed[rows, byte]
+        packed[rows, byte] = (col & 0x0F) | (value << 4) if odd else (col & 0xF0) | value
+
+    toks = [8 + i for i in range(t)]
+    set_nibble(w["emb"].packed, slice(None), 8)
+    set_nibble(w["emb"].packed, toks[bad], 15)
+    L = w["layers"][0]
+    L["ln1"][feature] = 1e36
+    set_nibble(L["wqkv"].packed, slice(0, (cfg.hq + 1) * dh), 8)
+    L["wqkv"].scale[(cfg.hq + 1) * dh:, feature // 32] = 65504
+    a, b = D.QuantDecoder(cfg, w, DEV), D.QuantDecoder(cfg, w, DEV)
+    for i, tok in enumerate(toks):
+        a.set_state(tok, i)
+        a.step()
+    b.feed(toks, 0)
+    assert bool(torch.isinf(b.vcache[0][bad * dh:(bad + 1) * dh]).any())
+    for name in ("kcache", "vcache"):
+        for li, (ca, cb) in enumerate(zip(getattr(a, name), getattr(b, name))):
+            assert torch.equal(torch.isfinite(cb[:t * dh]), torch.isfinite(ca[:t * dh])), (name, li)
+            ca, cb = ca[:bad * dh].float(), cb[:bad * dh].float()
+            assert bool(torch.isfinite(cb).all()) and float((cb - ca).norm() / ca.norm()) <= (3e-4 if li == 0 else 5e-3 * li), (name, li)
+
+
 @pytest.mark.parametrize("dh,pos,few,enough", [(256, 0, 2, 3), (256, 4000, 4, 5), (256, 16000, 8, 9), (64, 0, 2, 3), (64, 16000, 3, 4)])
 def test_decoder_feed_of_few_tokens_at_a_long_context_runs_the_step(monkeypatch, dh, pos, few, enough):
     """The prompt kernels walk the whole context in a few workgroups: below the measured number of tokens the step, which

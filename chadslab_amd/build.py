@@ -68,7 +68,7 @@ def build(verbose: bool = True, save_temps: bool = False) -> Path:
 # construction; nothing but the bench loads them.  name -> (source file, macro definition)
 ABLATIONS = {"stream": ("gemm_expert_i4g32.hip", "-DCHADQ_EXPERT_ABLATE=1"),   # expert GEMM: memory traffic without arithmetic
              "arith": ("gemm_expert_i4g32.hip", "-DCHADQ_EXPERT_ABLATE=2"),    # expert GEMM: arithmetic without weight loads
-             "nodequant": ("gemm_q_bf16.hip", "-DCHADQ_GEMM_ABLATE=1")}        # prefill GEMM (128 x 64 tile): no dequantisation
+             "nodequant": ("gemm_tile_q.hip", "-DCHADQ_GEMM_ABLATE=1")}        # prefill GEMM: no dequantisation
 
 
 def ablation_path(name: str) -> Path:

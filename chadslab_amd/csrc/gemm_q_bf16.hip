@@ -24,10 +24,6 @@
 #include "chadq_common.h"
 #include "gemm_tile_q.h"
 
-#ifndef CHADQ_GEMM_ABLATE
-#define CHADQ_GEMM_ABLATE 0  // measurement builds only: 1 = the dequantisation compiled out (packed words go to the matrix core as they are)
-#endif
-
 namespace chadq {
 
 struct FmtI4G32 {
@@ -227,10 +223,7 @@ __global__ __launch_bounds__(256) void gemm_q_bf16_kernel(const uint16_t *__rest
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             const u32x4 q = cq[nb];
-            if constexpr (CHADQ_GEMM_ABLATE == 1) {
-                const u32x4 raw = {q.x + (uint32_t)t, q.y, q.z, q.w};
-                __builtin_memcpy(&bf[set][t][nb], &raw, 16);
-            } else if constexpr (i4) {
+            if constexpr (i4) {
                 const uint32_t wsel = t == 0 ? q.x : t == 1 ? q.y : t == 2 ? q.z : q.w;
                 bf[set][t][nb] = dequant8_i4(wsel, cs[nb][0], cs[nb][1], cs[nb][2], cs[nb][3], c_mlo, c_mhi, c_magic);
             } else {
@@ -436,45 +429,13 @@ static int launch_gemm(const uint16_t *x, const void *wq, const typename F::scal
     return launch_gemm_g<F, 2, false, OUTF32>(x, wq, sc, y, M, N, K, groups, ngroups, st);
 }
 
-// Which tile.  A tile alone on a compute unit takes about as long as one on each of them, so a launch lasts as many rounds
-// of 256 tiles as it has, the last one 1/2 + fill/2 of a full one (measured: 0.65 at a quarter, 0.7-0.75 at a half).  A
-// full round of the 128 x 64 tile of this file takes 24 us per 4096 k (int8: 28), one of the 128 x 128 tile of
-// gemm_tile_q.hip 38, one of its 256 x 256 tile 114: the larger the tile, the less is fetched and dequantised per
-// product.  The rule takes the shortest and was the right one at every shape tried, e.g. at 4096 columns and k:
-// 512 rows 24 us (128 x 128: 27), 1024 rows 38 (128 x 64: 47), 2048 rows 74 (256 x 256: 78), 4096 rows 113 (144).
-enum GemmTile { TILE_128x64, TILE_128, TILE_256 };
-static GemmTile pick_tile(int M, int N, int K, bool int4) {
-    auto cost = [&](int bm, int bn, double full) {
-        const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn), rounds = (tiles + 255) / 256;
-        const double fill = (double)(tiles - (rounds - 1) * 256) / 256.0;
-        return full * ((double)(rounds - 1) + 0.5 + 0.5 * fill);
-    };
-    const double c64 = cost(128, 64, int4 ? 24.0 : 28.0), c128 = cost(128, 128, 38.0), c256 = cost(256, 256, 114.0);
-    if (!gemm_tile_q_ok(K) || (c64 <= c128 && c64 <= c256)) return TILE_128x64;
-    return c128 <= c256 ? TILE_128 : TILE_256;
-}
-
-// Whether the 64 x 64 tile (32 x 64 for at most 32 rows) of gemm_tile_q.hip takes the product: up to 64 rows, or a launch
-// whose 64 x 64 tiles all run at once.  The larger tiles then leave compute units idle and each lasts longer.  us, that
-// tile against what pick_tile gives: int4 128 x 4096 x 4096 (128 tiles) 12.9 / 19.6, 256 x 4096 x 4096 (256 tiles)
-// 15.9 / 20.3, 256 x 1024 x 1024 5.5 / 9.0, 512 x 2048 x 14336 46 / 61, 1000 x 1024 x 4096 15.0 / 20.3; int8 200 x 4096 x
-// 4096 15.2 / 23.1.  With a second round it is the slower one: 384 x 4096 x 4096 (384 tiles) 27.4 / 22.2.  Up to 64 rows it
-// wins in any number of rounds, because the other tiles are padded to 128 rows there and every round of theirs carries the
-// same weights: 33 x 20000 x 2048 (313 tiles) 15.4 / 23.7, 64 x 20000 x 2048 16.1 / 24.4, 48 x 32768 x 4096 (512) 27.5 / 41.6,
-// 64 x 256000 x 2048 (4000) 151 / 299, 64 x 16384 x 16384 (256) 63 / 87; int8 64 x 20000 x 2048 15.6 / 25.0, 64 x 256000 x
-// 2048 161 / 235.  Few weight rows leave most of the chip idle on either tile: 48 x 512 x 16384 (8 tiles) 36.3 / 56.5.
-static bool takes_small_tile(int M, int N, int K) {
-    const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
-    return gemm_tile_q_ok(K) && (M <= 64 || tiles <= 256);
-}
-
+// Products go to the tiles of gemm_tile_q.hip.  The 128 x 64 kernel of this file is left the rows of 2^22 k and more, which exceed
+// those tiles' offsets, and the grouped launch below.
 int gemm_i4g32_bf16_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N,
                              int K, hipStream_t st) {
     const int rc = activations_ok(M, K);  // the limit of the 128 x 64 tile, whichever tile is picked
     if (rc != 0) return rc;
-    if (takes_small_tile(M, N, K)) return gemm_tile_small_i4g32_launch(x, wp, sc, y, M, N, K, st);
-    const GemmTile t = pick_tile(M, N, K, true);
-    if (t != TILE_128x64) return gemm_tile_i4g32_launch(x, wp, sc, y, M, N, K, t == TILE_256, st);
+    if (gemm_tile_q_ok(K)) return gemm_tile_i4g32_launch(x, wp, sc, y, M, N, K, gemm_tile_pick(M, N, K, true), st);
     return launch_gemm<FmtI4G32, false>(x, wp, sc, y, M, N, K, nullptr, 0, st);
 }
 
@@ -482,9 +443,7 @@ int gemm_i8row_bf16_dispatch(const uint16_t *x, const int8_t *w8, const float *s
                              hipStream_t st) {
     const int rc = activations_ok(M, K);
     if (rc != 0) return rc;
-    if (takes_small_tile(M, N, K)) return gemm_tile_small_i8row_launch(x, w8, sc, y, M, N, K, st);
-    const GemmTile t = pick_tile(M, N, K, false);
-    if (t != TILE_128x64) return gemm_tile_i8row_launch(x, w8, sc, y, M, N, K, t == TILE_256, st);
+    if (gemm_tile_q_ok(K)) return gemm_tile_i8row_launch(x, w8, sc, y, M, N, K, gemm_tile_pick(M, N, K, false), st);
     return launch_gemm<FmtI8Row, false>(x, w8, sc, y, M, N, K, nullptr, 0, st);
 }
 

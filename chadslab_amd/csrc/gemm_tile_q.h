@@ -8,12 +8,12 @@ enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_GEGLU = 2 };
 }
 
 bool gemm_tile_q_ok(int K);
-// y bf16 [M,N]; big: 256 x 256 tiles, else 128 x 128
-int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, bool big, hipStream_t st);
-int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, bool big, hipStream_t st);
-// the same in tiles of 32 (at most 32 rows) or 64 rows x 64
-int gemm_tile_small_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, hipStream_t st);
-int gemm_tile_small_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, hipStream_t st);
+enum GemmTile { TILE_32x64, TILE_64x64, TILE_96x64, TILE_128x64, TILE_96x128, TILE_128x128, TILE_192x128, TILE_256x128, TILE_256x256 };
+// the tile (activation rows x weight rows) that takes the product in the shortest time
+GemmTile gemm_tile_pick(int M, int N, int K, bool int4);
+// y bf16 [M,N]; gemm_tile_q_ok(K)
+int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st);
+int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st);
 // int4 weights taken exactly (nothing rounded before the fp32 sums); K % 256 == 0, x, wp and sc 16-byte aligned
 constexpr int kExactMaxSplits = 8;
 int gemm_exact_splits(int M, int N, int K);  // K splits to use for gemm_exact_f32_launch

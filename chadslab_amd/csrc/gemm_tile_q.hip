@@ -1,41 +1,53 @@
 // Dequant-GEMM for many activation rows:  y[m,n] = sum_k x[m,k] * w[n,k],  x bf16 [M,K], int4 group-32 or int8 per-row
 // weights, fp32 accumulation on v_mfma_f32_32x32x16_bf16.
 //
-// What bounds it: the matrix cores, at the clock the power of all the work leaves (1.8-1.9 GHz here, 2.4 idle), and the
-// work beside them.  One wave alone on a SIMD issues a vector instruction every eight cycles or so and stalls at every
-// wait; two hide up to six vector instructions behind each 32-cycle MFMA (measured).  Hence eight waves per workgroup,
-// two per SIMD, each with a column block of 32 weight rows and all activation rows of the tile:
+// A workgroup's WM x WN x WK waves share a tile; a wave sums MB x NB blocks of 32 x 32, so that every weight it dequantises meets
+// 32 * MB activation rows; the WK waves of one result take KW (64 or 32) of a step's k each and meet in LDS at the end.
 //
-//   256 x 256 tile   eight waves side by side (WN = 8), 128 accumulators each; every weight is dequantised once per
-//                    256 activation rows.
-//   128 x 128 tile   four waves side by side, twice (WN = 4, WK = 2): the two halves of the workgroup take alternate
-//                    64-k blocks and meet in LDS at the end.  For grids that would leave the chip empty with the large one.
-//   64 x 64 tile     two waves side by side, four times (WN = 2, WK = 4); 32 x 64 for at most 32 rows.  For few rows and for
-//                    grids of one round (gemm_q_bf16.hip: takes_small_tile).
-//   exact weights    (HILO) 128, 64 or 32 rows x 128 weight rows, WN = 4, WK = 2, K possibly split over workgroups.
+//   256 x 256        WN = 8, MB = 8: eight waves side by side (or, exact weights and fewer rows, see the end of the file)
+//   256, 192 x 128   WM = WN = WK = 2, MB = 4 or 3, NB = 2
+//   128 x 128        int4: WN = 4, WK = 2, MB = 4; int8: WN = 2, WK = 4, MB = 4, NB = 2.   96 x 128: the latter with MB = 3
+//   128, 96 x 64     WN = 2, WK = 4, MB = 4 or 3, 32 k per wave and step.   64, 32 x 64: MB = 2 or 1, 64 k
+//   exact weights    256, 128 x 128: WN = 4, WK = 2, MB = 8 or 4.  64, 32 x 64: WN = 2, WK = 4; K possibly split over workgroups
 //
-//   * A (activations): global -> LDS by DMA, three stages of 64 * WK k, read back as fragments one or two slices (16 k)
+//   * A (activations): global -> LDS by DMA, ST stages of a step each, read back as fragments one or two slices (16 k)
 //     ahead of their MFMAs.  16-byte pieces of a 128-byte row segment are XOR-swizzled by row / 2: LDS has 64 banks, two
-//     segments cover them, so the key changes every second row (588 B/ns per compute unit; keyed by the row itself, 294).
-//   * B (weights): the packed bytes take the same road; lane (n, kq) reads back 32 k of its row and dequantises them one
-//     slice ahead into the MFMA operand: 17 vector instructions per 8 weights (int4) or 12 (int8).
-//   * int4 scales: 16 bytes (8 groups = 256 k) per row by DMA into an area of the wave's own, or, where K is no multiple
-//     of 256, two bytes per lane and step.
+//     segments cover them, so the key changes every second row (600 B/ns per compute unit; keyed by the row itself, 300).
+//   * B (weights): the packed bytes take the same road, one step further ahead; a lane reads the k of its row for the next step at
+//     the beginning of this one and dequantises them one slice ahead into the MFMA operand: 17 vector instructions per 8
+//     weights (int4) or 12 (int8).  int4 scales travel with them, the 16 bytes (256 k) that hold the step's, or, where K is no
+//     multiple of 256, two bytes per lane.
 //   * One barrier per step, in front of the last slices, whose fragments are in registers by then.
+//
+// What bounds it.  Large products: the matrix cores at the clock the power of all the work leaves (1.8 GHz; the counters have the
+// 256 x 256 tile at 71 % of its cycles in MFMAs; fed zeros 4096^3 takes 84 us, with data 113).  One round or less of small tiles: the
+// order of a wave's own instructions.  A wave issues one every four cycles at best, two of them on a SIMD run in step because of the
+// barrier, and whatever stands between two MFMAs stops both.  Hence a loop body without a branch (every wave requests the same
+// number of pieces, surplus ones into a place nobody reads), the requests dealt out one behind each MFMA (forty in a row behind the
+// barrier: +3 us of 24 at 512 x 4096 x 4096), the packed weights a step ahead (their LDS latency stood in front of the
+// dequantisation), stages as constants in an unrolled loop.  128 x 4096 x 4096, one tile on a quarter of the chip: 20.9 -> 17.1 us.
+// The requests alone take 13.8 us of the 22 at 512 rows; starting each workgroup at another k (16.4 -> 13.8 for them) gives the
+// whole kernel nothing.
 // The order inside a slice is given to the compiler's scheduler: left alone it issues all MFMAs of a slice, then all of
-// the dequantisation, and the two waves of a SIMD, which the barrier keeps in step, do the same thing at the same time.
+// the dequantisation, and the two waves of a SIMD do the same thing at the same time.
 //
-// Measured (us; the one-wave-per-SIMD tile and the 128 x 64 kernel this replaced at these sizes in brackets):
-//   int4 4096 x 14336 x 4096: 409 (486)   4096^3: 113 (129)   1000 x 4096 x 14336: 116 (143)   256 x 14336 x 4096: 33 (44)
-//   int8 4096^3: 110 (191)   1000 x 4096 x 14336: 111 (160)   512 x 4096 x 4096: 26.5 (27.4)
-// (the vendor's GEMM on bf16 weights: 328, 87, 113, 40; 88, 112, 25).  Tried and not kept: waves of 128 x 64 (every weight
-// dequantised by two waves), four-wave workgroups of 128 x 256, two per compute unit (both 2-4 % slower), waves that
-// alternate between a phase of MFMAs and one of LDS reads and dequantisation, the two of a SIMD in opposite phases (the
-// same time: what is left is power, not order - fed zeros, the same kernel takes 95 us at 4096^3).
+// Measured (us; the same tiles with the requests behind the barrier, or the 128 x 64 kernel of gemm_q_bf16.hip, in brackets):
+//   int4 512 x 4096 x 4096 22.2 (23.7)   1000 x 4096 x 14336 112 (118)   48 x 14336 x 4096 14.5 (15.8)   968 x 3200 x 7552 55 (55)
+//   3318 x 1792 x 3328 44 (54)   265 x 12544 x 1536 20 (28)   4096^3 114 (116)   4096 x 14336 x 4096 425 (420)
+//   int8 512 x 4096 x 4096 21.4 (28.0)   1000 x 4096 x 14336 107 (115)   858 x 6656 x 13408 174 (202)   1800 x 1664 x 15360 85 (101)
+// (the vendor's GEMM on bf16 weights: 512 x 4096 x 4096 25, 1000 x 4096 x 14336 112, 4096^3 88, 4096 x 14336 x 4096 328).
+// Tried and not kept: NB = 2 for the 256 x 256 tile (half the fragment reads, twice the dequantisation: 117-118 us at 4096^3), four
+// waves of 256 x 64 with 512 registers (115 there, but 10 % slower in a round that is not full), 64 x 128 tiles (25 us at 512 rows),
+// four-wave workgroups for the 128-row tiles (the same time), a stage more (the same), a stage less (28 us).
 //
-// HILO: the dequantised weight is kept exactly, as the sum of two bf16 operands (a 4-bit integer times an fp16 scale has
-// at most 15 significant bits), for callers that must not round weights; twice the matrix work.
-// The MFMA k-slot of a lane is free as long as A and B agree: slot group kq of slice t holds k = 32 kq + 8 t .. +7.
+// EXACT: no weight is rounded, for callers whose sums must be those of the decode step.  The operands are the integers (u - 8) / 2^9;
+// the scale of a group of 32 k is applied to its sum, one fp32 FMA per value.  That work, not the matrix cores, bounds it: 64 FMAs
+// and 2 x 19 instructions of unpacking per 32 k and 128 rows x 32 columns of a wave, 8 MFMAs beside them.  (The form before kept a
+// weight as the sum of two bf16 operands: twice the matrix work and 37 instructions per 8 weights.)  us, that form in brackets:
+// gate/up of a 2048 x 16384 layer, 256 tokens 45.5 (63.7; in 128-row tiles 61), down 30 (36.8).  As long as its sums are finite for
+// all finite activations (32 x 8 < 2^9) it errs by 8 / 2^24 of a group's largest activation at most where the weight there is 0.
+// The MFMA k-slot of a lane is free as long as A and B agree: slot group kq of slice t holds k = (KW / 2) kq + 8 t .. +7
+// (EXACT: 16 t + 8 kq .. +7).
 #include <type_traits>
 
 #include "chadq_common.h"
@@ -44,25 +56,37 @@
 namespace chadq {
 namespace tileq {
 
-constexpr int kStages = 3;
+#ifndef CHADQ_GEMM_ABLATE
+#define CHADQ_GEMM_ABLATE 0  // measurement builds only: 1 = the dequantisation compiled out (packed words go to the matrix core as they are)
+#endif
 
-template <bool I4, int WN, int WK, int WMB, bool GUARD>
+// WM waves along the rows, WN along the columns, WK along k; MB x NB blocks of 32 x 32 per wave; KW k per wave and step; ST stages
+template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD>
 struct Cfg {
-    static constexpr int NW = WN * WK, T = 64 * NW;
-    static constexpr int BM = 32 * WMB, BN = 32 * WN, KS = 64 * WK;  // tile, k per step
-    static constexpr int BB = (I4 ? 32 : 64) * WK;                   // packed bytes of a weight row per step
-    static constexpr int A_STAGE = BM * 128 * WK, B_STAGE = BN * BB, STAGE = A_STAGE + B_STAGE;
-    static constexpr int A_DMA = A_STAGE / (NW * 1024), B_DMA = B_STAGE / (NW * 1024);  // instructions per wave and step
-    static_assert(A_DMA * NW * 1024 == A_STAGE && B_DMA * NW * 1024 == B_STAGE, "whole DMA instructions per wave");
-    static constexpr int S_OFF = kStages * STAGE;
-    // scales of a wave, two buffers: 256 k (32 rows x 16 B, fetched twice), or (GUARD) one step (64 lanes x 4 B)
-    static constexpr int S_BUF = !I4 ? 0 : GUARD ? 256 : 1024, S_WAVE = 2 * S_BUF;
-    static constexpr int SPB = 4 / WK;                               // steps per 256 k
-    static constexpr int EP_PITCH = BN * 2 + 16;                     // result tile in LDS: bf16 rows, padded
-    static constexpr int OPER = S_OFF + NW * S_WAVE, EPI = BM * EP_PITCH, RED = WK == 4 ? BM * BN * 16 : WK > 1 ? BM * BN * 4 : 0;
+    static constexpr int NW = WM * WN * WK, T = 64 * NW;
+    static constexpr int BM = 32 * MB * WM, BN = 32 * NB * WN, KS = KW * WK;  // tile, k per step
+    static constexpr int SL = KW / 16;                                        // slices of 16 k (one MFMA) per step
+    static constexpr int BB = (I4 ? KW / 2 : KW) * WK;                        // packed bytes of a weight row per step
+    static constexpr int A_STAGE = BM * KS * 2, B_STAGE = BN * BB;
+    // int4 scales of a step: the 16 bytes (256 k) of every column that hold it, or (GUARD) 4 bytes per lane and block of each wave
+    static constexpr int S_STAGE = !I4 ? 0 : GUARD ? 256 * NB * NW : BN * 16;
+    static constexpr int STAGE = A_STAGE + B_STAGE + S_STAGE;
+    // DMA instructions per step: A_DMA of each wave for the activations; the BI of the weights and the SI of the scales are dealt
+    // to the waves, as many to each (BS_DMA; what is left over fetches nothing, into a place nobody reads: every wave has the
+    // same number of requests in flight, so the waits and the loop need no branch)
+    static constexpr int A_DMA = A_STAGE / (NW * 1024), BI = B_STAGE / 1024, SI = GUARD ? 0 : S_STAGE / 1024;
+    static constexpr int BS_DMA = (BI + SI + NW - 1) / NW, G_DMA = I4 && GUARD ? NB : 0, REQ = A_DMA + BS_DMA + G_DMA;
+    static_assert(A_DMA * NW * 1024 == A_STAGE && BI * 1024 == B_STAGE, "whole DMA instructions");
+    static constexpr bool DUMP = (BI + SI) % NW != 0;
+    static constexpr int DUMP_OFF = ST * STAGE;
+    static constexpr int SPB = 256 / KS;                                      // steps per 256 k
+    static constexpr int EP_PITCH = BN * 2 + 16;                              // result tile in LDS: bf16 rows, padded
+    static constexpr int OPER = ST * STAGE + (DUMP ? 1024 : 0), EPI = BM * EP_PITCH;
+    static constexpr int RED = WK == 4 ? NW * MB * 4096 : WK == 2 ? WM * WN * MB * 4096 : 0;  // one column block at a time
     static constexpr int LDS0 = OPER > EPI ? OPER : EPI, LDS = LDS0 > RED ? LDS0 : RED;
-    static constexpr int AHEAD = WMB > 4 ? 1 : 2;  // slices between a fragment's request and its MFMAs (what the registers allow)
+    static constexpr int AHEAD = MB * NB > 4 || SL == 2 ? 1 : 2;  // slices between a fragment's request and its MFMAs (what the registers allow)
     static_assert(LDS <= 163840, "one workgroup per compute unit");
+    static_assert(ST >= 3 && ST <= 6, "the stages that the last steps know");
 };
 
 // The bare barrier instruction (__syncthreads() would also wait for every outstanding request); the empty asm statements
@@ -89,43 +113,39 @@ __device__ __forceinline__ bf16x8 dequant8_i8(uint32_t a, uint32_t b) {
     return o;
 }
 
-// dequant8_i4 with nothing rounded: hi = the value cut off after 16 bits, lo = the rest (at most 8 bits)
-__device__ __forceinline__ void dequant8_i4_exact(uint32_t w, const float (&cs)[4], uint32_t mlo, uint32_t mhi, uint32_t magic, bf16x8 &hi,
-                                                  bf16x8 &lo) {
-    const f16x2 h0 = as_f16x2(and_or(w, mlo, magic)), h1 = as_f16x2(and_or(w, mhi, magic));
-    const uint32_t w8 = w >> 8;
-    const f16x2 h2 = as_f16x2(and_or(w8, mlo, magic)), h3 = as_f16x2(and_or(w8, mhi, magic));
-    float f[8];
-    f[0] = __builtin_fmaf((float)h0.x, cs[0], cs[2]), f[4] = __builtin_fmaf((float)h0.y, cs[0], cs[2]);
-    f[1] = __builtin_fmaf((float)h1.x, cs[1], cs[3]), f[5] = __builtin_fmaf((float)h1.y, cs[1], cs[3]);
-    f[2] = __builtin_fmaf((float)h2.x, cs[0], cs[2]), f[6] = __builtin_fmaf((float)h2.y, cs[0], cs[2]);
-    f[3] = __builtin_fmaf((float)h3.x, cs[1], cs[3]), f[7] = __builtin_fmaf((float)h3.y, cs[1], cs[3]);
-    uint32_t h[4], l[4];
+// 8 nibbles -> 8 bf16 (u - 8) / 2^9 in k order, exact: |u - 8| in a byte of its own is the e4m3 number |u - 8| / 2^9 (its low eight
+// values are the subnormals, the others the next binade, with the same spacing), the sign goes above it.  19 instructions.
+__device__ __forceinline__ bf16x8 signed8_i4(uint32_t w) {
+    uint32_t b[2];  // bytes of u0 u2 u4 u6, of u1 u3 u5 u7
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const uint32_t u0 = __float_as_uint(f[2 * e]), u1 = __float_as_uint(f[2 * e + 1]);
-        h[e] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-        const float r0 = f[2 * e] - __uint_as_float(u0 & 0xFFFF0000u), r1 = f[2 * e + 1] - __uint_as_float(u1 & 0xFFFF0000u);
-        l[e] = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), 0x07060302u);
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t v = h ? w >> 4 : w, u = v & 0x0F0F0F0Fu, n = ~v & 0x08080808u, m = n >> 3;  // n: 8 where u < 8
+        b[h] = ((u ^ (0x08080808u - m)) + m) | (n << 4);                                           // u - 8, or 7 - u + 1 and the sign
     }
-    __builtin_memcpy(&hi, h, 16);
-    __builtin_memcpy(&lo, l, 16);
+    const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u), hi = __builtin_amdgcn_perm(b[1], b[0], 0x07030602u);
+    const u32x4 r = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.f, false)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.f, true)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, false)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, true))};
+    bf16x8 o;
+    __builtin_memcpy(&o, &r, 16);
+    return o;
 }
 
 // EPI (what becomes of the sums): EPI_BF16 y bf16 [M,N], times the row scale for int8; EPI_F32 y fp32 [gridDim.y][M,N],
 // part blockIdx.y holding the sum over its kspan k; EPI_GEGLU the weight rows come in pairs (gate, up) of a feature and
 // h = bf16(gelu_tanh(gate) * up) goes to y as bf16 [M, N/2].
-template <bool I4, int WN, int WK, int WMB, bool GUARD, bool HILO, int EPI>
-__global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_tile_q_kernel(
+template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT, int EPI>
+__global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WM * WN * WK / 4, WM * WN * WK / 4))) void gemm_tile_q_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wq, const void *__restrict__ scv, void *__restrict__ yv, int M, int N,
     int K, int kspan) {
-    typedef Cfg<I4, WN, WK, WMB, GUARD> C;
-    constexpr int BM = C::BM, BN = C::BN, BB = C::BB, AHEAD = C::AHEAD;
+    typedef Cfg<I4, WM, WN, WK, MB, NB, KW, ST, GUARD> C;
+    constexpr int BM = C::BM, BN = C::BN, BB = C::BB, AHEAD = C::AHEAD, SL = C::SL;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nl = lane & 31, kq = lane >> 5;
-    const int wk = wave / WN, wn = wave % WN;
+    const int wn = wave % WN, wm = wave / WN % WM, wk = wave / (WN * WM);
     // workgroup i runs on XCD i % 8: deal the tiles so that one XCD walks consecutive n-tiles of the same m-panel
     const int tiles_n = (N + BN - 1) / BN, tiles = tiles_n * ((M + BM - 1) / BM);
     const int per_xcd = (tiles + 7) / 8;
@@ -146,268 +166,428 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
     const __amdgpu_buffer_rsrc_t brsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(wq) + (size_t)n0 * wrow, 0, nrows * wrow, 0x00020000);
     constexpr uint32_t kOut = 0x80000000u;
-    uint32_t aoff[C::A_DMA], boff[C::B_DMA];
-    int apc[C::A_DMA], bpc[C::B_DMA];
+    const __amdgpu_buffer_rsrc_t srsrc = __builtin_amdgcn_make_buffer_rsrc(
+        I4 ? const_cast<uint16_t *>(reinterpret_cast<const uint16_t *>(scv)) + (size_t)n0 * G : nullptr, 0, I4 ? nrows * G * 2 : 0, 0x00020000);
+    uint32_t aoff[C::A_DMA], boff[C::BS_DMA];
+    int apc[C::A_DMA], bpc[C::BS_DMA];
     constexpr int BPR = BB / 16;  // 16-byte pieces per weight row and step
-    // WK = 4: a row's 128 or 256 bytes span half or all of the banks, so its pieces are XOR-swizzled by the row as A's are
-    auto bkey = [](int r) { return WK < 4 ? 0 : BPR == 8 ? (r >> 1) & 7 : r & 15; };
+    // WK = 4: a row's 64 to 256 bytes span a quarter to all of the banks, so its pieces are XOR-swizzled by the row as A's are
+    auto bkey = [](int r) { return WK < 4 ? 0 : BPR == 4 ? (r >> 2) & 3 : BPR == 8 ? (r >> 1) & 7 : r & 15; };
 #pragma unroll
-    for (int q = 0; q < C::A_DMA; ++q) {  // 8 row segments of 128 B per instruction, [k half][row][128 B]
+    for (int q = 0; q < C::A_DMA; ++q) {  // 8 row segments of 128 B per instruction, [64 k][row][128 B]
         const int e = (q * C::NW + wave) * 8 + (lane >> 3), r = e % BM;
         apc[q] = e / BM * 128 + 16 * ((lane & 7) ^ ((r >> 1) & 7));
         aoff[q] = r < mrows ? (uint32_t)r * (uint32_t)(K * 2) + (uint32_t)apc[q] : kOut;
     }
 #pragma unroll
-    for (int q = 0; q < C::B_DMA; ++q) {  // 64 / BPR rows per instruction
-        const int r = (q * C::NW + wave) * (64 / BPR) + lane / BPR;
+    for (int q = 0; q < C::BS_DMA; ++q) {  // 64 / BPR weight rows, or the scales of 64, per instruction
+        const int e = q * C::NW + wave, r = e * (64 / BPR) + lane / BPR, c = (e - C::BI) * 64 + lane;
         bpc[q] = 16 * ((lane % BPR) ^ bkey(r));
-        boff[q] = r < nrows ? (uint32_t)r * (uint32_t)wrow + (uint32_t)bpc[q] : kOut;
+        if (e < C::BI) boff[q] = r < nrows ? (uint32_t)r * (uint32_t)wrow + (uint32_t)bpc[q] : kOut;
+        else boff[q] = e < C::BI + C::SI && c < nrows ? (uint32_t)c * (uint32_t)(G * 2) : kOut;
     }
-    const uint16_t *srow = nullptr;
-    if constexpr (I4) {
-        const int n = n0 + wn * 32 + nl;
-        srow = reinterpret_cast<const uint16_t *>(scv) + (size_t)(n < N ? n : N - 1) * G + (kbeg >> 5);
+    const uint16_t *srow[NB];  // GUARD: the scale rows of the lane's columns
+    if constexpr (I4 && GUARD) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const int n = n0 + (wn * NB + nb) * 32 + nl;
+            srow[nb] = reinterpret_cast<const uint16_t *>(scv) + (size_t)(n < N ? n : N - 1) * G + (kbeg >> 5);
+        }
     }
-    uint8_t *const slds = lds + C::S_OFF + wave * C::S_WAVE;
 
     auto dma = [&](const __amdgpu_buffer_rsrc_t &rsrc, uint32_t voff, int soff, uint8_t *dst) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)dst, 16, voff, soff, 0, 0);
     };
-    // GUARD: a piece past the end of its row is not fetched (zeros); whole pieces: K % 32 == 0 (int4), K % 16 == 0 (int8)
-    auto issue_a = [&](int step, int q0, int q1, uint8_t *stage) {
-#pragma unroll
-        for (int q = 0; q < C::A_DMA; ++q)
-            if (q >= q0 && q < q1) {
-                const int soff = kbeg * 2 + step * (2 * C::KS);
-                dma(arsrc, GUARD && soff + apc[q] >= K * 2 ? kOut : aoff[q], soff, stage + (q * C::NW + wave) * 1024);
-            }
+    // GUARD: a piece past the end of its row is not fetched (zeros); whole pieces: K % 32 == 0 (int4), K % 16 == 0 (int8).
+    // `whole`: the step is not the last one, so there is none.
+    auto issue_a = [&](int q, int step, uint8_t *stage, bool whole) {
+        const int soff = kbeg * 2 + step * (2 * C::KS);
+        dma(arsrc, GUARD && !whole && soff + apc[q] >= K * 2 ? kOut : aoff[q], soff, stage + (q * C::NW + wave) * 1024);
     };
-    auto issue_b = [&](int step, uint8_t *stage) {
-#pragma unroll
-        for (int q = 0; q < C::B_DMA; ++q) {
-            const int soff = (I4 ? kbeg >> 1 : kbeg) + step * BB;
-            dma(brsrc, GUARD && soff + bpc[q] >= wrow ? kOut : boff[q], soff, stage + C::A_STAGE + (q * C::NW + wave) * 1024);
+    auto issue_b = [&](int q, int step, uint8_t *stage, bool whole) {
+        const int boffs = (I4 ? kbeg >> 1 : kbeg) + step * BB, soffs = (kbeg >> 4) + step / C::SPB * 16;
+        const int e = q * C::NW + wave;
+        if (q >= C::BS_DMA) {  // GUARD, int4: scales
+            const int nb = q - C::BS_DMA, g = KW == 64 ? 2 * (step * WK + wk) + kq : step * WK + wk;
+            dma2_to_lds(srow[nb] + (g < G ? g : 0), stage + C::A_STAGE + C::B_STAGE + (wave * NB + nb) * 256);
+        } else if ((q + 1) * C::NW <= C::BI) {
+            dma(brsrc, GUARD && !whole && boffs + bpc[q] >= wrow ? kOut : boff[q], boffs, stage + C::A_STAGE + e * 1024);
+        } else {
+            const bool isb = e < C::BI, none = C::DUMP && e >= C::BI + C::SI;
+            const __amdgpu_buffer_rsrc_t rs = q * C::NW >= C::BI ? srsrc : isb ? brsrc : srsrc;
+            dma(rs, GUARD && !whole && isb && boffs + bpc[q] >= wrow ? kOut : boff[q], isb ? boffs : soffs,
+                none ? lds + C::DUMP_OFF : stage + C::A_STAGE + e * 1024);
         }
     };
-    auto issue_s = [&](int blk) {  // blk: 256-k block, or (GUARD) step
-        if constexpr (I4 && GUARD) {
-            const int g = 2 * (blk * WK + wk) + kq;
-            dma2_to_lds(srow + (g < G ? g : 0), slds + (blk & 1) * C::S_BUF);
-        } else if constexpr (I4) {
-            dma16_to_lds(srow + blk * 8, slds + (blk & 1) * C::S_BUF);
-        }
+    // The requests of a step: the weights and scales of step j+1 (the last step has none: its own once more, read by nobody), the
+    // activations of step j
+    auto request = [&](int r, int j, uint8_t *stage_b, uint8_t *stage_a, bool whole) {
+        if (r < C::REQ - C::A_DMA) issue_b(r, whole || j + 1 < steps ? j + 1 : j, stage_b, whole);
+        else issue_a(r - (C::REQ - C::A_DMA), j, stage_a, whole);
     };
 
-    // ---- fragment read offsets: row nl of a 32-row block, piece 4 kq + t; the lane's packed weights
-    uint32_t foff[4];
+    // ---- fragment read offsets: row nl of a 32-row block, the wave's pieces SL kq + t (EXACT: 2 t + kq, so that two slices are one
+    // scale group); the lane's packed weights
+    static_assert(!EXACT || (I4 && !GUARD && NB == 1), "exact weights: int4, whole blocks of 256 k, one column block");
+    uint32_t foff[SL];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) foff[t] = (uint32_t)(wk * BM * 128 + nl * 128 + (((4 * kq + t) ^ ((nl >> 1) & 7)) << 4));
-    constexpr int BQ = I4 ? 1 : 2;  // 16-byte pieces of a lane's 32 k
+    for (int t = 0; t < SL; ++t)
+        foff[t] = (uint32_t)(wk * KW / 64 * BM * 128 + (wm * MB * 32 + nl) * 128 +
+                             (((wk * KW % 64 / 8 + (EXACT ? 2 * t + kq : SL * kq + t)) ^ ((nl >> 1) & 7)) << 4));
+    constexpr int LB = I4 ? KW / 4 : KW / 2, BQ = EXACT ? KW / 32 : LB > 16 ? LB / 16 : 1;  // bytes of a lane's k, 16-byte pieces of them
     uint32_t woff[BQ];
 #pragma unroll
-    for (int e = 0; e < BQ; ++e) woff[e] = (uint32_t)(C::A_STAGE + (wn * 32 + nl) * BB + 16 * (((2 * wk + kq) * BQ + e) ^ bkey(wn * 32 + nl)));
+    for (int e = 0; e < BQ; ++e) {  // (a block of 32 rows further on has the same key)
+        const int b = (2 * wk + (EXACT ? 0 : kq)) * LB + 16 * e, r = wn * 32 * NB + nl;
+        woff[e] = (uint32_t)(C::A_STAGE + r * BB + 16 * (b / 16 ^ bkey(r)) + b % 16);
+    }
 
     const uint32_t c_mlo = vgpr_const(0x000F000Fu), c_mhi = vgpr_const(0x00F000F0u), c_magic = vgpr_const(0x64006400u);
 
-    f32x16 acc[WMB];
+    f32x16 acc[MB][NB];
 #pragma unroll
-    for (int a = 0; a < WMB; ++a)
+    for (int a = 0; a < MB; ++a)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[a][v] = 0.f;
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
 
-    u32x4 bq[BQ];  // the lane's packed weights of a step: 32 k
-    uint16_t sraw = 0;
-    float cs[4];
+    // Requests are spread over the MFMAs of a step, from the barrier on.  (A compute unit takes one in
+    // 16 cycles; forty of them behind a barrier keep every wave from its next MFMA for as long as a step should take.)
+    constexpr int NE = MB * NB, BAR = SL - AHEAD;          // MFMAs of a slice; the slice in front of which the barrier stands
+    constexpr int GR = KW / 32, Q = GR * MB, LOOK = 2;     // EXACT: scale groups of a step, pairs of MFMAs, pairs from the barrier on
+    static_assert(!EXACT || (Q >= LOOK && Q % 2 == 0), "the pairs behind the barrier are of the same step; two sums in turn");
+    constexpr bool UNROLL = !EXACT || MB > 2;
+    constexpr int NP = EXACT ? Q : SL * NE, AFTER = EXACT ? LOOK : AHEAD * NE;  // positions of a step, those behind its barrier
+    auto first = [](int p) { return (p * C::REQ + NP - 1) / NP; };  // the first request at position p or later
+
+    using T = std::true_type;
+    using F = std::false_type;
+    // ---- prologue
+#pragma unroll
+    for (int r = 0; r < C::REQ - C::A_DMA; ++r) issue_b(r, 0, lds, false);
+#pragma unroll
+    for (int j = 0; j < ST - 1; ++j)
+        if (j < steps)
+#pragma unroll
+            for (int r = 0; r < C::REQ; ++r) request(r, j, lds + (j + 1) * C::STAGE, lds + j * C::STAGE, false);
+    if (steps >= ST - 1) wait_vmcnt<(ST - 2) * C::REQ>();  // the activations of step 0, the weights of steps 0 and 1
+    else wait_vmcnt<0>();
+    wg_barrier();
+    auto run = [&](auto &step) {
+        // (stages as constants in the loop: their addresses cost nothing there; not worth the code for few rows, whose workgroups
+        // take a few steps each)
+        int i = 0;
+        for (; UNROLL && i + 2 * ST + 1 < steps; i += ST) {
+#pragma unroll
+            for (int u = 0; u < ST; ++u) step(i + u, u, std::integral_constant<int, ST - 2>{}, T{}, T{}, T{});
+        }
+        int slot = 0;
+        auto next = [&]() {
+            ++i;
+            slot = slot + 1 == ST ? 0 : slot + 1;
+        };
+        for (; i + ST < steps; next()) step(i, slot, std::integral_constant<int, ST - 2>{}, T{}, T{}, F{});
+        if (ST <= steps) step(i, slot, std::integral_constant<int, ST - 2>{}, T{}, F{}, F{}), next();
+        if (ST >= 6 && i + 4 < steps) step(i, slot, std::integral_constant<int, 3>{}, F{}, F{}, F{}), next();
+        if (ST >= 5 && i + 3 < steps) step(i, slot, std::integral_constant<int, 2>{}, F{}, F{}, F{}), next();
+        if (ST >= 4 && i + 2 < steps) step(i, slot, std::integral_constant<int, 1>{}, F{}, F{}, F{}), next();
+        if (i + 1 < steps) step(i, slot, std::integral_constant<int, 0>{}, F{}, F{}, F{}), next();
+        step(i, slot, std::integral_constant<int, -1>{}, F{}, F{}, F{});
+    };
+
+    if constexpr (EXACT) {
+    // Exact weights: integers (u - 8) / 2^9 as operands, two MFMAs from zero on per scale group and row block, and one fp32 FMA per
+    // value that applies the scale (times 2^9).  A pair of MFMAs runs beside the FMAs of the pair before it.
+    constexpr int RING = Q >= 4 ? 4 : 2;
+    uint32_t wv[GR][2], wnx[GR][2];  // the lane's packed words of a step [group][slice], of the next one
+    uint32_t sraw;                   // its scales
+    float sc2[GR], s_last = 0.f;     // ... as floats, that of the group whose sums are next
     auto fetch = [&](int step, const uint8_t *stage) {
 #pragma unroll
-        for (int e = 0; e < BQ; ++e) bq[e] = *reinterpret_cast<const u32x4 *>(stage + woff[e]);
-        if constexpr (I4) {
-            if (GUARD) sraw = *reinterpret_cast<const uint16_t *>(slds + (step & 1) * C::S_BUF + lane * 4);
-            else sraw = *reinterpret_cast<const uint16_t *>(slds + (step / C::SPB & 1) * C::S_BUF + nl * 16 + (((step * WK + wk) & 3) * 2 + kq) * 2);
-        }
-    };
-    auto prep = [&](int step) {  // scale -> FMA constants; int4 weights past the row's end read as u = 0 and get the scale 0
-        if constexpr (I4) {
-            const float s = (GUARD && kbeg + step * C::KS + wk * 64 + kq * 32 >= K) ? 0.f : f16_bits_to_f32(sraw);
-            cs[0] = s;
-            cs[1] = s * 0.0625f;
-            cs[2] = -1032.f * s;
-            cs[3] = -72.f * s;
-        }
-    };
-    bf16x8 bf[2], bl[2];
-    auto deq = [&](int t) {
-        if constexpr (I4 && HILO) dequant8_i4_exact(bq[0][t], cs, c_mlo, c_mhi, c_magic, bf[t & 1], bl[t & 1]);
-        else if constexpr (I4) bf[t & 1] = dequant8_i4(bq[0][t], cs[0], cs[1], cs[2], cs[3], c_mlo, c_mhi, c_magic);
-        else bf[t & 1] = dequant8_i8(bq[t >> 1][2 * (t & 1)], bq[t >> 1][2 * (t & 1) + 1]);
-    };
-    bf16x8 af[2 * AHEAD][WMB];
-    auto frags = [&](int t, const uint8_t *stage) {
+        for (int g = 0; g < GR; ++g)
 #pragma unroll
-        for (int mb = 0; mb < WMB; ++mb) af[t % (2 * AHEAD)][mb] = *reinterpret_cast<const bf16x8 *>(stage + mb * 4096 + foff[t]);
+            for (int e = 0; e < 2; ++e) wnx[g][e] = *reinterpret_cast<const uint32_t *>(stage + woff[g] + e * 8 + kq * 4);
+        const uint8_t *const sp = stage + C::A_STAGE + C::B_STAGE + (wn * 32 + nl) * 16;
+        if (GR == 2) sraw = *reinterpret_cast<const uint32_t *>(sp + ((step * WK + wk) & 3) * 4);
+        else sraw = *reinterpret_cast<const uint16_t *>(sp + ((step * WK + wk) & 7) * 2);
+    };
+    auto prep = [&]() {
+#pragma unroll
+        for (int g = 0; g < GR; ++g) {
+            wv[g][0] = wnx[g][0];
+            wv[g][1] = wnx[g][1];
+            sc2[g] = 512.f * f16_bits_to_f32((uint16_t)(sraw >> (16 * g)));
+        }
+    };
+    bf16x8 bo[2], bnx[2];  // operands of the present group, of the next one
+    bf16x8 af[RING][2];
+    auto frag = [&](int q, const uint8_t *stage) {  // of pair q: group q / MB, row block q % MB
+#pragma unroll
+        for (int e = 0; e < 2; ++e) af[q % RING][e] = *reinterpret_cast<const bf16x8 *>(stage + (q % MB) * 4096 + foff[2 * (q / MB) + e]);
+    };
+    f32x16 tmp[2];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) tmp[1][v] = 0.f;
+
+    fetch(0, lds);
+#pragma unroll
+    for (int q = 0; q < LOOK; ++q) frag(q, lds);
+    if (ST <= steps) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        wg_barrier();                        // step 0's weights have been read
+#pragma unroll
+        for (int r = 0; r < first(AFTER); ++r) request(r, ST - 1, lds, lds + (ST - 1) * C::STAGE, false);
+    }
+    prep();
+    bo[0] = signed8_i4(wv[0][0]);
+    bo[1] = signed8_i4(wv[0][1]);
+    auto step = [&](int i, int slot, auto pending_c, auto before_c, auto more_c, auto whole_c) {
+        constexpr bool whole = decltype(whole_c)::value, before = decltype(before_c)::value, more = decltype(more_c)::value;  // as below
+        constexpr int pending = decltype(pending_c)::value;
+        uint8_t *const cur = lds + slot * C::STAGE, *const nxt = lds + (slot + 1 == ST ? 0 : slot + 1) * C::STAGE;
+        uint8_t *const prv = lds + (slot == 0 ? ST - 1 : slot - 1) * C::STAGE;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int g = q / MB, mb = q % MB;
+            if (q == 0 && pending >= 0) fetch(i + 1, nxt);  // (in front of the barrier also where that is the first thing: MB = 1)
+            if (q == Q - LOOK && pending >= 0) {
+                wait_vmcnt<(pending > 0 ? pending * C::REQ : 0)>();
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+                wg_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const int p = q < Q - LOOK ? q + LOOK : q - (Q - LOOK);
+#pragma unroll
+            for (int r = first(p); r < first(p + 1); ++r) {
+                if (before && q < Q - LOOK) request(r, i + ST - 1, cur, prv, whole);
+                if (more && q >= Q - LOOK) request(r, i + ST, nxt, cur, whole);
+            }
+            f32x16 zero;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) zero[v] = 0.f;
+            tmp[q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[q % RING][0], bo[0], zero, 0, 0, 0);
+            tmp[q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[q % RING][1], bo[1], tmp[q & 1], 0, 0, 0);
+            if (q < Q - LOOK) frag(q + LOOK, cur);
+            else if (pending >= 0) frag(q - (Q - LOOK), nxt);
+            f32x16 &a = acc[(mb + MB - 1) % MB][0];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) a[v] = __builtin_fmaf(tmp[(q + 1) & 1][v], s_last, a[v]);
+            if (mb == 0) s_last = sc2[g];
+            // the next group's operands, a share beside each pair
+            if (g + 1 < GR || pending >= 0) {
+                if (g + 1 == GR && mb == (GR == 1 && MB > 2 ? 2 : 0)) prep();
+                if (mb == MB / 2 - (MB > 1)) bnx[0] = signed8_i4(wv[(g + 1) % GR][0]);
+                if (mb == MB - 1) bnx[1] = signed8_i4(wv[(g + 1) % GR][1]);
+            }
+            if (mb == MB - 1) {
+                bo[0] = bnx[0];
+                bo[1] = bnx[1];
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 5, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 60, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    run(step);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[MB - 1][0][v] = __builtin_fmaf(tmp[(Q - 1) & 1][v], s_last, acc[MB - 1][0][v]);
+    } else {
+    u32x4 bq[NB][BQ], bn[NB][BQ];  // the lane's packed weights of a step (int4 and 32 k: half of one), of the next one
+    uint16_t sraw[NB];
+    float cs[NB][4];
+    auto fetch = [&](int step, const uint8_t *stage) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+            for (int e = 0; e < BQ; ++e) {
+                const uint8_t *const p = stage + woff[e] + nb * 32 * BB;
+                if constexpr (LB == 8) {
+                    const u32x2 v = *reinterpret_cast<const u32x2 *>(p);
+                    bn[nb][e] = u32x4{v.x, v.y, 0u, 0u};
+                } else {
+                    bn[nb][e] = *reinterpret_cast<const u32x4 *>(p);
+                }
+            }
+                const uint8_t *const sp = stage + C::A_STAGE + C::B_STAGE;
+            if constexpr (I4 && GUARD) sraw[nb] = *reinterpret_cast<const uint16_t *>(sp + (wave * NB + nb) * 256 + lane * 4);
+            else if constexpr (I4)
+                sraw[nb] = *reinterpret_cast<const uint16_t *>(sp + ((wn * NB + nb) * 32 + nl) * 16 +
+                                                               (KW == 64 ? ((step * WK + wk) & 3) * 2 + kq : (step * WK + wk) & 7) * 2);
+        }
+    };
+    auto prep = [&](int step) {  // the fetched ones' turn; scale -> FMA constants; int4 weights past the row's end read as u = 0 and get the scale 0
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int e = 0; e < BQ; ++e) bq[nb][e] = bn[nb][e];
+        if constexpr (I4) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                const float s = (GUARD && kbeg + step * C::KS + wk * KW + kq * (KW / 2) >= K) ? 0.f : f16_bits_to_f32(sraw[nb]);
+                cs[nb][0] = s;
+                cs[nb][1] = s * 0.0625f;
+                cs[nb][2] = -1032.f * s;
+                cs[nb][3] = -72.f * s;
+            }
+        }
+    };
+    bf16x8 bf[2][NB];
+    auto deq = [&](int t) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            if constexpr (CHADQ_GEMM_ABLATE == 1) {
+                const u32x4 q = bq[nb][(I4 ? 0 : t >> 1) % BQ], raw = {q.x + (uint32_t)t, q.y, q.z, q.w};
+                __builtin_memcpy(&bf[t & 1][nb], &raw, 16);
+            } else if constexpr (I4) bf[t & 1][nb] = dequant8_i4(bq[nb][0][t], cs[nb][0], cs[nb][1], cs[nb][2], cs[nb][3], c_mlo, c_mhi, c_magic);
+            else bf[t & 1][nb] = dequant8_i8(bq[nb][t >> 1][2 * (t & 1)], bq[nb][t >> 1][2 * (t & 1) + 1]);
+        }
+    };
+    bf16x8 af[2 * AHEAD][MB];
+    auto frag = [&](int t, int mb, const uint8_t *stage) {
+        af[t % (2 * AHEAD)][mb] = *reinterpret_cast<const bf16x8 *>(stage + mb * 4096 + foff[t]);
     };
 
-    // ---- prologue: two stages and the scales they need
-    uint8_t *cur = lds, *nxt = lds + C::STAGE, *far = lds + 2 * C::STAGE;
-    issue_s(0);
-    if (GUARD || C::SPB == 1 ? steps > 1 : C::SPB == 2 && steps > 2) issue_s(1);
-    issue_b(0, cur);
-    issue_a(0, 0, C::A_DMA, cur);
-    if (steps > 1) {
-        issue_b(1, nxt);
-        issue_a(1, 0, C::A_DMA, nxt);
-        wait_vmcnt<C::A_DMA + C::B_DMA>();  // everything of step 0
-    } else {
-        wait_vmcnt<0>();
+    fetch(0, lds);
+#pragma unroll
+    for (int t = 0; t < AHEAD; ++t)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) frag(t, mb, lds);
+    if (ST <= steps) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        wg_barrier();                        // step 0's weights have been read
+#pragma unroll
+        for (int r = 0; r < first(AFTER); ++r) request(r, ST - 1, lds, lds + (ST - 1) * C::STAGE, false);
     }
-    wg_barrier();
-    fetch(0, cur);
-    frags(0, cur);
-    if (AHEAD == 2) frags(1, cur);
     prep(0);
     deq(0);
 
-    // Step i works on stage `cur` = i % 3 and requests step i+2 into `far`, which held step i-1: everybody has left that
-    // stage before the barrier of step i-1.  In front of the barrier a wave waits until no more than what it has
-    // requested during this step is outstanding: its part of stage i+1 and of the scales is then in LDS.
-    auto mfmas = [&](int t) {
-#pragma unroll
-        for (int mb = 0; mb < WMB; ++mb) {
-            acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[t % (2 * AHEAD)][mb], bf[t & 1], acc[mb], 0, 0, 0);
-            if (HILO) acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[t % (2 * AHEAD)][mb], bl[t & 1], acc[mb], 0, 0, 0);
-        }
+    // Step i works on stage i % ST and reads the packed weights of step i+1 at its beginning.  In front of its last slices, whose
+    // fragments are in registers, a wave waits until its part of the activations of step i+1 and of the weights of step i+2 is
+    // in LDS; the barrier says so for all of them, and that the activations of stage i and the weights of stage i+1 have been
+    // read: step i+ST's and step i+ST+1's are requested into their place, from here to the next barrier.
+    auto mfma = [&](int t, int e) {
+        const int mb = e / NB, nb = e % NB;
+        acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[t % (2 * AHEAD)][mb], bf[t & 1][nb], acc[mb][nb], 0, 0, 0);
     };
     // The order inside a slice: LDS reads with the first MFMAs, memory requests and the dequantisation spread over all of
     // them (mask 8: MFMA, 2: vector ALU, 0x100: LDS read, 0x20: vector memory).
-    constexpr int NM = WMB * (HILO ? 2 : 1), DQ = I4 ? (HILO ? 37 : 17) : 12;
+    constexpr int DQ = NB * (I4 ? 17 : 12);
     auto order = [&]() {
 #pragma unroll
-        for (int e = 0; e < NM; ++e) {
+        for (int e = 0; e < NE; ++e) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (e < WMB) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            if (e % 2 == 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, (DQ + NM - 1) / NM, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, (DQ + NE - 1) / NE, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto step = [&](int i, auto more1_c, auto more2_c) {
-        constexpr bool more1 = decltype(more1_c)::value, more2 = decltype(more2_c)::value;  // steps i+1, i+2 exist
-        constexpr int H = (C::A_DMA + C::B_DMA + 1) / 2 - C::B_DMA;
+    auto step = [&](int i, int slot, auto pending_c, auto before_c, auto more_c, auto whole_c) {
+        constexpr bool whole = decltype(whole_c)::value;     // everything it requests lies before the last step
+        constexpr int pending = decltype(pending_c)::value;  // further steps whose requests may be outstanding at the barrier; -1: the last step
+        constexpr bool before = decltype(before_c)::value;   // step i+ST-1 exists: the rest of its requests
+        constexpr bool more = decltype(more_c)::value;       // step i+ST exists
+        uint8_t *const cur = lds + slot * C::STAGE, *const nxt = lds + (slot + 1 == ST ? 0 : slot + 1) * C::STAGE;
+        uint8_t *const prv = lds + (slot == 0 ? ST - 1 : slot - 1) * C::STAGE;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            if (t == 4 - AHEAD && more1) {
-                if (more2) wait_vmcnt<C::A_DMA + C::B_DMA>();
-                else wait_vmcnt<0>();
-                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this stage has been read
+        for (int t = 0; t < SL; ++t) {
+            if (t == BAR && pending >= 0) {
+                wait_vmcnt<(pending > 0 ? pending * C::REQ : 0)>();
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
                 wg_barrier();
-                if (GUARD || C::SPB == 1) {
-                    if (more2) issue_s(i + 2);
-                } else if (I4 && (i + 3) % C::SPB == 0 && i + 3 < steps) {
-                    issue_s((i + 3) / C::SPB);
-                }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (t < 4 - AHEAD) frags(t + AHEAD, cur);
-            if (t == 0 && more2) {
-                issue_b(i + 2, far);
-                issue_a(i + 2, 0, H, far);
+#pragma unroll
+            for (int e = 0; e < NE; ++e) {
+                if (e < MB && t < BAR) frag(t + AHEAD, e, cur);
+                if (e < MB && t >= BAR && pending >= 0) frag(t - BAR, e, nxt);
+                if (t == 0 && e == 0 && pending >= 0) fetch(i + 1, nxt);
+                const int p = (t < BAR ? t + AHEAD : t - BAR) * NE + e;
+#pragma unroll
+                for (int r = first(p); r < first(p + 1); ++r) {
+                    if (before && t < BAR) request(r, i + ST - 1, cur, prv, whole);
+                    if (more && t >= BAR) request(r, i + ST, nxt, cur, whole);
+                }
+                mfma(t, e);
             }
-            if (t == 1 && more2) issue_a(i + 2, H < 0 ? 0 : H, C::A_DMA, far);
-            mfmas(t);
-            if (t < 3) deq(t + 1);
-            if (t == 4 - AHEAD && more1) fetch(i + 1, nxt);
-            if (t >= 4 - AHEAD && more1) frags(t + AHEAD - 4, nxt);
-            if (t == 3 && more1) {
+            if (t < SL - 1) deq(t + 1);
+            if (t == SL - 1 && pending >= 0) {
                 prep(i + 1);
                 deq(0);
             }
             order();
         }
-        uint8_t *const r = cur;
-        cur = nxt;
-        nxt = far;
-        far = r;
     };
-    using T = std::true_type;
-    using F = std::false_type;
-    int i = 0;
-    for (; i + 2 < steps; ++i) step(i, T{}, T{});
-    if (steps > 1) step(i++, T{}, F{});
-    step(i, F{}, F{});
+    run(step);
+    }
 
-    // ---- epilogue.  The lane holds, for every mb, column nl of rows 8*(v/4) + 4*kq + v%4 of a 32 x 32 block.
+    // ---- epilogue.  The lane holds, for every mb and nb, column nl of rows 8*(v/4) + 4*kq + v%4 of a 32 x 32 block.
     wg_barrier();  // every wave is done with the stages, which everything below reuses
-    // WK = 2: the two waves that hold the k halves of one result exchange halves of it through LDS and each finishes one:
-    // lower row blocks by the first, upper ones by the second.  (A tile of one row block: its upper eight values.)
-    // WK = 4: every wave leaves all of its values and finishes a quarter of the sums, added in the order of the k.
-    constexpr int PARTS = WK == 4 ? 4 : WMB == 1 ? 2 : WMB;    // units of exchange: row blocks, halves of the only one, quarters
-    constexpr int UV = WK == 4 ? WMB * 4 : WMB == 1 ? 8 : 16, PE = PARTS / WK;  // values per unit, units a wave finishes
-    auto val = [&](int u, int v) { return WMB == 1 ? acc[0][u * 8 + v] : acc[WMB == 1 ? 0 : u][v]; };
-    float res[PE][UV];
-    if constexpr (WK == 2) {
-        float *const red = reinterpret_cast<float *>(lds) + wn * (WMB * 1024) + lane * 4;
+    // A wave finishes 1/WK of its values, MB * 16 of them numbered (row block, v).  WK = 2: the two waves that hold the k halves of
+    // one result trade halves of it through LDS.  WK = 4: every wave leaves all of them and adds its quarter in the order of the k.
+    constexpr int UV = MB * 16 / WK;
+    float res[NB][UV];
 #pragma unroll
-        for (int u = 0; u < PE; ++u)
+    for (int nb = 0; nb < NB; ++nb) {
+        auto val = [&](int f) { return acc[f >> 4][nb][f & 15]; };
+        if constexpr (WK == 2) {
+            float *const red = reinterpret_cast<float *>(lds) + (wm * WN + wn) * (MB * 1024) + lane * 4;
 #pragma unroll
             for (int q = 0; q < UV / 4; ++q) {
                 f32x4 o;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = wk ? val(u, 4 * q + e) : val(PE + u, 4 * q + e);
-                *reinterpret_cast<f32x4 *>(red + ((wk * PE + u) * (UV / 4) + q) * 256) = o;
+                for (int e = 0; e < 4; ++e) o[e] = wk ? val(4 * q + e) : val(UV + 4 * q + e);
+                *reinterpret_cast<f32x4 *>(red + (wk * (UV / 4) + q) * 256) = o;
             }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < PE; ++u)
+            __syncthreads();
 #pragma unroll
             for (int q = 0; q < UV / 4; ++q) {
-                const f32x4 o = *reinterpret_cast<const f32x4 *>(red + (((1 - wk) * PE + u) * (UV / 4) + q) * 256);
+                const f32x4 o = *reinterpret_cast<const f32x4 *>(red + ((1 - wk) * (UV / 4) + q) * 256);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) res[u][4 * q + e] = (wk ? val(PE + u, 4 * q + e) : val(u, 4 * q + e)) + o[e];
+                for (int e = 0; e < 4; ++e) res[nb][4 * q + e] = (wk ? val(UV + 4 * q + e) : val(4 * q + e)) + o[e];
             }
-        __syncthreads();
-    } else if constexpr (WK == 4) {
-        float *const red = reinterpret_cast<float *>(lds) + lane * 4;
+            __syncthreads();
+        } else if constexpr (WK == 4) {
+            float *const red = reinterpret_cast<float *>(lds) + lane * 4;
 #pragma unroll
-        for (int q = 0; q < WMB * 4; ++q) {
-            const f32x4 o = {acc[q / 4][q % 4 * 4], acc[q / 4][q % 4 * 4 + 1], acc[q / 4][q % 4 * 4 + 2], acc[q / 4][q % 4 * 4 + 3]};
-            *reinterpret_cast<f32x4 *>(red + (wave * WMB * 4 + q) * 256) = o;
+            for (int q = 0; q < MB * 4; ++q)
+                *reinterpret_cast<f32x4 *>(red + (wave * MB * 4 + q) * 256) = f32x4{val(4 * q), val(4 * q + 1), val(4 * q + 2), val(4 * q + 3)};
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < UV / 4; ++q) {
+                f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int w = 0; w < WK; ++w)
+                    o += *reinterpret_cast<const f32x4 *>(red + (((w * WM + wm) * WN + wn) * MB * 4 + wk * (UV / 4) + q) * 256);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) res[nb][4 * q + e] = o[e];
+            }
+            __syncthreads();
+        } else {
+#pragma unroll
+            for (int v = 0; v < UV; ++v) res[nb][v] = val(v);
         }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < UV / 4; ++q) {
-            f32x4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int w = 0; w < WK; ++w) o += *reinterpret_cast<const f32x4 *>(red + ((w * WN + wn) * WMB * 4 + wk * (UV / 4) + q) * 256);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) res[0][4 * q + e] = o[e];
-        }
-        __syncthreads();
-    } else {
-#pragma unroll
-        for (int u = 0; u < PE; ++u)
-#pragma unroll
-            for (int v = 0; v < UV; ++v) res[u][v] = val(u, v);
     }
-    const int u0 = wk * PE;  // the wave's first unit
-    auto row_of = [&](int u, int v) {
-        if (WK == 4) {
-            const int f = u0 * UV + v, vv = f & 15;
-            return (f >> 4) * 32 + 8 * (vv >> 2) + 4 * kq + (vv & 3);
-        }
-        const int vv = WMB == 1 ? (u0 + u) * 8 + v : v;
-        return (WMB == 1 ? 0 : (u0 + u) * 32) + 8 * (vv >> 2) + 4 * kq + (vv & 3);
+    auto row_of = [&](int v) {
+        const int f = wk * UV + v, vv = f & 15;
+        return wm * MB * 32 + (f >> 4) * 32 + 8 * (vv >> 2) + 4 * kq + (vv & 3);
     };
     if constexpr (EPI == EPI_F32) {  // 128 contiguous bytes per row straight from the registers
         float *const y = reinterpret_cast<float *>(yv) + (size_t)blockIdx.y * M * N;
-        const int n = n0 + wn * 32 + nl;
 #pragma unroll
-        for (int u = 0; u < PE; ++u)
+        for (int nb = 0; nb < NB; ++nb) {
+            const int n = n0 + (wn * NB + nb) * 32 + nl;
 #pragma unroll
             for (int v = 0; v < UV; ++v) {
-                const int m = m0 + row_of(u, v);
-                if (m < M && n < N) y[(size_t)m * N + n] = res[u][v];
+                const int m = m0 + row_of(v);
+                if (m < M && n < N) y[(size_t)m * N + n] = res[nb][v];
             }
+        }
         return;
     }
     // bf16 results leave through a tile in LDS, as whole rows: neighbouring lanes first swap one value of each row pair
@@ -416,30 +596,32 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
     constexpr bool GE = EPI == EPI_GEGLU;
     constexpr int EP = C::EP_PITCH;
     const bool odd = lane & 1;
-    float colscale = 1.f;
-    if constexpr (!I4) {
-        const int n = n0 + wn * 32 + nl;
-        colscale = reinterpret_cast<const float *>(scv)[n < N ? n : N - 1];
-    }
 #pragma unroll
-    for (int u = 0; u < PE; ++u)
+    for (int nb = 0; nb < NB; ++nb) {
+        const int cb = (wn * NB + nb) * 32;  // the block's first column in the tile
+        float colscale = 1.f;
+        if constexpr (!I4) {
+            const int n = n0 + cb + nl;
+            colscale = reinterpret_cast<const float *>(scv)[n < N ? n : N - 1];
+        }
 #pragma unroll
         for (int v = 0; v < UV; v += 2) {
-            float a0 = res[u][v], a1 = res[u][v + 1];  // rows r and r+1, column nl
+            float a0 = res[nb][v], a1 = res[nb][v + 1];  // rows r and r+1, column nl
             if constexpr (!I4) {
                 a0 *= colscale;
                 a1 *= colscale;
             }
             const float send = odd ? a0 : a1;
             const float recv = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(send), 0xB1, 0xF, 0xF, false));  // lane ^ 1
-            const int row = row_of(u, v) + (odd ? 1 : 0);
+            const int row = row_of(v) + (odd ? 1 : 0);
             // even lane: row r, columns (nl, nl+1) = (own a0, neighbour's a0); odd lane: row r+1, columns (nl-1, nl)
             if constexpr (GE)
-                *reinterpret_cast<uint16_t *>(lds + row * EP + (wn * 16 + (nl >> 1)) * 2) =
+                *reinterpret_cast<uint16_t *>(lds + row * EP + (cb + nl) / 2 * 2) =
                     (uint16_t)f32_to_bf16_bits(gelu_tanh_dev(odd ? recv : a0) * (odd ? a1 : recv));
             else
-                *reinterpret_cast<uint32_t *>(lds + row * EP + (wn * 32 + (nl & ~1)) * 2) = odd ? pack_bf16_rne(recv, a1) : pack_bf16_rne(a0, recv);
+                *reinterpret_cast<uint32_t *>(lds + row * EP + (cb + (nl & ~1)) * 2) = odd ? pack_bf16_rne(recv, a1) : pack_bf16_rne(a0, recv);
         }
+    }
     __syncthreads();
     uint16_t *const y = reinterpret_cast<uint16_t *>(yv);
     constexpr int COLS = GE ? BN / 2 : BN, LPR = COLS / 8;  // 16-byte pieces (lanes) per tile row
@@ -459,18 +641,18 @@ __global__ __launch_bounds__(64 * WN * WK) __attribute__((amdgpu_waves_per_eu(2,
     }
 }
 
-template <bool I4, int WN, int WK, int WMB, bool GUARD, bool HILO = false, int EPI = EPI_BF16>
+template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT = false, int EPI = EPI_BF16>
 static int launch(const uint16_t *x, const uint8_t *wq, const void *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st) {
-    typedef Cfg<I4, WN, WK, WMB, GUARD> C;
+    typedef Cfg<I4, WM, WN, WK, MB, NB, KW, ST, GUARD> C;
     static std::atomic<bool> attr_set{false};  // setting it twice from two threads is harmless
     if (!attr_set.load(std::memory_order_acquire)) {
-        CHADQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tile_q_kernel<I4, WN, WK, WMB, GUARD, HILO, EPI>),
+        CHADQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tile_q_kernel<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, EXACT, EPI>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS));
         attr_set.store(true, std::memory_order_release);
     }
     const int tiles = ((N + C::BN - 1) / C::BN) * ((M + C::BM - 1) / C::BM);
-    hipLaunchKernelGGL((gemm_tile_q_kernel<I4, WN, WK, WMB, GUARD, HILO, EPI>), dim3((tiles + 7) / 8 * 8, ksplit), dim3(C::T), C::LDS, st, x,
-                       wq, sc, y, M, N, K, K / ksplit);
+    hipLaunchKernelGGL((gemm_tile_q_kernel<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, EXACT, EPI>), dim3((tiles + 7) / 8 * 8, ksplit), dim3(C::T), C::LDS, st,
+                       x, wq, sc, y, M, N, K, ksplit == 1 ? K : (K / 256 + ksplit - 1) / ksplit * 256);
     return hip_check(hipGetLastError(), "gemm_tile_q launch");
 }
 
@@ -479,64 +661,105 @@ static int launch(const uint16_t *x, const uint8_t *wq, const void *sc, void *y,
 // A tile's byte offsets are signed 32-bit in the descriptor: 256 rows of the wider matrix stay below 2 GiB.
 bool gemm_tile_q_ok(int K) { return K < (1 << 22); }
 
-int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, bool big,
+// Which tile.  A tile takes c0 + c1 * K / 4096 us on a chip full of them and less on one that is not: a round of f * 256 tiles b +
+// (1 - b) f of it.  Longer launches run at a lower clock, which costs the tiles differently: `a` us of work take a (1 + q a / (a +
+// 100)).  The constants are fitted to whole calls, every tile on 850 random products (65 to 4096 rows, 512 to 16384 columns and k);
+// the tile picked is 0.3 % slower on average than the best of all eight, 10 % at worst.  Up to 64 rows the smallest tiles win in
+// any number of rounds (the others are padded to 96 rows and every round of theirs carries the same weights): 33 x 20000 x 2048
+// 15.4 us (128 x 64: 23.7), 64 x 256000 x 2048 151 (299), 64 x 16384 x 16384 63 (87).
+struct TileCost {
+    GemmTile tile;
+    int bm, bn;
+    float c0, c1, b, q;
+};
+static const TileCost kCostI4[] = {{TILE_64x64, 64, 64, 2.2f, 9.7f, .68f, .27f},      {TILE_96x64, 96, 64, 2.3f, 13.6f, .72f, .36f},
+                                   {TILE_128x64, 128, 64, 2.6f, 16.5f, .70f, .37f},   {TILE_96x128, 96, 128, 4.2f, 21.0f, .71f, .41f},
+                                   {TILE_128x128, 128, 128, 3.9f, 23.9f, .65f, .54f}, {TILE_192x128, 192, 128, 5.1f, 37.0f, .70f, .50f},
+                                   {TILE_256x128, 256, 128, 5.8f, 46.1f, .69f, .42f}, {TILE_256x256, 256, 256, 8.1f, 87.3f, .63f, .13f}};
+static const TileCost kCostI8[] = {{TILE_64x64, 64, 64, 2.2f, 10.7f, .61f, .09f},     {TILE_96x64, 96, 64, 2.2f, 14.2f, .65f, .12f},
+                                   {TILE_128x64, 128, 64, 2.5f, 17.2f, .65f, .14f},   {TILE_96x128, 96, 128, 4.5f, 19.8f, .62f, .31f},
+                                   {TILE_128x128, 128, 128, 5.5f, 22.7f, .67f, .36f}, {TILE_192x128, 192, 128, 5.2f, 30.6f, .69f, .52f},
+                                   {TILE_256x128, 256, 128, 6.4f, 41.1f, .67f, .35f}, {TILE_256x256, 256, 256, 8.2f, 77.0f, .66f, .18f}};
+
+GemmTile gemm_tile_pick(int M, int N, int K, bool int4) {
+    if (M <= 64) return M <= 32 ? TILE_32x64 : TILE_64x64;
+    GemmTile best = TILE_64x64;
+    float best_cost = 0.f;
+    for (const TileCost &t : int4 ? kCostI4 : kCostI8) {
+        const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), rounds = (tiles + 255) / 256;
+        const float fill = (float)(tiles - (rounds - 1) * 256) / 256.f;
+        const float a = ((float)(rounds - 1) + t.b + (1.f - t.b) * fill) * (t.c0 + t.c1 * (float)K / 4096.f), cost = a * (1.f + t.q * a / (a + 100.f));
+        if (best_cost == 0.f || cost < best_cost) {
+            best = t.tile;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+template <bool I4, bool GUARD>
+static int launch_tile(const uint16_t *x, const uint8_t *w, const void *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st) {
+    switch (tile) {
+        case TILE_32x64: return tileq::launch<I4, 1, 2, 4, 1, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        case TILE_64x64: return tileq::launch<I4, 1, 2, 4, 2, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        case TILE_96x64: return tileq::launch<I4, 1, 2, 4, 3, 1, 32, GUARD ? 3 : 4, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        case TILE_128x64: return tileq::launch<I4, 1, 2, 4, 4, 1, 32, GUARD ? 3 : 4, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        case TILE_96x128: return tileq::launch<I4, 1, 2, 4, 3, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        case TILE_128x128:  // (the other form: int4 36.7 us against 36.3 at 1024 x 4096 x 4096, int8 113 against 107 at 1000 x 4096 x 14336)
+            if constexpr (I4) return tileq::launch<I4, 1, 4, 2, 4, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+            else return tileq::launch<I4, 1, 2, 4, 4, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        case TILE_192x128: return tileq::launch<I4, 2, 2, 2, 3, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        case TILE_256x128: return tileq::launch<I4, 2, 2, 2, 4, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        default: return tileq::launch<I4, 1, 8, 1, 8, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+    }
+}
+
+int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, GemmTile tile,
                            hipStream_t st) {
     const bool guard = K % 256 != 0 || !aligned16(sc);  // 16 bytes of scales at a time want aligned rows of them
-    if (big)
-        return guard ? tileq::launch<true, 8, 1, 8, true>(x, wp, sc, y, M, N, K, 1, st) : tileq::launch<true, 8, 1, 8, false>(x, wp, sc, y, M, N, K, 1, st);
-    return guard ? tileq::launch<true, 4, 2, 4, true>(x, wp, sc, y, M, N, K, 1, st) : tileq::launch<true, 4, 2, 4, false>(x, wp, sc, y, M, N, K, 1, st);
+    return guard ? launch_tile<true, true>(x, wp, sc, y, M, N, K, tile, st) : launch_tile<true, false>(x, wp, sc, y, M, N, K, tile, st);
 }
 
-int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, bool big, hipStream_t st) {
+int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st) {
     const uint8_t *w = reinterpret_cast<const uint8_t *>(w8);
-    if (big)
-        return K % 64 ? tileq::launch<false, 8, 1, 8, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 8, 1, 8, false>(x, w, sc, y, M, N, K, 1, st);
-    return K % 128 ? tileq::launch<false, 4, 2, 4, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 4, 2, 4, false>(x, w, sc, y, M, N, K, 1, st);
+    const int step = tile == TILE_32x64 || tile == TILE_64x64 ? 256 : tile == TILE_256x256 || tile == TILE_192x128 || tile == TILE_256x128 ? 64 : 128;
+    return K % step ? launch_tile<false, true>(x, w, sc, y, M, N, K, tile, st) : launch_tile<false, false>(x, w, sc, y, M, N, K, tile, st);
 }
 
-// At most 64 rows, or few enough tiles for one round: 32 or 64 rows x 64 weight rows, the eight waves two side by side and
-// four along K (256 k per step).
-// What bounds it is the operands' way into the compute unit: at 48 x 14336 x 4096 a workgroup pulls 393 KB of activations and
-// 147 KB of weights and scales, and these requests alone, nothing computed, take 10.1 of its 13.5 us in a queue of launches
-// (2.2 of them the launch; the weights alone 6.2).  As many weight rows per workgroup as the 128 x 64 kernel has (one
-// round of the chip up to 16384 of them), but twice the waves, a quarter of the steps and no padding to 128 rows.
-// us (the 128 x 64 kernel in brackets): int4 48 x 14336 x 4096 13.5 (21.0), 17 x 4096 x 4096 9.7 (18.1), 64 x 2048 x 14336
-// 36 (52), 64 x 32768 x 4096 28 (42), 64 x 1024 x 1024 5.5 (8.6); int8 48 x 14336 x 4096 13.6 (21.7).
-int gemm_tile_small_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, hipStream_t st) {
-    const bool guard = K % 256 != 0 || !aligned16(sc);
-    if (M <= 32)
-        return guard ? tileq::launch<true, 2, 4, 1, true>(x, wp, sc, y, M, N, K, 1, st) : tileq::launch<true, 2, 4, 1, false>(x, wp, sc, y, M, N, K, 1, st);
-    return guard ? tileq::launch<true, 2, 4, 2, true>(x, wp, sc, y, M, N, K, 1, st) : tileq::launch<true, 2, 4, 2, false>(x, wp, sc, y, M, N, K, 1, st);
-}
-
-int gemm_tile_small_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, hipStream_t st) {
-    const uint8_t *w = reinterpret_cast<const uint8_t *>(w8);
-    if (M <= 32)
-        return K % 256 ? tileq::launch<false, 2, 4, 1, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 2, 4, 1, false>(x, w, sc, y, M, N, K, 1, st);
-    return K % 256 ? tileq::launch<false, 2, 4, 2, true>(x, w, sc, y, M, N, K, 1, st) : tileq::launch<false, 2, 4, 2, false>(x, w, sc, y, M, N, K, 1, st);
-}
-
-// ---- exact weights (HILO), K % 256 == 0: the projections of a prompt, whose tokens must come out as the decode step's do.
-// Tiles of 32, 64 or 128 rows x 128 weight rows; with few rows the weight stream decides, not the padding.
+// ---- exact weights, K % 256 == 0: the projections of a prompt, whose tokens must come out as the decode step's do.
+// Tiles of 128 or 256 rows x 128 weight rows, or of 32 or 64 x 64: with few rows a workgroup waits for its weights, and what counts is
+// how many workgroups and steps wait at once (two workgroups per compute unit for at most 32 rows; the loop is not unrolled: the
+// code of a few steps is fetched as often as it is run).  Whole prompts in us, 128 weight rows for every number of tokens in brackets:
+// 24 tokens through 18 layers of 2048 x 16384 1152 (1343), 9 through 6 of 1280 x 3840 262 (321), 37 through 4 of 2048 x 8960 282 (311).
 template <int EPI>
 static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st) {
-    if (M <= 32) return tileq::launch<true, 4, 2, 1, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
-    if (M <= 64) return tileq::launch<true, 4, 2, 2, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
-    return tileq::launch<true, 4, 2, 4, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    if (M <= 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    if (M <= 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    if constexpr (EPI == tileq::EPI_GEGLU) {
+        // 256 rows dequantise a weight half as often: a full round takes 45 us per 2048 k, one of 128-row tiles 30
+        auto rounds = [&](int bm) {
+            const int tiles = ((M + bm - 1) / bm) * ((N + 127) / 128), full = (tiles - 1) / 256;
+            return (float)full + 0.65f + 0.35f / 256.f * (float)(tiles - full * 256);
+        };
+        if (rounds(256) * 45.f < rounds(128) * 30.f) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    }
+    return tileq::launch<true, 1, 4, 2, 4, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
 }
 
-// K splits that make the launch shortest: rounds of 256 workgroups times the k of each (and what a workgroup costs
-// besides, about 256 k worth).  At most kExactMaxSplits parts, each a multiple of 256 k.
+// K splits that make the launch shortest: rounds of workgroups times the k of each (and what a workgroup costs besides, about
+// 256 k worth).  At most kExactMaxSplits parts of whole 256-k blocks, the last one possibly shorter: with equal parts only, a down
+// projection of 8960 k had one part, 63 us of the 125 that its layer took for 37 tokens.
 int gemm_exact_splits(int M, int N, int K) {
-    const int bm = M <= 32 ? 32 : M <= 64 ? 64 : 128;
-    const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + 127) / 128);
+    const int bm = M <= 32 ? 32 : M <= 64 ? 64 : 128, blocks = K / 256;
+    const int bn = M <= 64 ? 64 : 128, wgs = M <= 32 ? 512 : 256;
+    const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
     int best = 1;
     int64_t best_cost = 0;
-    for (int s = 1; s <= kExactMaxSplits; s *= 2) {
-        if (K % (s * 256) != 0) break;
-        const int64_t cost = (tiles * s + 255) / 256 * (K / s + 256);
+    for (int s = 1; s <= kExactMaxSplits; ++s) {
+        const int per = (blocks + s - 1) / s, parts = (blocks + per - 1) / per;
+        const int64_t cost = (tiles * parts + wgs - 1) / wgs * (per + 1);
         if (s == 1 || cost < best_cost) {
-            best = s;
+            best = parts;
             best_cost = cost;
         }
     }

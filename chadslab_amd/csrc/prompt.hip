@@ -3,7 +3,7 @@
 // layer's weights are read once per chunk of tokens and the products run on the matrix cores.
 //
 // Nothing is rounded that the decode step does not round: activations become bf16 in the same four places (the two norms,
-// the attention vector, the gated activation), weights are taken exactly (gemm_tile_q.hip, HILO), sums, residual stream,
+// the attention vector, the gated activation), weights are taken exactly (gemm_tile_q.hip, EXACT), sums, residual stream,
 // rotation and softmax are fp32, K and V rows bf16.
 //
 // Per layer: residual add + RMSNorm | qkv product | rotation and cache rows | attention | output product | residual add +
@@ -82,11 +82,15 @@ __global__ __launch_bounds__(256) void prompt_add_norm_kernel(const float *res, 
 static void add_norm_launch(int rows, const float *res, float *res_out, const float *parts, int np, const float *w, uint16_t *y, int d,
                             float eps, hipStream_t st) {
 #define CHADQ_ADD_NORM(NP) hipLaunchKernelGGL(prompt_add_norm_kernel<NP>, dim3(rows), dim3(256), 0, st, res, res_out, parts, w, y, d, eps)
-    switch (np) {  // gemm_exact_splits gives powers of two up to kExactMaxSplits
+    switch (np) {  // at most kExactMaxSplits
         case 0: CHADQ_ADD_NORM(0); break;
         case 1: CHADQ_ADD_NORM(1); break;
         case 2: CHADQ_ADD_NORM(2); break;
+        case 3: CHADQ_ADD_NORM(3); break;
         case 4: CHADQ_ADD_NORM(4); break;
+        case 5: CHADQ_ADD_NORM(5); break;
+        case 6: CHADQ_ADD_NORM(6); break;
+        case 7: CHADQ_ADD_NORM(7); break;
         default: CHADQ_ADD_NORM(8); break;
     }
 #undef CHADQ_ADD_NORM
@@ -375,11 +379,13 @@ static size_t prompt_layout(uint8_t *base, int T, int d, int hq, int dh, int ffn
         const size_t n = (size_t)gemm_exact_splits(M, N, K) * M * N;
         parts = n > parts ? n : parts;
     };
-    need(T, (int)wq, d);
-    need(T, d, hq * dh);
-    need(T, d, ffn);
-    need(1, d, hq * dh);
-    need(1, d, ffn);
+    // (every number of rows up to T: a shorter chunk may come with the same workspace, and fewer rows take more splits)
+    for (int M = 32; M < T + 128; M += M < 128 ? M : 128) {
+        const int m = M < T ? M : T;
+        need(m, (int)wq, d);
+        need(m, d, hq * dh);
+        need(m, d, ffn);
+    }
     PromptWs w;
     w.x = (float *)take(t * d * 4);
     w.parts = (float *)take(parts * 4);

@@ -773,6 +773,14 @@ def test_decoder_prompt_in_chunks_equals_the_step_token_by_token(t, pos, layers,
     assert rel(b.logits, a.logits) <= 5e-3 * layers
 
 
+@pytest.mark.parametrize("t,pos,layers,d,hq,dh,ffn", [(9, 0, 2, 512, 4, 64, 1792), (50, 3, 1, 1280, 8, 128, 8960), (31, 0, 1, 2048, 8, 256, 768),
+                                                      (200, 0, 1, 256, 2, 128, 16384), (300, 0, 1, 1280, 8, 128, 8960)])
+def test_decoder_prompt_with_uneven_k_splits_and_256_row_tiles(t, pos, layers, d, hq, dh, ffn):
+    """K that no power of two divides into parts of whole blocks (7, 35 and 3 of 256 k), the gate/up product of more than 128
+    tokens in tiles of 256 rows, and a second chunk whose fewer rows take more splits than the first one's."""
+    test_decoder_prompt_in_chunks_equals_the_step_token_by_token(t, pos, layers, d, hq, dh, ffn)
+
+
 @pytest.mark.parametrize("t,bad,pos,d,hq,dh,ffn", [(16, (9,), 5, 512, 8, 64, 512), (21, (6, 13), 0, 256, 2, 128, 512), (40, (33, 39), 30, 256, 1, 256, 512),
                                                    (33, (0, 17, 31), 3, 768, 3, 256, 768), (300, (260, 270), 0, 256, 4, 64, 512)])
 def test_decoder_prompt_a_token_that_is_not_finite_reaches_no_earlier_token(t, bad, pos, d, hq, dh, ffn):

@@ -464,6 +464,18 @@ def test_gemm_eight_wave_tiles_every_row_and_column(ops, weight, m, n, k):
         assert np.sqrt(err.sum(axis=axis) / (ref ** 2).sum(axis=axis)).max() <= TOL_BF16
 
 
+@pytest.mark.parametrize("m,n,k", [(69, 3963, 32), (555, 1697, 96), (193, 4000, 512), (190, 4097, 1056),          # 96 x 64 tiles
+                                   (99, 8259, 32), (509, 3918, 96), (512, 4095, 512), (385, 5000, 1312),          # 128 x 64
+                                   (259, 8306, 512), (259, 6663, 1312), (276, 8097, 768),                         # 96 x 128
+                                   (390, 8279, 32), (1159, 3291, 160), (386, 11008, 256), (577, 5500, 544),       # 192 x 128
+                                   (588, 8210, 32), (635, 8317, 160), (600, 8300, 512), (513, 8193, 1312)])       # 256 x 128
+@pytest.mark.parametrize("weight", ["int4", "int8"])
+def test_gemm_tiles_between_64_and_256_rows(ops, weight, m, n, k):
+    """The sizes at which the other tiles of gemm_tile_q.hip are picked, ragged in rows, columns and k (from one step to more than
+    the unrolled loop takes); every row and column by itself, as above."""
+    test_gemm_eight_wave_tiles_every_row_and_column(ops, weight, m, n, k)
+
+
 @pytest.mark.parametrize("n", [64, 128, 512])
 def test_gemm_refuses_4_gib_of_activations_for_every_tile(ops, n):
     """One row below the limit is served and right in its last rows; at the limit the call is refused, whichever tile N picks."""

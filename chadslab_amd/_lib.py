@@ -83,6 +83,7 @@ class PromptLayerI4G32(ctypes.Structure):
 _STATUS_EXC = {-1: ValueError, -2: ValueError, -3: ValueError, -4: ValueError, -5: RuntimeError, -6: RuntimeError}
 
 _lib = None
+_native, _native_lib = None, None  # the host module, the library it is bound to
 
 
 class ChadqError(RuntimeError):
@@ -111,6 +112,34 @@ def load() -> ctypes.CDLL:
         )
     _lib = open_library(LIB_PATH)
     return _lib
+
+
+_NATIVE_ENTRIES = ("chadq_gemv_i4g32", "chadq_gemv_i4g32_bf16", "chadq_gemm_i4g32_bf16", "chadq_gemv_i8row", "chadq_gemv_i8row_bf16",
+                   "chadq_gemm_i8row_bf16", "chadq_moe_ffn_i4g32_workspace_bytes", "chadq_moe_ffn_i4g32", "chadq_moe_ffn_i4g32_tiled")
+
+
+def native():
+    """The host module (csrc/host_call.cpp), bound to the library that load() gives; raises if it has not been built."""
+    global _native, _native_lib
+    if _native_lib is not None and _native_lib is _lib:
+        return _native
+    lib = load()
+    if _native is None:
+        import importlib.machinery
+        import importlib.util
+
+        path = Path(__file__).resolve().parent / "_host_call.so"
+        if not path.exists():
+            raise ChadqError("%s not found: build it with `python -m chadslab_amd.build` (there is no fallback path)" % path)
+        import torch  # noqa: F401  (its libraries have to be loaded first)
+
+        loader = importlib.machinery.ExtensionFileLoader("chadslab_amd._host_call", str(path))
+        _native = importlib.util.module_from_spec(importlib.util.spec_from_loader("chadslab_amd._host_call", loader))
+    from .formats import QWeightInt4G32, QWeightInt4G32Tiles, QWeightInt8
+
+    _native.bind(tuple(ctypes.cast(getattr(lib, n), c_void_p).value for n in _NATIVE_ENTRIES), (QWeightInt4G32, QWeightInt8, QWeightInt4G32Tiles))
+    _native_lib = lib
+    return _native
 
 
 def check(rc: int, what: str) -> None:

@@ -15,6 +15,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 OBJ = PKG / "csrc" / "_obj"
 LIB = PKG / "libchadq.so"
+HOST = PKG / "_host_call.so"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -packed-fp32-ops: keep the compiler from forming packed fp32 arithmetic (v_pk_*_f32)
@@ -37,6 +38,25 @@ def _run(cmd):
         sys.stderr.write(err + "\n")
 
 
+def build_host(verbose: bool = True) -> Path:
+    """csrc/host_call.cpp -> _host_call.so: the plain calls of ops.py in C++ (host code only, against torch's own headers)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    inc = [sysconfig.get_paths()["include"], *cpp_extension.include_paths(), "/opt/rocm/include"]
+    lib = str(Path(torch.__file__).resolve().parent / "lib")
+    tmp = HOST.with_suffix(".so.tmp")
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), *("-isystem%s" % i for i in inc),
+          str(CSRC / "host_call.cpp"), "-o", str(tmp), "-L" + lib, "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"])
+    os.replace(tmp, HOST)
+    if verbose:
+        print("built %s" % HOST)
+    return HOST
+
+
 def build(verbose: bool = True, save_temps: bool = False) -> Path:
     srcs = sorted(CSRC.glob("*.hip"))
     if not srcs:
@@ -52,8 +72,10 @@ def build(verbose: bool = True, save_temps: bool = False) -> Path:
         _run(cmd)
         return o
 
-    with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        host = ex.submit(build_host, verbose)
         list(ex.map(one, zip(srcs, objs)))
+        host.result()
     tmp = LIB.with_suffix(".so.tmp")
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)])
     os.replace(tmp, LIB)

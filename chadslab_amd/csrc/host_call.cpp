@@ -1,0 +1,195 @@
+// The plain calls of chadslab_amd.ops (qlinear, moe_ffn) from the Python object to the C ABI in one native function.
+//
+// What bounds a small call is the host: a product of 2048 x 2048 on one token takes 2.9 us on the GPU and took 7.2 us of Python
+// (attribute look-ups, checks, the result's allocation, eight arguments through ctypes), a mixture of experts with sixteen experts
+// 59 us (96 tensors looked at one by one).  Here the same checks are C++: 4.9 us, and 28 us with the GPU the slower side.
+//
+// Only what needs nothing unusual is served: exact torch.Tensor objects on the current device, of the right types and shapes,
+// contiguous.  For everything else, also for a call that the library refuses, the functions return None before anything has been
+// launched, and the Python code behind them does what it always did: copies, casts, and the errors' texts.
+#include <ATen/ops/empty.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/chadq.h"
+
+namespace {
+
+typedef int (*product_fn)(const void *, const void *, const void *, void *, int, int, int, void *);
+typedef size_t (*moe_bytes_fn)(int, int, int, int, int);
+typedef int (*moe_fn)(const void *, const void *, const chadq_moe_expert_i4g32 *, void *, int, int, int, int, int, int, void *, size_t, void *);
+
+enum Entry { GEMV_I4, GEMV_I4_BF16, GEMM_I4, GEMV_I8, GEMV_I8_BF16, GEMM_I8, MOE_BYTES, MOE_ROWS, MOE_TILES, ENTRIES };
+void *g_entry[ENTRIES];                                // of the library in use (bind)
+PyObject *g_int4 = nullptr, *g_int8 = nullptr, *g_tiles = nullptr;  // the weight containers
+PyObject *s_packed, *s_scale, *s_w;
+constexpr int kGemvRows = 16, kMaxExperts = 16;
+
+// a dense GPU tensor that may be handed on as it is
+const at::Tensor *plain(PyObject *o, at::ScalarType type, int dim, int device) {
+    if (!o || !THPVariable_CheckExact(o)) return nullptr;
+    const at::Tensor &t = THPVariable_Unpack(o);
+    const c10::TensorImpl *const i = t.unsafeGetTensorImpl();
+    if (t.layout() != at::kStrided || !i->has_storage() || !t.is_cuda() || t.dim() != dim || t.scalar_type() != type || !t.is_contiguous() ||
+        t.get_device() != device || t.is_neg() || i->is_python_dispatch())
+        return nullptr;
+    return &t;
+}
+
+struct Ref {  // a new reference, dropped at the end of the scope
+    PyObject *p;
+    explicit Ref(PyObject *o) : p(o) {
+        if (!o) PyErr_Clear();
+    }
+    ~Ref() { Py_XDECREF(p); }
+    Ref(const Ref &) = delete;
+};
+
+// linear(x, weight, out_dtype) -> y, or None
+PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    if (n_args != 3) Py_RETURN_NONE;
+    PyObject *const qw = args[1];
+    const bool int4 = (PyObject *)Py_TYPE(qw) == g_int4;
+    if (!int4 && (PyObject *)Py_TYPE(qw) != g_int8) Py_RETURN_NONE;
+    if (!THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
+    const at::Tensor &xt = THPVariable_Unpack(args[0]);
+    if (!xt.is_cuda()) Py_RETURN_NONE;  // (before the device is asked for: there may be none)
+    const int dev = c10::hip::current_device();
+    const at::ScalarType x_type = xt.scalar_type();
+    if (x_type != at::kBFloat16 && (int4 || x_type != at::kFloat)) Py_RETURN_NONE;
+    const at::Tensor *const x = plain(args[0], x_type, 2, dev);
+    if (!x) Py_RETURN_NONE;
+    const Ref wo(PyObject_GetAttr(qw, int4 ? s_packed : s_w)), so(PyObject_GetAttr(qw, s_scale));
+    const at::Tensor *const w = plain(wo.p, int4 ? at::kByte : at::kChar, 2, dev);
+    const at::Tensor *const s = plain(so.p, int4 ? at::kHalf : at::kFloat, int4 ? 2 : 1, dev);
+    if (!w || !s) Py_RETURN_NONE;
+    const int64_t m = x->size(0), n = w->size(0), k = int4 ? w->size(1) * 2 : w->size(1);
+    if (m < 1 || m > INT_MAX || n < 1 || n > INT_MAX || k < 1 || k > INT_MAX || x->size(1) != k || s->size(0) != n || (int4 && s->size(1) * 32 != k))
+        Py_RETURN_NONE;
+    const bool gemv = m <= kGemvRows && (int4 || x_type == at::kFloat);
+    if (!gemv && x_type != at::kBFloat16) Py_RETURN_NONE;
+    at::ScalarType y_type = gemv ? at::kFloat : at::kBFloat16;
+    if (args[2] != Py_None) {
+        if (!THPDtype_Check(args[2])) Py_RETURN_NONE;
+        const at::ScalarType want = reinterpret_cast<THPDtype *>(args[2])->scalar_type;
+        if (want != y_type && want != at::kBFloat16) Py_RETURN_NONE;
+        y_type = want;
+    }
+    const Entry e = !gemv ? (int4 ? GEMM_I4 : GEMM_I8) : y_type == at::kFloat ? (int4 ? GEMV_I4 : GEMV_I8) : (int4 ? GEMV_I4_BF16 : GEMV_I8_BF16);
+    at::Tensor y = at::empty({m, n}, x->options().dtype(y_type).requires_grad(false));
+    if (!y.unsafeGetTensorImpl()->has_storage()) Py_RETURN_NONE;
+    const void *const xp = x->const_data_ptr(), *const wp = w->const_data_ptr(), *const sp = s->const_data_ptr();
+    void *const yp = y.mutable_data_ptr(), *const stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream();
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = reinterpret_cast<product_fn>(g_entry[e])(xp, wp, sp, yp, (int)m, (int)n, (int)k, stream);
+    Py_END_ALLOW_THREADS
+    if (rc != 0) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+// moe_ffn(x, logits, experts, top_k, renorm) -> y, or None
+PyObject *moe_ffn(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    if (n_args != 5 || !(PyList_CheckExact(args[2]) || PyTuple_CheckExact(args[2])) || !PyLong_CheckExact(args[3])) Py_RETURN_NONE;
+    if (!THPVariable_CheckExact(args[0]) || !THPVariable_Unpack(args[0]).is_cuda()) Py_RETURN_NONE;
+    const int dev = c10::hip::current_device();
+    const at::Tensor *const x = plain(args[0], at::kBFloat16, 2, dev), *const z = plain(args[1], at::kFloat, 2, dev);
+    const Py_ssize_t e = PySequence_Fast_GET_SIZE(args[2]);
+    const long top_k = PyLong_AsLong(args[3]);
+    if (top_k == -1 && PyErr_Occurred()) PyErr_Clear();
+    const int renorm = PyObject_IsTrue(args[4]);
+    if (renorm < 0) return nullptr;
+    if (!x || !z || e < 1 || e > kMaxExperts || top_k < 1 || top_k > e) Py_RETURN_NONE;
+    const int64_t t = x->size(0), h = x->size(1);
+    if (t < 1 || t > INT_MAX || h < 1 || h > INT_MAX || z->size(0) != t || z->size(1) != e) Py_RETURN_NONE;
+    chadq_moe_expert_i4g32 arr[kMaxExperts];
+    at::Tensor keep[kMaxExperts][6];  // alive until the call is launched
+    PyObject *kind = nullptr;
+    int64_t f = 0;
+    for (Py_ssize_t i = 0; i < e; ++i) {
+        PyObject *const triple = PySequence_Fast_GET_ITEM(args[2], i);
+        if (!(PyTuple_CheckExact(triple) || PyList_CheckExact(triple)) || PySequence_Fast_GET_SIZE(triple) != 3) Py_RETURN_NONE;
+        const void *p[6];
+        for (int j = 0; j < 3; ++j) {  // gate, up [F,H], down [H,F]
+            PyObject *const m = PySequence_Fast_GET_ITEM(triple, j);
+            if (!kind) kind = (PyObject *)Py_TYPE(m);
+            if ((PyObject *)Py_TYPE(m) != kind || (kind != g_int4 && kind != g_tiles)) Py_RETURN_NONE;
+            const Ref wo(PyObject_GetAttr(m, s_packed)), so(PyObject_GetAttr(m, s_scale));
+            const at::Tensor *const w = plain(wo.p, at::kByte, 2, dev), *const s = plain(so.p, at::kHalf, 2, dev);
+            if (!w || !s) Py_RETURN_NONE;
+            if (i == 0 && j == 0) f = w->size(0);
+            const int64_t n = j < 2 ? f : h, k = j < 2 ? h : f;
+            if (w->size(0) != n || w->size(1) * 2 != k || s->size(0) != n || s->size(1) * 32 != k) Py_RETURN_NONE;
+            keep[i][2 * j] = *w;
+            keep[i][2 * j + 1] = *s;
+            p[2 * j] = w->const_data_ptr();
+            p[2 * j + 1] = s->const_data_ptr();
+        }
+        arr[i] = chadq_moe_expert_i4g32{};
+        memcpy(&arr[i], p, sizeof(p));
+    }
+    static_assert(sizeof(chadq_moe_expert_i4g32) == 6 * sizeof(void *), "six pointers: gate, up and down with their scales");
+    if (f < 1 || f > INT_MAX) Py_RETURN_NONE;
+    const size_t need = reinterpret_cast<moe_bytes_fn>(g_entry[MOE_BYTES])((int)t, (int)h, (int)f, (int)e, (int)top_k);
+    if (need == 0) Py_RETURN_NONE;
+    at::Tensor ws = at::empty({(int64_t)need}, x->options().dtype(at::kByte).requires_grad(false));
+    at::Tensor y = at::empty({t, h}, x->options().requires_grad(false));
+    if (!ws.unsafeGetTensorImpl()->has_storage() || !y.unsafeGetTensorImpl()->has_storage()) Py_RETURN_NONE;
+    const void *const xp = x->const_data_ptr(), *const zp = z->const_data_ptr();
+    void *const yp = y.mutable_data_ptr(), *const wsp = ws.mutable_data_ptr(), *const stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream();
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = reinterpret_cast<moe_fn>(g_entry[kind == g_tiles ? MOE_TILES : MOE_ROWS])(xp, zp, arr, yp, (int)t, (int)h, (int)f, (int)e, (int)top_k, renorm,
+                                                                              wsp, need, stream);
+    Py_END_ALLOW_THREADS
+    if (rc != 0) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+// bind(addresses of the entry points in the order of Entry, (QWeightInt4G32, QWeightInt8, QWeightInt4G32Tiles))
+PyObject *bind(PyObject *, PyObject *args) {
+    PyObject *addr, *kinds;
+    if (!PyArg_ParseTuple(args, "O!O!", &PyTuple_Type, &addr, &PyTuple_Type, &kinds)) return nullptr;
+    if (PyTuple_GET_SIZE(addr) != ENTRIES || PyTuple_GET_SIZE(kinds) != 3) {
+        PyErr_SetString(PyExc_ValueError, "bind: one address per entry point and three containers");
+        return nullptr;
+    }
+    void *fresh[ENTRIES];
+    for (int i = 0; i < ENTRIES; ++i) {
+        fresh[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(addr, i));
+        if (!fresh[i]) {
+            if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: null address");
+            return nullptr;
+        }
+    }
+    memcpy(g_entry, fresh, sizeof(fresh));
+    PyObject **const slot[3] = {&g_int4, &g_int8, &g_tiles};
+    for (int i = 0; i < 3; ++i) {
+        PyObject *const k = PyTuple_GET_ITEM(kinds, i);
+        Py_INCREF(k);
+        Py_XSETREF(*slot[i], k);
+    }
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {{"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, "linear(x, weight, out_dtype) -> y, or None where the Python path has to look"},
+                         {"moe_ffn", (PyCFunction)(void (*)(void))moe_ffn, METH_FASTCALL, "moe_ffn(x, logits, experts, top_k, renorm) -> y, or None"},
+                         {"bind", bind, METH_VARARGS, "bind(addresses, containers)"},
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_call", nullptr, -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host_call(void) {
+    s_packed = PyUnicode_InternFromString("packed");
+    s_scale = PyUnicode_InternFromString("scale");
+    s_w = PyUnicode_InternFromString("w");
+    if (!s_packed || !s_scale || !s_w) return nullptr;
+    return PyModule_Create(&module);
+}

@@ -142,6 +142,10 @@ def qlinear(x: torch.Tensor, qw: QWeight, *, out_dtype: Optional[torch.dtype] = 
     out_dtype picks the result type.  The GEMV writes bf16 itself if that is asked for (the same sums rounded once); any
     other type than the kernel's native one is a cast.
     """
+    y = _lib.native().linear(x, qw, out_dtype)
+    if y is not None:
+        return y
+    # what the native path leaves: more dimensions, strided or misplaced tensors, other types, everything that raises
     x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     m = x2.size(0)
     use_gemv = m <= GEMV_MAX_M and not (isinstance(qw, QWeightInt8) and x2.dtype == torch.bfloat16)
@@ -196,7 +200,10 @@ def moe_ffn(x: torch.Tensor, logits: torch.Tensor, experts, *, top_k: int = 2, r
     some 16 tokens on).  Dequantised weights are rounded to bf16 (row order) or fp16 (tile order), so the two orders agree within
     rounding; at most 16 tokens take exact weights in row order and, where the experts hit hold at most 64 MB, in tile order
     too, with the same bits from both.  Returns bf16 [T,H]."""
-    lib = _lib.load()
+    y = _lib.native().moe_ffn(x, logits, experts, top_k, renorm)
+    if y is not None:
+        return y
+    lib = _lib.load()  # (as in qlinear)
     x = _dev(x, "x", torch.bfloat16)
     z = _dev(logits, "logits", torch.float32)
     t, h = x.shape

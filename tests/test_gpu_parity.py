@@ -644,6 +644,55 @@ def test_qlinear_bf16_result_is_the_fp32_one_rounded(ops, m, n, k):
         assert y.dtype == torch.bfloat16 and torch.equal(y, ops.qlinear(xv, qw).to(torch.bfloat16))
 
 
+def test_native_calls_serve_plain_tensors_and_leave_the_rest_to_python(ops):
+    """The C++ call takes exact, contiguous tensors of the right types and nothing else; both roads give the same bits, and what
+    only Python serves (or refuses) still is."""
+    from chadslab_amd import QWeightInt4G32, QWeightInt8, _lib
+
+    native = _lib.native()
+    _, _, xb, q4 = i4_case(31, 40, 96, 256)
+    x = bf16_tensor(xb)
+    x8, w8, s8, q8 = i8_case(32, 40, 96, 256)
+    xf = torch.from_numpy(x8).to(DEV)
+    for rows in (1, 16, 17, 40):  # the fp32 and bf16 GEMV, the GEMM
+        for dt in (None, torch.bfloat16) if rows > 16 else (None, torch.float32, torch.bfloat16):
+            y = native.linear(x[:rows], q4, dt)
+            ref = ops.qgemm(x[:rows], q4) if rows > 16 else ops.qgemv(x[:rows], q4)
+            assert y is not None and torch.equal(y, ref if dt is None else ref.to(dt))
+            y8 = native.linear(x[:rows] if rows > 16 else xf[:rows], q8, dt)
+            ref8 = ops.qgemm(x[:rows], q8) if rows > 16 else ops.qgemv(xf[:rows], q8)
+            assert y8 is not None and torch.equal(y8, ref8 if dt is None else ref8.to(dt))
+    wide = torch.cat([x, x], 1)
+    strided = QWeightInt4G32(torch.cat([q4.packed, q4.packed], 1)[:, :128], q4.scale)
+    for a, w, dt in ((wide[:, :256], q4, None), (x.view(4, 10, 256), q4, None), (x[:5], strided, None), (x, q4, torch.float32),
+                     (x[:3], q4, torch.float16)):
+        assert native.linear(a, w, dt) is None
+        y = ops.qlinear(a, w, out_dtype=dt)
+        a2 = a.reshape(-1, 256)
+        ref = ops.qgemm(a2, w) if a2.shape[0] > 16 else ops.qgemv(a2, w)
+        assert torch.equal(y.reshape(ref.shape), ref if dt is None else ref.to(dt))
+    for a, w in ((x.float(), q4), (xf[:20], q8), (x[:, :128], q4), (x.cpu(), q4), (x[:2].half(), q8), (x[:0], q4)):
+        assert native.linear(a, w, None) is None
+        with pytest.raises(ValueError):
+            ops.qlinear(a, w)
+    with pytest.raises((TypeError, AttributeError)):
+        ops.qlinear(x, q4.packed)
+
+    class Mine(torch.Tensor):
+        pass
+
+    assert native.linear(x.as_subclass(Mine), q4, None) is None
+    experts = [(i4_case(40 + i, 1, 256, 256)[3],) * 3 for i in range(4)]
+    z = torch.randn(5, 4, device=DEV)
+    y = native.moe_ffn(x[:5], z, experts, 2, True)
+    assert y is not None and torch.equal(y, ops.moe_ffn(x[:5], z, tuple(experts), top_k=2))
+    mixed = experts[:3] + [tuple(ops.to_tiles(w) for w in experts[3])]
+    for a, logits, ex, k in ((x[:5], z.double(), experts, 2), (wide[:5, :256], z, experts, 2), (x[:5], z[:, :3], experts, 2), (x[:5], z, mixed, 2),
+                             (x[:5], z, iter(experts), 2), (x[:5], z, experts, 5)):
+        assert native.moe_ffn(a, logits, ex, k, True) is None
+    assert torch.equal(ops.moe_ffn(wide[:5, :256], z, experts, top_k=2), y)
+
+
 def test_moe_route_matches_oracle(ops):
     r = rng(70)
     logits = r.standard_normal((300, 8)).astype(np.float32)

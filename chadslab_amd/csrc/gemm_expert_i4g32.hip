@@ -447,8 +447,14 @@ int expert_prep_h_launch(const uint16_t *h, const uint32_t *rowmax, int P, int K
 
 bool gemm_expert_ok(int H, int F) { return H % 256 == 0 && F % 256 == 0; }
 int gemm_expert_tile_rows() { return EX_MT; }
-// K splits of the down projection: four when every part is a multiple of 512 k, else one
-int gemm_expert_down_splits(int F) { return (F % (512 * 4) == 0) ? 4 : 1; }
+// K splits of the down projection: up to four parts of whole 512-k blocks, the last one possibly shorter.  (Four equal ones or none
+// left the down product of 64 tokens, 2048 x 5632 and 8 experts on 32 workgroups, 52 us of the call's 89; now the call takes 55.  20
+// tokens, 3072 x 12032, 8 experts top 1: 172 -> 105; in row order 30 tokens, 4096 x 7424, 4 experts 119 -> 78.)
+static int down_span(int F, int s) { return ((F + 511) / 512 + s - 1) / s * 512; }
+int gemm_expert_down_splits(int F) {
+    const int s = (F + 511) / 512 < 4 ? (F + 511) / 512 : 4, span = down_span(F, s);
+    return (F + span - 1) / span;
+}
 
 template <int MODE, int NB>
 static int expert_launch(const ExpertArgs &a, hipStream_t st) {
@@ -477,9 +483,13 @@ int gemm_expert_gateup(const GemmGroup *groups, const int32_t *tiles, const int3
 int gemm_expert_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int E, int H, int F, const uint16_t *ha,
                      const float *rs, const uint16_t *ghi, const uint16_t *glo, float *yp, int ksplit, size_t ysplit_stride,
                      hipStream_t st) {
-    ExpertArgs a = {groups, tiles, ha, rs, ghi, glo, nullptr, nullptr, yp, E, H, F, ((F >> 5) + 15) & ~15, F / ksplit, 0, ntiles, ksplit,
+    ExpertArgs a = {groups, tiles, ha, rs, ghi, glo, nullptr, nullptr, yp, E, H, F, ((F >> 5) + 15) & ~15, down_span(F, ksplit), 0, ntiles, ksplit,
                     ysplit_stride};
-    if (H % 512 == 0) {
+    // 128 rows per wave and one workgroup per compute unit, or, where that makes few workgroups, 64 rows and two.  (ntiles is the
+    // most that can exist, E + P / 96; about E + P / 192 of them do.)  us, 64 rows wherever fewer than 192 workgroups result / 128
+    // rows everywhere: 64 tokens of 2048 x 5632 54.7 / 59.5, 20 of 1024 x 1280 29.8 / 32.1, 256 of 4096 x 14336 (320) 265 either way.
+    const int likely = E + (ntiles - E) / 2;
+    if (H % 512 == 0 && (int64_t)likely * (H / 512) * ksplit >= 192) {
         a.nx = H / 512;
         return expert_launch<0, 4>(a, st);
     }

@@ -317,7 +317,7 @@ static int skinny_launch(const GemmGroup *groups, const int32_t *tiles, const in
     }
     const int pairs8 = (mtiles * ksplit + 7) / 8 * 8;  // (list entry, split) pairs, dealt to the 8 XCDs
     hipLaunchKernelGGL((gemm_skinny_i4g32_kernel<MODE>), dim3(pairs8 * ntiles), dim3(256), SK_LDS, st, groups, tiles, tok, E, N, K,
-                       K / ksplit, ystride, ntiles, mtiles, ksplit);
+                       (K / 256 + ksplit - 1) / ksplit * 256, ystride, ntiles, mtiles, ksplit);
     return hip_check(hipGetLastError(), "gemm_skinny launch");
 }
 

@@ -68,9 +68,9 @@ int gemm_expert_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, 
 bool moe_few_ok(int T, int H, int F, int E, int top_k, bool tiled);
 int moe_few_tile_rows();
 int moe_few_down_splits(int F);
-int moe_few_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int E, int F, int H, bool tiled,
+int moe_few_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int T, int E, int F, int H, bool tiled,
                    hipStream_t st);
-int moe_few_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int E, int H, int F, int nsplit, size_t split_stride, bool tiled,
+int moe_few_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int T, int E, int H, int F, int nsplit, size_t split_stride, bool tiled,
                  hipStream_t st);
 
 // Workgroup 0.  Phase 1: softmax + top-k per token.  Phase 2: stable counting sort of the pairs by expert.
@@ -381,11 +381,11 @@ int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe
     }
     if (rc) return rc;
     if (few) {
-        rc = moe_few_gateup(ws.groups, ws.tiles, ws.tok, ntiles, E, F, H, tiled, st);
+        rc = moe_few_gateup(ws.groups, ws.tiles, ws.tok, ntiles, T, E, F, H, tiled, st);
         if (rc) return rc;
         nsplit = moe_few_down_splits(F);
         static_assert(MOE_KSPLIT >= 4, "parts of the down product");
-        rc = moe_few_down(ws.groups, ws.tiles, ntiles, E, H, F, nsplit, (size_t)P * H, tiled, st);
+        rc = moe_few_down(ws.groups, ws.tiles, ntiles, T, E, H, F, nsplit, (size_t)P * H, tiled, st);
         if (rc) return rc;
     } else if (tiled) {
         // (the router's launch also made the fp16 form of the activations) gate/up with the SiLU gate, h to fp16, down split over K
@@ -399,7 +399,9 @@ int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe
     } else if (skinny) {
         rc = gemm_skinny_gateup(ws.groups, ws.tiles, ws.tok, ntiles, E, F, H, st);  // h = bf16(silu(gate) * up), [P,F]
         if (rc) return rc;
-        nsplit = (F % (256 * MOE_KSPLIT) == 0) ? MOE_KSPLIT : 1;
+        // parts of whole 256-k blocks, the last one possibly shorter
+        const int blocks = F / 256, per = (blocks + MOE_KSPLIT - 1) / MOE_KSPLIT;
+        nsplit = (blocks + per - 1) / per;
         rc = gemm_skinny_down(ws.groups, ws.tiles, ntiles, E, H, F, nsplit, (size_t)P * H, st);  // fp32 parts [nsplit][P,H]
         if (rc) return rc;
     } else {
@@ -409,7 +411,8 @@ int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe
         rc = gemm_i4g32_grouped(ws.groups + 2 * E, E, m_max, H, F, true, st);  // down: fp32 [P,H]
         if (rc) return rc;
     }
-    hipLaunchKernelGGL(moe_combine_kernel, dim3(1024), dim3(256), 0, st, ws.yp, ws.pos, ws.w, y, T, H, top_k, nsplit,
+    const int64_t quads = (int64_t)T * (H / 4);
+    hipLaunchKernelGGL(moe_combine_kernel, dim3(quads < 1024 * 256 ? (int)((quads + 255) / 256) : 1024), dim3(256), 0, st, ws.yp, ws.pos, ws.w, y, T, H, top_k, nsplit,
                        (size_t)P * H);
     return hip_check(hipGetLastError(), "moe act/combine launch");
 }

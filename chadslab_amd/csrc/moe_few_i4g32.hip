@@ -9,6 +9,10 @@
 //   * The four waves of a workgroup take the item's blocks of 256 k in turn; their sums meet in LDS once per item.
 //   * Everything goes straight to registers, one block ahead: 4 KiB of weights, the scales and the activation operands
 //     (which the caches serve).  Three waves per SIMD with one block ahead measured 4-8 % faster than two with two ahead.
+//   * Where an expert's rows of x or h fit into LDS (36 KB for all tokens at most: four of 4096 k) they are put there once per
+//     expert and K split, already in operand order, a workgroup's items are neighbours instead of a grid apart, and two blocks
+//     of weights are on their way: 32 of a block's 56 registers held activations, read again for every item.  4 tokens, 8 experts
+//     of 4096 x 14336: gate/up 87 -> 77 us, down 50 -> 49; four blocks in flight are no faster than three.
 //   * In row order a load takes whole 128-byte lines of 8 rows, not 64 bytes of 16 (gate/up 97 -> 87 us); two DPP moves
 //     per register pair put the halves in place.
 // Gate/up | down in us, 8 experts of 4096 x 14336, top 2, the skinny kernel in brackets: 4 tokens 87 | 50 (130 | 72),
@@ -33,6 +37,7 @@ namespace chadq {
 constexpr int FEW_ROWS = 16;     // activation rows of an expert
 constexpr int FEW_ENTRIES = 16;  // experts (one entry of the tile list each, as every expert has at most FEW_ROWS rows)
 constexpr int RB = 2;            // blocks of 16 weight rows per item
+constexpr int kXlBytes = 36 << 10;  // activations in LDS: three workgroups per compute unit with the 17 KB of the rest
 constexpr uint32_t kBeyond = 0x80000000u;
 constexpr int kRange = 0x7FFFFFFF;
 
@@ -53,7 +58,8 @@ __device__ __forceinline__ void order_x8(const uint32_t a[4], uint32_t o[4]) {
     o[3] = __builtin_amdgcn_perm(a[3], a[2], 0x07060302u);
 }
 
-template <int MODE, bool TILED>
+// XL: activations through LDS (at most kXlBytes of them), two blocks of weights on their way beside the one being summed
+template <int MODE, bool TILED, bool XL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void moe_few_i4g32_kernel(
     const GemmGroup *__restrict__ groups, const int32_t *__restrict__ tiles, const int32_t *__restrict__ tok, int ntiles, int E, int N,
     int K, int nsplit, size_t split_stride) {
@@ -93,7 +99,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     while (entries < ntiles && s_ent[entries].rows > 0) ++entries;
     entries = __builtin_amdgcn_readfirstlane(entries);
     const int ntn = MODE == 1 ? N / 16 : N / 32, per = MODE == 1 ? ntn : ntn * nsplit;
-    const int total = entries * per, stride = gridDim.x, nb = K >> 8;
+    const int all = entries * per, nb = K >> 8;
+    // items of a workgroup: every grid-th, or (XL: the activations change with the expert) a run of neighbours
+    const int stride = XL ? 1 : gridDim.x, begin = XL ? (int)((int64_t)blockIdx.x * all / gridDim.x) : blockIdx.x;
+    const int total = XL ? (int)((int64_t)(blockIdx.x + 1) * all / gridDim.x) : all;
     auto first_block = [&](int split) { return MODE == 1 ? split * nb : split * nb / nsplit; };
     auto blocks_of = [&](int item) {  // of each wave
         const int split = MODE == 1 ? 0 : item % per / ntn;
@@ -101,10 +110,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     };
 
     struct Block {  // 256 k = eight scale groups
-        u32x4 x[8], w[RB][2], s[RB];
+        u32x4 x[XL ? 1 : 8], w[RB][2], s[RB];
     };
     // ---- the request side
-    int l_item = blockIdx.x, l_i = 0, l_n = 0, l_kb = 0, l_end = 0;
+    int l_item = begin, l_i = 0, l_n = 0, l_kb = 0, l_end = 0;
     __amdgpu_buffer_rsrc_t wr[RB], sr[RB], xr;
     uint32_t woff = 0, soff = 0, xoff = 0;  // of the lane, in the first row block
     // the second row block: the same rows of the up matrix, or the next 16 rows
@@ -152,8 +161,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             for (int h = 0; h < 2; ++h)  // tile order: non-temporal (5 % faster at 4 tokens; in row order the same)
                 q.w[b][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[b], wv, kb * (TILED ? 4096u : 128u) + b * wblk + h * (TILED ? 2048u : 4u * K), TILED ? 2 : 0);
         }
+        if constexpr (!XL) {
 #pragma unroll
-        for (int g = 0; g < 8; ++g) q.x[g] = __builtin_amdgcn_raw_buffer_load_b128(xr, xv + 64u * g, kb * 512u, 0);
+            for (int g = 0; g < 8; ++g) q.x[g] = __builtin_amdgcn_raw_buffer_load_b128(xr, xv + 64u * g, kb * 512u, 0);
+        }
         l_kb += 4;
         if (++l_i == l_n) {
             l_item += stride;
@@ -167,7 +178,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         __builtin_memcpy(&bias, &v, 16);
     }
     // ---- the summing side
-    int c_item = blockIdx.x, c_i = 0, c_n = 0, par = 0;
+    int c_item = begin, c_i = 0, c_n = 0, par = 0;
     f32x4 acc[RB];
 #pragma unroll
     for (int b = 0; b < RB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -205,7 +216,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         }
         par ^= 1;
     };
+    // XL: the rows of an item's expert, the item's k, in operand order; rows without a token read a block of zeros
+    extern __shared__ __attribute__((aligned(16))) uint8_t s_x[];
+    int x_en = -1, x_split = -1, x_first = 0, x_last = 0;
+    uint32_t x_base = 0, x_mask = 0;
+    auto stage = [&]() {
+        const int en = c_item / per, split = c_item % per / ntn;
+        if (en == x_en && split == x_split) return;
+        x_en = en;
+        x_split = split;
+        x_first = first_block(split);
+        const int span = first_block(split + 1) - x_first, rows = s_ent[en].rows, pitch = span * 512 + 16;
+        x_last = span - 1;
+        const uint8_t *const src = reinterpret_cast<const uint8_t *>(s_ent[en].x) + (size_t)x_first * 512;
+        for (int p = tid; p < rows * span * 32; p += 256) {
+            const int m = p / (span * 32), c = p % (span * 32);
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(src + s_xoff[en][m] + c * 16);
+            const uint32_t a[4] = {v.x, v.y, v.z, v.w};
+            uint32_t o[4];
+            order_x8(a, o);
+            *reinterpret_cast<u32x4 *>(s_x + 512 + m * pitch + c * 16) = u32x4{o[0], o[1], o[2], o[3]};
+        }
+        if (tid < 32) *reinterpret_cast<u32x4 *>(s_x + tid * 16) = u32x4{0, 0, 0, 0};
+        x_base = (r < rows ? 512u + r * pitch : 0u) + 16u * j;
+        x_mask = r < rows ? ~0u : 0u;
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
     auto consume = [&](Block &q) {  // false after the workgroup's last item
+        uint32_t xa = 0;
+        if constexpr (XL) {
+            if (c_i == 0) stage();
+            const int kb = c_i * 4 + wave;  // (a block past the end: its weights and scales are zeros)
+            xa = x_base + ((uint32_t)(kb < x_last ? kb : x_last) * 512u & x_mask);
+        }
         if (!TILED) {  // the two loads trade halves: [h] then holds groups 4h .. 4h+3 of rows 0..15
 #pragma unroll
             for (int b = 0; b < RB; ++b)
@@ -233,12 +279,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             }
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const u32x4 xv = q.x[4 * h + t];
-                const uint32_t a[4] = {xv.x, xv.y, xv.z, xv.w};
-                uint32_t o[4];
-                order_x8(a, o);
                 bf16x8 av;
-                __builtin_memcpy(&av, o, 16);
+                if constexpr (XL) {
+                    av = *reinterpret_cast<const bf16x8 *>(s_x + xa + 64 * (4 * h + t));
+                } else {
+                    const u32x4 xv = q.x[4 * h + t];
+                    const uint32_t a[4] = {xv.x, xv.y, xv.z, xv.w};
+                    uint32_t o[4];
+                    order_x8(a, o);
+                    __builtin_memcpy(&av, o, 16);
+                }
                 const f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bias, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
                 for (int b = 0; b < RB; ++b) {
@@ -264,13 +314,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     if (l_item >= total) return;
     open();
     c_n = l_n;
-    Block q0, q1;
-    request(q0);
-    for (;;) {
-        request(q1);
-        if (!consume(q0)) break;
+    if constexpr (XL) {
+        Block q0, q1, q2;
         request(q0);
-        if (!consume(q1)) break;
+        request(q1);
+        for (;;) {
+            request(q2);
+            if (!consume(q0)) break;
+            request(q0);
+            if (!consume(q1)) break;
+            request(q1);
+            if (!consume(q2)) break;
+        }
+    } else {
+        Block q0, q1;
+        request(q0);
+        for (;;) {
+            request(q1);
+            if (!consume(q0)) break;
+            request(q0);
+            if (!consume(q1)) break;
+        }
     }
 }
 
@@ -295,25 +359,31 @@ int moe_few_tile_rows() { return FEW_ROWS; }
 int moe_few_down_splits(int F) { return F >= 4096 ? 4 : F >= 2048 ? 2 : 1; }
 
 template <int MODE, bool TILED>
-static int few_launch(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int E, int N, int K, int nsplit,
+static int few_launch(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int T, int E, int N, int K, int nsplit,
                       size_t split_stride, hipStream_t st) {
     const int64_t most = (int64_t)ntiles * (MODE == 1 ? N / 16 : N / 32 * nsplit);
-    hipLaunchKernelGGL((moe_few_i4g32_kernel<MODE, TILED>), dim3(most < 768 ? (int)most : 768), dim3(256), 0, st, groups, tiles, tok, ntiles,
-                       E, N, K, nsplit, split_stride);
+    const int nb = K / 256, x_bytes = 512 + T * ((nb + nsplit - 1) / nsplit * 512 + 16);
+    const dim3 grid(most < 768 ? (int)most : 768);
+    if (x_bytes <= kXlBytes)
+        hipLaunchKernelGGL((moe_few_i4g32_kernel<MODE, TILED, true>), grid, dim3(256), x_bytes, st, groups, tiles, tok, ntiles, E, N, K, nsplit,
+                           split_stride);
+    else
+        hipLaunchKernelGGL((moe_few_i4g32_kernel<MODE, TILED, false>), grid, dim3(256), 0, st, groups, tiles, tok, ntiles, E, N, K, nsplit,
+                           split_stride);
     return hip_check(hipGetLastError(), "moe_few launch");
 }
 
 // gate/up with the SiLU gate: h bf16 [P,F] through the down descriptors' x pointers
-int moe_few_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int E, int F, int H, bool tiled,
+int moe_few_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int T, int E, int F, int H, bool tiled,
                    hipStream_t st) {
-    return tiled ? few_launch<1, true>(groups, tiles, tok, ntiles, E, F, H, 1, 0, st) : few_launch<1, false>(groups, tiles, tok, ntiles, E, F, H, 1, 0, st);
+    return tiled ? few_launch<1, true>(groups, tiles, tok, ntiles, T, E, F, H, 1, 0, st) : few_launch<1, false>(groups, tiles, tok, ntiles, T, E, F, H, 1, 0, st);
 }
 
 // down: fp32 parts [nsplit][P,H]
-int moe_few_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int E, int H, int F, int nsplit, size_t split_stride, bool tiled,
+int moe_few_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int T, int E, int H, int F, int nsplit, size_t split_stride, bool tiled,
                  hipStream_t st) {
-    return tiled ? few_launch<0, true>(groups, tiles, nullptr, ntiles, E, H, F, nsplit, split_stride, st)
-                 : few_launch<0, false>(groups, tiles, nullptr, ntiles, E, H, F, nsplit, split_stride, st);
+    return tiled ? few_launch<0, true>(groups, tiles, nullptr, ntiles, T, E, H, F, nsplit, split_stride, st)
+                 : few_launch<0, false>(groups, tiles, nullptr, ntiles, T, E, H, F, nsplit, split_stride, st);
 }
 
 }  // namespace chadq

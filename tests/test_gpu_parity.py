@@ -860,6 +860,19 @@ def test_moe_ffn_few_tokens(ops, t, h, f, e, top_k):
         assert O.rel_l2(O.bf16_to_f32(v), ref) <= TOL_BF16
 
 
+@pytest.mark.parametrize("t,h,f,e,top_k", [(4, 4096, 3584, 8, 2), (1, 512, 2816, 16, 4), (5, 2048, 7424, 3, 2), (2, 1536, 256, 2, 1), (9, 1024, 4864, 4, 4)])
+def test_moe_ffn_few_tokens_activations_through_lds(ops, t, h, f, e, top_k):
+    """Activations of an expert small enough for LDS, in one of the two products or in both; workgroups whose run of items crosses
+    from one expert or K split to the next; K splits of uneven length."""
+    test_moe_ffn_few_tokens(ops, t, h, f, e, top_k)
+
+
+@pytest.mark.parametrize("t,h,f,e,top_k", [(20, 512, 1280, 4, 2), (33, 1024, 2816, 3, 2), (70, 768, 5632, 8, 1), (260, 512, 3328, 2, 2), (40, 1536, 2304, 16, 4)])
+def test_moe_ffn_down_products_in_uneven_k_splits(ops, t, h, f, e, top_k):
+    """F that no power of two divides into parts of whole blocks, in both weight orders; 64 and 128 weight rows per wave."""
+    test_moe_ffn_tiled_agrees_with_row_major_and_oracle(ops, t, h, f, e, top_k)
+
+
 @pytest.mark.parametrize("big", [0.0, 3e37, -2.9e38])
 def test_moe_ffn_few_tokens_large_activations(ops, big):
     """One activation near the top of bf16's range in some tokens (its gate weights have the scale 0, so that the gate stays

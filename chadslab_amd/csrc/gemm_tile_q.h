@@ -14,12 +14,15 @@ GemmTile gemm_tile_pick(int M, int N, int K, bool int4);
 // y bf16 [M,N]; gemm_tile_q_ok(K)
 int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st);
 int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st);
-// int4 weights taken exactly (nothing rounded before the fp32 sums); K % 256 == 0, x, wp and sc 16-byte aligned
+// int4 weights taken exactly (nothing rounded before the fp32 sums); K % 256 == 0, x, wp and sc 16-byte aligned unless it says otherwise
 constexpr int kExactMaxSplits = 8;
 int gemm_exact_splits(int M, int N, int K);  // K splits to use for gemm_exact_f32_launch
 // y_parts fp32 [ksplit][M,N]
 int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
                           hipStream_t st);
+// y [M,N] fp32 or bf16, at most 32 rows, any K % 32 == 0 with gemm_tile_q_ok(K), any alignment of the scales
+int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, bool bf16_out,
+                               hipStream_t st);
 // weight rows in (gate, up) pairs: h[m,i] = bf16(gelu_tanh(y[m,2i]) * y[m,2i+1]), [M, N/2]
 int gemm_exact_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st);
 

@@ -228,7 +228,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 
     // ---- fragment read offsets: row nl of a 32-row block, the wave's pieces SL kq + t (EXACT: 2 t + kq, so that two slices are one
     // scale group); the lane's packed weights
-    static_assert(!EXACT || (I4 && !GUARD && NB == 1), "exact weights: int4, whole blocks of 256 k, one column block");
+    static_assert(!EXACT || (I4 && NB == 1 && (!GUARD || KW == 64)), "exact weights: int4, one column block");
     uint32_t foff[SL];
 #pragma unroll
     for (int t = 0; t < SL; ++t)
@@ -301,23 +301,25 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     // value that applies the scale (times 2^9).  A pair of MFMAs runs beside the FMAs of the pair before it.
     constexpr int RING = Q >= 4 ? 4 : 2;
     uint32_t wv[GR][2], wnx[GR][2];  // the lane's packed words of a step [group][slice], of the next one
-    uint32_t sraw;                   // its scales
+    uint32_t sraw[GR];               // its scales
     float sc2[GR], s_last = 0.f;     // ... as floats, that of the group whose sums are next
     auto fetch = [&](int step, const uint8_t *stage) {
 #pragma unroll
         for (int g = 0; g < GR; ++g)
 #pragma unroll
             for (int e = 0; e < 2; ++e) wnx[g][e] = *reinterpret_cast<const uint32_t *>(stage + woff[g] + e * 8 + kq * 4);
-        const uint8_t *const sp = stage + C::A_STAGE + C::B_STAGE + (wn * 32 + nl) * 16;
-        if (GR == 2) sraw = *reinterpret_cast<const uint32_t *>(sp + ((step * WK + wk) & 3) * 4);
-        else sraw = *reinterpret_cast<const uint16_t *>(sp + ((step * WK + wk) & 7) * 2);
+        const uint8_t *const sp = stage + C::A_STAGE + C::B_STAGE;
+#pragma unroll
+        for (int g = 0; g < GR; ++g)
+            sraw[g] = *reinterpret_cast<const uint16_t *>(GUARD ? sp + wave * 256 + (nl + 32 * g) * 4
+                                                                : sp + (wn * 32 + nl) * 16 + ((step * WK + wk) * GR + g & 7) * 2);
     };
-    auto prep = [&]() {
+    auto prep = [&](int step) {
 #pragma unroll
         for (int g = 0; g < GR; ++g) {
             wv[g][0] = wnx[g][0];
             wv[g][1] = wnx[g][1];
-            sc2[g] = 512.f * f16_bits_to_f32((uint16_t)(sraw >> (16 * g)));
+            sc2[g] = (GUARD && kbeg + step * C::KS + wk * KW + 32 * g >= K) ? 0.f : 512.f * f16_bits_to_f32((uint16_t)sraw[g]);
         }
     };
     bf16x8 bo[2], bnx[2];  // operands of the present group, of the next one
@@ -339,7 +341,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
         for (int r = 0; r < first(AFTER); ++r) request(r, ST - 1, lds, lds + (ST - 1) * C::STAGE, false);
     }
-    prep();
+    prep(0);
     bo[0] = signed8_i4(wv[0][0]);
     bo[1] = signed8_i4(wv[0][1]);
     auto step = [&](int i, int slot, auto pending_c, auto before_c, auto more_c, auto whole_c) {
@@ -377,7 +379,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             if (mb == 0) s_last = sc2[g];
             // the next group's operands, a share beside each pair
             if (g + 1 < GR || pending >= 0) {
-                if (g + 1 == GR && mb == (GR == 1 && MB > 2 ? 2 : 0)) prep();
+                if (g + 1 == GR && mb == (GR == 1 && MB > 2 ? 2 : 0)) prep(i + 1);
                 if (mb == MB / 2 - (MB > 1)) bnx[0] = signed8_i4(wv[(g + 1) % GR][0]);
                 if (mb == MB - 1) bnx[1] = signed8_i4(wv[(g + 1) % GR][1]);
             }
@@ -744,6 +746,14 @@ static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc
         if (rounds(256) * 45.f < rounds(128) * 30.f) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
     }
     return tileq::launch<true, 1, 4, 2, 4, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+}
+
+// Decode products of at most 32 rows whose K (or scales) the GEMV of gemv_i4g32_mfma.hip does not take: y fp32 or bf16 [M,N] in one
+// pass over the weights.
+int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, bool bf16_out,
+                               hipStream_t st) {
+    return bf16_out ? tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, true, true, tileq::EPI_BF16>(x, wp, sc, y, M, N, K, 1, st)
+                    : tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, true, true, tileq::EPI_F32>(x, wp, sc, y, M, N, K, 1, st);
 }
 
 // K splits that make the launch shortest: rounds of workgroups times the k of each (and what a workgroup costs besides, about

@@ -12,6 +12,7 @@
 // fp32 for integer-valued x, so integer accumulation is bit-exact.  The 64 partial sums of a row are
 // folded with DPP adds; no LDS is used.
 #include "chadq_common.h"
+#include "gemm_tile_q.h"
 
 namespace chadq {
 
@@ -158,6 +159,12 @@ static void launch_rows(const uint16_t *x, const uint8_t *wp, const uint16_t *sc
 
 int gemv_i4g32_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K,
                         bool bf16_out, hipStream_t st) {
+    // Five rows and more (three of more than 4096 k): one pass over the weights on the matrix cores, weights taken exactly there
+    // too.  The kernels of this file stream them once per pair of rows, the generic one once per row.  us, here / there, for 4, 8
+    // and 16 rows: 4096 x 4064 12.4 / 13.0, 24.8 / 13.1, 49.5 / 13.3; 8192 x 8160 37.4 / 24.4, 70.9 / 24.6, 137 / 24.7; 2 rows of
+    // the latter 20.4 / 24.0.
+    if (M >= (K <= 4096 ? 5 : 3) && M <= 32 && gemm_tile_q_ok(K) && aligned16(x) && aligned16(wp))
+        return gemm_exact_few_rows_launch(x, wp, sc, y, M, N, K, bf16_out, st);
     if (K <= 4096) {
         // rows per wave: enough waves to fill 256 CUs several times over, few enough to keep loads deep
         const bool big = N >= 8192;

@@ -227,6 +227,22 @@ def test_gemv_int4_zero_weights_and_special_scales(ops):
         assert np.array_equal(ops.qgemv(bf16_tensor(O.f32_to_bf16(e)), qw).cpu().numpy()[0], d[:, kk])
 
 
+# K not a multiple of 256: the matrix cores take five rows and more (three of more than 4096 k), whole and part scale groups of a step
+@pytest.mark.parametrize("m,n,k", [(5, 1, 32), (16, 65, 96), (7, 63, 1056), (16, 200, 4064), (3, 130, 4128), (5, 31, 4128), (3, 77, 8160),
+                                   (16, 77, 8160)])
+def test_gemv_int4_other_k_several_rows(ops, m, n, k):
+    packed, s, xb, q4 = i4_case(80 + m, m, n, k)
+    ref = O.qgemm_int4g32_f64(xb, packed, s)
+    # every product is exact; what is left is the fp32 sum of at most k terms and the scales' products
+    u = np.stack([packed & 15, packed >> 4], 2).reshape(n, k).astype(np.float64) - 8
+    mag = np.abs(O.bf16_to_f32(xb)).astype(np.float64) @ (np.abs(u) * np.repeat(s.astype(np.float64), 32, 1)).T
+    x = bf16_tensor(xb)
+    y = ops.qgemv(x, q4).cpu().numpy()
+    assert (np.abs(y - ref) <= (k / 8 + 8) * 2.0**-24 * mag).all()
+    yb = ops.qlinear(x, q4, out_dtype=torch.bfloat16)
+    assert (np.abs(O.bf16_to_f32(bits(yb)) - ref) <= 2.0**-8 * np.abs(ref) + (k / 8 + 8) * 2.0**-24 * mag).all()
+
+
 # ------------------------------------------------------------------ GEMV int8 (config 0)
 @pytest.mark.parametrize("m,n,k", [(1, 16384, 2048), (1, 64, 16), (3, 100, 1040), (2, 77, 4096), (16, 40, 256),
                                    # rows of 2049..8192 k (4 or 8 chunks per row), and beyond (the general kernel)

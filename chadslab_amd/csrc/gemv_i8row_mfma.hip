@@ -5,7 +5,7 @@
 // The fp32 activations are what has to change shape: per activation row and per 2048 k, x is written in fixed point
 // with a power-of-two scale, X = rint(x * 2^(20 - e)) with 2^e <= max|x| < 2^(e+1) (|X| <= 2^21), and X as three
 // balanced base-256 digits, X = a0 * 2^16 + a1 * 2^8 + a2 with -128 <= a <= 127.  Each digit is one int8 operand
-// row; the three int32 dot products are exact and meet again in fp32: y = s[n] * sum over blocks 2^(e-20) * (D0 *
+// row; the three int32 dot products are exact and meet again in float64: y = s[n] * sum over blocks 2^(e-20) * (D0 *
 // 2^16 + D1 * 2^8 + D2).  What is dropped is at most 2^-21 of the block's largest |x| per element, so a result is off by
 // at most scale[n] * sum over blocks of 2^-21 * max_block|x| * sum_{k in block} |W[n,k]| (the result is held to a 1e-3
 // relative tolerance; one outlier among the activations costs the small elements of its block their low bits, also
@@ -22,12 +22,20 @@
 //   A = activations.  SETS <= 2 (M <= 4, M <= 8): operand row 4q + d of set s is digit d of activation row 4s + q
 //       (row 4q + 3 is zero), so the three digit sums of a result sit in one lane's accumulator registers.  SETS = 3
 //       (M <= 16): set d holds digit d of all 16 rows.
-// Workgroup = 8 waves on 64 weight rows: wave (rw, kh) multiplies rows 16 rw .. 16 rw + 15 with the kh-th 1024 k of
-// every 2048, so at K <= 2048 a wave's 16 loads - all of its weights - are in flight from the start and nothing
-// about the activations can stall the stream.  The 512 threads turn 2048 k of all M activation rows into operand
+// Workgroup = 8 waves on RWS = 1, 2 or 4 blocks of 16 weight rows: wave (rw, kh) multiplies block rw with the kh-th of
+// 8 / RWS parts of every 2048 k, so at K <= 2048 a wave's loads - all of its weights - are in flight from the start and
+// nothing about the activations can stall the stream.  The 512 threads turn 2048 k of all M activation rows into operand
 // order in LDS (SETS x 32 KiB); the activation loads are issued before the weight loads because memory returns in
 // order.  Longer rows repeat this per 2048 k with the ring refilled as it is consumed (every load unconditional:
-// addresses past the end are clamped and their activations staged as zeros).  The two K halves meet in LDS at the end.
+// addresses past the end are clamped and their activations staged as zeros).  The K parts meet in LDS at the end.
+//
+// What bounds it is how fast one CU takes its weights, about 40 bytes per ns: 3.8 us per 64 rows and 2048 k, however
+// few the workgroups are.  So the rows are dealt out until the 256 CUs have one workgroup each: 16 to a workgroup up to
+// 4096 rows, 32 up to 8192, else 64.  us at 16 / 32 / 64 rows (64 was all there was), 1 and 16 activation rows:
+// 2048 x 2048 4.8 / 4.2 / 5.8 and 8.1 / 8.7 / 10.9; 4096 x 4096 6.9 / 7.2 / 10.2 and 16.4 / 17.0 / 21.1; 2048 x 16384
+// 14.7 / 19.1 / 32.9 and 47 / 50 / 65; 8192 x 4096 10.8 / 9.0 / 11.0 and 32 / 18 / 21; 16384 x 2048 9.6 / 7.1 / 7.4 and
+// 29 / 17 / 12.  Activations requested two 2048-blocks ahead gave nothing (and spilled at 16 rows).  M plays no part in
+// the rule: a row's result does not depend on how many rows come with it.
 #include <type_traits>
 
 #include "chadq_common.h"
@@ -36,9 +44,11 @@ namespace chadq {
 
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 
-template <int SETS>
+// RWS: blocks of 16 weight rows per workgroup (1, 2 or 4), each shared by 8 / RWS waves
+template <int SETS, int RWS>
 struct GemvI8Cfg {
-    static constexpr int PAIRS = 8;                       // 128-k pair-steps per wave and round (1024 k)
+    static constexpr int PAIRS = 8;                       // 128-k pair-steps per round (1024 k)
+    static constexpr int KHS = 8 / RWS, STEPS = 16 / KHS; // waves of a row block, pair-steps of each per 2048 k
     static constexpr int PAIR_BYTES = SETS * 2048;        // A operands of one pair-step: SETS x 2 MFMAs x 1 KiB
     static constexpr int BUF_BYTES = PAIRS * PAIR_BYTES;  // one round's operands: SETS x 16 KiB
     static constexpr int MROWS = SETS == 3 ? 16 : 4 * SETS;  // activation rows the staging covers
@@ -46,8 +56,8 @@ struct GemvI8Cfg {
     static constexpr int XIT = 128 / PARTS;               // 16-k pieces a thread stages per 2048 k: 1 / 2 / 4
     static constexpr int RES = SETS == 3 ? 4 : SETS;      // results per lane
     static constexpr int AMAX_OFF = 2 * BUF_BYTES;        // [MROWS][8 waves] largest |x| bits
-    static constexpr int FOLD_OFF = AMAX_OFF + 16 * 8 * 4;  // [4 row blocks][64 lanes] x 16 B from the upper K half
-    static constexpr int LDS = FOLD_OFF + 4 * 64 * 16;
+    static constexpr int FOLD_OFF = AMAX_OFF + 16 * 8 * 4;  // [waves but the first of each row block][RES][64 lanes] float64
+    static constexpr int LDS = FOLD_OFF + (8 - RWS) * RES * 64 * 8;
 };
 
 // lanes 8..15 of every row of 16 take src from the lane 8 below, lanes 0..7 keep old (BANKS = 0xC); or lanes 0..7 take
@@ -57,26 +67,26 @@ __device__ __forceinline__ int half_row_merge(uint32_t old, uint32_t src) {
     return __builtin_amdgcn_update_dpp((int)old, (int)src, 0x128, 0xF, BANKS, false);
 }
 
-template <int SETS>
+template <int SETS, int RWS>
 __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__restrict__ x, const int8_t *w8,
                                                               const float *sc, float *__restrict__ y, int M, int N,
                                                               int K, int bf16_out) {
-    using C = GemvI8Cfg<SETS>;
+    using C = GemvI8Cfg<SETS, RWS>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint32_t *amax = reinterpret_cast<uint32_t *>(smem + C::AMAX_OFF);
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int rw = wave & 3, kh = wave >> 2;
+    const int rw = wave % RWS, kh = wave / RWS;
     const int c = lane & 15, g = lane >> 4;
-    const int n0 = blockIdx.x * 64 + rw * 16;
+    const int n0 = blockIdx.x * (16 * RWS) + rw * 16;
     // the two loads of a pair-step: rows (c & 7) and 8 + (c & 7) of the wave's 16, piece (c >> 3) + 2g of 128 bytes;
     // rows past the end are clamped, computed and never stored
     const int rx = (n0 + (c & 7) < N) ? n0 + (c & 7) : N - 1, ry = (n0 + 8 + (c & 7) < N) ? n0 + 8 + (c & 7) : N - 1;
     const unsigned char *wbase = reinterpret_cast<const unsigned char *>(w8) + 16 * ((c >> 3) + 2 * g);
     const unsigned char *wpx = wbase + (size_t)rx * K, *wpy = wbase + (size_t)ry * K;
     const int pairs = K >> 7, supers = (K + 2047) >> 11;
-    auto pair_off = [&](int sr, int t) {  // byte offset of pair-step t of this wave's round in 2048-block sr
-        const int p = (sr * 2 + kh) * C::PAIRS + t;
+    auto pair_off = [&](int sr, int t) {  // byte offset of pair-step t of this wave in 2048-block sr
+        const int p = sr * 16 + kh * C::STEPS + t;
         return (size_t)((p < pairs) ? p : pairs - 1) * 128;
     };
 
@@ -180,9 +190,9 @@ __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__res
     };
 
     request_x(0);
-    u32x4 ring[2 * C::PAIRS];
+    u32x4 ring[2 * C::STEPS];
 #pragma unroll
-    for (int t = 0; t < C::PAIRS; ++t) {
+    for (int t = 0; t < C::STEPS; ++t) {
         ring[2 * t] = load_nt_b128(wpx + pair_off(0, t));
         ring[2 * t + 1] = load_nt_b128(wpy + pair_off(0, t));
     }
@@ -194,16 +204,17 @@ __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__res
     if (supers > 1) request_x(1);
     __syncthreads();
 
-    float yacc[C::RES];
+    double yacc[C::RES];
 #pragma unroll
-    for (int r = 0; r < C::RES; ++r) yacc[r] = 0.f;
-    const unsigned char *abuf = smem + kh * C::BUF_BYTES;
-    auto multiply = [&](int sr, auto refill) {  // this wave's 1024 k of 2048-block sr; refill: request the next block's
+    for (int r = 0; r < C::RES; ++r) yacc[r] = 0.;
+    const int t0 = kh * C::STEPS % C::PAIRS;  // the wave's first pair-step in its round of 1024 k
+    const unsigned char *abuf = smem + kh * C::STEPS / C::PAIRS * C::BUF_BYTES + t0 * C::PAIR_BYTES;
+    auto multiply = [&](int sr, auto refill) {  // this wave's part of 2048-block sr; refill: request the next block's
         i32x4 acc[SETS][2];
 #pragma unroll
         for (int s = 0; s < SETS; ++s) acc[s][0] = acc[s][1] = i32x4{0, 0, 0, 0};
 #pragma unroll
-        for (int t = 0; t < C::PAIRS; ++t) {
+        for (int t = 0; t < C::STEPS; ++t) {
             // wait for this pair-step's weights, then put the request for the next 2048-block in the queue
             asm volatile("" : "+v"(ring[2 * t]), "+v"(ring[2 * t + 1]));
             const u32x4 wx = ring[2 * t], wy = ring[2 * t + 1];
@@ -221,28 +232,25 @@ __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__res
             for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
                 for (int s = 0; s < SETS; ++s) {
-                    const int slot = (SETS == 3) ? lane : (lane ^ (jj + 2 * (t & 1)));
+                    const int slot = (SETS == 3) ? lane : (lane ^ (jj + 2 * (t & 1)));  // (t0 is even)
                     const i32x4 av = *reinterpret_cast<const i32x4 *>(abuf + t * C::PAIR_BYTES + (s * 2 + jj) * 1024 + slot * 16);
                     acc[s][jj] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, jj ? b1 : b0, acc[s][jj], 0, 0, 0);
                 }
         }
-        // the block's digit sums -> fp32 with the block's scales.  D0 * 2^16 + D1 * 2^8 + D2 can need more than the 24
-        // bits of a float before its terms cancel, so the three are combined in float64 (exact: below 2^53) and rounded
-        // to fp32 once
-        auto combine = [](int d0, int d1, int d2) {
-            return (float)__builtin_fma((double)d0, 65536.0, __builtin_fma((double)d1, 256.0, (double)d2));
-        };
+        // the digit sums meet in float64, where D0 * 2^16 + D1 * 2^8 + D2 (more than the 24 bits of a float before its
+        // terms cancel) and its product with the block's power of two are exact; the waves' sums are rounded to fp32 once
+        auto combine = [](int d0, int d1, int d2) { return __builtin_fma((double)d0, 65536.0, __builtin_fma((double)d1, 256.0, (double)d2)); };
         if constexpr (SETS == 3) {
             const i32x4 e0 = acc[0][0] + acc[0][1], e1 = acc[1][0] + acc[1][1], e2 = acc[2][0] + acc[2][1];
             const int q0[4] = {e0.x, e0.y, e0.z, e0.w}, q1[4] = {e1.x, e1.y, e1.z, e1.w}, q2[4] = {e2.x, e2.y, e2.z, e2.w};
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                yacc[r] = __builtin_fmaf(bscale[r], combine(q0[r], q1[r], q2[r]), yacc[r]);
+                yacc[r] = __builtin_fma((double)bscale[r], combine(q0[r], q1[r], q2[r]), yacc[r]);
         } else {
 #pragma unroll
             for (int s = 0; s < SETS; ++s) {
                 const i32x4 e = acc[s][0] + acc[s][1];
-                yacc[s] = __builtin_fmaf(bscale[s], combine(e.x, e.y, e.z), yacc[s]);
+                yacc[s] = __builtin_fma((double)bscale[s], combine(e.x, e.y, e.z), yacc[s]);
             }
         }
     };
@@ -255,44 +263,48 @@ __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__res
     }
     multiply(supers - 1, std::false_type{});
 
-    // the upper K half hands its sums over
-    f32x4 *fold = reinterpret_cast<f32x4 *>(smem + C::FOLD_OFF) + rw * 64 + lane;
+    // the other waves of the row block hand their sums over
+    double *const fold = reinterpret_cast<double *>(smem + C::FOLD_OFF) + rw * C::RES * 64 + lane;
     if (kh) {
-        f32x4 o = {0.f, 0.f, 0.f, 0.f};
-        o.x = yacc[0];
-        if constexpr (C::RES > 1) o.y = yacc[1];
-        if constexpr (C::RES > 2) {
-            o.z = yacc[2];
-            o.w = yacc[3];
-        }
-        *fold = o;
+#pragma unroll
+        for (int r = 0; r < C::RES; ++r) fold[((kh - 1) * RWS * C::RES + r) * 64] = yacc[r];
     }
     __syncthreads();
     if (kh) return;
-    const f32x4 o = *fold;
-    const float other[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+    for (int h = 0; h < C::KHS - 1; ++h)
+#pragma unroll
+        for (int r = 0; r < C::RES; ++r) yacc[r] += fold[(h * RWS * C::RES + r) * 64];
     const int n = n0 + c;
     const float scale = (n < N) ? sc[n] : 0.f;
 #pragma unroll
     for (int r = 0; r < C::RES; ++r) {
         const int m = (SETS == 3) ? 4 * g + r : 4 * r + g;
-        if (m < M && n < N) store_sum(y, (size_t)m * N + n, (yacc[r] + other[r]) * scale, bf16_out);
+        if (m < M && n < N) store_sum(y, (size_t)m * N + n, (float)yacc[r] * scale, bf16_out);
     }
 }
 
 bool gemv_i8row_mfma_ok(int M, int K) { return M >= 1 && M <= 16 && K % 128 == 0; }
 
-template <int SETS>
+template <int SETS, int RWS>
 static int launch_i8_mfma(const float *x, const int8_t *w8, const float *sc, float *y, int M, int N, int K, bool bf16_out, hipStream_t st) {
-    using C = GemvI8Cfg<SETS>;
+    using C = GemvI8Cfg<SETS, RWS>;
     static std::atomic<bool> attr_set{false};  // setting it twice from two threads is harmless
     if (!attr_set.load(std::memory_order_acquire)) {
-        CHADQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_i8row_mfma_kernel<SETS>),
+        CHADQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_i8row_mfma_kernel<SETS, RWS>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS));
         attr_set.store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL(gemv_i8row_mfma_kernel<SETS>, dim3((N + 63) / 64), dim3(512), C::LDS, st, x, w8, sc, y, M, N, K, (int)bf16_out);
+    hipLaunchKernelGGL((gemv_i8row_mfma_kernel<SETS, RWS>), dim3((N + 16 * RWS - 1) / (16 * RWS)), dim3(512), C::LDS, st, x, w8, sc, y, M, N, K,
+                       (int)bf16_out);
     return hip_check(hipGetLastError(), "gemv_i8row_mfma launch");
+}
+
+template <int SETS>
+static int launch_i8_mfma(const float *x, const int8_t *w8, const float *sc, float *y, int M, int N, int K, bool bf16_out, hipStream_t st) {
+    if (N <= 4096) return launch_i8_mfma<SETS, 1>(x, w8, sc, y, M, N, K, bf16_out, st);
+    if (N <= 8192) return launch_i8_mfma<SETS, 2>(x, w8, sc, y, M, N, K, bf16_out, st);
+    return launch_i8_mfma<SETS, 4>(x, w8, sc, y, M, N, K, bf16_out, st);
 }
 
 // 1..16 activation rows, K a multiple of 128 (x and w8 16-byte aligned as for every int8 GEMV)

@@ -266,6 +266,18 @@ def test_gemv_int8_matrix_core(ops, m, n, k):
     assert O.rel_l2(y, O.qgemv_int8_f64(x, w, s)) <= TOL_F32
 
 
+# 16, 32 or 64 weight rows to a workgroup: either side of each line, ragged, with less k than its waves have parts
+@pytest.mark.parametrize("n", [4096, 4097, 8192, 8205])
+@pytest.mark.parametrize("m,k", [(1, 128), (4, 2048), (6, 2176), (16, 4224)])
+def test_gemv_int8_matrix_core_rows_per_workgroup(ops, m, n, k):
+    x, w, s, q8 = i8_case(340 + m + n, m, n, k)
+    y = ops.qgemv(torch.from_numpy(x).to(DEV), q8).cpu().numpy()
+    ref = O.qgemv_int8_f64(x, w, s)
+    # every element: fixed point drops at most 2^-21 of the row's largest |x| per product, the one rounding to fp32 and the scale 2^-23
+    bound = 2.0**-21 * np.abs(x).max(1)[:, None] * (np.abs(w.astype(np.float64)).sum(1) * s)[None] + 2.0**-22 * np.abs(ref)
+    assert (np.abs(y - ref) <= bound).all()
+
+
 @pytest.mark.parametrize("m,n,k", [(2, 300, 2048), (2, 300, 2064), (1, 100, 4096), (5, 333, 4096), (8, 64, 2048), (16, 70, 6144),
                                    (11, 90, 128)])
 def test_gemv_int8_integer_exact(ops, m, n, k):

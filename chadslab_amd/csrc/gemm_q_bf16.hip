@@ -1,6 +1,7 @@
 // Prefill dequant-GEMM:  y[m,n] = bf16( sum_k x[m,k] * w[n,k] ),  x bf16 [M,K], fp32 accumulate on MFMA.
 //   int4 group-32:  w = bf16_rne((u-8) * scale[n,k/32])          (dequantised to bf16 for the matrix core)
 //   int8 per-row :  w = W[n,k] exactly in bf16, scale[n] applied to the fp32 accumulator afterwards
+// For rows of 2^22 k and more and for grouped launches; other products take the tiles of gemm_tile_q.hip.
 //
 // Workgroup = 4 waves, output tile 128 x 64, and the four waves split K: wave w owns every fourth slice of
 // K and accumulates a full 128 x 64 partial tile (8 accumulators of v_mfma_f32_32x32x16_bf16).  That choice

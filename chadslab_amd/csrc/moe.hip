@@ -73,6 +73,52 @@ int moe_few_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t 
 int moe_few_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int T, int E, int H, int F, int nsplit, size_t split_stride, bool tiled,
                  hipStream_t st);
 
+// Token t: softmax over its E logits, the top_k largest (the lowest index wins ties) and their weights; s_e: the choices in LDS too.
+__device__ __forceinline__ void route_token(const float *__restrict__ logits, int32_t *__restrict__ idx, float *__restrict__ w, int t, int E,
+                                            int top_k, int renorm, uint8_t *s_e) {
+    // the token's logits go to registers once (every load in flight together); places past E hold -inf and are
+    // never candidates
+    const float *z = logits + (size_t)t * E;
+    float zr[MOE_MAX_E];
+#pragma unroll
+    for (int e = 0; e < MOE_MAX_E; ++e) zr[e] = (e < E) ? z[e] : -INFINITY;
+    float mx = zr[0];
+#pragma unroll
+    for (int e = 1; e < MOE_MAX_E; ++e)
+        if (e < E) mx = fmaxf(mx, zr[e]);
+    float sum = 0.f;
+#pragma unroll
+    for (int e = 0; e < MOE_MAX_E; ++e)
+        if (e < E) sum += __expf(zr[e] - mx);
+    uint32_t taken = 0;
+    int chosen[MOE_MAX_K];
+    float pw[MOE_MAX_K], wsum = 0.f;
+#pragma unroll
+    for (int j = 0; j < MOE_MAX_K; ++j) {
+        if (j < top_k) {
+            int best = -1;
+            float bv = 0.f;
+#pragma unroll
+            for (int e = 0; e < MOE_MAX_E; ++e)
+                if (e < E && !((taken >> e) & 1u) && (best < 0 || zr[e] > bv)) {  // strict >: the lowest index wins ties
+                    best = e;
+                    bv = zr[e];
+                }
+            taken |= 1u << best;
+            chosen[j] = best;
+            pw[j] = __expf(bv - mx) / sum;
+            wsum += pw[j];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < MOE_MAX_K; ++j)
+        if (j < top_k) {
+            idx[(size_t)t * top_k + j] = chosen[j];
+            w[(size_t)t * top_k + j] = renorm ? pw[j] / wsum : pw[j];
+            if (s_e) s_e[t * top_k + j] = (uint8_t)chosen[j];
+        }
+}
+
 // Workgroup 0.  Phase 1: softmax + top-k per token.  Phase 2: stable counting sort of the pairs by expert.
 // Phase 3: descriptors.  idx/w may be the caller's arrays (chadq_moe_route) with everything else null.
 // Workgroups 1..T (launched for the tile-order path only, prep_x != nullptr): workgroup t+1 turns row t of the
@@ -114,47 +160,7 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const float *__restrict
     }
 
     for (int t = tid; t < T; t += B) {
-        // the token's logits go to registers once (every load in flight together); places past E hold -inf and are
-        // never candidates
-        const float *z = logits + (size_t)t * E;
-        float zr[MOE_MAX_E];
-#pragma unroll
-        for (int e = 0; e < MOE_MAX_E; ++e) zr[e] = (e < E) ? z[e] : -INFINITY;
-        float mx = zr[0];
-#pragma unroll
-        for (int e = 1; e < MOE_MAX_E; ++e)
-            if (e < E) mx = fmaxf(mx, zr[e]);
-        float sum = 0.f;
-#pragma unroll
-        for (int e = 0; e < MOE_MAX_E; ++e)
-            if (e < E) sum += __expf(zr[e] - mx);
-        uint32_t taken = 0;
-        int chosen[MOE_MAX_K];
-        float pw[MOE_MAX_K], wsum = 0.f;
-#pragma unroll
-        for (int j = 0; j < MOE_MAX_K; ++j) {
-            if (j < top_k) {
-                int best = -1;
-                float bv = 0.f;
-#pragma unroll
-                for (int e = 0; e < MOE_MAX_E; ++e)
-                    if (e < E && !((taken >> e) & 1u) && (best < 0 || zr[e] > bv)) {  // strict >: the lowest index wins ties
-                        best = e;
-                        bv = zr[e];
-                    }
-                taken |= 1u << best;
-                chosen[j] = best;
-                pw[j] = __expf(bv - mx) / sum;
-                wsum += pw[j];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < MOE_MAX_K; ++j)
-            if (j < top_k) {
-                idx[(size_t)t * top_k + j] = chosen[j];
-                w[(size_t)t * top_k + j] = renorm ? pw[j] / wsum : pw[j];
-                if (in_lds) s_e[t * top_k + j] = (uint8_t)chosen[j];
-            }
+        route_token(logits, idx, w, t, E, top_k, renorm, in_lds ? s_e : nullptr);
     }
     if (!ws.pos) return;  // routing only
     if (prep_x)
@@ -241,6 +247,59 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(const float *__restrict
             if (cls_rem == c && at < ntiles_max) ws.tiles[at] = e | (nfull << 16);
         }
         for (int n = total + tid; n < ntiles_max; n += B) ws.tiles[n] = -1;
+    }
+}
+
+// The same for a few tokens (at most 64 pairs, one token tile per expert): one wave, a lane per token and then per pair.
+// What bounds it is the chain of memory and LDS round trips and barriers; here it is logits -> LDS -> stores.  An expert's
+// place among the rows and in the tile list comes from the ballots of the experts before it.  The whole call, us, with the
+// general router in brackets: 4 tokens, 8 experts of 4096 x 14336 126.5 (128.5), 1 token 61 (63), 2 tokens of 1024 x 2816 22.5 (25).
+__global__ __launch_bounds__(64) void moe_route_few_kernel(const float *__restrict__ logits, int T, int E, int top_k, int renorm, MoeWs ws,
+                                                           MoeExperts ex, int H, int F, const uint16_t *__restrict__ x) {
+    __shared__ uint8_t s_e[64];
+    const int lane = threadIdx.x, P = T * top_k;
+    GemmGroup gg{x, nullptr, nullptr, nullptr, 0, 0}, gu = gg, gd = gg;
+    if (lane < E) {  // the pointers sit in the kernel-argument buffer: asked for now, used at the end
+        gg.w = ex.wg[lane];
+        gg.sc = ex.sg[lane];
+        gu.w = ex.wu[lane];
+        gu.sc = ex.su[lane];
+        gd.w = ex.wd[lane];
+        gd.sc = ex.sd[lane];
+    }
+    if (lane < T) route_token(logits, ws.idx, ws.w, lane, E, top_k, renorm, s_e);
+    __syncthreads();
+    const int e_mine = lane < P ? (int)s_e[lane] : -1;
+    int row = 0, o = 0, m = 0, tile = -1, first = 0, ntiles = 0;
+    for (int e = 0; e < E; ++e) {
+        const unsigned long long hit = __ballot(e_mine == e);
+        const int n = __popcll(hit);
+        if (e_mine == e) row = first + __popcll(hit & ((1ull << lane) - 1ull));
+        if (lane == e) {
+            o = first;
+            m = n;
+        }
+        if (lane == ntiles && n > 0) tile = e;
+        first += n;
+        ntiles += n > 0;
+    }
+    if (lane < P) {
+        ws.pos[lane] = row;
+        ws.tok[row] = lane / top_k;
+    }
+    if (lane < E) {
+        ws.cnt[lane] = m;
+        ws.cnt[E + lane] = o;
+        ws.tiles[lane] = tile;
+        gg.y = ws.g + (size_t)o * F;
+        gu.y = ws.u + (size_t)o * F;
+        gd.x = ws.h + (size_t)o * F;
+        gd.y = ws.yp + (size_t)o * H;
+        gg.M = gu.M = gd.M = m;
+        gg.pad = gu.pad = o;
+        ws.groups[lane] = gg;
+        ws.groups[E + lane] = gu;
+        ws.groups[2 * E + lane] = gd;
     }
 }
 
@@ -368,7 +427,10 @@ int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe
     if (tiled && !skinny) return fail(CHADQ_ERR_ALIGN, "moe_ffn (tiled): weights and scales must be 16-byte aligned, H and F multiples of 256");
     const int route_threads = P <= 256 ? 256 : P <= 512 ? 512 : 1024;
     int rc;
-    if (skinny) {  // the router also lists the token tiles; gate/up read the activations through tok
+    if (few && P <= 64) {  // tile_rows == 16 >= T: one tile per expert hit, ntiles == E
+        hipLaunchKernelGGL(moe_route_few_kernel, dim3(1), dim3(64), 0, st, logits, T, E, top_k, renorm, ws, ex, H, F, x);
+        rc = hip_check(hipGetLastError(), "moe route launch");
+    } else if (skinny) {  // the router also lists the token tiles; gate/up read the activations through tok
         const bool prep = tiled && !few;
         hipLaunchKernelGGL(moe_route_kernel, dim3(prep ? 1 + T : 1), dim3(route_threads), 0, st, logits, ws.idx, ws.w, T, E, top_k, renorm,
                            ws, ex, H, F, x, tile_rows, ntiles, prep ? x : nullptr);

@@ -895,6 +895,13 @@ def test_moe_ffn_few_tokens_activations_through_lds(ops, t, h, f, e, top_k):
     test_moe_ffn_few_tokens(ops, t, h, f, e, top_k)
 
 
+@pytest.mark.parametrize("t,h,f,e,top_k", [(16, 256, 512, 5, 4), (13, 256, 512, 7, 5), (16, 512, 256, 16, 8), (16, 256, 256, 1, 1), (8, 512, 512, 16, 8),
+                                           (1, 256, 256, 16, 8)])
+def test_moe_ffn_few_tokens_routed_by_one_wave(ops, t, h, f, e, top_k):
+    """64 pairs of token and expert and fewer take the one-wave router, 65 and more the general one; every expert hit or few, one alone."""
+    test_moe_ffn_few_tokens(ops, t, h, f, e, top_k)
+
+
 @pytest.mark.parametrize("t,h,f,e,top_k", [(20, 512, 1280, 4, 2), (33, 1024, 2816, 3, 2), (70, 768, 5632, 8, 1), (260, 512, 3328, 2, 2), (40, 1536, 2304, 16, 4)])
 def test_moe_ffn_down_products_in_uneven_k_splits(ops, t, h, f, e, top_k):
     """F that no power of two divides into parts of whole blocks, in both weight orders; 64 and 128 weight rows per wave."""

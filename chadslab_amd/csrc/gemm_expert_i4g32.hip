@@ -447,12 +447,12 @@ int expert_prep_h_launch(const uint16_t *h, const uint32_t *rowmax, int P, int K
 
 bool gemm_expert_ok(int H, int F) { return H % 256 == 0 && F % 256 == 0; }
 int gemm_expert_tile_rows() { return EX_MT; }
-// K splits of the down projection: up to four parts of whole 512-k blocks, the last one possibly shorter.  (Four equal ones or none
+// K splits of the down projection: up to `most` parts of whole 512-k blocks, the last one possibly shorter.  (Four equal ones or none
 // left the down product of 64 tokens, 2048 x 5632 and 8 experts on 32 workgroups, 52 us of the call's 89; now the call takes 55.  20
 // tokens, 3072 x 12032, 8 experts top 1: 172 -> 105; in row order 30 tokens, 4096 x 7424, 4 experts 119 -> 78.)
 static int down_span(int F, int s) { return ((F + 511) / 512 + s - 1) / s * 512; }
-int gemm_expert_down_splits(int F) {
-    const int s = (F + 511) / 512 < 4 ? (F + 511) / 512 : 4, span = down_span(F, s);
+int gemm_expert_down_splits(int F, int most) {
+    const int s = (F + 511) / 512 < most ? (F + 511) / 512 : most, span = down_span(F, s);
     return (F + span - 1) / span;
 }
 

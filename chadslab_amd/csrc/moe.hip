@@ -55,7 +55,7 @@ int gemm_skinny_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, 
 // weights in tile order (gemm_expert_i4g32.hip)
 bool gemm_expert_ok(int H, int F);
 int gemm_expert_tile_rows();
-int gemm_expert_down_splits(int F);
+int gemm_expert_down_splits(int F, int most);
 int expert_prep_h_launch(const uint16_t *h, const uint32_t *rowmax, int P, int K, uint16_t *dst, float *rs, uint16_t *ghi, uint16_t *glo,
                          hipStream_t st);
 int gemm_expert_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int E, int F, int H,
@@ -399,6 +399,16 @@ int moe_route_launch(const float *logits, int32_t *idx, float *w, int T, int E, 
 // tiled: the experts' weights and scales are in the tile order of chadq_repack_i4g32_tiles (the skinny kernel only)
 bool moe_ffn_tiled_ok(int H, int F) { return gemm_expert_ok(H, F); }
 
+// K splits, at most, of a down product whose F four equal parts do not fit: while the launch stays below some 400 workgroups of 96
+// token rows x 256 weight rows (beyond that the fp32 parts cost more than the workgroups bring).  Whole call in tile order, us, with
+// 1 / 2 / up to 4 splits, 8 experts: 256 tokens top 2 of 2304 x 1280 (72 workgroups unsplit) 69.6 / 67.5 / 65.8; 455 top 2 of 2048 x
+// 8960 (128) 213 / 179 / 186; 455 top 4 of it (192) 307 / 297 / 311; 455 top 4 of 2304 x 1280 (216) 89.7 / 100 / 101.
+static int uneven_splits(int P, int H, int E) {
+    const int hit = P < E ? P : E, rows = (P + hit - 1) / hit;
+    const int64_t wgs = (int64_t)hit * ((rows + 95) / 96) * (H / 256);
+    return wgs * 2 > 400 ? 1 : wgs * 3 > 400 ? 2 : wgs * 4 > 400 ? 3 : MOE_KSPLIT;
+}
+
 int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe_expert_i4g32 *experts, uint16_t *y,
                          int T, int H, int F, int E, int top_k, int renorm, void *workspace, bool tiled, hipStream_t st) {
     MoeWs ws;
@@ -455,14 +465,14 @@ int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe
         if (rc) return rc;
         rc = expert_prep_h_launch(ws.h, ws.rowmax, P, F, ws.ha, ws.rsh, ws.ghh, ws.ghl, st);
         if (rc) return rc;
-        nsplit = gemm_expert_down_splits(F);
+        nsplit = gemm_expert_down_splits(F, F % (512 * MOE_KSPLIT) == 0 ? MOE_KSPLIT : uneven_splits(P, H, E));
         rc = gemm_expert_down(ws.groups, ws.tiles, ntiles, E, H, F, ws.ha, ws.rsh, ws.ghh, ws.ghl, ws.yp, nsplit, (size_t)P * H, st);
         if (rc) return rc;
     } else if (skinny) {
         rc = gemm_skinny_gateup(ws.groups, ws.tiles, ws.tok, ntiles, E, F, H, st);  // h = bf16(silu(gate) * up), [P,F]
         if (rc) return rc;
         // parts of whole 256-k blocks, the last one possibly shorter
-        const int blocks = F / 256, per = (blocks + MOE_KSPLIT - 1) / MOE_KSPLIT;
+        const int blocks = F / 256, most = F % (256 * MOE_KSPLIT) == 0 ? MOE_KSPLIT : uneven_splits(P, H, E), per = (blocks + most - 1) / most;
         nsplit = (blocks + per - 1) / per;
         rc = gemm_skinny_down(ws.groups, ws.tiles, ntiles, E, H, F, nsplit, (size_t)P * H, st);  // fp32 parts [nsplit][P,H]
         if (rc) return rc;

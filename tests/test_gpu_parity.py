@@ -902,7 +902,8 @@ def test_moe_ffn_few_tokens_routed_by_one_wave(ops, t, h, f, e, top_k):
     test_moe_ffn_few_tokens(ops, t, h, f, e, top_k)
 
 
-@pytest.mark.parametrize("t,h,f,e,top_k", [(20, 512, 1280, 4, 2), (33, 1024, 2816, 3, 2), (70, 768, 5632, 8, 1), (260, 512, 3328, 2, 2), (40, 1536, 2304, 16, 4)])
+@pytest.mark.parametrize("t,h,f,e,top_k", [(20, 512, 1280, 4, 2), (33, 1024, 2816, 3, 2), (70, 768, 5632, 8, 1), (260, 512, 3328, 2, 2), (40, 1536, 2304, 16, 4),
+                                           (200, 3072, 1280, 8, 4), (150, 2304, 1792, 8, 2), (120, 3072, 3328, 8, 1)])
 def test_moe_ffn_down_products_in_uneven_k_splits(ops, t, h, f, e, top_k):
     """F that no power of two divides into parts of whole blocks, in both weight orders; 64 and 128 weight rows per wave."""
     test_moe_ffn_tiled_agrees_with_row_major_and_oracle(ops, t, h, f, e, top_k)

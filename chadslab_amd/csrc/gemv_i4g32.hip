@@ -157,13 +157,26 @@ static void launch_rows(const uint16_t *x, const uint8_t *wp, const uint16_t *sc
                        (int)bf16_out);
 }
 
+// Whether M rows go to the matrix cores: one pass over the weights by workgroups of 64 weight rows, weights taken exactly there too.  The
+// kernels of this file stream the weights once per pair of rows in a launch each, the generic one (beyond 4096 k) once per row.
+// us, here / there: 8 rows of 4096 x 4064 24.8 / 13.1, of 8192 x 8160 70.9 / 24.6; 5 of 128 x 96 7.3 / 3.8.  But a workgroup there walks all of
+// K by itself, 2.45 us per 1000 k, however few weight rows there are; here they cost less the fewer they are: 4 rows of 1024 x 14368 14.8 /
+// 39.5, of 4096 x 8160 20.4 / 23.9, 5 of 1024 x 4064 9.0 / 13.4, 8 of it 12.8 / 13.4.  The terms below are these kernels' times, within 10 %
+// on 32 to 32000 weight rows and 32 to 14368 k where the two are near each other.
+bool gemv_on_matrix_cores(int M, int N, int K) {
+    if (M < (K <= 4096 ? 5 : 3)) return false;
+    const float there = 3.7f + 2.45e-3f * (float)K, n = (float)N;
+    if (K <= 4096) {
+        const float streamed = n * (K <= 2048 ? 2048.f : 4096.f) - 4e6f;  // beyond what hides behind a launch
+        return (float)((M + 1) / 2) * (2.5f + 1e-4f * (float)K + (streamed > 0.f ? 2.6e-7f * streamed : 0.f)) > there;
+    }
+    const float few = 0.36f + 5e-5f * n, many = 0.03f + 2.7e-4f * n;  // us per row and 2048 k: latency, then the CUs' arithmetic
+    return 1.2f + (float)(M * ((K + 2047) / 2048)) * (few > many ? few : many) > there;
+}
+
 int gemv_i4g32_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K,
                         bool bf16_out, hipStream_t st) {
-    // Five rows and more (three of more than 4096 k): one pass over the weights on the matrix cores, weights taken exactly there
-    // too.  The kernels of this file stream them once per pair of rows, the generic one once per row.  us, here / there, for 4, 8
-    // and 16 rows: 4096 x 4064 12.4 / 13.0, 24.8 / 13.1, 49.5 / 13.3; 8192 x 8160 37.4 / 24.4, 70.9 / 24.6, 137 / 24.7; 2 rows of
-    // the latter 20.4 / 24.0.
-    if (M >= (K <= 4096 ? 5 : 3) && M <= 32 && gemm_tile_q_ok(K) && aligned16(x) && aligned16(wp))
+    if (M <= 32 && gemm_tile_q_ok(K) && aligned16(x) && aligned16(wp) && gemv_on_matrix_cores(M, N, K))
         return gemm_exact_few_rows_launch(x, wp, sc, y, M, N, K, bf16_out, st);
     if (K <= 4096) {
         // rows per wave: enough waves to fill 256 CUs several times over, few enough to keep loads deep

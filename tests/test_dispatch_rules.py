@@ -1,0 +1,21 @@
+"""Which kernel a call takes: the rules by size, asked directly on the host (C++ functions of libchadq.so).  No GPU."""
+import ctypes
+
+from chadslab_amd import _lib
+
+def _rule(symbol, result=ctypes.c_int):
+    fn = _lib.load()[symbol]
+    fn.restype = result
+    return fn
+
+
+def test_gemv_of_k_that_256_does_not_divide_takes_the_matrix_cores_where_they_are_faster():
+    fn = _rule("_ZN5chadq20gemv_on_matrix_coresEiii", ctypes.c_bool)
+    # us, streamed once per pair of rows (beyond 4096 k: per row) / on the matrix cores
+    for m, n, k in ((3, 32, 14368), (4, 1024, 14368), (3, 2048, 8160), (4, 4096, 8160), (8, 512, 6176), (5, 32, 4064), (5, 1024, 4064),
+                    (8, 512, 4064), (5, 128, 2080)):  # 9.9 / 38, 14.8 / 39.5, 9.7 / 23.8, 20.4 / 23.9, 13.2 / 19.2, 8.4 / 13, 9.0 / 13.4, 12.4 / 13.3, 8.1 / 8.9
+        assert not fn(m, n, k), (m, n, k)
+    for m, n, k in ((5, 32, 32), (16, 128, 96), (5, 2048, 2080), (8, 4096, 4064), (16, 1024, 4064), (4, 11008, 6176), (8, 8192, 8160), (16, 1024, 8160),
+                    (3, 32000, 14368)):               # 7.2 / 3.7, 19 / 3.8, 11.1 / 9.0, 26 / 13.8, 24 / 13.5, 46 / 21, 71 / 24.6, 27.8 / 23.9, 207 / 81
+        assert fn(m, n, k), (m, n, k)
+    assert not any(fn(m, 4096, 4064) for m in range(1, 5)) and not any(fn(m, 32000, 14368) for m in (1, 2))

@@ -68,9 +68,9 @@ int gemm_expert_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, 
 bool moe_few_ok(int T, int H, int F, int E, int top_k, bool tiled);
 int moe_few_tile_rows();
 int moe_few_down_splits(int F);
-int moe_few_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int T, int E, int F, int H, bool tiled,
+int moe_few_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int T, int E, int top_k, int F, int H, bool tiled,
                    hipStream_t st);
-int moe_few_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int T, int E, int H, int F, int nsplit, size_t split_stride, bool tiled,
+int moe_few_down(const GemmGroup *groups, const int32_t *tiles, int ntiles, int T, int E, int top_k, int H, int F, int nsplit, size_t split_stride, bool tiled,
                  hipStream_t st);
 
 // Token t: softmax over its E logits, the top_k largest (the lowest index wins ties) and their weights; s_e: the choices in LDS too.
@@ -453,11 +453,11 @@ int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe
     }
     if (rc) return rc;
     if (few) {
-        rc = moe_few_gateup(ws.groups, ws.tiles, ws.tok, ntiles, T, E, F, H, tiled, st);
+        rc = moe_few_gateup(ws.groups, ws.tiles, ws.tok, ntiles, T, E, top_k, F, H, tiled, st);
         if (rc) return rc;
         nsplit = moe_few_down_splits(F);
         static_assert(MOE_KSPLIT >= 4, "parts of the down product");
-        rc = moe_few_down(ws.groups, ws.tiles, ntiles, T, E, H, F, nsplit, (size_t)P * H, tiled, st);
+        rc = moe_few_down(ws.groups, ws.tiles, ntiles, T, E, top_k, H, F, nsplit, (size_t)P * H, tiled, st);
         if (rc) return rc;
     } else if (tiled) {
         // (the router's launch also made the fp16 form of the activations) gate/up with the SiLU gate, h to fp16, down split over K

@@ -19,3 +19,25 @@ def test_gemv_of_k_that_256_does_not_divide_takes_the_matrix_cores_where_they_ar
                     (3, 32000, 14368)):               # 7.2 / 3.7, 19 / 3.8, 11.1 / 9.0, 26 / 13.8, 24 / 13.5, 46 / 21, 71 / 24.6, 27.8 / 23.9, 207 / 81
         assert fn(m, n, k), (m, n, k)
     assert not any(fn(m, 4096, 4064) for m in range(1, 5)) and not any(fn(m, 32000, 14368) for m in (1, 2))
+
+
+def test_few_token_experts_stage_activations_only_where_workgroups_have_items_enough():
+    fn = _rule("_ZN5chadq19moe_few_through_ldsEiiiii", ctypes.c_bool)  # (tokens, experts, top k, items of an expert, blocks of 256 k of each)
+
+    def gate_up(t, e, top_k, h, f):
+        return fn(t, e, top_k, f // 16, h // 256)
+
+    def down(t, e, top_k, h, f):
+        parts = 4 if f >= 4096 else 2 if f >= 2048 else 1
+        return fn(t, e, top_k, h // 32 * parts, -(-(f // 256) // parts))
+
+    # whole calls, us, through LDS / straight to registers: 28 / 21, 40 / 32.5, 23 / 20 (one or two items per workgroup, or none)
+    for size in ((2, 8, 1, 2304, 1536), (14, 4, 2, 1280, 4352), (3, 8, 1, 1280, 1280)):
+        assert not gate_up(*size) and not down(*size)
+    assert gate_up(4, 8, 2, 4096, 14336) and down(4, 8, 2, 4096, 14336)  # 135 / 150
+    assert gate_up(6, 8, 2, 256, 12288)                                  # 40 / 43
+    # never more LDS than leaves three workgroups on a compute unit: 18304 bytes are the kernel's own, dealt out in pieces of 1280
+    for t in range(1, 17):
+        for span in range(1, 65):
+            x_bytes = 512 + t * (span * 512 + 16)
+            assert fn(t, 16, 4, 100000, span) == (3 * -(-(18304 + x_bytes) // 1280) * 1280 <= 163840)

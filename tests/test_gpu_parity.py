@@ -890,9 +890,45 @@ def test_moe_ffn_few_tokens(ops, t, h, f, e, top_k):
 
 @pytest.mark.parametrize("t,h,f,e,top_k", [(4, 4096, 3584, 8, 2), (1, 512, 2816, 16, 4), (5, 2048, 7424, 3, 2), (2, 1536, 256, 2, 1), (9, 1024, 4864, 4, 4)])
 def test_moe_ffn_few_tokens_activations_through_lds(ops, t, h, f, e, top_k):
-    """Activations of an expert small enough for LDS, in one of the two products or in both; workgroups whose run of items crosses
-    from one expert or K split to the next; K splits of uneven length."""
+    """Activations of an expert small enough for LDS, with few items to a workgroup; K splits of uneven length."""
     test_moe_ffn_few_tokens(ops, t, h, f, e, top_k)
+
+
+@pytest.mark.parametrize("t,h,f,e,top_k,gate,down", [(6, 256, 12288, 8, 2, True, False), (16, 512, 8960, 16, 4, True, False), (16, 2560, 4096, 16, 8, False, True),
+                                                     (5, 3328, 10496, 8, 2, True, True), (3, 2304, 9984, 16, 4, True, True)])
+def test_moe_ffn_few_tokens_many_items_are_summed_as_one_by_one(ops, t, h, f, e, top_k, gate, down):
+    """Where the activations go through LDS, in one of the two products or in both, every token's result has the bits of a call with that token
+    alone, which reads them straight to registers: workgroups whose run of items crosses from one expert or K split to the next, K splits of
+    uneven length, all tokens on the same experts and tokens spread over all of them."""
+    import ctypes
+
+    from chadslab_amd import QWeightInt4G32, _lib
+
+    fn = _lib.load()["_ZN5chadq19moe_few_through_ldsEiiiii"]
+    fn.restype = ctypes.c_bool
+    parts = 4 if f >= 4096 else 2 if f >= 2048 else 1
+    rule = [(fn(n, e, top_k, f // 16, h // 256), fn(n, e, top_k, h // 32 * parts, -(-(f // 256) // parts))) for n in (t, 1)]
+    assert rule[0] == (gate, down) and rule[0] != rule[1]
+    g = torch.Generator(device=DEV)
+    g.manual_seed(9500 + t)
+
+    def matrix(n, k):
+        return QWeightInt4G32(torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g),
+                              torch.exp(torch.randn(n, k // 32, device=DEV, generator=g) * 0.5 - 5.0).half())
+
+    experts = [(matrix(f, h), matrix(f, h), matrix(h, f)) for _ in range(e)]
+    x = torch.randn(t, h, device=DEV, generator=g).bfloat16()
+    z = torch.randn(t, e, device=DEV, generator=g)
+    same = z.clone()
+    same[:, -top_k:] += 30.0
+    for logits in (z, same):
+        y = ops.moe_ffn(x, logits, experts, top_k=top_k)
+        assert bool(torch.isfinite(y).all()) and bool(y.any())
+        differ = 0
+        for i in range(t):
+            one = ops.moe_ffn(x[i:i + 1], logits[i:i + 1], experts, top_k=top_k)
+            differ += int((one[0].view(torch.int16) != y[i].view(torch.int16)).sum())
+        assert differ == 0
 
 
 @pytest.mark.parametrize("t,h,f,e,top_k", [(16, 256, 512, 5, 4), (13, 256, 512, 7, 5), (16, 512, 256, 16, 8), (16, 256, 256, 1, 1), (8, 512, 512, 16, 8),

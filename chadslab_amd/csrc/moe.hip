@@ -400,12 +400,17 @@ int moe_route_launch(const float *logits, int32_t *idx, float *w, int T, int E, 
 bool moe_ffn_tiled_ok(int H, int F) { return gemm_expert_ok(H, F); }
 
 // K splits, at most, of a down product whose F four equal parts do not fit: while the launch stays below some 400 workgroups of 96
-// token rows x 256 weight rows (beyond that the fp32 parts cost more than the workgroups bring).  Whole call in tile order, us, with
-// 1 / 2 / up to 4 splits, 8 experts: 256 tokens top 2 of 2304 x 1280 (72 workgroups unsplit) 69.6 / 67.5 / 65.8; 455 top 2 of 2048 x
-// 8960 (128) 213 / 179 / 186; 455 top 4 of it (192) 307 / 297 / 311; 455 top 4 of 2304 x 1280 (216) 89.7 / 100 / 101.
-static int uneven_splits(int P, int H, int E) {
+// token rows x 256 weight rows (beyond that the fp32 parts cost more than the workgroups bring), and from 100 workgroups on only if F is
+// long.  Whole call in tile order, us, with 1 / 2 / up to 4 splits, 8 experts: 256 tokens top 2 of 2304 x 1280 (72 workgroups unsplit) 69.6 /
+// 67.5 / 65.8; 455 top 2 of 2048 x 8960 (128) 213 / 179 / 186; 455 top 4 of it (192) 307 / 297 / 311; 455 top 4 of 2304 x 1280 (216) 89.7 / 100
+// / 101.  Short F in many workgroups, 1 / as many as fit: 375 top 4 of 2304 x 768 in row order (144) 67.0 / 71.6, 422 top 4 of 4 experts of
+// 2560 x 1536 (200) 85.4 / 96.3.  Both orders follow the rule: of 1600 calls in either, 17 to 900 tokens, none is more than 4 % slower than
+// unsplit and the mean 20 % faster.  (Four equal parts are taken whatever the number of rows.  The same rule for them too: -20 % at
+// F = 1024 in row order and 150 workgroups, but +10 to +18 % at 3072 to 8192, where the last of three or two parts is short.)
+int moe_uneven_splits(int P, int H, int F, int E) {
     const int hit = P < E ? P : E, rows = (P + hit - 1) / hit;
     const int64_t wgs = (int64_t)hit * ((rows + 95) / 96) * (H / 256);
+    if (F < 4096 && wgs >= 100) return 1;
     return wgs * 2 > 400 ? 1 : wgs * 3 > 400 ? 2 : wgs * 4 > 400 ? 3 : MOE_KSPLIT;
 }
 
@@ -465,14 +470,14 @@ int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe
         if (rc) return rc;
         rc = expert_prep_h_launch(ws.h, ws.rowmax, P, F, ws.ha, ws.rsh, ws.ghh, ws.ghl, st);
         if (rc) return rc;
-        nsplit = gemm_expert_down_splits(F, F % (512 * MOE_KSPLIT) == 0 ? MOE_KSPLIT : uneven_splits(P, H, E));
+        nsplit = gemm_expert_down_splits(F, F % (512 * MOE_KSPLIT) == 0 ? MOE_KSPLIT : moe_uneven_splits(P, H, F, E));
         rc = gemm_expert_down(ws.groups, ws.tiles, ntiles, E, H, F, ws.ha, ws.rsh, ws.ghh, ws.ghl, ws.yp, nsplit, (size_t)P * H, st);
         if (rc) return rc;
     } else if (skinny) {
         rc = gemm_skinny_gateup(ws.groups, ws.tiles, ws.tok, ntiles, E, F, H, st);  // h = bf16(silu(gate) * up), [P,F]
         if (rc) return rc;
         // parts of whole 256-k blocks, the last one possibly shorter
-        const int blocks = F / 256, most = F % (256 * MOE_KSPLIT) == 0 ? MOE_KSPLIT : uneven_splits(P, H, E), per = (blocks + most - 1) / most;
+        const int blocks = F / 256, most = F % (256 * MOE_KSPLIT) == 0 ? MOE_KSPLIT : moe_uneven_splits(P, H, F, E), per = (blocks + most - 1) / most;
         nsplit = (blocks + per - 1) / per;
         rc = gemm_skinny_down(ws.groups, ws.tiles, ntiles, E, H, F, nsplit, (size_t)P * H, st);  // fp32 parts [nsplit][P,H]
         if (rc) return rc;

@@ -41,3 +41,10 @@ def test_few_token_experts_stage_activations_only_where_workgroups_have_items_en
         for span in range(1, 65):
             x_bytes = 512 + t * (span * 512 + 16)
             assert fn(t, 16, 4, 100000, span) == (3 * -(-(18304 + x_bytes) // 1280) * 1280 <= 163840)
+
+
+def test_expert_down_product_of_short_k_is_not_split_among_many_workgroups():
+    fn = _rule("_ZN5chadq17moe_uneven_splitsEiiii")  # (pairs, H, F, experts)
+    assert fn(4 * 375, 2304, 768, 8) == 1 and fn(4 * 422, 2560, 1536, 4) == 1  # 67.0 us (split 71.6), 85.4 (96.3)
+    assert fn(2 * 256, 2304, 1280, 8) == 4                                     # 65.8 (69.6)
+    assert fn(2 * 455, 2048, 8960, 8) == 3 and fn(4 * 455, 2304, 1280, 8) == 1

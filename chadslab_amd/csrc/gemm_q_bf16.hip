@@ -436,7 +436,7 @@ int gemm_i4g32_bf16_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_
                              int K, hipStream_t st) {
     const int rc = activations_ok(M, K);  // the limit of the 128 x 64 tile, whichever tile is picked
     if (rc != 0) return rc;
-    if (gemm_tile_q_ok(K)) return gemm_tile_i4g32_launch(x, wp, sc, y, M, N, K, gemm_tile_pick(M, N, K, true), st);
+    if (gemm_tile_q_ok(K)) return gemm_tile_i4g32_launch(x, wp, sc, y, M, N, K, gemm_tile_pick(M, N, K, true, K % 256 != 0 || !aligned16(sc)), st);
     return launch_gemm<FmtI4G32, false>(x, wp, sc, y, M, N, K, nullptr, 0, st);
 }
 
@@ -444,7 +444,7 @@ int gemm_i8row_bf16_dispatch(const uint16_t *x, const int8_t *w8, const float *s
                              hipStream_t st) {
     const int rc = activations_ok(M, K);
     if (rc != 0) return rc;
-    if (gemm_tile_q_ok(K)) return gemm_tile_i8row_launch(x, w8, sc, y, M, N, K, gemm_tile_pick(M, N, K, false), st);
+    if (gemm_tile_q_ok(K)) return gemm_tile_i8row_launch(x, w8, sc, y, M, N, K, gemm_tile_pick(M, N, K, false, K % 128 != 0), st);
     return launch_gemm<FmtI8Row, false>(x, w8, sc, y, M, N, K, nullptr, 0, st);
 }
 

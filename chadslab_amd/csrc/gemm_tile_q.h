@@ -8,9 +8,11 @@ enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_GEGLU = 2 };
 }
 
 bool gemm_tile_q_ok(int K);
-enum GemmTile { TILE_32x64, TILE_64x64, TILE_96x64, TILE_128x64, TILE_96x128, TILE_128x128, TILE_192x128, TILE_256x128, TILE_256x256 };
-// the tile (activation rows x weight rows) that takes the product in the shortest time
-GemmTile gemm_tile_pick(int M, int N, int K, bool int4);
+enum GemmTile { TILE_32x64, TILE_64x64, TILE_96x64, TILE_128x64, TILE_96x128, TILE_128x128, TILE_192x128, TILE_256x128, TILE_256x256,
+                SHORT_32x64, SHORT_64x64, SHORT_128x128, SHORT_256x256 };
+// the tile (activation rows x weight rows) that takes the product in the shortest time; guard: K no multiple of the tiles' steps, or int4
+// scales that are not 16-byte aligned
+GemmTile gemm_tile_pick(int M, int N, int K, bool int4, bool guard);
 // y bf16 [M,N]; gemm_tile_q_ok(K)
 int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st);
 int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st);

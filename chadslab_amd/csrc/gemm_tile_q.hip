@@ -9,6 +9,7 @@
 //   128 x 128        int4: WN = 4, WK = 2, MB = 4; int8: WN = 2, WK = 4, MB = 4, NB = 2.   96 x 128: the latter with MB = 3
 //   128, 96 x 64     WN = 2, WK = 4, MB = 4 or 3, 32 k per wave and step.   64, 32 x 64: MB = 2 or 1, 64 k
 //   exact weights    256, 128 x 128: WN = 4, WK = 2, MB = 8 or 4.  64, 32 x 64: WN = 2, WK = 4; K possibly split over workgroups
+//   SHORT            32, 64 x 64, 128 x 128 (WN = 4, WK = 2, MB = 4) and, int4, 256 x 256 with another loop, for few steps (short_k)
 //
 //   * A (activations): global -> LDS by DMA, ST stages of a step each, read back as fragments one or two slices (16 k)
 //     ahead of their MFMAs.  16-byte pieces of a 128-byte row segment are XOR-swizzled by row / 2: LDS has 64 banks, two
@@ -38,7 +39,9 @@
 // (the vendor's GEMM on bf16 weights: 512 x 4096 x 4096 25, 1000 x 4096 x 14336 112, 4096^3 88, 4096 x 14336 x 4096 328).
 // Tried and not kept: NB = 2 for the 256 x 256 tile (half the fragment reads, twice the dequantisation: 117-118 us at 4096^3), four
 // waves of 256 x 64 with 512 registers (115 there, but 10 % slower in a round that is not full), 64 x 128 tiles (25 us at 512 rows),
-// four-wave workgroups for the 128-row tiles (the same time), a stage more (the same), a stage less (28 us).
+// four-wave workgroups for the 128-row tiles (the same time), a stage more (the same), a stage less (28 us)  For few steps:
+// one body for all of them with its conditions at run time (24 x 1024 x 1120 6.5 us, five bodies 5.8, SHORT 5.2), no unrolled loop, no
+// second request of the last step's weights (both nothing from two steps on).
 //
 // EXACT: no weight is rounded, for callers whose sums must be those of the decode step.  The operands are the integers (u - 8) / 2^9;
 // the scale of a group of 32 k is applied to its sum, one fp32 FMA per value.  That work, not the matrix cores, bounds it: 64 FMAs
@@ -61,7 +64,8 @@ namespace tileq {
 #endif
 
 // WM waves along the rows, WN along the columns, WK along k; MB x NB blocks of 32 x 32 per wave; KW k per wave and step; ST stages
-template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD>
+// SHORT: the loop for few steps
+template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool SHORT>
 struct Cfg {
     static constexpr int NW = WM * WN * WK, T = 64 * NW;
     static constexpr int BM = 32 * MB * WM, BN = 32 * NB * WN, KS = KW * WK;  // tile, k per step
@@ -69,7 +73,7 @@ struct Cfg {
     static constexpr int BB = (I4 ? KW / 2 : KW) * WK;                        // packed bytes of a weight row per step
     static constexpr int A_STAGE = BM * KS * 2, B_STAGE = BN * BB;
     // int4 scales of a step: the 16 bytes (256 k) of every column that hold it, or (GUARD) 4 bytes per lane and block of each wave
-    static constexpr int S_STAGE = !I4 ? 0 : GUARD ? 256 * NB * NW : BN * 16;
+    static constexpr int S_STAGE = !I4 || SHORT ? 0 : GUARD ? 256 * NB * NW : BN * 16;
     static constexpr int STAGE = A_STAGE + B_STAGE + S_STAGE;
     // DMA instructions per step: A_DMA of each wave for the activations; the BI of the weights and the SI of the scales are dealt
     // to the waves, as many to each (BS_DMA; what is left over fetches nothing, into a place nobody reads: every wave has the
@@ -79,9 +83,12 @@ struct Cfg {
     static_assert(A_DMA * NW * 1024 == A_STAGE && BI * 1024 == B_STAGE, "whole DMA instructions");
     static constexpr bool DUMP = (BI + SI) % NW != 0;
     static constexpr int DUMP_OFF = ST * STAGE;
+    // SHORT: the scales of a wave behind the stages, two buffers: 256 k (32 rows x 16 B, fetched twice), or (GUARD) one step (64 lanes x 4 B)
+    static constexpr int S_BUF = !I4 || !SHORT ? 0 : GUARD ? 256 : 1024, S_OFF = ST * STAGE;
+    static_assert(!SHORT || (!DUMP && WM == 1 && NB == 1 && KW == 64 && ST == 3), "what that loop knows");
     static constexpr int SPB = 256 / KS;                                      // steps per 256 k
     static constexpr int EP_PITCH = BN * 2 + 16;                              // result tile in LDS: bf16 rows, padded
-    static constexpr int OPER = ST * STAGE + (DUMP ? 1024 : 0), EPI = BM * EP_PITCH;
+    static constexpr int OPER = ST * STAGE + (DUMP ? 1024 : 0) + 2 * NW * S_BUF, EPI = BM * EP_PITCH;
     static constexpr int RED = WK == 4 ? NW * MB * 4096 : WK == 2 ? WM * WN * MB * 4096 : 0;  // one column block at a time
     static constexpr int LDS0 = OPER > EPI ? OPER : EPI, LDS = LDS0 > RED ? LDS0 : RED;
     static constexpr int AHEAD = MB * NB > 4 || SL == 2 ? 1 : 2;  // slices between a fragment's request and its MFMAs (what the registers allow)
@@ -135,11 +142,11 @@ __device__ __forceinline__ bf16x8 signed8_i4(uint32_t w) {
 // EPI (what becomes of the sums): EPI_BF16 y bf16 [M,N], times the row scale for int8; EPI_F32 y fp32 [gridDim.y][M,N],
 // part blockIdx.y holding the sum over its kspan k; EPI_GEGLU the weight rows come in pairs (gate, up) of a feature and
 // h = bf16(gelu_tanh(gate) * up) goes to y as bf16 [M, N/2].
-template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT, int EPI>
+template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT, int EPI, bool SHORT>
 __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WM * WN * WK / 4, WM * WN * WK / 4))) void gemm_tile_q_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wq, const void *__restrict__ scv, void *__restrict__ yv, int M, int N,
     int K, int kspan) {
-    typedef Cfg<I4, WM, WN, WK, MB, NB, KW, ST, GUARD> C;
+    typedef Cfg<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, SHORT> C;
     constexpr int BM = C::BM, BN = C::BN, BB = C::BB, AHEAD = C::AHEAD, SL = C::SL;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -183,7 +190,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     for (int q = 0; q < C::BS_DMA; ++q) {  // 64 / BPR weight rows, or the scales of 64, per instruction
         const int e = q * C::NW + wave, r = e * (64 / BPR) + lane / BPR, c = (e - C::BI) * 64 + lane;
         bpc[q] = 16 * ((lane % BPR) ^ bkey(r));
-        if (e < C::BI) boff[q] = r < nrows ? (uint32_t)r * (uint32_t)wrow + (uint32_t)bpc[q] : kOut;
+        if (SHORT || e < C::BI) boff[q] = r < nrows ? (uint32_t)r * (uint32_t)wrow + (uint32_t)bpc[q] : kOut;
         else boff[q] = e < C::BI + C::SI && c < nrows ? (uint32_t)c * (uint32_t)(G * 2) : kOut;
     }
     const uint16_t *srow[NB];  // GUARD: the scale rows of the lane's columns
@@ -264,16 +271,18 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     using T = std::true_type;
     using F = std::false_type;
     // ---- prologue
+    if constexpr (!SHORT) {
 #pragma unroll
-    for (int r = 0; r < C::REQ - C::A_DMA; ++r) issue_b(r, 0, lds, false);
+        for (int r = 0; r < C::REQ - C::A_DMA; ++r) issue_b(r, 0, lds, false);
 #pragma unroll
-    for (int j = 0; j < ST - 1; ++j)
-        if (j < steps)
+        for (int j = 0; j < ST - 1; ++j)
+            if (j < steps)
 #pragma unroll
-            for (int r = 0; r < C::REQ; ++r) request(r, j, lds + (j + 1) * C::STAGE, lds + j * C::STAGE, false);
-    if (steps >= ST - 1) wait_vmcnt<(ST - 2) * C::REQ>();  // the activations of step 0, the weights of steps 0 and 1
-    else wait_vmcnt<0>();
-    wg_barrier();
+                for (int r = 0; r < C::REQ; ++r) request(r, j, lds + (j + 1) * C::STAGE, lds + j * C::STAGE, false);
+        if (steps >= ST - 1) wait_vmcnt<(ST - 2) * C::REQ>();  // the activations of step 0, the weights of steps 0 and 1
+        else wait_vmcnt<0>();
+        wg_barrier();
+    }
     auto run = [&](auto &step) {
         // (stages as constants in the loop: their addresses cost nothing there; not worth the code for few rows, whose workgroups
         // take a few steps each)
@@ -398,6 +407,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[MB - 1][0][v] = __builtin_fmaf(tmp[(Q - 1) & 1][v], s_last, acc[MB - 1][0][v]);
     } else {
+    uint8_t *const slds = lds + C::S_OFF + 2 * wave * C::S_BUF;  // SHORT
     u32x4 bq[NB][BQ], bn[NB][BQ];  // the lane's packed weights of a step (int4 and 32 k: half of one), of the next one
     uint16_t sraw[NB];
     float cs[NB][4];
@@ -414,8 +424,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
                     bn[nb][e] = *reinterpret_cast<const u32x4 *>(p);
                 }
             }
-                const uint8_t *const sp = stage + C::A_STAGE + C::B_STAGE;
-            if constexpr (I4 && GUARD) sraw[nb] = *reinterpret_cast<const uint16_t *>(sp + (wave * NB + nb) * 256 + lane * 4);
+            const uint8_t *const sp = stage + C::A_STAGE + C::B_STAGE;
+            if constexpr (I4 && SHORT)
+                sraw[nb] = *reinterpret_cast<const uint16_t *>(
+                    slds + (GUARD ? (step & 1) * C::S_BUF + lane * 4 : (step / C::SPB & 1) * C::S_BUF + nl * 16 + (((step * WK + wk) & 3) * 2 + kq) * 2));
+            else if constexpr (I4 && GUARD) sraw[nb] = *reinterpret_cast<const uint16_t *>(sp + (wave * NB + nb) * 256 + lane * 4);
             else if constexpr (I4)
                 sraw[nb] = *reinterpret_cast<const uint16_t *>(sp + ((wn * NB + nb) * 32 + nl) * 16 +
                                                                (KW == 64 ? ((step * WK + wk) & 3) * 2 + kq : (step * WK + wk) & 7) * 2);
@@ -453,19 +466,23 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         af[t % (2 * AHEAD)][mb] = *reinterpret_cast<const bf16x8 *>(stage + mb * 4096 + foff[t]);
     };
 
-    fetch(0, lds);
+    auto frags = [&](int t, const uint8_t *stage) {
 #pragma unroll
-    for (int t = 0; t < AHEAD; ++t)
+        for (int mb = 0; mb < MB; ++mb) frag(t, mb, stage);
+    };
+    auto begin = [&]() {
+        fetch(0, lds);
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) frag(t, mb, lds);
-    if (ST <= steps) {
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-        wg_barrier();                        // step 0's weights have been read
+        for (int t = 0; t < AHEAD; ++t) frags(t, lds);
+        if (!SHORT && ST <= steps) {
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+            wg_barrier();                        // step 0's weights have been read
 #pragma unroll
-        for (int r = 0; r < first(AFTER); ++r) request(r, ST - 1, lds, lds + (ST - 1) * C::STAGE, false);
-    }
-    prep(0);
-    deq(0);
+            for (int r = 0; r < first(AFTER); ++r) request(r, ST - 1, lds, lds + (ST - 1) * C::STAGE, false);
+        }
+        prep(0);
+        deq(0);
+    };
 
     // Step i works on stage i % ST and reads the packed weights of step i+1 at its beginning.  In front of its last slices, whose
     // fragments are in registers, a wave waits until its part of the activations of step i+1 and of the weights of step i+2 is
@@ -478,6 +495,97 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     // The order inside a slice: LDS reads with the first MFMAs, memory requests and the dequantisation spread over all of
     // them (mask 8: MFMA, 2: vector ALU, 0x100: LDS read, 0x20: vector memory).
     constexpr int DQ = NB * (I4 ? 17 : 12);
+    if constexpr (SHORT) {
+        // Few steps: everything of a step is requested together, two steps ahead, half of the activations a slice later, and the packed
+        // weights are read with the step's first fragments.  Half the code and no request in front of the first MFMA that
+        // it does not wait for: what a product of a few steps takes longest for is its way to the first MFMA and the code that it
+        // runs through once.
+        const uint16_t *const srow1 = reinterpret_cast<const uint16_t *>(scv) + (size_t)(n0 + wn * 32 + nl < N ? n0 + wn * 32 + nl : N - 1) * G;
+        auto issue_s = [&](int blk) {  // blk: 256-k block, or (GUARD) step
+            if constexpr (I4 && GUARD) {
+                const int g = 2 * (blk * WK + wk) + kq;
+                dma2_to_lds(srow1 + (g < G ? g : 0), slds + (blk & 1) * C::S_BUF);
+            } else if constexpr (I4) {
+                dma16_to_lds(srow1 + blk * 8, slds + (blk & 1) * C::S_BUF);
+            }
+        };
+        auto issue = [&](int step, uint8_t *stage, bool b, int q0, int q1) {
+#pragma unroll
+            for (int q = 0; q < C::BS_DMA; ++q)
+                if (b) issue_b(q, step, stage, false);
+#pragma unroll
+            for (int q = 0; q < C::A_DMA; ++q)
+                if (q >= q0 && q < q1) issue_a(q, step, stage, false);
+        };
+        constexpr int STEP = C::A_DMA + C::BS_DMA;  // requests of a step, its scales aside
+        uint8_t *cur = lds, *nxt = lds + C::STAGE, *far = lds + 2 * C::STAGE;
+        issue_s(0);
+        if (GUARD || C::SPB == 1 ? steps > 1 : C::SPB == 2 && steps > 2) issue_s(1);
+        issue(0, cur, true, 0, C::A_DMA);
+        if (steps > 1) {
+            issue(1, nxt, true, 0, C::A_DMA);
+            wait_vmcnt<STEP>();  // everything of step 0
+        } else {
+            wait_vmcnt<0>();
+        }
+        wg_barrier();
+        begin();
+        auto order = [&]() {
+#pragma unroll
+            for (int e = 0; e < MB; ++e) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                if (e % 2 == 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (DQ + MB - 1) / MB, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // Step i works on stage `cur` = i % 3 and requests step i+2 into `far`, which held step i-1: everybody has left that stage before
+        // the barrier of step i-1.  In front of the barrier a wave waits until no more than what it has requested during this step is
+        // outstanding: its part of stage i+1 and of the scales is then in LDS.
+        auto step = [&](int i, auto more1_c, auto more2_c) {
+            constexpr bool more1 = decltype(more1_c)::value, more2 = decltype(more2_c)::value;  // steps i+1, i+2 exist
+            constexpr int H = (STEP + 1) / 2 - C::BS_DMA < 0 ? 0 : (STEP + 1) / 2 - C::BS_DMA;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if (t == BAR && more1) {
+                    if (more2) wait_vmcnt<STEP>();
+                    else wait_vmcnt<0>();
+                    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this stage has been read
+                    wg_barrier();
+                    if (GUARD || C::SPB == 1) {
+                        if (more2) issue_s(i + 2);
+                    } else if (I4 && (i + 3) % C::SPB == 0 && i + 3 < steps) {
+                        issue_s((i + 3) / C::SPB);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (t < BAR) frags(t + AHEAD, cur);
+                if (t == 0 && more2) issue(i + 2, far, true, 0, H);
+                if (t == 1 && more2) issue(i + 2, far, false, H, C::A_DMA);
+#pragma unroll
+                for (int e = 0; e < MB; ++e) mfma(t, e);
+                if (t < 3) deq(t + 1);
+                if (t == BAR && more1) fetch(i + 1, nxt);
+                if (t >= BAR && more1) frags(t - BAR, nxt);
+                if (t == 3 && more1) {
+                    prep(i + 1);
+                    deq(0);
+                }
+                order();
+            }
+            uint8_t *const r = cur;
+            cur = nxt;
+            nxt = far;
+            far = r;
+        };
+        int i = 0;
+        for (; i + 2 < steps; ++i) step(i, T{}, T{});
+        if (steps > 1) step(i++, T{}, F{});
+        step(i, F{}, F{});
+    } else {
+    begin();
     auto order = [&]() {
 #pragma unroll
         for (int e = 0; e < NE; ++e) {
@@ -526,6 +634,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         }
     };
     run(step);
+    }
     }
 
     // ---- epilogue.  The lane holds, for every mb and nb, column nl of rows 8*(v/4) + 4*kq + v%4 of a 32 x 32 block.
@@ -576,8 +685,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         }
     }
     auto row_of = [&](int v) {
-        const int f = wk * UV + v, vv = f & 15;
-        return wm * MB * 32 + (f >> 4) * 32 + 8 * (vv >> 2) + 4 * kq + (vv & 3);
+        auto at = [](int f) { return (f >> 4) * 32 + 8 * ((f & 15) >> 2) + (f & 3); };
+        // (where no carry goes between the two parts of the number, the second part of the row is a constant)
+        return wm * MB * 32 + 4 * kq + (16 % UV == 0 || UV % 16 == 0 ? at(wk * UV) + at(v) : at(wk * UV + v));
     };
     if constexpr (EPI == EPI_F32) {  // 128 contiguous bytes per row straight from the registers
         float *const y = reinterpret_cast<float *>(yv) + (size_t)blockIdx.y * M * N;
@@ -643,17 +753,17 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     }
 }
 
-template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT = false, int EPI = EPI_BF16>
+template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT = false, int EPI = EPI_BF16, bool SHORT = false>
 static int launch(const uint16_t *x, const uint8_t *wq, const void *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st) {
-    typedef Cfg<I4, WM, WN, WK, MB, NB, KW, ST, GUARD> C;
+    typedef Cfg<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, SHORT> C;
     static std::atomic<bool> attr_set{false};  // setting it twice from two threads is harmless
     if (!attr_set.load(std::memory_order_acquire)) {
-        CHADQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tile_q_kernel<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, EXACT, EPI>),
+        CHADQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tile_q_kernel<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, EXACT, EPI, SHORT>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS));
         attr_set.store(true, std::memory_order_release);
     }
     const int tiles = ((N + C::BN - 1) / C::BN) * ((M + C::BM - 1) / C::BM);
-    hipLaunchKernelGGL((gemm_tile_q_kernel<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, EXACT, EPI>), dim3((tiles + 7) / 8 * 8, ksplit), dim3(C::T), C::LDS, st,
+    hipLaunchKernelGGL((gemm_tile_q_kernel<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, EXACT, EPI, SHORT>), dim3((tiles + 7) / 8 * 8, ksplit), dim3(C::T), C::LDS, st,
                        x, wq, sc, y, M, N, K, ksplit == 1 ? K : (K / 256 + ksplit - 1) / ksplit * 256);
     return hip_check(hipGetLastError(), "gemm_tile_q launch");
 }
@@ -664,39 +774,73 @@ static int launch(const uint16_t *x, const uint8_t *wq, const void *sc, void *y,
 bool gemm_tile_q_ok(int K) { return K < (1 << 22); }
 
 // Which tile.  A tile takes c0 + c1 * K / 4096 us on a chip full of them and less on one that is not: a round of f * 256 tiles b +
-// (1 - b) f of it.  Longer launches run at a lower clock, which costs the tiles differently: `a` us of work take a (1 + q a / (a +
-// 100)).  The constants are fitted to whole calls, every tile on 850 random products (65 to 4096 rows, 512 to 16384 columns and k);
-// the tile picked is 0.3 % slower on average than the best of all eight, 10 % at worst.  Up to 64 rows the smallest tiles win in
-// any number of rounds (the others are padded to 96 rows and every round of theirs carries the same weights): 33 x 20000 x 2048
-// 15.4 us (128 x 64: 23.7), 64 x 256000 x 2048 151 (299), 64 x 16384 x 16384 63 (87).
+// (1 - b) f of it; s is what a launch takes besides.  Longer launches run at a lower clock, which costs the tiles differently: `a` us of
+// work take a (1 + q a / (a + 100)).  The constants are fitted to whole calls, every tile on 4600 random products (65 to 7000 rows, 64 to
+// 33000 columns, 32 to 18000 k), for whole and for guarded steps (K no multiple of a step, or int4 scales that are not aligned), whose
+// requests cost the tiles of two column blocks per wave more.  The tile picked is 0.2 % slower on average than the best of all, 7 % in
+// one case of a hundred.  (With constants of products of 512 k and more only, the picks below that were up to 40 % off: 193 x 12160 x
+// 128 int8 6.5 us on 128 x 128 tiles, 8.8 on 128 x 64.)  Up to 64 rows the smallest tiles win in any number of rounds (the others are
+// padded to 96 rows and every round of theirs carries the same weights): 33 x 20000 x 2048 15.4 us (128 x 64: 23.7), 64 x 256000 x 2048
+// 151 (299), 64 x 16384 x 16384 63 (87).
 struct TileCost {
     GemmTile tile;
-    int bm, bn;
-    float c0, c1, b, q;
+    int bm, bn, ks;  // ks: k of a step
+    float s, c0, c1, b, q;
 };
-static const TileCost kCostI4[] = {{TILE_64x64, 64, 64, 2.2f, 9.7f, .68f, .27f},      {TILE_96x64, 96, 64, 2.3f, 13.6f, .72f, .36f},
-                                   {TILE_128x64, 128, 64, 2.6f, 16.5f, .70f, .37f},   {TILE_96x128, 96, 128, 4.2f, 21.0f, .71f, .41f},
-                                   {TILE_128x128, 128, 128, 3.9f, 23.9f, .65f, .54f}, {TILE_192x128, 192, 128, 5.1f, 37.0f, .70f, .50f},
-                                   {TILE_256x128, 256, 128, 5.8f, 46.1f, .69f, .42f}, {TILE_256x256, 256, 256, 8.1f, 87.3f, .63f, .13f}};
-static const TileCost kCostI8[] = {{TILE_64x64, 64, 64, 2.2f, 10.7f, .61f, .09f},     {TILE_96x64, 96, 64, 2.2f, 14.2f, .65f, .12f},
-                                   {TILE_128x64, 128, 64, 2.5f, 17.2f, .65f, .14f},   {TILE_96x128, 96, 128, 4.5f, 19.8f, .62f, .31f},
-                                   {TILE_128x128, 128, 128, 5.5f, 22.7f, .67f, .36f}, {TILE_192x128, 192, 128, 5.2f, 30.6f, .69f, .52f},
-                                   {TILE_256x128, 256, 128, 6.4f, 41.1f, .67f, .35f}, {TILE_256x256, 256, 256, 8.2f, 77.0f, .66f, .18f}};
+static const TileCost kCost[2][2][8] = {  // [int8, int4][whole steps, guarded]
+    {{{TILE_64x64, 64, 64, 256, 1.89f, 2.51f, 10.61f, 0.67f, -0.03f}, {TILE_96x64, 96, 64, 128, 1.88f, 3.11f, 12.80f, 0.72f, 0.18f},
+      {TILE_128x64, 128, 64, 128, 0.00f, 5.66f, 15.04f, 0.76f, 0.18f}, {TILE_96x128, 96, 128, 128, 0.00f, 8.21f, 21.96f, 0.51f, -0.02f},
+      {TILE_128x128, 128, 128, 128, 0.00f, 7.28f, 28.37f, 0.62f, -0.06f}, {TILE_192x128, 192, 128, 64, 1.36f, 6.81f, 40.17f, 0.62f, 0.00f},
+      {TILE_256x128, 256, 128, 64, 2.00f, 7.67f, 53.01f, 0.55f, -0.03f}, {TILE_256x256, 256, 256, 64, 1.77f, 9.47f, 105.38f, 0.53f, -0.11f}},
+     {{TILE_64x64, 64, 64, 256, 2.05f, 2.18f, 11.35f, 0.67f, 0.24f}, {TILE_96x64, 96, 64, 128, 1.52f, 3.45f, 14.81f, 0.71f, 0.19f},
+      {TILE_128x64, 128, 64, 128, 1.14f, 4.22f, 16.36f, 0.71f, 0.62f}, {TILE_96x128, 96, 128, 128, 0.00f, 7.63f, 24.52f, 0.61f, -0.04f},
+      {TILE_128x128, 128, 128, 128, 0.36f, 6.35f, 31.52f, 0.65f, -0.08f}, {TILE_192x128, 192, 128, 64, 1.83f, 5.69f, 44.59f, 0.66f, -0.00f},
+      {TILE_256x128, 256, 128, 64, 1.86f, 7.58f, 56.05f, 0.51f, -0.03f}, {TILE_256x256, 256, 256, 64, 1.56f, 9.07f, 119.73f, 0.48f, -0.18f}}},
+    {{{TILE_64x64, 64, 64, 256, 1.93f, 2.66f, 10.60f, 0.70f, -0.03f}, {TILE_96x64, 96, 64, 128, 2.47f, 2.71f, 13.49f, 0.70f, 0.26f},
+      {TILE_128x64, 128, 64, 128, 0.00f, 5.42f, 16.04f, 0.80f, 0.18f}, {TILE_96x128, 96, 128, 128, 0.00f, 7.28f, 22.22f, 0.66f, 0.06f},
+      {TILE_128x128, 128, 128, 128, 2.36f, 3.88f, 30.34f, 0.54f, 0.02f}, {TILE_192x128, 192, 128, 64, 2.96f, 4.86f, 48.02f, 0.48f, 0.01f},
+      {TILE_256x128, 256, 128, 64, 2.58f, 5.85f, 62.65f, 0.50f, -0.09f}, {TILE_256x256, 256, 256, 64, 2.21f, 8.13f, 111.38f, 0.50f, -0.07f}},
+     {{TILE_64x64, 64, 64, 256, 1.84f, 2.38f, 11.89f, 0.74f, 0.11f}, {TILE_96x64, 96, 64, 128, 0.63f, 4.46f, 15.47f, 0.81f, 0.37f},
+      {TILE_128x64, 128, 64, 128, 1.41f, 3.75f, 19.00f, 0.80f, 0.21f}, {TILE_96x128, 96, 128, 128, 0.00f, 6.78f, 27.90f, 0.73f, 0.06f},
+      {TILE_128x128, 128, 128, 128, 1.92f, 3.88f, 31.22f, 0.65f, 0.07f}, {TILE_192x128, 192, 128, 64, 0.00f, 8.48f, 47.18f, 0.61f, 0.28f},
+      {TILE_256x128, 256, 128, 64, 1.29f, 7.12f, 70.92f, 0.64f, -0.06f}, {TILE_256x256, 256, 256, 64, 2.70f, 7.41f, 114.01f, 0.48f, -0.05f}}},
+};
 
-GemmTile gemm_tile_pick(int M, int N, int K, bool int4) {
-    if (M <= 64) return M <= 32 ? TILE_32x64 : TILE_64x64;
-    GemmTile best = TILE_64x64;
-    float best_cost = 0.f;
-    for (const TileCost &t : int4 ? kCostI4 : kCostI8) {
-        const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), rounds = (tiles + 255) / 256;
-        const float fill = (float)(tiles - (rounds - 1) * 256) / 256.f;
-        const float a = ((float)(rounds - 1) + t.b + (1.f - t.b) * fill) * (t.c0 + t.c1 * (float)K / 4096.f), cost = a * (1.f + t.q * a / (a + 100.f));
-        if (best_cost == 0.f || cost < best_cost) {
-            best = t.tile;
-            best_cost = cost;
+// K up to which the loop for few steps is the faster one (it also is for the first steps of the others, hence no clear line: within 2 %
+// of each other for a third of the value on both sides).  us, that loop / the other: 24 x 1024 x 1120 int4 5.2 / 5.8, 48 x 1024 x 512 4.7 / 4.9,
+// 24 x 1024 x 512 int8 3.85 / 4.05, 247 x 13952 x 96 int8 6.7 / 7.8; 48 x 4096 x 8192 int4 21.7 / 19.0, 100 x 1024 x 4096 13.0 / 11.8.
+static int short_k(GemmTile t, bool int4, bool guard) {
+    switch (t) {
+        case TILE_32x64: return int4 ? (guard ? 8192 : 3584) : guard ? 2560 : 3584;
+        case TILE_64x64: return int4 && guard ? 4096 : 1792;
+        case TILE_128x128: return int4 ? (guard ? 1536 : 768) : guard ? 1536 : 1792;
+        case TILE_256x256: return int4 ? (guard ? 1280 : 512) : 0;
+        default: return 0;
+    }
+}
+
+GemmTile gemm_tile_pick(int M, int N, int K, bool int4, bool guard) {
+    GemmTile best = M <= 32 ? TILE_32x64 : TILE_64x64;
+    if (M > 64) {
+        float best_cost = 0.f;
+        for (const TileCost &t : kCost[int4][guard]) {
+            const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), rounds = (tiles + 255) / 256;
+            const float fill = (float)(tiles - (rounds - 1) * 256) / 256.f, k = (float)((K + t.ks - 1) / t.ks) * (float)t.ks;
+            const float a = t.s + ((float)(rounds - 1) + t.b + (1.f - t.b) * fill) * (t.c0 + t.c1 * k / 4096.f), cost = a * (1.f + t.q * a / (a + 100.f));
+            if (best_cost == 0.f || cost < best_cost) {
+                best = t.tile;
+                best_cost = cost;
+            }
         }
     }
-    return best;
+    if (K > short_k(best, int4, guard)) return best;
+    switch (best) {
+        case TILE_32x64: return SHORT_32x64;
+        case TILE_64x64: return SHORT_64x64;
+        case TILE_128x128: return SHORT_128x128;
+        case TILE_256x256: return SHORT_256x256;
+        default: return best;
+    }
 }
 
 template <bool I4, bool GUARD>
@@ -712,8 +856,15 @@ static int launch_tile(const uint16_t *x, const uint8_t *w, const void *sc, uint
             else return tileq::launch<I4, 1, 2, 4, 4, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
         case TILE_192x128: return tileq::launch<I4, 2, 2, 2, 3, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
         case TILE_256x128: return tileq::launch<I4, 2, 2, 2, 4, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
-        default: return tileq::launch<I4, 1, 8, 1, 8, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        case TILE_256x256: return tileq::launch<I4, 1, 8, 1, 8, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        case SHORT_32x64: return tileq::launch<I4, 1, 2, 4, 1, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, 1, st);
+        case SHORT_64x64: return tileq::launch<I4, 1, 2, 4, 2, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, 1, st);
+        case SHORT_128x128: return tileq::launch<I4, 1, 4, 2, 4, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, 1, st);
+        case SHORT_256x256:
+            if constexpr (I4) return tileq::launch<I4, 1, 8, 1, 8, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, 1, st);
+            break;
     }
+    return fail(CHADQ_ERR_SHAPE, "gemm: no tile %d", (int)tile);
 }
 
 int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, GemmTile tile,
@@ -724,7 +875,9 @@ int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t 
 
 int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st) {
     const uint8_t *w = reinterpret_cast<const uint8_t *>(w8);
-    const int step = tile == TILE_32x64 || tile == TILE_64x64 ? 256 : tile == TILE_256x256 || tile == TILE_192x128 || tile == TILE_256x128 ? 64 : 128;
+    const bool k256 = tile == TILE_32x64 || tile == TILE_64x64 || tile == SHORT_32x64 || tile == SHORT_64x64;
+    const bool k64 = tile == TILE_256x256 || tile == TILE_192x128 || tile == TILE_256x128;
+    const int step = k256 ? 256 : k64 ? 64 : 128;  // k of a step
     return K % step ? launch_tile<false, true>(x, w, sc, y, M, N, K, tile, st) : launch_tile<false, false>(x, w, sc, y, M, N, K, tile, st);
 }
 

@@ -1,12 +1,51 @@
 """Which kernel a call takes: the rules by size, asked directly on the host (C++ functions of libchadq.so).  No GPU."""
 import ctypes
 
+import pytest
+
 from chadslab_amd import _lib
+
+TILES = ["32x64", "64x64", "96x64", "128x64", "96x128", "128x128", "192x128", "256x128", "256x256",
+         "short 32x64", "short 64x64", "short 128x128", "short 256x256"]
+
 
 def _rule(symbol, result=ctypes.c_int):
     fn = _lib.load()[symbol]
     fn.restype = result
     return fn
+
+
+def _tile(m, n, k, int4, guard):
+    fn = _rule("_ZN5chadq14gemm_tile_pickEiiibb")
+    fn.argtypes = [ctypes.c_int] * 3 + [ctypes.c_bool] * 2
+    return TILES[fn(m, n, k, int4, guard)]
+
+
+def test_gemm_tile_of_few_k_is_not_one_fitted_to_many():
+    """Products of a few steps, each with its time on the tile given here and on the one that constants fitted to 512 k and more gave."""
+    assert _tile(193, 12160, 128, False, False) == "short 128x128"  # 6.5 us, on 128 x 64 8.8
+    assert _tile(2690, 256, 256, False, False) == "short 64x64"     # 4.3, on 96 x 64 5.1
+    assert _tile(1865, 1728, 256, False, False) == "short 128x128"  # 8.1, on 192 x 128 9.8
+    assert _tile(24, 1024, 1120, True, True) == "short 32x64"       # 5.2, with the other loop 5.8
+    assert _tile(48, 1024, 512, True, False) == "short 64x64"       # 4.7, with the other loop 4.9
+    # and many k still take the loop that is the faster one there
+    assert _tile(48, 14336, 4096, True, False) == "64x64"
+    assert _tile(512, 4096, 4096, True, False) == "128x64"
+    assert _tile(1000, 4096, 14336, False, False) == "128x128"
+    assert _tile(4096, 14336, 4096, True, False) == "256x256"
+
+
+@pytest.mark.parametrize("int4", [True, False])
+@pytest.mark.parametrize("guard", [True, False])
+def test_gemm_tile_fits_the_rows_and_every_tile_is_somebodys(int4, guard):
+    seen = set()
+    for m in (1, 17, 32, 33, 64, 65, 70, 100, 129, 190, 250, 300, 385, 512, 700, 1000, 1500, 2049, 4096, 7000):
+        for n in (1, 64, 257, 1024, 2048, 3000, 4096, 5000, 8192, 11008, 14336, 20000, 33000):
+            for k in (32, 96, 256, 512, 800, 1024, 1504, 2048, 4096, 8192, 14336):
+                tile = _tile(m, n, k, int4, guard)
+                seen.add(tile)
+                assert tile.endswith("32x64") == (m <= 32) and (m > 64 or tile.endswith(("32x64", "64x64")))
+    assert seen == set(TILES) - (set() if int4 else {"short 256x256"})
 
 
 def test_gemv_of_k_that_256_does_not_divide_takes_the_matrix_cores_where_they_are_faster():

@@ -470,7 +470,7 @@ def test_gemm_int4_many_rows_tile(ops, m, n, k):
     assert O.rel_l2(y, O.qgemm_int4g32_f64(xb, packed, s)) <= TOL_BF16
 
 
-@pytest.mark.parametrize("m,n,k", [(385, 8200, 64), (641, 4100, 96), (1025, 4095, 32), (1024, 4096, 384), (897, 4223, 1312),  # 128 x 128 tiles
+@pytest.mark.parametrize("m,n,k", [(385, 8200, 64), (641, 4100, 96), (1025, 4095, 32), (1024, 4096, 384), (897, 4223, 1312),  # some of each
                                    (3841, 3847, 32), (4096, 4097, 288), (3840, 4096, 256),                                # 256 x 256
                                    (17, 100, 32), (32, 515, 512), (33, 1000, 4352), (64, 64, 256), (63, 4097, 1056),      # 64 x 64, at most 64 rows
                                    (65, 100, 32), (128, 8192, 64), (129, 5440, 1056), (1000, 1000, 288), (2049, 447, 512)])   # and in one round
@@ -492,16 +492,65 @@ def test_gemm_eight_wave_tiles_every_row_and_column(ops, weight, m, n, k):
         assert np.sqrt(err.sum(axis=axis) / (ref ** 2).sum(axis=axis)).max() <= TOL_BF16
 
 
-@pytest.mark.parametrize("m,n,k", [(69, 3963, 32), (555, 1697, 96), (193, 4000, 512), (190, 4097, 1056),          # 96 x 64 tiles
-                                   (99, 8259, 32), (509, 3918, 96), (512, 4095, 512), (385, 5000, 1312),          # 128 x 64
-                                   (259, 8306, 512), (259, 6663, 1312), (276, 8097, 768),                         # 96 x 128
-                                   (390, 8279, 32), (1159, 3291, 160), (386, 11008, 256), (577, 5500, 544),       # 192 x 128
-                                   (588, 8210, 32), (635, 8317, 160), (600, 8300, 512), (513, 8193, 1312)])       # 256 x 128
+@pytest.mark.parametrize("m,n,k", [(69, 3963, 32), (555, 1697, 96), (193, 4000, 512), (190, 4097, 1056),
+                                   (99, 8259, 32), (509, 3918, 96), (512, 4095, 512), (385, 5000, 1312),
+                                   (259, 8306, 512), (259, 6663, 1312), (276, 8097, 768),
+                                   (390, 8279, 32), (1159, 3291, 160), (386, 11008, 256), (577, 5500, 544),
+                                   (588, 8210, 32), (635, 8317, 160), (600, 8300, 512), (513, 8193, 1312)])
 @pytest.mark.parametrize("weight", ["int4", "int8"])
 def test_gemm_tiles_between_64_and_256_rows(ops, weight, m, n, k):
-    """The sizes at which the other tiles of gemm_tile_q.hip are picked, ragged in rows, columns and k (from one step to more than
-    the unrolled loop takes); every row and column by itself, as above."""
+    """Grids of one to a few rounds, where the rule by size weighs all tiles against each other, ragged in rows, columns and k; every row and
+    column by itself, as above.  (Each tile at the sizes where it can go wrong: test_gemm_each_tile_by_itself.)"""
     test_gemm_eight_wave_tiles_every_row_and_column(ops, weight, m, n, k)
+
+
+TILES = [("32x64", 256), ("64x64", 256), ("96x64", 128), ("128x64", 128), ("96x128", 128), ("128x128", 128), ("192x128", 64), ("256x128", 64),
+         ("256x256", 64), ("short 32x64", 256), ("short 64x64", 256), ("short 128x128", 128), ("short 256x256", 64)]  # k of a step
+
+
+@pytest.mark.parametrize("tile", range(len(TILES)), ids=[t[0] for t in TILES])
+@pytest.mark.parametrize("weight", ["int4", "int8"])
+def test_gemm_each_tile_by_itself(ops, weight, tile):
+    """Every tile at ragged ends of rows and columns, whichever the rule by size would take: k of one step, of as many as there are stages, of
+    more than the unrolled loop takes and in between, with and without a remainder; int4 scales that are not 16-byte aligned."""
+    import ctypes
+
+    from chadslab_amd import _lib
+
+    name, step = TILES[tile]
+    if name == "short 256x256" and weight == "int8":
+        pytest.skip("not built: never the faster one")
+    launch = _lib.load()["_ZN5chadq22gemm_tile_i4g32_launchEPKtPKhS1_PtiiiNS_8GemmTileEP12ihipStream_t" if weight == "int4" else
+                         "_ZN5chadq22gemm_tile_i8row_launchEPKtPKaPKfPtiiiNS_8GemmTileEP12ihipStream_t"]
+    launch.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 + [ctypes.c_void_p]
+    bm, bn = (int(v) for v in name.split()[-1].split("x"))
+    if weight == "int4":
+        ks = [256, 512, 768, 1024, 2304, 2560] + [32, 96, step + 32, 2 * step + 160, 4 * step + 96, 9 * step + 32, 1056]
+    else:
+        ks = [step * i for i in (1, 2, 3, 4, 6, 9, 10)] + [16, 48, step + 16, 2 * step + 144, 4 * step + 80, 9 * step + 16]
+    for i, k in enumerate(ks):
+        m, n = ((bm + 3, bn + 5), (2 * bm - 1, 3), (bm, 2 * bn))[i % 3]
+        seed = 660 + 100 * tile + i
+        if weight == "int4":
+            packed, s, xb, q = i4_case(seed, m, n, k)
+            w, sc = q.packed, q.scale
+            wv = O.bf16_to_f32(O.f32_to_bf16(O.dequant_int4g32(packed, s))).astype(np.float64)  # as the matrix cores get them
+        else:
+            xf, wn, s, q = i8_case(seed, m, n, k)
+            xb = O.f32_to_bf16(xf)
+            w, sc, wv = q.w, q.scale, wn * s.astype(np.float64)[:, None]
+        xv = O.bf16_to_f32(xb).astype(np.float64)
+        ref, mag = xv @ wv.T, np.abs(xv) @ np.abs(wv).T
+        x = bf16_tensor(xb)
+        scales = [sc]
+        if weight == "int4" and k % 256 == 0:
+            scales.append(torch.cat((sc.new_zeros(1), sc.reshape(-1)))[1:])
+        for sv in scales:
+            y = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+            assert launch(x.data_ptr(), w.data_ptr(), sv.data_ptr(), y.data_ptr(), m, n, k, tile, torch.cuda.current_stream().cuda_stream) == 0
+            assert bool((y[m] == 7).all()), ("a row too many", k)
+            # the products are exact in fp32: the fp32 sum of at most k terms, the rounding to bf16
+            assert (np.abs(O.bf16_to_f32(bits(y[:m])) - ref) <= 2.0**-8 * np.abs(ref) + (k / 8 + 8) * 2.0**-24 * mag).all(), (m, n, k)
 
 
 @pytest.mark.parametrize("n", [64, 128, 512])

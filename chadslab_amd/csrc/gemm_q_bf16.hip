@@ -448,10 +448,9 @@ int gemm_i8row_bf16_dispatch(const uint16_t *x, const int8_t *w8, const float *s
     return launch_gemm<FmtI8Row, false>(x, w8, sc, y, M, N, K, nullptr, 0, st);
 }
 
-// One launch over `ngroups` int4 group-32 products that share N and K; m_max bounds every group's row count.
-int gemm_i4g32_grouped(const GemmGroup *groups, int ngroups, int m_max, int N, int K, bool out_f32, hipStream_t st) {
-    if (out_f32) return launch_gemm<FmtI4G32, true>(nullptr, nullptr, nullptr, nullptr, m_max, N, K, groups, ngroups, st);
-    return launch_gemm<FmtI4G32, false>(nullptr, nullptr, nullptr, nullptr, m_max, N, K, groups, ngroups, st);
+// One launch over `ngroups` int4 group-32 products that share N and K, fp32 results; m_max bounds every group's row count.
+int gemm_i4g32_grouped(const GemmGroup *groups, int ngroups, int m_max, int N, int K, hipStream_t st) {
+    return launch_gemm<FmtI4G32, true>(nullptr, nullptr, nullptr, nullptr, m_max, N, K, groups, ngroups, st);
 }
 
 }  // namespace chadq

@@ -45,7 +45,7 @@ struct MoeWs {  // workspace carved up on the host
 
 constexpr int MOE_KSPLIT = 4;
 
-int gemm_i4g32_grouped(const GemmGroup *groups, int ngroups, int m_max, int N, int K, bool out_f32, hipStream_t st);
+int gemm_i4g32_grouped(const GemmGroup *groups, int ngroups, int m_max, int N, int K, hipStream_t st);
 bool gemm_skinny_ok(int H, int F);
 int gemm_skinny_tile_rows();
 int gemm_skinny_gateup(const GemmGroup *groups, const int32_t *tiles, const int32_t *tok, int ntiles, int E, int F, int H,
@@ -482,10 +482,10 @@ int moe_ffn_i4g32_launch(const uint16_t *x, const float *logits, const chadq_moe
         rc = gemm_skinny_down(ws.groups, ws.tiles, ntiles, E, H, F, nsplit, (size_t)P * H, st);  // fp32 parts [nsplit][P,H]
         if (rc) return rc;
     } else {
-        rc = gemm_i4g32_grouped(ws.groups, 2 * E, m_max, F, H, true, st);  // gate and up: fp32 [P,F] each
+        rc = gemm_i4g32_grouped(ws.groups, 2 * E, m_max, F, H, st);  // gate and up: fp32 [P,F] each
         if (rc) return rc;
         hipLaunchKernelGGL(moe_act_kernel, dim3(2048), dim3(256), 0, st, ws.g, ws.u, ws.h, (int64_t)P * F / 4);
-        rc = gemm_i4g32_grouped(ws.groups + 2 * E, E, m_max, H, F, true, st);  // down: fp32 [P,H]
+        rc = gemm_i4g32_grouped(ws.groups + 2 * E, E, m_max, H, F, st);  // down: fp32 [P,H]
         if (rc) return rc;
     }
     const int64_t quads = (int64_t)T * (H / 4);

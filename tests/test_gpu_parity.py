@@ -553,6 +553,24 @@ def test_gemm_each_tile_by_itself(ops, weight, tile):
             assert (np.abs(O.bf16_to_f32(bits(y[:m])) - ref) <= 2.0**-8 * np.abs(ref) + (k / 8 + 8) * 2.0**-24 * mag).all(), (m, n, k)
 
 
+@pytest.mark.parametrize("more", [0, 1])
+@pytest.mark.parametrize("weight", ["int4", "int8"])
+def test_gemm_of_rows_beyond_the_tiles_offsets(ops, weight, more):
+    """K of 2^22 and more: the 128 x 64 kernel of gemm_q_bf16.hip, with and without a remainder of its step."""
+    m, n = 5, 3
+    if weight == "int4":
+        k = 2 ** 22 + 32 * more
+        packed, s, xb, q = i4_case(690 + more, m, n, k)
+        w = (np.stack([packed & 15, packed >> 4], 2).reshape(n, k) - 8.0) * np.repeat(s.astype(np.float64), 32, 1)
+    else:
+        k = 2 ** 22 + 16 * more
+        xf, wn, s, q = i8_case(690 + more, m, n, k)
+        xb = O.f32_to_bf16(xf)
+        w = wn * s.astype(np.float64)[:, None]
+    y = O.bf16_to_f32(bits(ops.qgemm(bf16_tensor(xb), q)))
+    assert O.rel_l2(y, O.bf16_to_f32(xb).astype(np.float64) @ w.T) <= TOL_BF16
+
+
 @pytest.mark.parametrize("n", [64, 128, 512])
 def test_gemm_refuses_4_gib_of_activations_for_every_tile(ops, n):
     """One row below the limit is served and right in its last rows; at the limit the call is refused, whichever tile N picks."""

@@ -137,7 +137,8 @@ def native():
         _native = importlib.util.module_from_spec(importlib.util.spec_from_loader("chadslab_amd._host_call", loader))
     from .formats import QWeightInt4G32, QWeightInt4G32Tiles, QWeightInt8
 
-    _native.bind(tuple(ctypes.cast(getattr(lib, n), c_void_p).value for n in _NATIVE_ENTRIES), (QWeightInt4G32, QWeightInt8, QWeightInt4G32Tiles))
+    _native.bind(tuple(ctypes.cast(getattr(lib, n), c_void_p).value for n in _NATIVE_ENTRIES), (QWeightInt4G32, QWeightInt8, QWeightInt4G32Tiles),
+                 check)
     _native_lib = lib
     return _native
 

@@ -5,8 +5,10 @@
 // 59 us (96 tensors looked at one by one).  Here the same checks are C++: 4.9 us, and 28 us with the GPU the slower side.
 //
 // Only what needs nothing unusual is served: exact torch.Tensor objects on the current device, of the right types and shapes,
-// contiguous.  For everything else, also for a call that the library refuses, the functions return None before anything has been
-// launched, and the Python code behind them does what it always did: copies, casts, and the errors' texts.
+// contiguous.  For everything else, also for a call whose arguments the library refuses, the functions return None before anything has
+// been launched, and the Python code behind them does what it always did: copies, casts, and the errors' texts.  An error of the
+// device or of a launch is raised here and now, with the library's text: kernels of the call may be queued, and a second attempt
+// would find another error than the one that was reported.
 #include <ATen/ops/empty.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -22,8 +24,12 @@ typedef size_t (*moe_bytes_fn)(int, int, int, int, int);
 typedef int (*moe_fn)(const void *, const void *, const chadq_moe_expert_i4g32 *, void *, int, int, int, int, int, int, void *, size_t, void *);
 
 enum Entry { GEMV_I4, GEMV_I4_BF16, GEMM_I4, GEMV_I8, GEMV_I8_BF16, GEMM_I8, MOE_BYTES, MOE_ROWS, MOE_TILES, ENTRIES };
+const char *const kEntryNames[ENTRIES] = {"chadq_gemv_i4g32", "chadq_gemv_i4g32_bf16", "chadq_gemm_i4g32_bf16", "chadq_gemv_i8row", "chadq_gemv_i8row_bf16",
+                                          "chadq_gemm_i8row_bf16", "chadq_moe_ffn_i4g32_workspace_bytes", "chadq_moe_ffn_i4g32",
+                                          "chadq_moe_ffn_i4g32_tiled"};
 void *g_entry[ENTRIES];                                // of the library in use (bind)
 PyObject *g_int4 = nullptr, *g_int8 = nullptr, *g_tiles = nullptr;  // the weight containers
+PyObject *g_check = nullptr;                           // _lib.check(status, name): raises
 PyObject *s_packed, *s_scale, *s_w;
 constexpr int kGemvRows = 16, kMaxExperts = 16;
 
@@ -46,6 +52,12 @@ struct Ref {  // a new reference, dropped at the end of the scope
     ~Ref() { Py_XDECREF(p); }
     Ref(const Ref &) = delete;
 };
+
+// What becomes of a call that did not succeed (the text of the error belongs to this thread)
+PyObject *failed(int rc, const char *name) {
+    if (rc != CHADQ_ERR_HIP && rc != CHADQ_ERR_DEVICE) Py_RETURN_NONE;
+    return PyObject_CallFunction(g_check, "is", rc, name);
+}
 
 // linear(x, weight, out_dtype) -> y, or None
 PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
@@ -87,7 +99,7 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     Py_BEGIN_ALLOW_THREADS
     rc = reinterpret_cast<product_fn>(g_entry[e])(xp, wp, sp, yp, (int)m, (int)n, (int)k, stream);
     Py_END_ALLOW_THREADS
-    if (rc != 0) Py_RETURN_NONE;
+    if (rc != 0) return failed(rc, kEntryNames[e]);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -140,24 +152,24 @@ PyObject *moe_ffn(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     at::Tensor ws = at::empty({(int64_t)need}, x->options().dtype(at::kByte).requires_grad(false));
     at::Tensor y = at::empty({t, h}, x->options().requires_grad(false));
     if (!ws.unsafeGetTensorImpl()->has_storage() || !y.unsafeGetTensorImpl()->has_storage()) Py_RETURN_NONE;
+    const Entry entry = kind == g_tiles ? MOE_TILES : MOE_ROWS;
     const void *const xp = x->const_data_ptr(), *const zp = z->const_data_ptr();
     void *const yp = y.mutable_data_ptr(), *const wsp = ws.mutable_data_ptr(), *const stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream();
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = reinterpret_cast<moe_fn>(g_entry[kind == g_tiles ? MOE_TILES : MOE_ROWS])(xp, zp, arr, yp, (int)t, (int)h, (int)f, (int)e, (int)top_k, renorm,
-                                                                              wsp, need, stream);
+    rc = reinterpret_cast<moe_fn>(g_entry[entry])(xp, zp, arr, yp, (int)t, (int)h, (int)f, (int)e, (int)top_k, renorm, wsp, need, stream);
     Py_END_ALLOW_THREADS
-    if (rc != 0) Py_RETURN_NONE;
+    if (rc != 0) return failed(rc, kEntryNames[entry]);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
 
-// bind(addresses of the entry points in the order of Entry, (QWeightInt4G32, QWeightInt8, QWeightInt4G32Tiles))
+// bind(addresses of the entry points in the order of Entry, (QWeightInt4G32, QWeightInt8, QWeightInt4G32Tiles), check)
 PyObject *bind(PyObject *, PyObject *args) {
-    PyObject *addr, *kinds;
-    if (!PyArg_ParseTuple(args, "O!O!", &PyTuple_Type, &addr, &PyTuple_Type, &kinds)) return nullptr;
-    if (PyTuple_GET_SIZE(addr) != ENTRIES || PyTuple_GET_SIZE(kinds) != 3) {
-        PyErr_SetString(PyExc_ValueError, "bind: one address per entry point and three containers");
+    PyObject *addr, *kinds, *check;
+    if (!PyArg_ParseTuple(args, "O!O!O", &PyTuple_Type, &addr, &PyTuple_Type, &kinds, &check)) return nullptr;
+    if (PyTuple_GET_SIZE(addr) != ENTRIES || PyTuple_GET_SIZE(kinds) != 3 || !PyCallable_Check(check)) {
+        PyErr_SetString(PyExc_ValueError, "bind: one address per entry point, three containers and a function");
         return nullptr;
     }
     void *fresh[ENTRIES];
@@ -175,12 +187,14 @@ PyObject *bind(PyObject *, PyObject *args) {
         Py_INCREF(k);
         Py_XSETREF(*slot[i], k);
     }
+    Py_INCREF(check);
+    Py_XSETREF(g_check, check);
     Py_RETURN_NONE;
 }
 
 PyMethodDef methods[] = {{"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, "linear(x, weight, out_dtype) -> y, or None where the Python path has to look"},
                          {"moe_ffn", (PyCFunction)(void (*)(void))moe_ffn, METH_FASTCALL, "moe_ffn(x, logits, experts, top_k, renorm) -> y, or None"},
-                         {"bind", bind, METH_VARARGS, "bind(addresses, containers)"},
+                         {"bind", bind, METH_VARARGS, "bind(addresses, containers, check)"},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_call", nullptr, -1, methods};
 

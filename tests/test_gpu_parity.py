@@ -788,6 +788,44 @@ def test_native_calls_serve_plain_tensors_and_leave_the_rest_to_python(ops):
     assert torch.equal(ops.moe_ffn(wide[:5, :256], z, experts, top_k=2), y)
 
 
+@pytest.mark.parametrize("status,error", [(-5, RuntimeError), (-6, RuntimeError)])
+def test_native_calls_raise_a_device_error_at_the_first_attempt(ops, status, error):
+    """An entry point that reports a failed launch (-5) or device (-6) is called once and its error is the one that is raised; a refused
+    argument (any other status) is left to the Python road."""
+    import ctypes
+
+    from chadslab_amd import QWeightInt4G32, QWeightInt8, QWeightInt4G32Tiles, _lib
+
+    native = _lib.native()
+    calls = []
+    product = ctypes.CFUNCTYPE(ctypes.c_int, *[ctypes.c_void_p] * 4, *[ctypes.c_int] * 3, ctypes.c_void_p)
+    moe = ctypes.CFUNCTYPE(ctypes.c_int, *[ctypes.c_void_p] * 4, *[ctypes.c_int] * 6, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p)
+
+    def fail(*args):
+        calls.append(args)
+        return status
+
+    p, m = product(fail), moe(fail)
+    real = {n: ctypes.cast(getattr(_lib.load(), n), ctypes.c_void_p).value for n in _lib._NATIVE_ENTRIES}
+    fake = [real[n] if "workspace" in n else ctypes.cast(m if "moe" in n else p, ctypes.c_void_p).value for n in _lib._NATIVE_ENTRIES]
+    q = QWeightInt4G32(torch.zeros(256, 128, dtype=torch.uint8, device=DEV), torch.ones(256, 8, dtype=torch.float16, device=DEV))
+    x = torch.ones(3, 256, dtype=torch.bfloat16, device=DEV)
+    try:
+        native.bind(tuple(fake), (QWeightInt4G32, QWeightInt8, QWeightInt4G32Tiles), _lib.check)
+        with pytest.raises(error, match="chadq_gemv_i4g32 failed"):
+            ops.qlinear(x, q)
+        assert len(calls) == 1
+        with pytest.raises(error, match="chadq_moe_ffn_i4g32 failed"):
+            ops.moe_ffn(x, torch.zeros(3, 1, device=DEV), [(q, q, q)], top_k=1)
+        assert len(calls) == 2
+        status = -2
+        assert native.linear(x, q, None) is None and len(calls) == 3
+    finally:
+        _lib._native_lib = None
+        _lib.native()
+    assert torch.equal(ops.qlinear(x, q), torch.full((3, 256), -2048.0, device=DEV))
+
+
 def test_moe_route_matches_oracle(ops):
     r = rng(70)
     logits = r.standard_normal((300, 8)).astype(np.float32)

@@ -114,8 +114,12 @@ PyObject *moe_ffn(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     const Py_ssize_t e = PySequence_Fast_GET_SIZE(args[2]);
     const long top_k = PyLong_AsLong(args[3]);
     if (top_k == -1 && PyErr_Occurred()) PyErr_Clear();
-    const int renorm = PyObject_IsTrue(args[4]);
-    if (renorm < 0) return nullptr;
+    // (other objects than True, False and ints go through Python's int())
+    if (!PyBool_Check(args[4]) && !PyLong_CheckExact(args[4])) Py_RETURN_NONE;
+    int overflow = 0;
+    const long renorm_value = PyLong_AsLongAndOverflow(args[4], &overflow);
+    if (overflow || renorm_value < INT_MIN || renorm_value > INT_MAX) Py_RETURN_NONE;
+    const int renorm = (int)renorm_value;
     if (!x || !z || e < 1 || e > kMaxExperts || top_k < 1 || top_k > e) Py_RETURN_NONE;
     const int64_t t = x->size(0), h = x->size(1);
     if (t < 1 || t > INT_MAX || h < 1 || h > INT_MAX || z->size(0) != t || z->size(1) != e) Py_RETURN_NONE;

@@ -788,6 +788,22 @@ def test_native_calls_serve_plain_tensors_and_leave_the_rest_to_python(ops):
     assert torch.equal(ops.moe_ffn(wide[:5, :256], z, experts, top_k=2), y)
 
 
+def test_moe_ffn_reads_renorm_as_int_does(ops):
+    """0.5 is 0, None has no int: what is no bool and no int goes the way of int(renorm), whichever road serves the call."""
+    from chadslab_amd import _lib
+
+    experts = [(i4_case(44 + i, 1, 256, 256)[3],) * 3 for i in range(4)]
+    x, z = torch.randn(5, 256, device=DEV).bfloat16(), torch.randn(5, 4, device=DEV)
+    yes, no = (ops.moe_ffn(x, z, experts, renorm=v) for v in (True, False))
+    assert not torch.equal(yes, no)
+    for value, same in ((1, yes), (-3, yes), (0, no), (0.5, no), (1.5, yes), (np.bool_(True), yes), (torch.tensor(0), no)):
+        assert torch.equal(ops.moe_ffn(x, z, experts, renorm=value), same), value
+    for value in (0.5, None, "1", np.bool_(True), 2 ** 40):
+        assert _lib.native().moe_ffn(x, z, experts, 2, value) is None
+    with pytest.raises(TypeError):
+        ops.moe_ffn(x, z, experts, renorm=None)
+
+
 @pytest.mark.parametrize("status,error", [(-5, RuntimeError), (-6, RuntimeError)])
 def test_native_calls_raise_a_device_error_at_the_first_attempt(ops, status, error):
     """An entry point that reports a failed launch (-5) or device (-6) is called once and its error is the one that is raised; a refused

@@ -53,6 +53,13 @@ struct Ref {  // a new reference, dropped at the end of the scope
     Ref(const Ref &) = delete;
 };
 
+// The interpreter lock is given up for as long as this lives, as torch.empty and ctypes do: an allocation may wait for the device (the
+// allocator gives cached memory back and asks again) or run a hook that wants the lock on a thread that another allocation waits for.
+struct WithoutLock {
+    PyThreadState *const state = PyEval_SaveThread();
+    ~WithoutLock() { PyEval_RestoreThread(state); }
+};
+
 // What becomes of a call that did not succeed (the text of the error belongs to this thread)
 PyObject *failed(int rc, const char *name) {
     if (rc != CHADQ_ERR_HIP && rc != CHADQ_ERR_DEVICE) Py_RETURN_NONE;
@@ -91,14 +98,17 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
         y_type = want;
     }
     const Entry e = !gemv ? (int4 ? GEMM_I4 : GEMM_I8) : y_type == at::kFloat ? (int4 ? GEMV_I4 : GEMV_I8) : (int4 ? GEMV_I4_BF16 : GEMV_I8_BF16);
-    at::Tensor y = at::empty({m, n}, x->options().dtype(y_type).requires_grad(false));
-    if (!y.unsafeGetTensorImpl()->has_storage()) Py_RETURN_NONE;
-    const void *const xp = x->const_data_ptr(), *const wp = w->const_data_ptr(), *const sp = s->const_data_ptr();
-    void *const yp = y.mutable_data_ptr(), *const stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream();
+    const at::Tensor keep[3] = {*x, *w, *s};  // whatever another thread does with the objects
+    const product_fn fn = reinterpret_cast<product_fn>(g_entry[e]);
+    at::Tensor y;
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = reinterpret_cast<product_fn>(g_entry[e])(xp, wp, sp, yp, (int)m, (int)n, (int)k, stream);
-    Py_END_ALLOW_THREADS
+    {
+        const WithoutLock free;
+        y = at::empty({m, n}, keep[0].options().dtype(y_type).requires_grad(false));
+        if (!y.unsafeGetTensorImpl()->has_storage()) rc = CHADQ_ERR_NULL;
+        else rc = fn(keep[0].const_data_ptr(), keep[1].const_data_ptr(), keep[2].const_data_ptr(), y.mutable_data_ptr(), (int)m, (int)n, (int)k,
+                     c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream());
+    }
     if (rc != 0) return failed(rc, kEntryNames[e]);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
@@ -153,16 +163,19 @@ PyObject *moe_ffn(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     if (f < 1 || f > INT_MAX) Py_RETURN_NONE;
     const size_t need = reinterpret_cast<moe_bytes_fn>(g_entry[MOE_BYTES])((int)t, (int)h, (int)f, (int)e, (int)top_k);
     if (need == 0) Py_RETURN_NONE;
-    at::Tensor ws = at::empty({(int64_t)need}, x->options().dtype(at::kByte).requires_grad(false));
-    at::Tensor y = at::empty({t, h}, x->options().requires_grad(false));
-    if (!ws.unsafeGetTensorImpl()->has_storage() || !y.unsafeGetTensorImpl()->has_storage()) Py_RETURN_NONE;
     const Entry entry = kind == g_tiles ? MOE_TILES : MOE_ROWS;
-    const void *const xp = x->const_data_ptr(), *const zp = z->const_data_ptr();
-    void *const yp = y.mutable_data_ptr(), *const wsp = ws.mutable_data_ptr(), *const stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream();
+    const moe_fn fn = reinterpret_cast<moe_fn>(g_entry[entry]);
+    const at::Tensor xk = *x, zk = *z;  // as keep
+    at::Tensor ws, y;
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = reinterpret_cast<moe_fn>(g_entry[entry])(xp, zp, arr, yp, (int)t, (int)h, (int)f, (int)e, (int)top_k, renorm, wsp, need, stream);
-    Py_END_ALLOW_THREADS
+    {
+        const WithoutLock free;
+        ws = at::empty({(int64_t)need}, xk.options().dtype(at::kByte).requires_grad(false));
+        y = at::empty({t, h}, xk.options().requires_grad(false));
+        if (!ws.unsafeGetTensorImpl()->has_storage() || !y.unsafeGetTensorImpl()->has_storage()) rc = CHADQ_ERR_NULL;
+        else rc = fn(xk.const_data_ptr(), zk.const_data_ptr(), arr, y.mutable_data_ptr(), (int)t, (int)h, (int)f, (int)e, (int)top_k, renorm,
+                     ws.mutable_data_ptr(), need, c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream());
+    }
     if (rc != 0) return failed(rc, kEntryNames[entry]);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS

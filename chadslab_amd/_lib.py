@@ -118,8 +118,29 @@ _NATIVE_ENTRIES = ("chadq_gemv_i4g32", "chadq_gemv_i4g32_bf16", "chadq_gemm_i4g3
                    "chadq_gemm_i8row_bf16", "chadq_moe_ffn_i4g32_workspace_bytes", "chadq_moe_ffn_i4g32", "chadq_moe_ffn_i4g32_tiled")
 
 
+HOST_PATH = Path(__file__).resolve().parent / "_host_call.so"
+
+
+class _NoHostModule:
+    """In the place of a host module that is missing or was built for another torch: every call takes ops.py's own road to the same
+    kernels, some 3 us slower."""
+
+    @staticmethod
+    def bind(addresses, containers, check):
+        pass
+
+    @staticmethod
+    def linear(x, weight, out_dtype):
+        return None
+
+    @staticmethod
+    def moe_ffn(x, logits, experts, top_k, renorm):
+        return None
+
+
 def native():
-    """The host module (csrc/host_call.cpp), bound to the library that load() gives; raises if it has not been built."""
+    """The host module (csrc/host_call.cpp), bound to the library that load() gives.  Where it cannot be loaded the calls go without it, and a
+    warning says so once: it holds no kernels."""
     global _native, _native_lib
     if _native_lib is not None and _native_lib is _lib:
         return _native
@@ -128,13 +149,17 @@ def native():
         import importlib.machinery
         import importlib.util
 
-        path = Path(__file__).resolve().parent / "_host_call.so"
-        if not path.exists():
-            raise ChadqError("%s not found: build it with `python -m chadslab_amd.build` (there is no fallback path)" % path)
         import torch  # noqa: F401  (its libraries have to be loaded first)
 
-        loader = importlib.machinery.ExtensionFileLoader("chadslab_amd._host_call", str(path))
-        _native = importlib.util.module_from_spec(importlib.util.spec_from_loader("chadslab_amd._host_call", loader))
+        loader = importlib.machinery.ExtensionFileLoader("chadslab_amd._host_call", str(HOST_PATH))
+        try:
+            _native = importlib.util.module_from_spec(importlib.util.spec_from_loader("chadslab_amd._host_call", loader))
+        except ImportError as e:
+            import warnings
+
+            warnings.warn("calls take some 3 us longer without the host module (`python -m chadslab_amd.build` builds it): %s" % e,
+                          RuntimeWarning, stacklevel=3)
+            _native = _NoHostModule
     from .formats import QWeightInt4G32, QWeightInt4G32Tiles, QWeightInt8
 
     _native.bind(tuple(ctypes.cast(getattr(lib, n), c_void_p).value for n in _NATIVE_ENTRIES), (QWeightInt4G32, QWeightInt8, QWeightInt4G32Tiles),

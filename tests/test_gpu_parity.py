@@ -788,6 +788,38 @@ def test_native_calls_serve_plain_tensors_and_leave_the_rest_to_python(ops):
     assert torch.equal(ops.moe_ffn(wide[:5, :256], z, experts, top_k=2), y)
 
 
+def test_dimensions_and_casts_of_qlinear_stay_on_the_native_call(ops, monkeypatch):
+    """An x of any number of dimensions, strided or not, and a result of another type: the same bits as the product of the same rows,
+    and the product itself is the native one."""
+    _, _, xb, q4 = i4_case(33, 40, 96, 256)
+    x = bf16_tensor(xb)
+    x8, _, _, q8 = i8_case(34, 40, 96, 256)
+    xf = torch.from_numpy(x8).to(DEV)
+    cases = []
+    for a, q in ((x, q4), (x[:1], q4), (x[:16], q4), (x, q8), (xf[:16], q8), (xf[:1], q8)):
+        y = ops.qgemm(a, q) if a.shape[0] > 16 else ops.qgemv(a, q)
+        half = ops.qlinear(a, q, out_dtype=torch.bfloat16)
+        rows = a.shape[0]
+        shapes = [(rows, 256), (1, rows, 256)] + [(rows // 4, 2, 2, 256)] * (rows % 4 == 0) + [(256,)] * (rows == 1)
+        for shape in shapes:
+            for dt in (None, torch.float32, torch.bfloat16, torch.float16, torch.float64):
+                cases.append((a.view(shape), q, dt, (half if dt == torch.bfloat16 else y if dt is None else y.to(dt)).view(*shape[:-1], 96)))
+    wide = torch.cat([x, x], 1)
+    turned, part, parts = x.view(8, 5, 256).transpose(0, 1), wide[:, :256], wide.view(8, 5, 512)[..., 256:]
+    for a in (turned, part, parts, part[:3]):  # strided
+        rows = a.reshape(-1, 256).contiguous()
+        cases.append((a, q4, None, (ops.qgemm if len(rows) > 16 else ops.qgemv)(rows, q4).view(*a.shape[:-1], 96)))
+
+    def left(*args, **kw):
+        raise AssertionError("the product went through Python")
+
+    for name in ("_gemv", "qgemv", "qgemm"):
+        monkeypatch.setattr(ops, name, left)
+    for a, q, dt, ref in cases:
+        y = ops.qlinear(a, q, out_dtype=dt)
+        assert y.dtype == ref.dtype and torch.equal(y, ref), (a.shape, dt)
+
+
 def test_moe_ffn_reads_renorm_as_int_does(ops):
     """0.5 is 0, None has no int: what is no bool and no int goes the way of int(renorm), whichever road serves the call."""
     from chadslab_amd import _lib

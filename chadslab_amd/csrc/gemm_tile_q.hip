@@ -886,6 +886,29 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
 // how many workgroups and steps wait at once (two workgroups per compute unit for at most 32 rows; the loop is not unrolled: the
 // code of a few steps is fetched as often as it is run).  Whole prompts in us, 128 weight rows for every number of tokens in brackets:
 // 24 tokens through 18 layers of 2048 x 16384 1152 (1343), 9 through 6 of 1280 x 3840 262 (321), 37 through 4 of 2048 x 8960 282 (311).
+struct ExactCost {
+    int bm, bn;  // tile
+    float s, c0, c1, d0, d1, b, c2;
+};
+static const ExactCost kExact32 = {32, 64, 4.87f, -1.63f, .694f, 1.42f, .694f, .870f, .216f}, kExact64 = {64, 64, 2.75f, 1.42f, .779f, 1.42f, .779f, .904f, .284f},
+                       kExact128 = {128, 128, 3.84f, 1.29f, 2.55f, 1.29f, 2.55f, .950f, .184f};
+
+// us that a launch takes in `parts` K splits of `per` 256-k blocks.  Tiles go to the XCDs in turn, each in all its splits, and a round is over
+// when the fullest XCD has dealt its workgroups to its 32 compute units: 33 tiles in 7 parts are 231 workgroups, but 35 on one XCD.  A tile
+// takes c0 + c1 * per in the first round and d0 + d1 * per in a further one (of the tiles of 32 rows two fit on a compute unit), the last
+// round b + (1 - b) f of it if it is full to f; s is what a launch takes besides, c2 what a MB of fp32 parts takes to be written.  Fitted to 3900
+// random products in every number of splits (2 to 700 rows, 128 to 8192 weight rows, 256 to 24000 k): 4 % standard deviation.
+static float exact_us(const ExactCost &t, int M, int N, int per, int parts) {
+    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), fullest = (tiles + 7) / 8 * parts, rounds = (fullest + 31) / 32;
+    const float last = t.b + (1.f - t.b) * (float)(fullest - (rounds - 1) * 32) / 32.f, first = t.c0 + t.c1 * (float)per;
+    const float mb = 4e-6f * (float)(tiles * parts) * (float)(t.bm * t.bn);
+    return t.s + (rounds == 1 ? last * first : first + ((float)(rounds - 2) + last) * (t.d0 + t.d1 * (float)per)) + t.c2 * mb;
+}
+
+static float exact_f32_us(int M, int N, int per, int parts) {
+    return exact_us(M <= 32 ? kExact32 : M <= 64 ? kExact64 : kExact128, M, N, per, parts);
+}
+
 template <int EPI>
 static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st) {
     if (M <= 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
@@ -909,21 +932,22 @@ int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint1
                     : tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, true, true, tileq::EPI_F32>(x, wp, sc, y, M, N, K, 1, st);
 }
 
-// K splits that make the launch shortest: rounds of workgroups times the k of each (and what a workgroup costs besides, about
-// 256 k worth).  At most kExactMaxSplits parts of whole 256-k blocks, the last one possibly shorter: with equal parts only, a down
-// projection of 8960 k had one part, 63 us of the 125 that its layer took for 37 tokens.
+// The K splits of a product, whole 256-k blocks each, the last one possibly shorter.  (With equal parts only, a down projection of 8960 k had
+// one part, 63 us of the 125 that its layer took for 37 tokens.)  kRead: us that the next kernel takes for a MB of parts.  Rounds of 256
+// workgroups (512 for up to 32 rows) times the k of each, as the splits were chosen by before, miss how tiles fall to the XCDs, what half a
+// chip costs and what the parts cost.  us, so chosen / now: 265 x 1344 x 7168 in 7 parts 31.6 / in 6 20.5, 552 x 1280 x 5120 in 5 32.1 / in 4 20.7,
+// 22 x 4480 x 1024 in 4 6.4 / in 2 4.9.  M counts in whole tiles only: prompt_layout asks for every number of them.
 int gemm_exact_splits(int M, int N, int K) {
-    const int bm = M <= 32 ? 32 : M <= 64 ? 64 : 128, blocks = K / 256;
-    const int bn = M <= 64 ? 64 : 128, wgs = M <= 32 ? 512 : 256;
-    const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    constexpr float kRead = .4f;
+    const int blocks = K / 256, rows = M <= 32 ? 32 : (M + 63) / 64 * 64;
     int best = 1;
-    int64_t best_cost = 0;
+    float best_us = 0.f;
     for (int s = 1; s <= kExactMaxSplits; ++s) {
         const int per = (blocks + s - 1) / s, parts = (blocks + per - 1) / per;
-        const int64_t cost = (tiles * parts + wgs - 1) / wgs * (per + 1);
-        if (s == 1 || cost < best_cost) {
+        const float us = exact_f32_us(M, N, per, parts) + kRead * 4e-6f * (float)rows * (float)N * (float)parts;
+        if (s == 1 || us < best_us) {
             best = parts;
-            best_cost = cost;
+            best_us = us;
         }
     }
     return best;

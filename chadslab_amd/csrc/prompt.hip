@@ -379,8 +379,8 @@ static size_t prompt_layout(uint8_t *base, int T, int d, int hq, int dh, int ffn
         const size_t n = (size_t)gemm_exact_splits(M, N, K) * M * N;
         parts = n > parts ? n : parts;
     };
-    // (every number of rows up to T: a shorter chunk may come with the same workspace, and fewer rows take more splits)
-    for (int M = 32; M < T + 128; M += M < 128 ? M : 128) {
+    // (every number of row tiles up to T: a shorter chunk may come with the same workspace, and fewer rows can take more splits)
+    for (int M = 32; M < T + 64; M += M < 64 ? M : 64) {
         const int m = M < T ? M : T;
         need(m, (int)wq, d);
         need(m, d, hq * dh);

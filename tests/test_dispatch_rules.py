@@ -87,3 +87,30 @@ def test_expert_down_product_of_short_k_is_not_split_among_many_workgroups():
     assert fn(4 * 375, 2304, 768, 8) == 1 and fn(4 * 422, 2560, 1536, 4) == 1  # 67.0 us (split 71.6), 85.4 (96.3)
     assert fn(2 * 256, 2304, 1280, 8) == 4                                     # 65.8 (69.6)
     assert fn(2 * 455, 2048, 8960, 8) == 3 and fn(4 * 455, 2304, 1280, 8) == 1
+
+
+def test_splits_of_exact_products_count_the_workgroups_of_the_fullest_xcd():
+    """us, in the parts that rounds of 256 (512) workgroups gave / in those given here."""
+    fn = _rule("_ZN5chadq17gemm_exact_splitsEiii")
+    fn.argtypes = [ctypes.c_int] * 3
+    assert fn(552, 1280, 5120) != 5   # 35 tiles: 25 workgroups in 5 parts on each XCD that has 5 tiles, 15 more than the others; 32.1 / 20.7 in 4
+    assert fn(265, 1344, 7168) != 7   # 31.6 / 20.5 in 6
+    assert fn(266, 3520, 3072) != 3   # 31.6 / 22.0 in 2
+    assert fn(22, 4480, 1024) == 2    # 4: 6.4 / 4.9
+    assert fn(55, 128, 256) == 1 and fn(152, 384, 22016) == 8 and fn(4096, 2048, 2048) == 1
+
+
+@pytest.mark.parametrize("d,hq,dh,ffn", [(2048, 8, 256, 16384), (256, 16, 128, 256), (1280, 4, 128, 6400), (512, 1, 256, 768)])
+def test_prompt_workspace_covers_shorter_chunks(d, hq, dh, ffn):
+    """A workspace for T tokens serves fewer as well, the last layer's single row among them, in however many parts they are summed."""
+    lib = _lib.load()
+    splits = _rule("_ZN5chadq17gemm_exact_splitsEiii")
+    splits.argtypes = [ctypes.c_int] * 3
+    size = [lib.chadq_prompt_i4g32_workspace_bytes(t, d, hq, dh, ffn) for t in range(1, 400)]
+    assert size == sorted(size)
+    most = 0
+    for t in range(1, 400):
+        parts = [splits(t, n, k) * t * n for n, k in (((hq + 2) * dh, d), (d, hq * dh), (d, ffn))] + [splits(1, n, k) * n for n, k in ((d, hq * dh), (d, ffn))]
+        most = max(most, *parts)
+        rest = t * (4 * d + 4 * hq * dh + 2 * max(d, hq * dh) + 2 * ffn)
+        assert size[t - 1] >= 4 * most + rest

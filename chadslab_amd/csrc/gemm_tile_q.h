@@ -19,6 +19,8 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
 // int4 weights taken exactly (nothing rounded before the fp32 sums); K % 256 == 0, x, wp and sc 16-byte aligned unless it says otherwise
 constexpr int kExactMaxSplits = 8;
 int gemm_exact_splits(int M, int N, int K);  // K splits to use for gemm_exact_f32_launch
+// rows of the tile that the two launches below take for `parts` K splits of `per` 256-k blocks; *us: what the launch takes
+int gemm_exact_tile(int M, int N, int per, int parts, bool geglu, float *us);
 // y_parts fp32 [ksplit][M,N]
 int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
                           hipStream_t st);

@@ -882,7 +882,7 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
 }
 
 // ---- exact weights, K % 256 == 0: the projections of a prompt, whose tokens must come out as the decode step's do.
-// Tiles of 128 or 256 rows x 128 weight rows, or of 32 or 64 x 64: with few rows a workgroup waits for its weights, and what counts is
+// Tiles of 128 or 256 rows x 128 weight rows, or of 32 or 64 x 64: in few tiles a workgroup waits for its weights, and what counts is
 // how many workgroups and steps wait at once (two workgroups per compute unit for at most 32 rows; the loop is not unrolled: the
 // code of a few steps is fetched as often as it is run).  Whole prompts in us, 128 weight rows for every number of tokens in brackets:
 // 24 tokens through 18 layers of 2048 x 16384 1152 (1343), 9 through 6 of 1280 x 3840 262 (321), 37 through 4 of 2048 x 8960 282 (311).
@@ -891,13 +891,15 @@ struct ExactCost {
     float s, c0, c1, d0, d1, b, c2;
 };
 static const ExactCost kExact32 = {32, 64, 4.87f, -1.63f, .694f, 1.42f, .694f, .870f, .216f}, kExact64 = {64, 64, 2.75f, 1.42f, .779f, 1.42f, .779f, .904f, .284f},
-                       kExact128 = {128, 128, 3.84f, 1.29f, 2.55f, 1.29f, 2.55f, .950f, .184f};
+                       kExact128 = {128, 128, 3.84f, 1.29f, 2.55f, 1.29f, 2.55f, .950f, .184f}, kGeglu64 = {64, 64, 1.88f, 2.55f, .891f, 2.55f, .891f, .856f, 0.f},
+                       kGeglu128 = {128, 128, 1.58f, 4.65f, 2.76f, 4.65f, 2.76f, .884f, 0.f}, kGeglu256 = {256, 128, 1.54f, 7.74f, 3.58f, 7.74f, 3.58f, .847f, 0.f};
 
 // us that a launch takes in `parts` K splits of `per` 256-k blocks.  Tiles go to the XCDs in turn, each in all its splits, and a round is over
 // when the fullest XCD has dealt its workgroups to its 32 compute units: 33 tiles in 7 parts are 231 workgroups, but 35 on one XCD.  A tile
 // takes c0 + c1 * per in the first round and d0 + d1 * per in a further one (of the tiles of 32 rows two fit on a compute unit), the last
 // round b + (1 - b) f of it if it is full to f; s is what a launch takes besides, c2 what a MB of fp32 parts takes to be written.  Fitted to 3900
-// random products in every number of splits (2 to 700 rows, 128 to 8192 weight rows, 256 to 24000 k): 4 % standard deviation.
+// random products in every number of splits (2 to 700 rows, 128 to 8192 weight rows, 256 to 24000 k) and 2300 gated ones: 2 to 4 % standard
+// deviation.
 static float exact_us(const ExactCost &t, int M, int N, int per, int parts) {
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), fullest = (tiles + 7) / 8 * parts, rounds = (fullest + 31) / 32;
     const float last = t.b + (1.f - t.b) * (float)(fullest - (rounds - 1) * 32) / 32.f, first = t.c0 + t.c1 * (float)per;
@@ -905,21 +907,34 @@ static float exact_us(const ExactCost &t, int M, int N, int per, int parts) {
     return t.s + (rounds == 1 ? last * first : first + ((float)(rounds - 2) + last) * (t.d0 + t.d1 * (float)per)) + t.c2 * mb;
 }
 
-static float exact_f32_us(int M, int N, int per, int parts) {
-    return exact_us(M <= 32 ? kExact32 : M <= 64 ? kExact64 : kExact128, M, N, per, parts);
+// The tile (its rows) that takes a product in the shortest time.  64 rows reach the chip's compute units where 128 leave most of them idle, and
+// take a third of the time per k; 256 dequantise a weight half as often.  us, 64 / 128 rows: 101 x 128 x 2048 in eight parts 4.7 / 7.6, 158 x 5120 x
+// 2304 in one 12.1 / 27.9, 432 x 5120 x 1536 24.4 / 21.8; gate/up, 64 / 128 / 256 rows: 101 x 8192 x 2048 11.7 / 25.9 / 32.7, 237 x 32512 x 1792 71.6 /
+// 49.7 / 38.3.  (In few steps the loop of 128 rows also takes 0.6 us more than the one with all requests of a step in a row did.)  A prompt of
+// 256 tokens through 18 layers of 2048 x 16384 2518 -> 2320.
+int gemm_exact_tile(int M, int N, int per, int parts, bool geglu, float *us) {
+    if (M <= 32) return *us = exact_us(kExact32, M, N, per, parts), 32;
+    const ExactCost *const t[3] = {geglu ? &kGeglu64 : &kExact64, geglu ? &kGeglu128 : &kExact128, &kGeglu256};
+    int best = 0;
+    *us = exact_us(*t[0], M, N, per, parts);
+    for (int i = 1; i < (M <= 64 ? 1 : geglu ? 3 : 2); ++i) {
+        const float u = exact_us(*t[i], M, N, per, parts);
+        if (u < *us) {
+            best = i;
+            *us = u;
+        }
+    }
+    return t[best]->bm;
 }
 
 template <int EPI>
 static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st) {
-    if (M <= 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
-    if (M <= 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    float us;
+    const int rows = gemm_exact_tile(M, N, (K / 256 + ksplit - 1) / ksplit, ksplit, EPI == tileq::EPI_GEGLU, &us);
+    if (rows == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    if (rows == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
     if constexpr (EPI == tileq::EPI_GEGLU) {
-        // 256 rows dequantise a weight half as often: a full round takes 45 us per 2048 k, one of 128-row tiles 30
-        auto rounds = [&](int bm) {
-            const int tiles = ((M + bm - 1) / bm) * ((N + 127) / 128), full = (tiles - 1) / 256;
-            return (float)full + 0.65f + 0.35f / 256.f * (float)(tiles - full * 256);
-        };
-        if (rounds(256) * 45.f < rounds(128) * 30.f) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+        if (rows == 256) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
     }
     return tileq::launch<true, 1, 4, 2, 4, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
 }
@@ -944,7 +959,9 @@ int gemm_exact_splits(int M, int N, int K) {
     float best_us = 0.f;
     for (int s = 1; s <= kExactMaxSplits; ++s) {
         const int per = (blocks + s - 1) / s, parts = (blocks + per - 1) / per;
-        const float us = exact_f32_us(M, N, per, parts) + kRead * 4e-6f * (float)rows * (float)N * (float)parts;
+        float us;
+        gemm_exact_tile(M, N, per, parts, false, &us);
+        us += kRead * 4e-6f * (float)rows * (float)N * (float)parts;
         if (s == 1 || us < best_us) {
             best = parts;
             best_us = us;

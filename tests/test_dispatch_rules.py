@@ -114,3 +114,19 @@ def test_prompt_workspace_covers_shorter_chunks(d, hq, dh, ffn):
         most = max(most, *parts)
         rest = t * (4 * d + 4 * hq * dh + 2 * max(d, hq * dh) + 2 * ffn)
         assert size[t - 1] >= 4 * most + rest
+
+
+def test_exact_products_take_the_tile_that_reaches_the_compute_units():
+    """us in tiles of 64 / 128 (/ 256) rows."""
+    fn = _rule("_ZN5chadq15gemm_exact_tileEiiiibPf")
+    fn.argtypes = [ctypes.c_int] * 4 + [ctypes.c_bool, ctypes.POINTER(ctypes.c_float)]
+
+    def rows(m, n, per, parts, gated):
+        return fn(m, n, per, parts, gated, ctypes.byref(ctypes.c_float()))
+
+    assert rows(101, 128, 1, 8, False) == 64      # 4.7 / 7.6
+    assert rows(158, 5120, 9, 1, False) == 64     # 12.1 / 27.9
+    assert rows(432, 5120, 6, 1, False) == 128    # 24.4 / 21.8
+    assert rows(101, 8192, 8, 1, True) == 64      # 11.7 / 25.9 / 32.7
+    assert rows(256, 32768, 8, 1, True) == 256
+    assert rows(64, 32768, 8, 1, True) == 64 and rows(32, 32768, 8, 1, True) == 32 and rows(9, 64, 1, 1, False) == 32

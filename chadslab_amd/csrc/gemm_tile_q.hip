@@ -948,12 +948,13 @@ int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint1
 }
 
 // The K splits of a product, whole 256-k blocks each, the last one possibly shorter.  (With equal parts only, a down projection of 8960 k had
-// one part, 63 us of the 125 that its layer took for 37 tokens.)  kRead: us that the next kernel takes for a MB of parts.  Rounds of 256
-// workgroups (512 for up to 32 rows) times the k of each, as the splits were chosen by before, miss how tiles fall to the XCDs, what half a
-// chip costs and what the parts cost.  us, so chosen / now: 265 x 1344 x 7168 in 7 parts 31.6 / in 6 20.5, 552 x 1280 x 5120 in 5 32.1 / in 4 20.7,
-// 22 x 4480 x 1024 in 4 6.4 / in 2 4.9.  M counts in whole tiles only: prompt_layout asks for every number of them.
+// one part, 63 us of the 125 that its layer took for 37 tokens.)  Rounds of 256 workgroups (512 for up to 32 rows) times the k of each, as the
+// splits were chosen by before, miss how tiles fall to the XCDs, what half a chip costs and what the parts cost.  us, so chosen / in other
+// parts of the same tiles: 265 x 1344 x 7168 in 7 31.6 / in 6 20.5, 552 x 1280 x 5120 in 5 32.1 / in 4 20.7, 22 x 4480 x 1024 in 4 6.4 / in 2
+// 4.9.  kRead: what a MB of parts costs the next kernel.  256 tokens through 18 layers of 2048 x 16384, us, with 0 / 0.2 / 0.4 us per MB 2188 / 2166 /
+// 2181, through 12 of 1536 x 12288 1180 / 1158 / 1163.  M counts in whole tiles only: prompt_layout asks for every number of them.
 int gemm_exact_splits(int M, int N, int K) {
-    constexpr float kRead = .4f;
+    constexpr float kRead = .2f;
     const int blocks = K / 256, rows = M <= 32 ? 32 : (M + 63) / 64 * 64;
     int best = 1;
     float best_us = 0.f;

@@ -11,8 +11,19 @@
 //     (which the caches serve).  Three waves per SIMD with one block ahead measured 4-8 % faster than two with two ahead.
 //   * Where an expert's rows of x or h fit into LDS and a workgroup has items enough (few_launch), they are put there once per
 //     expert and K split, already in operand order, a workgroup's items are neighbours instead of a grid apart, and two blocks
-//     of weights are on their way: 32 of a block's 56 registers held activations, read again for every item.  4 tokens, 8 experts
-//     of 4096 x 14336: gate/up 87 -> 77 us, down 50 -> 49; four blocks in flight are no faster than three.
+//     of weights are on their way: a block's activations are 32 registers to its weights' 24, read again for every item.  4 tokens, 8
+//     experts of 4096 x 14336: gate/up 87 -> 77 us, down 50 -> 49; four blocks in flight are no faster than three.
+//   * Otherwise the registers of the activations are single: a piece is requested again for the next block as soon as its MFMAs have
+//     been issued (the caches are nearer than the memory the weights come from).
+//   * At most four tokens (FEW): the 16 rows of the A operand are four tokens of four scale groups, each lane group's row non-zero only
+//     where it meets that group's words, so the weights are used in the registers they arrived in (no exchange between lanes), the
+//     sums of four groups come out in one register each and one FMA per four groups and row is left of four: 188 vector instructions per
+//     4 KiB instead of 275.  The whole call, us, before in brackets: 4 tokens, 8 experts of 4096 x 14336 119 (134), with `stream` as
+//     below; 2 tokens 86 (98); 3 of 16 of 2304 x 12032 69 (78), 3 of 4 of 3328 x 2816 25.6 (27.5).  What is left at 4 tokens is the stream:
+//     with the arithmetic taken out the call takes 108.
+//   * `stream`: weights are requested non-temporal where all experts together do not fit into the 256 MB memory-side cache by far.  Row order,
+//     us, 4 tokens of 8 experts with / without: 4096 x 14336 (793 MB) 117 / 125, 4096 x 8192 (453 MB) 85.1 / 88.2, 2048 x 14336 (396 MB) 70.9 /
+//     70.1, 3072 x 7168 (297 MB) 59.4 / 57.8, 1024 x 2048 19.8 / 19.0: the line is at 400 MB.
 //   * In row order a load takes whole 128-byte lines of 8 rows, not 64 bytes of 16 (gate/up 97 -> 87 us); two DPP moves
 //     per register pair put the halves in place.
 // Gate/up | down in us, 8 experts of 4096 x 14336, top 2, the skinny kernel in brackets: 4 tokens 87 | 50 (130 | 72),
@@ -20,7 +31,9 @@
 // down product is slower here; the whole call is the quicker one all the same, 84.6 against 88.5); 1 token of 1024 x 2048
 // 5.2 | 4.5 (12.8 | 7.0).
 // Arithmetic: v_mfma_f32_16x16x32_bf16 on unscaled weights.  A lane holds a whole scale group of its weight row (16
-// bytes); the lanes' words are exchanged (v_permlane16_swap, v_permlane32_swap) so that one MFMA holds one scale group;
+// bytes); the lanes' words are exchanged (v_permlane16_swap, v_permlane32_swap) so that one MFMA holds one scale group (FEW: four MFMAs
+// take the four words of a lane in turn; one MFMA adds its lane groups' eight products in that order too, so both forms have the same bits,
+// and both keep a sum per scale group modulo 4 and add those at the end of an item);
 // nibbles become the bf16 value u / 2^9 (unpack8_fp8), another MFMA of the same activations with the constant -8 / 2^9 takes
 // the 8 off beforehand for both of the item's row blocks, one fp32 FMA per value applies the scale and the finished sum is
 // multiplied by 2^9: weights are exact.  32 x 15 < 2^9, so every group's sum is finite for all finite activations, and it
@@ -60,11 +73,12 @@ __device__ __forceinline__ void order_x8(const uint32_t a[4], uint32_t o[4]) {
     o[3] = __builtin_amdgcn_perm(a[3], a[2], 0x07060302u);
 }
 
-// XL: activations through LDS (at most kXlBytes of them), two blocks of weights on their way beside the one being summed
-template <int MODE, bool TILED, bool XL>
+// XL: activations through LDS (at most kXlBytes of them), two blocks of weights on their way beside the one being summed.  FEW: no expert
+// has more than four rows.  stream: weights are not kept in the caches (tile order: never).
+template <int MODE, bool TILED, bool XL, bool FEW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void moe_few_i4g32_kernel(
     const GemmGroup *__restrict__ groups, const int32_t *__restrict__ tiles, const int32_t *__restrict__ tok, int ntiles, int E, int N,
-    int K, int nsplit, size_t split_stride) {
+    int K, int nsplit, int stream, size_t split_stride) {
     struct Entry {
         const void *w[2], *s[2], *x;
         void *y;
@@ -113,11 +127,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     };
 
     struct Block {  // 256 k = eight scale groups
-        u32x4 x[XL ? 1 : 8], w[RB][2], s[RB];
+        u32x4 w[RB][2], s[RB];
     };
+    // The activations of the block being summed (FEW), or of half of it; a place is refilled as soon as it has been used.
+    u32x4 xq[XL ? 1 : FEW ? 8 : 4];
     // ---- the request side
     int l_item = begin, l_i = 0, l_n = 0, l_kb = 0, l_end = 0;
-    __amdgpu_buffer_rsrc_t wr[RB], sr[RB], xr;
+    __amdgpu_buffer_rsrc_t wr[RB], sr[RB], xr, x_rsrc;
+    __amdgpu_buffer_rsrc_t x_rsrc0;
+    uint32_t x_voff = kBeyond, x_kb = 0, x_voff0 = kBeyond, x_kb0 = 0;  // where the activations of the last block requested and of the one before it are
     uint32_t woff = 0, soff = 0, xoff = 0;  // of the lane, in the first row block
     // the second row block: the same rows of the up matrix, or the next 16 rows
     const uint32_t wblk = MODE == 1 ? 0u : TILED ? 256u : 8u * K, sblk = MODE == 1 ? 0u : TILED ? 128u : (uint32_t)K;
@@ -133,7 +151,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         l_n = blocks_of(l_item);
         l_i = 0;
         xr = __builtin_amdgcn_make_buffer_rsrc(uniform(s_ent[en].x), 0, kRange, 0x00020000);
-        xoff = s_xoff[en][r] + 16u * j;
+        xoff = FEW ? (r >> 2) == j ? s_xoff[en][r & 3] + 64u * j : kBeyond : s_xoff[en][r] + 16u * j;
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             wr[b] = __builtin_amdgcn_make_buffer_rsrc(uniform(s_ent[en].w[b]), 0, kRange, 0x00020000);
@@ -149,30 +167,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         }
     };
     auto request = [&](Block &q) {
-        if (l_item >= total) return;
+        x_rsrc0 = x_rsrc;
+        x_voff0 = x_voff;
+        x_kb0 = x_kb;
+        if (l_item >= total) {
+            x_voff = kBeyond;
+            return;
+        }
         const uint32_t kb = l_kb, beyond = l_kb < l_end ? 0u : kBeyond, wv = woff | beyond, sv = soff | beyond, xv = xoff | beyond;
 #pragma unroll
         for (int b = 0; b < RB; ++b) {
             if (TILED) {
                 const uint32_t sk = kb * 512u + b * sblk;
-                const u32x2 ev = __builtin_amdgcn_raw_buffer_load_b64(sr[b], sv, sk, 0), od = __builtin_amdgcn_raw_buffer_load_b64(sr[b], sv + 256u, sk, 0);
+                const u32x2 ev = __builtin_amdgcn_raw_buffer_load_b64(sr[b], sv, sk, 0), od = __builtin_amdgcn_raw_buffer_load_b64(sr[b], sv, sk + 256u, 0);
                 q.s[b] = u32x4{ev.x, ev.y, od.x, od.y};
             } else {
                 q.s[b] = __builtin_amdgcn_raw_buffer_load_b128(sr[b], sv, kb * 16u + b * sblk, 0);
             }
 #pragma unroll
-            for (int h = 0; h < 2; ++h)  // tile order: non-temporal (5 % faster at 4 tokens; in row order the same)
-                q.w[b][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[b], wv, kb * (TILED ? 4096u : 128u) + b * wblk + h * (TILED ? 2048u : 4u * K), TILED ? 2 : 0);
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t at = kb * (TILED ? 4096u : 128u) + b * wblk + h * (TILED ? 2048u : 4u * K);
+                if (TILED || stream) q.w[b][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[b], wv, at, 2);
+                else q.w[b][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[b], wv, at, 0);
+            }
         }
         if constexpr (!XL) {
-#pragma unroll
-            for (int g = 0; g < 8; ++g) q.x[g] = __builtin_amdgcn_raw_buffer_load_b128(xr, xv + 64u * g, kb * 512u, 0);
+            x_rsrc = xr;
+            x_voff = xv;
+            x_kb = kb;
         }
         l_kb += 4;
         if (++l_i == l_n) {
             l_item += stride;
             if (l_item < total) open();
         }
+    };
+
+    auto request_x = [&](int g, bool last) {  // piece g of the last block requested, or of the one before it
+        const uint32_t at = FEW ? 256u * (g >> 2) + 16u * (g & 3) : 64u * g;
+        xq[FEW ? g : g & 3] = last ? __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, x_voff, x_kb * 512u + at, 0)
+                                   : __builtin_amdgcn_raw_buffer_load_b128(x_rsrc0, x_voff0, x_kb0 * 512u + at, 0);
     };
 
     bf16x8 bias;
@@ -182,14 +216,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
     // ---- the summing side
     int c_item = begin, c_i = 0, c_n = 0, par = 0;
-    f32x4 acc[RB];
+    constexpr int NC = FEW ? 1 : 4;
+    f32x4 acc[RB][NC];  // [row block][scale group modulo 4]; at most four rows: [row block][0], the lane's groups
 #pragma unroll
-    for (int b = 0; b < RB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int t = 0; t < NC; ++t) acc[b][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto finish = [&]() {
 #pragma unroll
         for (int b = 0; b < RB; ++b) {
-            s_red[par][wave][b][lane] = acc[b];
-            acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            f32x4 v;
+            if constexpr (FEW) {  // the four lane groups' sums meet, (0 + 1) + (2 + 3) as below
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t a = __float_as_uint(acc[b][0][e]);
+                    const u32x2 h = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+                    const uint32_t c = __float_as_uint(__uint_as_float(h.x) + __uint_as_float(h.y));
+                    const u32x2 q = __builtin_amdgcn_permlane32_swap(c, c, false, false);
+                    v[e] = __uint_as_float(q.x) + __uint_as_float(q.y);
+                }
+            } else {
+                v = (acc[b][0] + acc[b][1 % NC]) + (acc[b][2 % NC] + acc[b][3 % NC]);
+            }
+            s_red[par][wave][b][lane] = v;
+#pragma unroll
+            for (int t = 0; t < NC; ++t) acc[b][t] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
         // the bare barrier instruction: __syncthreads() would also wait for every load in flight.  Two buffers: the next
         // item's sums go to the other one, and nobody writes to this one again before the barrier of that item.
@@ -241,8 +292,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             *reinterpret_cast<u32x4 *>(s_x + 512 + m * pitch + c * 16) = u32x4{o[0], o[1], o[2], o[3]};
         }
         if (tid < 32) *reinterpret_cast<u32x4 *>(s_x + tid * 16) = u32x4{0, 0, 0, 0};
-        x_base = (r < rows ? 512u + r * pitch : 0u) + 16u * j;
-        x_mask = r < rows ? ~0u : 0u;
+        const bool mine = FEW ? (r >> 2) == j && (r & 3) < rows : r < rows;
+        x_base = FEW ? (mine ? 512u + (r & 3) * pitch + 64u * j : 0u) : (mine ? 512u + r * pitch : 0u) + 16u * j;
+        x_mask = mine ? ~0u : 0u;
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
@@ -265,6 +317,52 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
                     q.w[b][1][e] = (uint32_t)__builtin_amdgcn_update_dpp(hi, lo, 0x128, 0xF, 0x3, false);  // ... into lanes 0..7
                 }
         }
+        auto operand = [&](int g, int at) {  // piece g of the block's activations (`at`: its place in LDS)
+            bf16x8 av;
+            if constexpr (XL) {
+                av = *reinterpret_cast<const bf16x8 *>(s_x + xa + at);
+            } else {
+                const u32x4 v = xq[FEW ? g : g & 3];
+                const uint32_t a[4] = {v.x, v.y, v.z, v.w};
+                uint32_t o[4];
+                order_x8(a, o);
+                __builtin_memcpy(&av, o, 16);
+            }
+            return av;
+        };
+        if constexpr (FEW) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                bf16x8 av[4];
+                f32x4 d[RB] = {};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    av[e] = operand(4 * h + e, 256 * h + 16 * e);
+                    d[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[e], bias, d[0], 0, 0, 0);
+                }
+#pragma unroll
+                for (int b = 1; b < RB; ++b) d[b] = d[0];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int b = 0; b < RB; ++b) {
+                        uint32_t p[4];
+                        unpack8_fp8(q.w[b][h][e], p);
+                        bf16x8 bv;
+                        __builtin_memcpy(&bv, p, 16);
+                        d[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[e], bv, d[b], 0, 0, 0);
+                    }
+#pragma unroll
+                for (int b = 0; b < RB; ++b) {  // the lane's group: 4h + j
+                    const u32x4 s = q.s[b];
+                    const uint32_t sw = TILED ? (j & 1 ? s[2 + h] : s[h]) : (j & 2 ? s[2 * h + 1] : s[2 * h]);
+                    acc[b][0] += d[b] * f16_bits_to_f32((uint16_t)(sw >> ((TILED ? j >> 1 : j & 1) * 16)));
+                }
+                if constexpr (!XL)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) request_x(4 * h + e, true);
+            }
+        } else {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             uint32_t word[RB][4];  // [row block][group]
@@ -282,16 +380,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             }
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                bf16x8 av;
-                if constexpr (XL) {
-                    av = *reinterpret_cast<const bf16x8 *>(s_x + xa + 64 * (4 * h + t));
-                } else {
-                    const u32x4 xv = q.x[4 * h + t];
-                    const uint32_t a[4] = {xv.x, xv.y, xv.z, xv.w};
-                    uint32_t o[4];
-                    order_x8(a, o);
-                    __builtin_memcpy(&av, o, 16);
-                }
+                const bf16x8 av = operand(4 * h + t, 64 * (4 * h + t));
+                if constexpr (!XL) request_x(4 * (h ^ 1) + t, h == 1);
                 const f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bias, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
                 for (int b = 0; b < RB; ++b) {
@@ -301,9 +391,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
                     __builtin_memcpy(&bv, p, 16);
                     const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, d0, 0, 0, 0);
                     const uint32_t sw = q.s[b][TILED ? 2 * (t & 1) + h : 2 * h + (t >> 1)];  // group 4h + t
-                    acc[b] += d * f16_bits_to_f32((uint16_t)((TILED ? t >> 1 : t & 1) ? sw >> 16 : sw & 0xFFFFu));
+                    acc[b][t] += d * f16_bits_to_f32((uint16_t)((TILED ? t >> 1 : t & 1) ? sw >> 16 : sw & 0xFFFFu));
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);  // (else the halves' words are all in registers at once, more than there are)
+        }
         }
         if (++c_i == c_n) {
             finish();
@@ -332,6 +424,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     } else {
         Block q0, q1;
         request(q0);
+#pragma unroll
+        for (int g = 0; g < (FEW ? 8 : 4); ++g) request_x(g, true);
         for (;;) {
             request(q1);
             if (!consume(q0)) break;
@@ -385,12 +479,19 @@ static int few_launch(const GemmGroup *groups, const int32_t *tiles, const int32
     const int64_t most = (int64_t)ntiles * per;
     const int span = (K / 256 + nsplit - 1) / nsplit, x_bytes = few_x_bytes(T, span);
     const dim3 grid(most < 768 ? (int)most : 768);
-    if (moe_few_through_lds(T, E, top_k, per, span))
-        hipLaunchKernelGGL((moe_few_i4g32_kernel<MODE, TILED, true>), grid, dim3(256), x_bytes, st, groups, tiles, tok, ntiles, E, N, K, nsplit,
-                           split_stride);
-    else
-        hipLaunchKernelGGL((moe_few_i4g32_kernel<MODE, TILED, false>), grid, dim3(256), 0, st, groups, tiles, tok, ntiles, E, N, K, nsplit,
-                           split_stride);
+    const int stream = (int64_t)E * N * K * 27 / 16 > (int64_t)400 << 20;  // all experts' bytes
+    const bool lds = moe_few_through_lds(T, E, top_k, per, span);
+#define CHADQ_FEW(XL, FEW)                                                                                                                        \
+    hipLaunchKernelGGL((moe_few_i4g32_kernel<MODE, TILED, XL, FEW>), grid, dim3(256), XL ? x_bytes : 0, st, groups, tiles, tok, ntiles, E, N, K, \
+                       nsplit, stream, split_stride)
+    if (T <= 4) {
+        if (lds) CHADQ_FEW(true, true);
+        else CHADQ_FEW(false, true);
+    } else {
+        if (lds) CHADQ_FEW(true, false);
+        else CHADQ_FEW(false, false);
+    }
+#undef CHADQ_FEW
     return hip_check(hipGetLastError(), "moe_few launch");
 }
 

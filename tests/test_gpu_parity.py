@@ -1134,6 +1134,32 @@ def test_moe_ffn_few_tokens_many_items_are_summed_as_one_by_one(ops, t, h, f, e,
         assert differ == 0
 
 
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("t,h,f,e,top_k", [(2, 256, 256, 1, 1), (4, 256, 512, 2, 2), (4, 1280, 2304, 3, 2), (5, 256, 256, 1, 1), (5, 2560, 1280, 2, 1), (8, 512, 4352, 2, 2),
+                                           (13, 1024, 768, 1, 1), (16, 768, 2816, 2, 2)])
+def test_moe_ffn_up_to_four_tokens_and_more_have_the_bits_of_one(ops, t, h, f, e, top_k, tiled):
+    """At most four tokens are summed with four scale groups side by side, more with one group after the other: the same order of additions,
+    so a token's bits do not depend on how many came with it."""
+    from chadslab_amd import QWeightInt4G32
+
+    g = torch.Generator(device=DEV)
+    g.manual_seed(9600 + t + h)
+
+    def matrix(n, k):
+        w = QWeightInt4G32(torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g),
+                           torch.exp(torch.randn(n, k // 32, device=DEV, generator=g) * 0.5 - 5.0).half())
+        return ops.to_tiles(w) if tiled else w
+
+    experts = [(matrix(f, h), matrix(f, h), matrix(h, f)) for _ in range(e)]
+    x = torch.randn(t, h, device=DEV, generator=g).bfloat16()
+    z = torch.randn(t, e, device=DEV, generator=g)
+    y = ops.moe_ffn(x, z, experts, top_k=top_k)
+    assert bool(torch.isfinite(y).all()) and bool(y.any())
+    for i in range(t):
+        one = ops.moe_ffn(x[i:i + 1], z[i:i + 1], experts, top_k=top_k)
+        assert torch.equal(one[0].view(torch.int16), y[i].view(torch.int16)), i
+
+
 @pytest.mark.parametrize("t,h,f,e,top_k", [(16, 256, 512, 5, 4), (13, 256, 512, 7, 5), (16, 512, 256, 16, 8), (16, 256, 256, 1, 1), (8, 512, 512, 16, 8),
                                            (1, 256, 256, 16, 8)])
 def test_moe_ffn_few_tokens_routed_by_one_wave(ops, t, h, f, e, top_k):

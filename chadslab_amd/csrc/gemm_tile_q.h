@@ -17,6 +17,9 @@ GemmTile gemm_tile_pick(int M, int N, int K, bool int4, bool guard);
 int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st);
 int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st);
 // int4 weights taken exactly (nothing rounded before the fp32 sums); K % 256 == 0, x, wp and sc 16-byte aligned unless it says otherwise
+// The two products below take activations that carry this factor (exact but for magnitudes below 2^-121), and the second one's result
+// carries it too: their operands are (u - 8) / 2^4, and with it no group's sum overflows while the activations are finite (32 x 8 < 2^9).
+constexpr float kExactX = 0x1p-5f;
 constexpr int kExactMaxSplits = 8;
 int gemm_exact_splits(int M, int N, int K);  // K splits to use for gemm_exact_f32_launch
 // rows of the tile that the two launches below take for `parts` K splits of `per` 256-k blocks; *us: what the launch takes
@@ -27,7 +30,7 @@ int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *
 // y [M,N] fp32 or bf16, at most 32 rows, any K % 32 == 0 with gemm_tile_q_ok(K), any alignment of the scales
 int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, bool bf16_out,
                                hipStream_t st);
-// weight rows in (gate, up) pairs: h[m,i] = bf16(gelu_tanh(y[m,2i]) * y[m,2i+1]), [M, N/2]
+// weight rows in (gate, up) pairs: h[m,i] = bf16(gelu_tanh(y[m,2i]) * y[m,2i+1]) * kExactX, [M, N/2]
 int gemm_exact_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st);
 
 }  // namespace chadq

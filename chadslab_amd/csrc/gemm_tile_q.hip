@@ -8,7 +8,7 @@
 //   256, 192 x 128   WM = WN = WK = 2, MB = 4 or 3, NB = 2
 //   128 x 128        int4: WN = 4, WK = 2, MB = 4; int8: WN = 2, WK = 4, MB = 4, NB = 2.   96 x 128: the latter with MB = 3
 //   128, 96 x 64     WN = 2, WK = 4, MB = 4 or 3, 32 k per wave and step.   64, 32 x 64: MB = 2 or 1, 64 k
-//   exact weights    256, 128 x 128: WN = 4, WK = 2, MB = 8 or 4.  64, 32 x 64: WN = 2, WK = 4; K possibly split over workgroups
+//   exact weights    256, 128 x 128: WN = 4, WK = 2, MB = 8 or 4.  128, 64, 32 x 64: WN = 2, WK = 4; K possibly split over workgroups
 //   SHORT            32, 64 x 64, 128 x 128 (WN = 4, WK = 2, MB = 4) and, int4, 256 x 256 with another loop, for few steps (short_k)
 //
 //   * A (activations): global -> LDS by DMA, ST stages of a step each, read back as fragments one or two slices (16 k)
@@ -43,11 +43,14 @@
 // one body for all of them with its conditions at run time (24 x 1024 x 1120 6.5 us, five bodies 5.8, SHORT 5.2), no unrolled loop, no
 // second request of the last step's weights (both nothing from two steps on).
 //
-// EXACT: no weight is rounded, for callers whose sums must be those of the decode step.  The operands are the integers (u - 8) / 2^9;
-// the scale of a group of 32 k is applied to its sum, one fp32 FMA per value.  That work, not the matrix cores, bounds it: 64 FMAs
-// and 2 x 19 instructions of unpacking per 32 k and 128 rows x 32 columns of a wave, 8 MFMAs beside them.  (The form before kept a
-// weight as the sum of two bf16 operands: twice the matrix work and 37 instructions per 8 weights.)  us, that form in brackets:
-// gate/up of a 2048 x 16384 layer, 256 tokens 45.5 (63.7; in 128-row tiles 61), down 30 (36.8).  Its sums are finite for all finite
+// EXACT: no weight is rounded, for callers whose sums must be those of the decode step.  The operands are integers, (u - 8) / 2^4 for
+// activations that carry 2^-5, (u - 8) / 2^9 for others; the scale of a group of 32 k is applied to its sum, one fp32 FMA per value.
+// Unpacking takes 14 instructions per 8 weights where the activations carry the factor (signed nibbles to fp32, the upper halves paired), 19
+// where not (by way of e4m3): gate/up of a 2048 x 16384 layer, 24 / 100 / 256 tokens 16.6 -> 15 / 30.2 -> 29 / 50.4 -> 43-46 us in a stream of that
+// product alone.  What bounds it is everything together, at the clock its power leaves (1.8 GHz): of 42 us at 256 tokens the FMAs taken out
+// leave 34, the LDS reads of the activations 33, their requests 37, the unpacking 42; reading three or four row blocks ahead, other
+// orders of a pair's instructions and waves of 128 x 64 (half the LDS reads, twice the unpacking: 48) give nothing.
+// (An earlier form kept a weight as the sum of two bf16 operands: twice the matrix work, 63.7 us.)  Its sums are finite for all finite
 // activations (32 x 8 < 2^9), and a weight of 0 is the operand 0: a large activation beside it leaves the other products their low bits.
 // The MFMA k-slot of a lane is free as long as A and B agree: slot group kq of slice t holds k = (KW / 2) kq + 8 t .. +7
 // (EXACT: 16 t + 8 kq .. +7).
@@ -139,9 +142,25 @@ __device__ __forceinline__ bf16x8 signed8_i4(uint32_t w) {
     return o;
 }
 
+// The same as (u - 8) / 2^4, for activations that carry the factor 2^-5: v_cvt_off_f32_i4 takes a signed nibble, u ^ 8, of any byte.  14
+// instructions.
+__device__ __forceinline__ bf16x8 signed8_i4_16th(uint32_t w) {
+    const uint32_t lo = w ^ 0x88888888u;
+    uint32_t hi = lo >> 4;
+    asm("" : "+v"(hi));  // (else the shift is merged with that of each byte, and no byte select of the conversion is left)
+    u32x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        r[e] = __builtin_amdgcn_perm(__float_as_uint(__builtin_amdgcn_cvt_off_f32_i4((hi >> (8 * e)) & 255u)),
+                                     __float_as_uint(__builtin_amdgcn_cvt_off_f32_i4((lo >> (8 * e)) & 255u)), 0x07060302u);
+    bf16x8 o;
+    __builtin_memcpy(&o, &r, 16);
+    return o;
+}
+
 // EPI (what becomes of the sums): EPI_BF16 y bf16 [M,N], times the row scale for int8; EPI_F32 y fp32 [gridDim.y][M,N],
 // part blockIdx.y holding the sum over its kspan k; EPI_GEGLU the weight rows come in pairs (gate, up) of a feature and
-// h = bf16(gelu_tanh(gate) * up) goes to y as bf16 [M, N/2].
+// h = bf16(gelu_tanh(gate) * up) goes to y as bf16 [M, N/2], times kExactX for the exact product that reads it.
 template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT, int EPI, bool SHORT>
 __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WM * WN * WK / 4, WM * WN * WK / 4))) void gemm_tile_q_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wq, const void *__restrict__ scv, void *__restrict__ yv, int M, int N,
@@ -306,9 +325,13 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     };
 
     if constexpr (EXACT) {
-    // Exact weights: integers (u - 8) / 2^9 as operands, two MFMAs from zero on per scale group and row block, and one fp32 FMA per
-    // value that applies the scale (times 2^9).  A pair of MFMAs runs beside the FMAs of the pair before it.
+    // Exact weights: integers as operands, two MFMAs from zero on per scale group and row block, and one fp32 FMA per
+    // value that applies the scale (times 2^9, what operands and activations leave out).  A pair of MFMAs runs beside the FMAs of the pair before it.
     constexpr int RING = Q >= 4 ? 4 : 2;
+    // The row block beside whose MFMAs the next group's words are taken over (a step of one group: when they have arrived) and the one, not
+    // before it, beside which the first half of their operands is made
+    constexpr int PREP = GR > 1 || MB <= 2 ? 0 : MB > 4 ? 2 : 1, HALF = MB <= 2 ? 0 : MB > 4 ? MB / 2 - 1 : GR > 1 ? 1 : 2;
+    static_assert(MB <= 4 || MB == 8, "the row blocks these are right for");
     uint32_t wv[GR][2], wnx[GR][2];  // the lane's packed words of a step [group][slice], of the next one
     uint32_t sraw[GR];               // its scales
     float sc2[GR], s_last = 0.f;     // ... as floats, that of the group whose sums are next
@@ -332,6 +355,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         }
     };
     bf16x8 bo[2], bnx[2];  // operands of the present group, of the next one
+    auto operand = [](uint32_t w) { return GUARD ? signed8_i4(w) : signed8_i4_16th(w); };
     bf16x8 af[RING][2];
     auto frag = [&](int q, const uint8_t *stage) {  // of pair q: group q / MB, row block q % MB
 #pragma unroll
@@ -351,8 +375,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         for (int r = 0; r < first(AFTER); ++r) request(r, ST - 1, lds, lds + (ST - 1) * C::STAGE, false);
     }
     prep(0);
-    bo[0] = signed8_i4(wv[0][0]);
-    bo[1] = signed8_i4(wv[0][1]);
+    bo[0] = operand(wv[0][0]);
+    bo[1] = operand(wv[0][1]);
     auto step = [&](int i, int slot, auto pending_c, auto before_c, auto more_c, auto whole_c) {
         constexpr bool whole = decltype(whole_c)::value, before = decltype(before_c)::value, more = decltype(more_c)::value;  // as below
         constexpr int pending = decltype(pending_c)::value;
@@ -388,9 +412,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             if (mb == 0) s_last = sc2[g];
             // the next group's operands, a share beside each pair
             if (g + 1 < GR || pending >= 0) {
-                if (g + 1 == GR && mb == (GR == 1 && MB > 2 ? 2 : 0)) prep(i + 1);
-                if (mb == MB / 2 - (MB > 1)) bnx[0] = signed8_i4(wv[(g + 1) % GR][0]);
-                if (mb == MB - 1) bnx[1] = signed8_i4(wv[(g + 1) % GR][1]);
+                if (g + 1 == GR && mb == PREP) prep(i + 1);
+                if (mb == HALF) bnx[0] = operand(wv[(g + 1) % GR][0]);
+                if (mb == MB - 1) bnx[1] = operand(wv[(g + 1) % GR][1]);
             }
             if (mb == MB - 1) {
                 bo[0] = bnx[0];
@@ -729,7 +753,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             // even lane: row r, columns (nl, nl+1) = (own a0, neighbour's a0); odd lane: row r+1, columns (nl-1, nl)
             if constexpr (GE)
                 *reinterpret_cast<uint16_t *>(lds + row * EP + (cb + nl) / 2 * 2) =
-                    (uint16_t)f32_to_bf16_bits(gelu_tanh_dev(odd ? recv : a0) * (odd ? a1 : recv));
+                    (uint16_t)pack_bf16_rne(gelu_tanh_dev(odd ? recv : a0) * (odd ? a1 : recv) * kExactX, 0.f);
             else
                 *reinterpret_cast<uint32_t *>(lds + row * EP + (cb + (nl & ~1)) * 2) = odd ? pack_bf16_rne(recv, a1) : pack_bf16_rne(a0, recv);
         }
@@ -882,7 +906,7 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
 }
 
 // ---- exact weights, K % 256 == 0: the projections of a prompt, whose tokens must come out as the decode step's do.
-// Tiles of 128 or 256 rows x 128 weight rows, or of 32 or 64 x 64: in few tiles a workgroup waits for its weights, and what counts is
+// Tiles of 128 or 256 rows x 128 weight rows, or of 32 to 128 x 64: in few tiles a workgroup waits for its weights, and what counts is
 // how many workgroups and steps wait at once (two workgroups per compute unit for at most 32 rows; the loop is not unrolled: the
 // code of a few steps is fetched as often as it is run).  Whole prompts in us, 128 weight rows for every number of tokens in brackets:
 // 24 tokens through 18 layers of 2048 x 16384 1152 (1343), 9 through 6 of 1280 x 3840 262 (321), 37 through 4 of 2048 x 8960 282 (311).
@@ -890,16 +914,18 @@ struct ExactCost {
     int bm, bn;  // tile
     float s, c0, c1, d0, d1, b, c2;
 };
-static const ExactCost kExact32 = {32, 64, 4.87f, -1.63f, .694f, 1.42f, .694f, .870f, .216f}, kExact64 = {64, 64, 2.75f, 1.42f, .779f, 1.42f, .779f, .904f, .284f},
-                       kExact128 = {128, 128, 3.84f, 1.29f, 2.55f, 1.29f, 2.55f, .950f, .184f}, kGeglu64 = {64, 64, 1.88f, 2.55f, .891f, 2.55f, .891f, .856f, 0.f},
-                       kGeglu128 = {128, 128, 1.58f, 4.65f, 2.76f, 4.65f, 2.76f, .884f, 0.f}, kGeglu256 = {256, 128, 1.54f, 7.74f, 3.58f, 7.74f, 3.58f, .847f, 0.f};
+static const ExactCost kExact32 = {32, 64, 4.87f, -1.63f, .694f, 1.42f, .694f, .870f, .216f};
+static const ExactCost kExact[3] = {{64, 64, 1.33f, 2.61f, .817f, 2.61f, .817f, .787f, .023f}, {128, 64, 1.66f, 3.52f, 1.144f, 3.52f, 1.144f, .784f, .043f},
+                                    {128, 128, 2.86f, 1.75f, 2.64f, 1.75f, 2.64f, .883f, .170f}};
+static const ExactCost kGeglu[4] = {{64, 64, 1.10f, 2.61f, .860f, 2.61f, .860f, .801f, 0.f}, {128, 64, 1.12f, 3.88f, 1.197f, 3.88f, 1.197f, .808f, 0.f},
+                                    {128, 128, .75f, 4.60f, 2.871f, 4.60f, 2.871f, .823f, 0.f}, {256, 128, .75f, 7.18f, 3.784f, 7.18f, 3.784f, .798f, 0.f}};
 
 // us that a launch takes in `parts` K splits of `per` 256-k blocks.  Tiles go to the XCDs in turn, each in all its splits, and a round is over
 // when the fullest XCD has dealt its workgroups to its 32 compute units: 33 tiles in 7 parts are 231 workgroups, but 35 on one XCD.  A tile
 // takes c0 + c1 * per in the first round and d0 + d1 * per in a further one (of the tiles of 32 rows two fit on a compute unit), the last
-// round b + (1 - b) f of it if it is full to f; s is what a launch takes besides, c2 what a MB of fp32 parts takes to be written.  Fitted to 3900
-// random products in every number of splits (2 to 700 rows, 128 to 8192 weight rows, 256 to 24000 k) and 2300 gated ones: 2 to 4 % standard
-// deviation.
+// round b + (1 - b) f of it if it is full to f; s is what a launch takes besides, c2 what a MB of fp32 parts takes to be written.  The
+// constants of 64 rows and more are fitted to 18700 random products in every number of splits (33 to 700 rows, 128 to 8192 weight rows, 256 to
+// 16000 k) and 8900 gated ones, 2 to 5 % standard deviation; the tile and splits they pick take 0.2 % more than the best of all on average.
 static float exact_us(const ExactCost &t, int M, int N, int per, int parts) {
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), fullest = (tiles + 7) / 8 * parts, rounds = (fullest + 31) / 32;
     const float last = t.b + (1.f - t.b) * (float)(fullest - (rounds - 1) * 32) / 32.f, first = t.c0 + t.c1 * (float)per;
@@ -910,32 +936,36 @@ static float exact_us(const ExactCost &t, int M, int N, int per, int parts) {
 // The tile (its rows) that takes a product in the shortest time.  64 rows reach the chip's compute units where 128 leave most of them idle, and
 // take a third of the time per k; 256 dequantise a weight half as often.  us, 64 / 128 rows: 101 x 128 x 2048 in eight parts 4.7 / 7.6, 158 x 5120 x
 // 2304 in one 12.1 / 27.9, 432 x 5120 x 1536 24.4 / 21.8; gate/up, 64 / 128 / 256 rows: 101 x 8192 x 2048 11.7 / 25.9 / 32.7, 237 x 32512 x 1792 71.6 /
-// 49.7 / 38.3.  (In few steps the loop of 128 rows also takes 0.6 us more than the one with all requests of a step in a row did.)  A prompt of
+// 49.7 / 38.3.  128 x 64 has the unpacking of 128 rows in as many workgroups as half the rows would make: 256 x 2048 x 16384 in four parts 27.2, in 64 x 64
+// tiles in two 31.5, in 128 x 128 in eight 30.0; without it the products of more than 64 rows would take 3 % longer on average, gated ones 4 %.
+// (Three stages; four are 2 % slower.)  (In few steps the loop of 128 rows also takes 0.6 us more than the one with all requests of a step in a row did.)  A prompt of
 // 256 tokens through 18 layers of 2048 x 16384 2518 -> 2320.
-int gemm_exact_tile(int M, int N, int per, int parts, bool geglu, float *us) {
-    if (M <= 32) return *us = exact_us(kExact32, M, N, per, parts), 32;
-    const ExactCost *const t[3] = {geglu ? &kGeglu64 : &kExact64, geglu ? &kGeglu128 : &kExact128, &kGeglu256};
+static const ExactCost &exact_pick(int M, int N, int per, int parts, bool geglu, float *us) {
+    const ExactCost *const t = M <= 32 ? &kExact32 : geglu ? kGeglu : kExact;
     int best = 0;
-    *us = exact_us(*t[0], M, N, per, parts);
-    for (int i = 1; i < (M <= 64 ? 1 : geglu ? 3 : 2); ++i) {
-        const float u = exact_us(*t[i], M, N, per, parts);
+    *us = exact_us(t[0], M, N, per, parts);
+    for (int i = 1; i < (M <= 64 ? 1 : geglu ? 4 : 3); ++i) {
+        const float u = exact_us(t[i], M, N, per, parts);
         if (u < *us) {
             best = i;
             *us = u;
         }
     }
-    return t[best]->bm;
+    return t[best];
 }
+
+int gemm_exact_tile(int M, int N, int per, int parts, bool geglu, float *us) { return exact_pick(M, N, per, parts, geglu, us).bm; }
 
 template <int EPI>
 static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st) {
     float us;
-    const int rows = gemm_exact_tile(M, N, (K / 256 + ksplit - 1) / ksplit, ksplit, EPI == tileq::EPI_GEGLU, &us);
-    if (rows == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
-    if (rows == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    const ExactCost &t = exact_pick(M, N, (K / 256 + ksplit - 1) / ksplit, ksplit, EPI == tileq::EPI_GEGLU, &us);
+    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
     if constexpr (EPI == tileq::EPI_GEGLU) {
-        if (rows == 256) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+        if (t.bm == 256) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
     }
+    if (t.bn == 64) return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
     return tileq::launch<true, 1, 4, 2, 4, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
 }
 
@@ -951,10 +981,10 @@ int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint1
 // one part, 63 us of the 125 that its layer took for 37 tokens.)  Rounds of 256 workgroups (512 for up to 32 rows) times the k of each, as the
 // splits were chosen by before, miss how tiles fall to the XCDs, what half a chip costs and what the parts cost.  us, so chosen / in other
 // parts of the same tiles: 265 x 1344 x 7168 in 7 31.6 / in 6 20.5, 552 x 1280 x 5120 in 5 32.1 / in 4 20.7, 22 x 4480 x 1024 in 4 6.4 / in 2
-// 4.9.  kRead: what a MB of parts costs the next kernel.  256 tokens through 18 layers of 2048 x 16384, us, with 0 / 0.2 / 0.4 us per MB 2188 / 2166 /
-// 2181, through 12 of 1536 x 12288 1180 / 1158 / 1163.  M counts in whole tiles only: prompt_layout asks for every number of them.
+// 4.9.  kRead: what a MB of parts costs the next kernel.  34 prompts, geometric mean against the earlier kernels, with 0.2 / 0.35 / 0.5 / 0.7 us per MB 1.011 /
+// 1.030 / 1.011 / 1.026.  M counts in whole tiles only: prompt_layout asks for every number of them.
 int gemm_exact_splits(int M, int N, int K) {
-    constexpr float kRead = .2f;
+    constexpr float kRead = .35f;
     const int blocks = K / 256, rows = M <= 32 ? 32 : (M + 63) / 64 * 64;
     int best = 1;
     float best_us = 0.f;

@@ -34,7 +34,7 @@ __global__ __launch_bounds__(256) void prompt_embed_kernel(const int32_t *__rest
 }
 
 // One row per workgroup: r = res + the np parts (part p of row t at parts + (p * rows + t) * d, added in order), kept in
-// res_out if there were any (may be res), then, if y, y = bf16(r / sqrt(mean(r^2) + eps) * w).  d % 4 == 0, d <= 2048.
+// res_out if there were any (may be res), then, if y, y = bf16(r / sqrt(mean(r^2) + eps) * w) * kExactX.  d % 4 == 0, d <= 2048.
 // NP: the number of parts, so that every load is in flight before the first sum (one memory round trip, not np of them).
 template <int NP>
 __global__ __launch_bounds__(256) void prompt_add_norm_kernel(const float *res, float *res_out, const float *__restrict__ parts,
@@ -68,12 +68,13 @@ __global__ __launch_bounds__(256) void prompt_add_norm_kernel(const float *res, 
     if ((tid & 63) == 63) s_ss[tid >> 6] = ss;
     __syncthreads();
     const float rinv = rsqrtf((s_ss[0] + s_ss[1] + s_ss[2] + s_ss[3]) / (float)d + eps);
+    auto bits = [](float v) { return f32_to_bf16_bits(v * kExactX); };
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int i = tid + 256 * j;
         if (i < nv) {
-            const uint32_t lo = f32_to_bf16_bits(r[j].x * rinv * wv[j].x) | (f32_to_bf16_bits(r[j].y * rinv * wv[j].y) << 16);
-            const uint32_t hi = f32_to_bf16_bits(r[j].z * rinv * wv[j].z) | (f32_to_bf16_bits(r[j].w * rinv * wv[j].w) << 16);
+            const uint32_t lo = bits(r[j].x * rinv * wv[j].x) | (bits(r[j].y * rinv * wv[j].y) << 16);
+            const uint32_t hi = bits(r[j].z * rinv * wv[j].z) | (bits(r[j].w * rinv * wv[j].w) << 16);
             reinterpret_cast<u32x2 *>(y + (size_t)blockIdx.x * d)[i] = u32x2{lo, hi};
         }
     }
@@ -345,8 +346,8 @@ __global__ __launch_bounds__(256) void prompt_attn_kernel(const float *__restric
             den += __expf(s_m[w][r] - M) * s_l[w][r];
             v += reinterpret_cast<const f32x4 *>(s_v[w])[i];
         }
-        const u32x2 ob = {f32_to_bf16_bits(v.x / den) | (f32_to_bf16_bits(v.y / den) << 16),
-                          f32_to_bf16_bits(v.z / den) | (f32_to_bf16_bits(v.w / den) << 16)};
+        auto bits = [&](float o) { return f32_to_bf16_bits(o / den * kExactX); };  // (for the exact product that reads them)
+        const u32x2 ob = {bits(v.x) | (bits(v.y) << 16), bits(v.z) | (bits(v.w) << 16)};
         *reinterpret_cast<u32x2 *>(out + (size_t)r0 * DH + 4 * i) = ob;
     }
 }

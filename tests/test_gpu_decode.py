@@ -1131,3 +1131,56 @@ def test_decoder_refuses_positions_past_the_cache_and_tokens_outside_the_table()
         dec.feed([1, 300], 0)                         # token outside [0, vocab)
     with pytest.raises(ValueError):
         dec.generate(-1, 0, 1)
+
+
+def _exact_weights(n, k, g):
+    p = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+    s = torch.exp(torch.randn(n, k // 32, device=DEV, generator=g) * 0.5 - 5.0).half()
+    u = torch.stack((p & 15, p >> 4), -1).reshape(n, k).double() - 8
+    return p, s, u * s.double().repeat_interleave(32, 1)
+
+
+@pytest.mark.parametrize("m,n,k,parts", [(1, 64, 256, 1), (31, 200, 768, 3), (33, 192, 1024, 2), (70, 64, 512, 2), (129, 700, 2816, 3), (128, 2048, 4096, 4),
+                                         (255, 2048, 2048, 8), (200, 2000, 1280, 1), (300, 8192, 2048, 1), (257, 4096, 256, 1), (512, 4096, 512, 1)])
+def test_exact_products_of_every_tile(m, n, k, parts):
+    """The prompt's products against float64, tiles of 32 x 64, 64 x 64, 128 x 64 and 128 x 128, from one step to many, ragged rows and columns,
+    parts of uneven length.  Sums in fp32 of k / 32 groups: a few roundings of 2^-24 each; a group taken twice or left out is 2^-5 and more."""
+    import ctypes
+
+    from chadslab_amd import _lib
+
+    fn = _lib.load()["_ZN5chadq21gemm_exact_f32_launchEPKtPKhS1_PfiiiiP12ihipStream_t"]
+    fn.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 + [ctypes.c_void_p]
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + n)
+    p, s, w = _exact_weights(n, k, g)
+    x = torch.randn(m, k, device=DEV, generator=g).bfloat16()
+    scaled = (x.float() * 2.0 ** -5).bfloat16()  # the factor these products expect
+    y = torch.full((parts, m, n), float("nan"), device=DEV)
+    assert fn(scaled.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, parts, torch.cuda.current_stream().cuda_stream) == 0
+    ref = x.double() @ w.t()
+    err = (y.double().sum(0) - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= 2.0 ** -20, float(err.max())
+
+
+@pytest.mark.parametrize("m,n,k", [(9, 256, 256), (40, 4096, 768), (100, 8192, 1024), (65, 16384, 256), (128, 16384, 512), (129, 16384, 2048), (300, 4096, 1280),
+                                   (256, 32768, 512), (200, 32000, 2048), (512, 8192, 256)])
+def test_exact_gated_products_of_every_tile(m, n, k):
+    """Gate and up rows in pairs: gelu_tanh(gate) * up rounded once to bf16, times 2^-5; tiles of 32 to 256 rows.  2^-9 per rounding, 1.66e-3 over all."""
+    import ctypes
+
+    from chadslab_amd import _lib
+
+    fn = _lib.load()["_ZN5chadq23gemm_exact_geglu_launchEPKtPKhS1_PtiiiP12ihipStream_t"]
+    fn.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 3 + [ctypes.c_void_p]
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + n)
+    p, s, w = _exact_weights(n, k, g)
+    x = (torch.randn(m, k, device=DEV, generator=g) * 0.5).bfloat16()
+    scaled = (x.float() * 2.0 ** -5).bfloat16()
+    h = torch.full((m, n // 2), float("nan"), device=DEV, dtype=torch.bfloat16)
+    assert fn(scaled.data_ptr(), p.data_ptr(), s.data_ptr(), h.data_ptr(), m, n, k, torch.cuda.current_stream().cuda_stream) == 0
+    y = x.double() @ w.t()
+    ref = torch.nn.functional.gelu(y[:, 0::2], approximate="tanh") * y[:, 1::2]
+    err = (h.double() * 32 - ref).norm(dim=1) / ref.norm(dim=1)
+    assert float(err.max()) <= 2.0 ** -8, float(err.max())

@@ -160,11 +160,17 @@ __device__ __forceinline__ bf16x8 signed8_i4_16th(uint32_t w) {
 
 // EPI (what becomes of the sums): EPI_BF16 y bf16 [M,N], times the row scale for int8; EPI_F32 y fp32 [gridDim.y][M,N],
 // part blockIdx.y holding the sum over its kspan k; EPI_GEGLU the weight rows come in pairs (gate, up) of a feature and
-// h = bf16(gelu_tanh(gate) * up) goes to y as bf16 [M, N/2], times kExactX for the exact product that reads it.
+// h = bf16(gelu_tanh(gate) * up) goes to y as bf16 [M, N/2], times kExactX for the exact product that reads it.  EPI_QKV (WN = 2, WK = 4): as
+// QkvOut says; a tile's columns are 32 of a head's first half and the 32 of its second half that they are rotated with.
+// (A type of its own per epilogue: a name formed from the unnamed enumeration would not be the same for the host's and the device's compiler.)
+template <int EPI>
+struct MoreOut {};
+template <>
+struct MoreOut<EPI_QKV> : QkvOut {};
 template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT, int EPI, bool SHORT>
 __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WM * WN * WK / 4, WM * WN * WK / 4))) void gemm_tile_q_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wq, const void *__restrict__ scv, void *__restrict__ yv, int M, int N,
-    int K, int kspan) {
+    int K, int kspan, MoreOut<EPI> qkv) {
     typedef Cfg<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, SHORT> C;
     constexpr int BM = C::BM, BN = C::BN, BB = C::BB, AHEAD = C::AHEAD, SL = C::SL;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -177,7 +183,14 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     const int per_xcd = (tiles + 7) / 8;
     const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (tile >= tiles) return;
-    const int m0 = (tile / tiles_n) * BM, n0 = (tile % tiles_n) * BN;
+    const int m0 = (tile / tiles_n) * BM;
+    int n0 = (tile % tiles_n) * BN, half = 32;  // the tile's first weight row; (EPI_QKV) how far its second 32 are from there
+    if constexpr (EPI == EPI_QKV) {
+        static_assert(WM == 1 && WN == 2 && WK == 4 && NB == 1 && !GUARD, "what the rotation knows");
+        half = qkv.dh >> 1;
+        const int per_head = half >> 5, tn = tile % tiles_n;
+        n0 = tn / per_head * qkv.dh + tn % per_head * 32;
+    }
     const int kbeg = EPI == EPI_BF16 ? 0 : blockIdx.y * kspan;                                        // a multiple of 256
     const int kn = EPI == EPI_BF16 ? K : (K - kbeg < kspan ? K - kbeg : kspan);                       // k of this workgroup
     const int G = K >> 5, steps = (kn + C::KS - 1) / C::KS;
@@ -186,7 +199,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     // ---- requests.  Buffer form of the DMA: the tile's first row in a resource descriptor, the lane's place in a 32-bit
     // offset that never changes, the step in the scalar offset.  A row past the matrix is requested beyond the
     // descriptor's range and arrives as zeros (its products are not stored; multipliers fed zeros draw less power).
-    const int mrows = M - m0 < BM ? M - m0 : BM, nrows = N - n0 < BN ? N - n0 : BN;
+    const int mrows = M - m0 < BM ? M - m0 : BM, nrows = EPI == EPI_QKV ? half + 32 : N - n0 < BN ? N - n0 : BN;
+    auto wrow_at = [&](int r) { return EPI == EPI_QKV ? (r & 31) + (r >> 5) * half : r; };  // of the tile's column r, behind n0
     const __amdgpu_buffer_rsrc_t arsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(x) + (size_t)m0 * K, 0, mrows * K * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t brsrc =
@@ -207,10 +221,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     }
 #pragma unroll
     for (int q = 0; q < C::BS_DMA; ++q) {  // 64 / BPR weight rows, or the scales of 64, per instruction
-        const int e = q * C::NW + wave, r = e * (64 / BPR) + lane / BPR, c = (e - C::BI) * 64 + lane;
+        const int e = q * C::NW + wave, r = e * (64 / BPR) + lane / BPR, c = (e - C::BI) * 64 + lane, rw = wrow_at(r), cw = wrow_at(c);
         bpc[q] = 16 * ((lane % BPR) ^ bkey(r));
-        if (SHORT || e < C::BI) boff[q] = r < nrows ? (uint32_t)r * (uint32_t)wrow + (uint32_t)bpc[q] : kOut;
-        else boff[q] = e < C::BI + C::SI && c < nrows ? (uint32_t)c * (uint32_t)(G * 2) : kOut;
+        if (SHORT || e < C::BI) boff[q] = rw < nrows ? (uint32_t)rw * (uint32_t)wrow + (uint32_t)bpc[q] : kOut;
+        else boff[q] = e < C::BI + C::SI && cw < nrows ? (uint32_t)cw * (uint32_t)(G * 2) : kOut;
     }
     const uint16_t *srow[NB];  // GUARD: the scale rows of the lane's columns
     if constexpr (I4 && GUARD) {
@@ -666,6 +680,49 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     // A wave finishes 1/WK of its values, MB * 16 of them numbered (row block, v).  WK = 2: the two waves that hold the k halves of
     // one result trade halves of it through LDS.  WK = 4: every wave leaves all of them and adds its quarter in the order of the k.
     constexpr int UV = MB * 16 / WK;
+    auto row_of = [&](int v) {
+        auto at = [](int f) { return (f >> 4) * 32 + 8 * ((f & 15) >> 2) + (f & 3); };
+        // (where no carry goes between the two parts of the number, the second part of the row is a constant)
+        return wm * MB * 32 + 4 * kq + (16 % UV == 0 || UV % 16 == 0 ? at(wk * UV) + at(v) : at(wk * UV + v));
+    };
+    if constexpr (EPI == EPI_QKV) {
+        // as WK = 4 below, but a wave adds up both halves of its pairs of columns: each of the two waves of a pair then writes one of them
+        const int head = n0 / qkv.dh, j = n0 % qkv.dh + nl;
+        float cs[UV], sn[UV];
+#pragma unroll
+        for (int v = 0; v < UV; ++v) {
+            const int m = m0 + row_of(v);
+            const float *const t = qkv.table + ((size_t)(qkv.pos + (m < M ? m : M - 1)) * half + j) * 2;
+            cs[v] = t[0];
+            sn[v] = t[1];
+        }
+        float *const red = reinterpret_cast<float *>(lds) + lane * 4;
+#pragma unroll
+        for (int q = 0; q < MB * 4; ++q) {
+            auto val = [&](int f) { return acc[f >> 4][0][f & 15]; };
+            *reinterpret_cast<f32x4 *>(red + (wave * MB * 4 + q) * 256) = f32x4{val(4 * q), val(4 * q + 1), val(4 * q + 2), val(4 * q + 3)};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < UV / 4; ++q) {
+            f32x4 o[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int w = 0; w < WK; ++w) o[h] += *reinterpret_cast<const f32x4 *>(red + ((w * WN + h) * MB * 4 + wk * (UV / 4) + q) * 256);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int v = 4 * q + e, m = m0 + row_of(v);
+                if (m >= M) continue;
+                const float a = o[0][e], b = o[1][e];
+                const float r = head > qkv.hq ? (wn ? b : a) : wn ? b * cs[v] + a * sn[v] : a * cs[v] - b * sn[v];
+                const int at = j + wn * half;
+                if (head < qkv.hq) qkv.q[((size_t)m * qkv.hq + head) * qkv.dh + at] = r;
+                else (head == qkv.hq ? qkv.kc : qkv.vc)[(size_t)(qkv.pos + m) * qkv.dh + at] = (uint16_t)f32_to_bf16_bits(r);
+            }
+        }
+        return;
+    }
     float res[NB][UV];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
@@ -708,11 +765,6 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             for (int v = 0; v < UV; ++v) res[nb][v] = val(v);
         }
     }
-    auto row_of = [&](int v) {
-        auto at = [](int f) { return (f >> 4) * 32 + 8 * ((f & 15) >> 2) + (f & 3); };
-        // (where no carry goes between the two parts of the number, the second part of the row is a constant)
-        return wm * MB * 32 + 4 * kq + (16 % UV == 0 || UV % 16 == 0 ? at(wk * UV) + at(v) : at(wk * UV + v));
-    };
     if constexpr (EPI == EPI_F32) {  // 128 contiguous bytes per row straight from the registers
         float *const y = reinterpret_cast<float *>(yv) + (size_t)blockIdx.y * M * N;
 #pragma unroll
@@ -778,7 +830,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 }
 
 template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT = false, int EPI = EPI_BF16, bool SHORT = false>
-static int launch(const uint16_t *x, const uint8_t *wq, const void *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st) {
+static int launch(const uint16_t *x, const uint8_t *wq, const void *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st,
+                  MoreOut<EPI> qkv = {}) {
     typedef Cfg<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, SHORT> C;
     static std::atomic<bool> attr_set{false};  // setting it twice from two threads is harmless
     if (!attr_set.load(std::memory_order_acquire)) {
@@ -788,7 +841,7 @@ static int launch(const uint16_t *x, const uint8_t *wq, const void *sc, void *y,
     }
     const int tiles = ((N + C::BN - 1) / C::BN) * ((M + C::BM - 1) / C::BM);
     hipLaunchKernelGGL((gemm_tile_q_kernel<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, EXACT, EPI, SHORT>), dim3((tiles + 7) / 8 * 8, ksplit), dim3(C::T), C::LDS, st,
-                       x, wq, sc, y, M, N, K, ksplit == 1 ? K : (K / 256 + ksplit - 1) / ksplit * 256);
+                       x, wq, sc, y, M, N, K, ksplit == 1 ? K : (K / 256 + ksplit - 1) / ksplit * 256, qkv);
     return hip_check(hipGetLastError(), "gemm_tile_q launch");
 }
 
@@ -917,7 +970,7 @@ struct ExactCost {
 static const ExactCost kExact32 = {32, 64, 4.87f, -1.63f, .694f, 1.42f, .694f, .870f, .216f};
 static const ExactCost kExact[3] = {{64, 64, 1.33f, 2.61f, .817f, 2.61f, .817f, .787f, .023f}, {128, 64, 1.66f, 3.52f, 1.144f, 3.52f, 1.144f, .784f, .043f},
                                     {128, 128, 2.86f, 1.75f, 2.64f, 1.75f, 2.64f, .883f, .170f}};
-static const ExactCost kGeglu[4] = {{64, 64, 1.10f, 2.61f, .860f, 2.61f, .860f, .801f, 0.f}, {128, 64, 1.12f, 3.88f, 1.197f, 3.88f, 1.197f, .808f, 0.f},
+static const ExactCost kGeglu[4] = {{64, 64, 1.10f, 2.61f, .860f, 2.61f, .860f, .801f, 0.f}, {128, 64, 2.f, 3.88f, 1.197f, 3.88f, 1.197f, .808f, 0.f},
                                     {128, 128, .75f, 4.60f, 2.871f, 4.60f, 2.871f, .823f, 0.f}, {256, 128, .75f, 7.18f, 3.784f, 7.18f, 3.784f, .798f, 0.f}};
 
 // us that a launch takes in `parts` K splits of `per` 256-k blocks.  Tiles go to the XCDs in turn, each in all its splits, and a round is over
@@ -925,7 +978,8 @@ static const ExactCost kGeglu[4] = {{64, 64, 1.10f, 2.61f, .860f, 2.61f, .860f, 
 // takes c0 + c1 * per in the first round and d0 + d1 * per in a further one (of the tiles of 32 rows two fit on a compute unit), the last
 // round b + (1 - b) f of it if it is full to f; s is what a launch takes besides, c2 what a MB of fp32 parts takes to be written.  The
 // constants of 64 rows and more are fitted to 18700 random products in every number of splits (33 to 700 rows, 128 to 8192 weight rows, 256 to
-// 16000 k) and 8900 gated ones, 2 to 5 % standard deviation; the tile and splits they pick take 0.2 % more than the best of all on average.
+// 16000 k) and 8900 gated ones, 2 to 5 % standard deviation (128 x 64, gated: 0.9 us more than fitted, for prompts of 70 to 128 tokens took 1 % longer with it where the
+// fit has it even with 128 x 128); the tile and splits they pick take 0.2 % more than the best of all on average.
 static float exact_us(const ExactCost &t, int M, int N, int per, int parts) {
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), fullest = (tiles + 7) / 8 * parts, rounds = (fullest + 31) / 32;
     const float last = t.b + (1.f - t.b) * (float)(fullest - (rounds - 1) * 32) / 32.f, first = t.c0 + t.c1 * (float)per;
@@ -981,10 +1035,10 @@ int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint1
 // one part, 63 us of the 125 that its layer took for 37 tokens.)  Rounds of 256 workgroups (512 for up to 32 rows) times the k of each, as the
 // splits were chosen by before, miss how tiles fall to the XCDs, what half a chip costs and what the parts cost.  us, so chosen / in other
 // parts of the same tiles: 265 x 1344 x 7168 in 7 31.6 / in 6 20.5, 552 x 1280 x 5120 in 5 32.1 / in 4 20.7, 22 x 4480 x 1024 in 4 6.4 / in 2
-// 4.9.  kRead: what a MB of parts costs the next kernel.  34 prompts, geometric mean against the earlier kernels, with 0.2 / 0.35 / 0.5 / 0.7 us per MB 1.011 /
-// 1.030 / 1.011 / 1.026.  M counts in whole tiles only: prompt_layout asks for every number of them.
+// 4.9.  kRead: what a MB of parts costs the next kernel: with 0.35 us per MB the down product of 128 tokens, 2048 x 16384, is in eight parts of 128 x
+// 64 tiles and the prompt of 18 layers takes 1640-1680 us, with 0.7 in four of 64 x 64 1569-1607.  M counts in whole tiles only: prompt_layout asks for every number of them.
 int gemm_exact_splits(int M, int N, int K) {
-    constexpr float kRead = .35f;
+    constexpr float kRead = .7f;
     const int blocks = K / 256, rows = M <= 32 ? 32 : (M + 63) / 64 * 64;
     int best = 1;
     float best_us = 0.f;
@@ -999,6 +1053,30 @@ int gemm_exact_splits(int M, int N, int K) {
         }
     }
     return best;
+}
+
+// q, k and v of a prompt with the rotation and the cache rows in the epilogue: tiles of 64 weight rows, K in one part.
+static const ExactCost &qkv_pick(int M, int N, int K) {
+    return M <= 32 ? kExact32 : M <= 64 || exact_us(kExact[0], M, N, K / 256, 1) <= exact_us(kExact[1], M, N, K / 256, 1) ? kExact[0] : kExact[1];
+}
+
+// What the parts bring may be more than the launch that adds and rotates them takes, 1 to 1.9 us in a queue (its own time is 5 us, most of it the
+// way of the parts through memory, which the next kernel has to itself otherwise).  us, in the epilogue / in parts and a launch: 18 layers of
+// 2048 x 16384, 24 tokens (four parts) 1088 / 1058, 256 (one) 2085 / 2134; 3 layers of 1792 x 10752, 212 tokens 313 / 325; 6 of 1024 x 4864, 35 tokens
+// (four) 283 / 277; 4 of 512 x 3840, 4 tokens (two) 203 / 208.
+bool gemm_exact_qkv_pays(int M, int N, int K) {
+    const int parts = gemm_exact_splits(M, N, K), per = (K / 256 + parts - 1) / parts;
+    float us;
+    gemm_exact_tile(M, N, per, parts, false, &us);
+    return exact_us(qkv_pick(M, N, K), M, N, K / 256, 1) <= us + 1.f;
+}
+
+int gemm_exact_qkv_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, const QkvOut &out, int M, int K, hipStream_t st) {
+    const int N = (out.hq + 2) * out.dh;
+    const ExactCost &t = qkv_pick(M, N, K);
+    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, 1, st, {out});
+    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, 1, st, {out});
+    return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, 1, st, {out});
 }
 
 int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,

@@ -6,7 +6,8 @@
 // the attention vector, the gated activation), weights are taken exactly (gemm_tile_q.hip, EXACT), sums, residual stream,
 // rotation and softmax are fp32, K and V rows bf16.
 //
-// Per layer: residual add + RMSNorm | qkv product | rotation and cache rows | attention | output product | residual add +
+// Per layer: residual add + RMSNorm | qkv product | rotation and cache rows, by a launch of their own where the
+// product is split over K, else in its epilogue | attention | output product | residual add +
 // RMSNorm | gate/up product with the GeGLU in its epilogue | down product.  Products with few tiles are split over K; the
 // kernel that consumes them adds the parts, in order.  In the last layer everything behind the cache rows runs for the last
 // token only: nothing else of it is ever read.
@@ -410,6 +411,7 @@ int prompt_i4g32_launch(const chadq_prompt_layer_i4g32 *layers, int n_layers, co
     PromptWs ws;
     prompt_layout(reinterpret_cast<uint8_t *>(workspace), T, d, hq, dh, ffn, &ws);
     const int wq = (hq + 2) * dh;
+    const bool rotated = gemm_exact_qkv_pays(T, wq, d);  // q and k are, by the product's epilogue
     hipLaunchKernelGGL(prompt_embed_kernel, dim3(T), dim3(256), 0, st, tokens, emb, semb, ws.x, d, V);
     int np = 0, rc;  // parts pending for the residual stream
     int rows = T;
@@ -422,9 +424,13 @@ int prompt_i4g32_launch(const chadq_prompt_layer_i4g32 *layers, int n_layers, co
     for (int li = 0; li < n_layers; ++li) {
         const chadq_prompt_layer_i4g32 &L = layers[li];
         add_norm_launch(T, x, x, ws.parts, np, L.ln1, ws.xn, d, eps, st);
-        np = gemm_exact_splits(T, wq, d);
-        CHADQ_STEP(gemm_exact_f32_launch(ws.xn, L.wqkv, L.sqkv, ws.parts, T, wq, d, np, st));
-        hipLaunchKernelGGL(prompt_rope_kernel, dim3(T, hq + 2), dim3(128), 0, st, ws.parts, np, rope_table, ws.q, L.kcache, L.vcache, hq, dh, pos);
+        if (rotated) {
+            CHADQ_STEP(gemm_exact_qkv_launch(ws.xn, L.wqkv, L.sqkv, QkvOut{rope_table, ws.q, L.kcache, L.vcache, hq, dh, pos}, T, d, st));
+        } else {
+            np = gemm_exact_splits(T, wq, d);
+            CHADQ_STEP(gemm_exact_f32_launch(ws.xn, L.wqkv, L.sqkv, ws.parts, T, wq, d, np, st));
+            hipLaunchKernelGGL(prompt_rope_kernel, dim3(T, hq + 2), dim3(128), 0, st, ws.parts, np, rope_table, ws.q, L.kcache, L.vcache, hq, dh, pos);
+        }
         const float *q = ws.q;
         if (li == n_layers - 1) {  // of the last layer only the last token goes on
             rows = 1;

@@ -130,3 +130,9 @@ def test_exact_products_take_the_tile_that_reaches_the_compute_units():
     assert rows(101, 8192, 8, 1, True) == 64      # 11.7 / 25.9 / 32.7
     assert rows(256, 32768, 8, 1, True) == 256
     assert rows(64, 32768, 8, 1, True) == 64 and rows(32, 32768, 8, 1, True) == 32 and rows(9, 64, 1, 1, False) == 32
+
+
+def test_prompt_projections_are_rotated_where_they_are_written_unless_parts_pay():
+    fn = _rule("_ZN5chadq19gemm_exact_qkv_paysEiii", ctypes.c_bool)  # (tokens, (hq + 2) * dh, d)
+    assert fn(256, 2560, 2048) and fn(212, 2560, 1792) and fn(4, 1280, 512)          # us a prompt 2085 / 2134, 313 / 325, 203 / 208
+    assert not fn(24, 2560, 2048) and not fn(35, 640, 1024) and not fn(7, 1536, 1536)  # 1088 / 1058, 283 / 277

@@ -1184,3 +1184,42 @@ def test_exact_gated_products_of_every_tile(m, n, k):
     ref = torch.nn.functional.gelu(y[:, 0::2], approximate="tanh") * y[:, 1::2]
     err = (h.double() * 32 - ref).norm(dim=1) / ref.norm(dim=1)
     assert float(err.max()) <= 2.0 ** -8, float(err.max())
+
+
+@pytest.mark.parametrize("m,pos,d,hq,dh", [(1, 0, 256, 1, 64), (7, 5, 512, 4, 64), (32, 1, 256, 3, 128), (33, 100, 768, 2, 256), (64, 0, 512, 8, 64), (65, 9, 1024, 8, 128),
+                                           (256, 33, 2048, 8, 256), (200, 0, 256, 16, 64), (129, 77, 2048, 8, 256)])
+def test_exact_qkv_product_rotates_and_fills_the_caches(m, pos, d, hq, dh):
+    """q, k and v with the rotation in the product's epilogue, against float64: every tile, every head size, ragged rows; cache rows outside
+    pos .. pos + m - 1 keep their bits.  q in fp32 (2^-20 as the plain products), k and v rounded to bf16 (2^-8)."""
+    import ctypes
+
+    from chadslab_amd import _lib
+
+    class Out(ctypes.Structure):
+        _fields_ = [("table", ctypes.c_void_p), ("q", ctypes.c_void_p), ("kc", ctypes.c_void_p), ("vc", ctypes.c_void_p), ("hq", ctypes.c_int),
+                    ("dh", ctypes.c_int), ("pos", ctypes.c_int)]
+
+    fn = _lib.load()["_ZN5chadq21gemm_exact_qkv_launchEPKtPKhS1_RKNS_6QkvOutEiiP12ihipStream_t"]
+    fn.argtypes = [ctypes.c_void_p] * 3 + [ctypes.POINTER(Out), ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + d)
+    n, ctx, half = (hq + 2) * dh, pos + m + 3, dh // 2
+    p, s, w = _exact_weights(n, d, g)
+    x = torch.randn(m, d, device=DEV, generator=g).bfloat16()
+    scaled = (x.float() * 2.0 ** -5).bfloat16()
+    table = torch.randn(ctx, half, 2, device=DEV, generator=g)  # (any pair of factors: the epilogue only applies them)
+    q = torch.full((m, hq, dh), float("nan"), device=DEV)
+    kc, vc = (torch.full((ctx, dh), 7.0, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    out = Out(table.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), hq, dh, pos)
+    assert fn(scaled.data_ptr(), p.data_ptr(), s.data_ptr(), ctypes.byref(out), m, d, torch.cuda.current_stream().cuda_stream) == 0
+    y = (x.double() @ w.t()).reshape(m, hq + 2, 2, half)
+    cs, sn = table[pos:pos + m, None, :, 0].double(), table[pos:pos + m, None, :, 1].double()
+    rot = torch.stack((y[:, :, 0] * cs - y[:, :, 1] * sn, y[:, :, 1] * cs + y[:, :, 0] * sn), 2).reshape(m, hq + 2, dh)
+
+    def off(got, ref):
+        return float(((got.double() - ref).norm(dim=-1) / ref.norm(dim=-1)).max())
+
+    assert off(q, rot[:, :hq]) <= 2.0 ** -20
+    assert off(kc[pos:pos + m], rot[:, hq]) <= 2.0 ** -8 and off(vc[pos:pos + m], y[:, hq + 1].reshape(m, dh)) <= 2.0 ** -8
+    for c in (kc, vc):
+        assert bool((c[:pos] == 7).all()) and bool((c[pos + m:] == 7).all())

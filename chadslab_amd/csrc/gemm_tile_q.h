@@ -31,7 +31,7 @@ int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *
 int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, bool bf16_out,
                                hipStream_t st);
 // The product of a prompt's M tokens with [q heads | k | v] (hq + 2 heads of dh, in whole K): q and k rotated at positions pos + m (table as
-// chadq_rope_table writes it), q fp32 [M][hq*dh], k and v as bf16 rows pos + m of the caches.
+// chadq_rope_table writes it), q fp32 [M][hq*dh], k and v as bf16 rows pos + m of the caches.  x carries kExactX.
 struct QkvOut {
     const float *table;
     float *q;
@@ -40,7 +40,11 @@ struct QkvOut {
 };
 bool gemm_exact_qkv_pays(int M, int N, int K);  // against the plain product and a launch for the rest
 int gemm_exact_qkv_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, const QkvOut &out, int M, int K, hipStream_t st);
-// weight rows in (gate, up) pairs: h[m,i] = bf16(gelu_tanh(y[m,2i]) * y[m,2i+1]) * kExactX, [M, N/2]
+int gemm_exact_scaled_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
+                                 hipStream_t st);
+// weight rows in (gate, up) pairs: h[m,i] = bf16(gelu_tanh(y[m,2i]) * y[m,2i+1]), [M, N/2]
 int gemm_exact_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st);
+
+int gemm_exact_scaled_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st);
 
 }  // namespace chadq

@@ -160,13 +160,20 @@ __device__ __forceinline__ bf16x8 signed8_i4_16th(uint32_t w) {
 
 // EPI (what becomes of the sums): EPI_BF16 y bf16 [M,N], times the row scale for int8; EPI_F32 y fp32 [gridDim.y][M,N],
 // part blockIdx.y holding the sum over its kspan k; EPI_GEGLU the weight rows come in pairs (gate, up) of a feature and
-// h = bf16(gelu_tanh(gate) * up) goes to y as bf16 [M, N/2], times kExactX for the exact product that reads it.  EPI_QKV (WN = 2, WK = 4): as
+// h = bf16(gelu_tanh(gate) * up) goes to y as bf16 [M, N/2], times the factor of the activations (ExactX).  EPI_QKV (WN = 2, WK = 4): as
 // QkvOut says; a tile's columns are 32 of a head's first half and the 32 of its second half that they are rotated with.
 // (A type of its own per epilogue: a name formed from the unnamed enumeration would not be the same for the host's and the device's compiler.)
 template <int EPI>
 struct MoreOut {};
 template <>
 struct MoreOut<EPI_QKV> : QkvOut {};
+struct ExactX {
+    float x = 1.f;  // the factor that the activations (and a gated result) carry
+};
+template <>
+struct MoreOut<EPI_F32> : ExactX {};
+template <>
+struct MoreOut<EPI_GEGLU> : ExactX {};
 template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT, int EPI, bool SHORT>
 __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WM * WN * WK / 4, WM * WN * WK / 4))) void gemm_tile_q_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wq, const void *__restrict__ scv, void *__restrict__ yv, int M, int N,
@@ -340,7 +347,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
 
     if constexpr (EXACT) {
     // Exact weights: integers as operands, two MFMAs from zero on per scale group and row block, and one fp32 FMA per
-    // value that applies the scale (times 2^9, what operands and activations leave out).  A pair of MFMAs runs beside the FMAs of the pair before it.
+    // value that applies the scale.  A pair of MFMAs runs beside the FMAs of the pair before it.
     constexpr int RING = Q >= 4 ? 4 : 2;
     // The row block beside whose MFMAs the next group's words are taken over (a step of one group: when they have arrived) and the one, not
     // before it, beside which the first half of their operands is made
@@ -349,6 +356,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     uint32_t wv[GR][2], wnx[GR][2];  // the lane's packed words of a step [group][slice], of the next one
     uint32_t sraw[GR];               // its scales
     float sc2[GR], s_last = 0.f;     // ... as floats, that of the group whose sums are next
+    float undo = 512.f;              // what operands and activations leave out
+    if constexpr (!GUARD && EPI != EPI_QKV) undo = 16.f / qkv.x;
     auto fetch = [&](int step, const uint8_t *stage) {
 #pragma unroll
         for (int g = 0; g < GR; ++g)
@@ -365,7 +374,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         for (int g = 0; g < GR; ++g) {
             wv[g][0] = wnx[g][0];
             wv[g][1] = wnx[g][1];
-            sc2[g] = (GUARD && kbeg + step * C::KS + wk * KW + 32 * g >= K) ? 0.f : 512.f * f16_bits_to_f32((uint16_t)sraw[g]);
+            sc2[g] = (GUARD && kbeg + step * C::KS + wk * KW + 32 * g >= K) ? 0.f : undo * f16_bits_to_f32((uint16_t)sraw[g]);
         }
     };
     bf16x8 bo[2], bnx[2];  // operands of the present group, of the next one
@@ -805,7 +814,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             // even lane: row r, columns (nl, nl+1) = (own a0, neighbour's a0); odd lane: row r+1, columns (nl-1, nl)
             if constexpr (GE)
                 *reinterpret_cast<uint16_t *>(lds + row * EP + (cb + nl) / 2 * 2) =
-                    (uint16_t)pack_bf16_rne(gelu_tanh_dev(odd ? recv : a0) * (odd ? a1 : recv) * kExactX, 0.f);
+                    (uint16_t)pack_bf16_rne(gelu_tanh_dev(odd ? recv : a0) * (odd ? a1 : recv) * qkv.x, 0.f);
             else
                 *reinterpret_cast<uint32_t *>(lds + row * EP + (cb + (nl & ~1)) * 2) = odd ? pack_bf16_rne(recv, a1) : pack_bf16_rne(a0, recv);
         }
@@ -969,16 +978,17 @@ struct ExactCost {
 };
 static const ExactCost kExact32 = {32, 64, 4.87f, -1.63f, .694f, 1.42f, .694f, .870f, .216f};
 static const ExactCost kExact[3] = {{64, 64, 1.33f, 2.61f, .817f, 2.61f, .817f, .787f, .023f}, {128, 64, 1.66f, 3.52f, 1.144f, 3.52f, 1.144f, .784f, .043f},
-                                    {128, 128, 2.86f, 1.75f, 2.64f, 1.75f, 2.64f, .883f, .170f}};
+                                    {128, 128, 2.75f, 1.75f, 2.64f, 1.75f, 2.64f, .883f, .170f}};
 static const ExactCost kGeglu[4] = {{64, 64, 1.10f, 2.61f, .860f, 2.61f, .860f, .801f, 0.f}, {128, 64, 2.f, 3.88f, 1.197f, 3.88f, 1.197f, .808f, 0.f},
-                                    {128, 128, .75f, 4.60f, 2.871f, 4.60f, 2.871f, .823f, 0.f}, {256, 128, .75f, 7.18f, 3.784f, 7.18f, 3.784f, .798f, 0.f}};
+                                    {128, 128, .75f, 4.60f, 2.871f, 4.60f, 2.871f, .823f, 0.f}, {256, 128, 1.4f, 7.18f, 3.784f, 7.18f, 3.784f, .798f, 0.f}};
 
 // us that a launch takes in `parts` K splits of `per` 256-k blocks.  Tiles go to the XCDs in turn, each in all its splits, and a round is over
 // when the fullest XCD has dealt its workgroups to its 32 compute units: 33 tiles in 7 parts are 231 workgroups, but 35 on one XCD.  A tile
 // takes c0 + c1 * per in the first round and d0 + d1 * per in a further one (of the tiles of 32 rows two fit on a compute unit), the last
 // round b + (1 - b) f of it if it is full to f; s is what a launch takes besides, c2 what a MB of fp32 parts takes to be written.  The
 // constants of 64 rows and more are fitted to 18700 random products in every number of splits (33 to 700 rows, 128 to 8192 weight rows, 256 to
-// 16000 k) and 8900 gated ones, 2 to 5 % standard deviation (128 x 64, gated: 0.9 us more than fitted, for prompts of 70 to 128 tokens took 1 % longer with it where the
+// 16000 k) and 8900 gated ones, 2 to 5 % standard deviation (two numbers of the 128-row tiles and one of the gated 256 moved by 0.1 to 0.9 us
+// where tiles are even; 128 x 64, gated, by 0.9: prompts of 70 to 128 tokens took 1 % longer with it where the
 // fit has it even with 128 x 128); the tile and splits they pick take 0.2 % more than the best of all on average.
 static float exact_us(const ExactCost &t, int M, int N, int per, int parts) {
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), fullest = (tiles + 7) / 8 * parts, rounds = (fullest + 31) / 32;
@@ -999,6 +1009,7 @@ static const ExactCost &exact_pick(int M, int N, int per, int parts, bool geglu,
     int best = 0;
     *us = exact_us(t[0], M, N, per, parts);
     for (int i = 1; i < (M <= 64 ? 1 : geglu ? 4 : 3); ++i) {
+        if (i == 1 && per < 4) continue;  // (128 x 64: a step of it is 128 k, and 64 x 64 reach more compute units for the same unpacking)
         const float u = exact_us(t[i], M, N, per, parts);
         if (u < *us) {
             best = i;
@@ -1011,16 +1022,17 @@ static const ExactCost &exact_pick(int M, int N, int per, int parts, bool geglu,
 int gemm_exact_tile(int M, int N, int per, int parts, bool geglu, float *us) { return exact_pick(M, N, per, parts, geglu, us).bm; }
 
 template <int EPI>
-static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st) {
+static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, void *y, int M, int N, int K, int ksplit, float factor, hipStream_t st) {
     float us;
+    const tileq::MoreOut<EPI> more{{factor}};
     const ExactCost &t = exact_pick(M, N, (K / 256 + ksplit - 1) / ksplit, ksplit, EPI == tileq::EPI_GEGLU, &us);
-    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
-    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st, more);
+    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st, more);
     if constexpr (EPI == tileq::EPI_GEGLU) {
-        if (t.bm == 256) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+        if (t.bm == 256) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st, more);
     }
-    if (t.bn == 64) return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
-    return tileq::launch<true, 1, 4, 2, 4, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st);
+    if (t.bn == 64) return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st, more);
+    return tileq::launch<true, 1, 4, 2, 4, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st, more);
 }
 
 // Decode products of at most 32 rows whose K (or scales) the GEMV of gemv_i4g32_mfma.hip does not take: y fp32 or bf16 [M,N] in one
@@ -1081,11 +1093,20 @@ int gemm_exact_qkv_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *
 
 int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
                           hipStream_t st) {
-    return launch_exact<tileq::EPI_F32>(x, wp, sc, y_parts, M, N, K, ksplit, st);
+    return launch_exact<tileq::EPI_F32>(x, wp, sc, y_parts, M, N, K, ksplit, 1.f, st);
+}
+
+int gemm_exact_scaled_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
+                                 hipStream_t st) {
+    return launch_exact<tileq::EPI_F32>(x, wp, sc, y_parts, M, N, K, ksplit, kExactX, st);
 }
 
 int gemm_exact_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st) {
-    return launch_exact<tileq::EPI_GEGLU>(x, wp, sc, h, M, N, K, 1, st);
+    return launch_exact<tileq::EPI_GEGLU>(x, wp, sc, h, M, N, K, 1, 1.f, st);
+}
+
+int gemm_exact_scaled_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st) {
+    return launch_exact<tileq::EPI_GEGLU>(x, wp, sc, h, M, N, K, 1, kExactX, st);
 }
 
 }  // namespace chadq

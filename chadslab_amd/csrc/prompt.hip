@@ -428,7 +428,7 @@ int prompt_i4g32_launch(const chadq_prompt_layer_i4g32 *layers, int n_layers, co
             CHADQ_STEP(gemm_exact_qkv_launch(ws.xn, L.wqkv, L.sqkv, QkvOut{rope_table, ws.q, L.kcache, L.vcache, hq, dh, pos}, T, d, st));
         } else {
             np = gemm_exact_splits(T, wq, d);
-            CHADQ_STEP(gemm_exact_f32_launch(ws.xn, L.wqkv, L.sqkv, ws.parts, T, wq, d, np, st));
+            CHADQ_STEP(gemm_exact_scaled_f32_launch(ws.xn, L.wqkv, L.sqkv, ws.parts, T, wq, d, np, st));
             hipLaunchKernelGGL(prompt_rope_kernel, dim3(T, hq + 2), dim3(128), 0, st, ws.parts, np, rope_table, ws.q, L.kcache, L.vcache, hq, dh, pos);
         }
         const float *q = ws.q;
@@ -439,11 +439,11 @@ int prompt_i4g32_launch(const chadq_prompt_layer_i4g32 *layers, int n_layers, co
         }
         CHADQ_STEP(prompt_attn_launch(q, L.kcache, L.vcache, ws.xn, rows, pos + T - rows, hq, dh, st));
         np = gemm_exact_splits(rows, d, hq * dh);
-        CHADQ_STEP(gemm_exact_f32_launch(ws.xn, L.wo, L.so, ws.parts, rows, d, hq * dh, np, st));
+        CHADQ_STEP(gemm_exact_scaled_f32_launch(ws.xn, L.wo, L.so, ws.parts, rows, d, hq * dh, np, st));
         add_norm_launch(rows, x, x, ws.parts, np, L.ln2, ws.xn, d, eps, st);
-        CHADQ_STEP(gemm_exact_geglu_launch(ws.xn, L.wgu, L.sgu, ws.h, rows, 2 * ffn, d, st));
+        CHADQ_STEP(gemm_exact_scaled_geglu_launch(ws.xn, L.wgu, L.sgu, ws.h, rows, 2 * ffn, d, st));
         np = gemm_exact_splits(rows, d, ffn);
-        CHADQ_STEP(gemm_exact_f32_launch(ws.h, L.wd, L.sd, ws.parts, rows, d, ffn, np, st));
+        CHADQ_STEP(gemm_exact_scaled_f32_launch(ws.h, L.wd, L.sd, ws.parts, rows, d, ffn, np, st));
     }
 #undef CHADQ_STEP
     add_norm_launch(1, x, x_last, ws.parts, np, (const float *)nullptr, (uint16_t *)nullptr, d, eps, st);

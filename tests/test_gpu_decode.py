@@ -1149,7 +1149,7 @@ def test_exact_products_of_every_tile(m, n, k, parts):
 
     from chadslab_amd import _lib
 
-    fn = _lib.load()["_ZN5chadq21gemm_exact_f32_launchEPKtPKhS1_PfiiiiP12ihipStream_t"]
+    fn = _lib.load()["_ZN5chadq28gemm_exact_scaled_f32_launchEPKtPKhS1_PfiiiiP12ihipStream_t"]
     fn.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 + [ctypes.c_void_p]
     g = torch.Generator(device=DEV)
     g.manual_seed(m + n)
@@ -1171,7 +1171,7 @@ def test_exact_gated_products_of_every_tile(m, n, k):
 
     from chadslab_amd import _lib
 
-    fn = _lib.load()["_ZN5chadq23gemm_exact_geglu_launchEPKtPKhS1_PtiiiP12ihipStream_t"]
+    fn = _lib.load()["_ZN5chadq30gemm_exact_scaled_geglu_launchEPKtPKhS1_PtiiiP12ihipStream_t"]
     fn.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 3 + [ctypes.c_void_p]
     g = torch.Generator(device=DEV)
     g.manual_seed(m + n)

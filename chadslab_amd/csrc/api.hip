@@ -58,6 +58,8 @@ int gemv_i4g32_mfma_dispatch(const uint16_t *, const uint8_t *, const uint16_t *
 int gemv_i8row_dispatch(const float *, const int8_t *, const float *, float *, int, int, int, bool fp32_only, bool bf16_out, hipStream_t);
 int gemm_i4g32_bf16_dispatch(const uint16_t *, const uint8_t *, const uint16_t *, uint16_t *, int, int, int,
                              hipStream_t);
+size_t gemm_parts_bytes(int, int, int, bool);
+int gemm_ws_dispatch(const uint16_t *, const uint8_t *, const void *, uint16_t *, int, int, int, bool, float *, size_t, hipStream_t);
 int gemm_i8row_bf16_dispatch(const uint16_t *, const int8_t *, const float *, uint16_t *, int, int, int,
                              hipStream_t);
 
@@ -282,6 +284,28 @@ int chadq_gemm_i8row_bf16(const uint16_t *x_bf16, const int8_t *w8, const float 
     CHADQ_REQUIRE(x_bf16 && w8 && scale && y_bf16, CHADQ_ERR_NULL, "chadq_gemm_i8row_bf16: null pointer");
     CHADQ_REQUIRE(aligned16(x_bf16) && aligned16(w8), CHADQ_ERR_ALIGN, "chadq_gemm_i8row_bf16: x and w8 must be 16-byte aligned");
     return gemm_i8row_bf16_dispatch(x_bf16, w8, scale, y_bf16, M, N, K, st);
+}
+
+size_t chadq_gemm_bf16_workspace_bytes(int M, int N, int K, int int8_weights) { return gemm_parts_bytes(M, N, K, !int8_weights); }
+
+int chadq_gemm_i4g32_bf16_ws(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, uint16_t *y_bf16, int M, int N, int K, void *workspace,
+                             size_t workspace_bytes, void *stream) {
+    ENTER();
+    CHADQ_REQUIRE(M >= 0 && N >= 0 && K >= 32 && K % 32 == 0, CHADQ_ERR_SHAPE, "chadq_gemm_i4g32_bf16_ws: M=%d N=%d K=%d (K must be a positive multiple of 32)", M, N, K);
+    if (M == 0 || N == 0) return 0;
+    CHADQ_REQUIRE(x_bf16 && wp && scale_f16 && y_bf16, CHADQ_ERR_NULL, "chadq_gemm_i4g32_bf16_ws: null pointer");
+    CHADQ_REQUIRE(aligned16(x_bf16) && aligned16(wp) && aligned16(workspace), CHADQ_ERR_ALIGN, "chadq_gemm_i4g32_bf16_ws: x, wp and workspace must be 16-byte aligned");
+    return gemm_ws_dispatch(x_bf16, wp, scale_f16, y_bf16, M, N, K, true, reinterpret_cast<float *>(workspace), workspace_bytes, st);
+}
+
+int chadq_gemm_i8row_bf16_ws(const uint16_t *x_bf16, const int8_t *w8, const float *scale, uint16_t *y_bf16, int M, int N, int K, void *workspace,
+                             size_t workspace_bytes, void *stream) {
+    ENTER();
+    CHADQ_REQUIRE(M >= 0 && N >= 0 && K >= 16 && K % 16 == 0, CHADQ_ERR_SHAPE, "chadq_gemm_i8row_bf16_ws: M=%d N=%d K=%d (K must be a positive multiple of 16)", M, N, K);
+    if (M == 0 || N == 0) return 0;
+    CHADQ_REQUIRE(x_bf16 && w8 && scale && y_bf16, CHADQ_ERR_NULL, "chadq_gemm_i8row_bf16_ws: null pointer");
+    CHADQ_REQUIRE(aligned16(x_bf16) && aligned16(w8) && aligned16(workspace), CHADQ_ERR_ALIGN, "chadq_gemm_i8row_bf16_ws: x, w8 and workspace must be 16-byte aligned");
+    return gemm_ws_dispatch(x_bf16, reinterpret_cast<const uint8_t *>(w8), scale, y_bf16, M, N, K, false, reinterpret_cast<float *>(workspace), workspace_bytes, st);
 }
 
 static bool moe_sizes_ok(int T, int H, int F, int E, int top_k) {

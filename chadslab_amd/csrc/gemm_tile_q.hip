@@ -256,7 +256,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
         const int e = q * C::NW + wave;
         if (q >= C::BS_DMA) {  // GUARD, int4: scales
             const int nb = q - C::BS_DMA, g = KW == 64 ? 2 * (step * WK + wk) + kq : step * WK + wk;
-            dma2_to_lds(srow[nb] + (g < G ? g : 0), stage + C::A_STAGE + C::B_STAGE + (wave * NB + nb) * 256);
+            dma2_to_lds(srow[nb] + (g < G - (kbeg >> 5) ? g : 0), stage + C::A_STAGE + C::B_STAGE + (wave * NB + nb) * 256);
         } else if ((q + 1) * C::NW <= C::BI) {
             dma(brsrc, GUARD && !whole && boffs + bpc[q] >= wrow ? kOut : boff[q], boffs, stage + C::A_STAGE + e * 1024);
         } else {
@@ -905,14 +905,22 @@ static int short_k(GemmTile t, bool int4, bool guard) {
     }
 }
 
+// us of `tiles` workgroups of t, `wgs` of them counted for the fill of the last round (the same number where nothing is split), k each
+static float tile_us(const TileCost &t, int64_t wgs, int k) {
+    const int64_t rounds = (wgs + 255) / 256;
+    const float fill = (float)(wgs - (rounds - 1) * 256) / 256.f, kk = (float)((k + t.ks - 1) / t.ks) * (float)t.ks;
+    const float a = t.s + ((float)(rounds - 1) + t.b + (1.f - t.b) * fill) * (t.c0 + t.c1 * kk / 4096.f);
+    return a * (1.f + t.q * a / (a + 100.f));
+}
+
+static int64_t tiles_of(const TileCost &t, int M, int N) { return (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn); }
+
 GemmTile gemm_tile_pick(int M, int N, int K, bool int4, bool guard) {
     GemmTile best = M <= 32 ? TILE_32x64 : TILE_64x64;
     if (M > 64) {
         float best_cost = 0.f;
         for (const TileCost &t : kCost[int4][guard]) {
-            const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), rounds = (tiles + 255) / 256;
-            const float fill = (float)(tiles - (rounds - 1) * 256) / 256.f, k = (float)((K + t.ks - 1) / t.ks) * (float)t.ks;
-            const float a = t.s + ((float)(rounds - 1) + t.b + (1.f - t.b) * fill) * (t.c0 + t.c1 * k / 4096.f), cost = a * (1.f + t.q * a / (a + 100.f));
+            const float cost = tile_us(t, tiles_of(t, M, N), K);
             if (best_cost == 0.f || cost < best_cost) {
                 best = t.tile;
                 best_cost = cost;
@@ -965,6 +973,91 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
     const bool k64 = tile == TILE_256x256 || tile == TILE_192x128 || tile == TILE_256x128;
     const int step = k256 ? 256 : k64 ? 64 : 128;  // k of a step
     return K % step ? launch_tile<false, true>(x, w, sc, y, M, N, K, tile, st) : launch_tile<false, false>(x, w, sc, y, M, N, K, tile, st);
+}
+
+// ---- few tiles and a long K: the product in parts of whole 256-k blocks, one fp32 matrix each, added by a second launch.  A workgroup's walk
+// through K is what such a product takes: 48 x 4096 x 14336 is 64 workgroups of 56 steps, 35 us.  us, in one part / in parts, the launch that adds
+// them included: int4 81 x 1280 x 14080 29.1 / 14.2 (six), 62 x 1536 x 11264 23.2 / 12.5 (eight), 26 x 5542 x 11776 21.6 / 15.2 (two), 46 x 6528 x 4928
+// 14.7 / 13.6 (two); int8 250 x 640 x 9760 25.3 / 13.3 (six), 152 x 1280 x 14336 30.0 / 18.0 (four), 235 x 768 x 4352 11.2 / 11.1 (five).  Of 120 random
+// products of 17 to 1200 rows 32 are split, none of them slower, the mean of all 9 % faster.  The model of gemm_tile_pick, with what the parts
+// cost on top, has to find 7 % in it.
+static const TileCost kCost32 = {TILE_32x64, 32, 64, 256, 1.9f, 2.2f, 7.6f, 0.75f, 0.f};
+
+int gemm_split_parts(int M, int N, int K, bool int4, bool guard, GemmTile *tile) {
+    constexpr float kSum = 2.5f, kMB = .3f;  // us of the second launch, of a MB of parts
+    constexpr int kMost = 8;
+    if (M < 17 || K < 1024 || K >= (1 << 22) || (int64_t)((M + 63) / 64) * ((N + 63) / 64) > 200) return 1;  // (what costs no time on the host)
+    float whole = 0.f, best = 0.f;
+    int parts = 1;
+    auto split = [&](const TileCost &t) {
+        const int64_t tiles = tiles_of(t, M, N);
+        const int blocks = (K + 255) / 256;
+        for (int s = 2; s <= kMost && s <= blocks; ++s) {
+            const int per = (blocks + s - 1) / s;
+            if ((blocks + per - 1) / per != s) continue;
+            // (tiles go to the XCDs in turn, each in all its parts)
+            const float us = tile_us(t, (tiles + 7) / 8 * 8 * s, per * 256) + kSum + kMB * 4e-6f * (float)M * (float)N * (float)s;
+            if (best == 0.f || us < best) {
+                best = us;
+                parts = s;
+                *tile = t.tile;
+            }
+        }
+    };
+    if (M <= 32) {
+        whole = tile_us(kCost32, tiles_of(kCost32, M, N), K);
+        split(kCost32);
+    } else {
+        for (const TileCost &t : kCost[int4][guard]) {
+            if (M <= 64 && t.tile != TILE_64x64) continue;
+            const float us = tile_us(t, tiles_of(t, M, N), K);
+            if (whole == 0.f || us < whole) whole = us;
+            if (t.tile == TILE_64x64 || t.tile == TILE_128x64) split(t);
+        }
+    }
+    return best != 0.f && best < .93f * whole ? parts : 1;
+}
+
+// y[m,n] = bf16(sum of the parts, in order, times the row scale of int8 weights); V columns per thread
+template <int V>
+__global__ __launch_bounds__(256) void gemm_sum_parts_kernel(const float *__restrict__ parts, const float *__restrict__ scale, uint16_t *__restrict__ y, int N,
+                                                             int64_t total, int np) {
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+    if (i >= total) return;
+    typedef float vec __attribute__((ext_vector_type(V)));
+    vec p[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+        if (s < np) p[s] = *reinterpret_cast<const vec *>(parts + s * total + i);
+    vec a = p[0];
+#pragma unroll
+    for (int s = 1; s < 8; ++s)
+        if (s < np) a += p[s];
+    if (scale) a *= *reinterpret_cast<const vec *>(scale + i % N);
+    if constexpr (V == 4) *reinterpret_cast<u32x2 *>(y + i) = u32x2{pack_bf16_rne(a[0], a[1]), pack_bf16_rne(a[2], a[3])};
+    else y[i] = (uint16_t)pack_bf16_rne(a[0], 0.f);
+}
+
+template <bool I4, bool GUARD>
+static int launch_parts(const uint16_t *x, const uint8_t *w, const void *sc, float *parts, int M, int N, int K, GemmTile tile, int np, hipStream_t st) {
+    switch (tile) {
+        case TILE_32x64: return tileq::launch<I4, 1, 2, 4, 1, 1, 64, 3, GUARD, false, tileq::EPI_F32>(x, w, sc, parts, M, N, K, np, st);
+        case TILE_64x64: return tileq::launch<I4, 1, 2, 4, 2, 1, 64, 3, GUARD, false, tileq::EPI_F32>(x, w, sc, parts, M, N, K, np, st);
+        default: return tileq::launch<I4, 1, 2, 4, 4, 1, 32, GUARD ? 3 : 4, GUARD, false, tileq::EPI_F32>(x, w, sc, parts, M, N, K, np, st);
+    }
+}
+
+int gemm_tile_parts_launch(const uint16_t *x, const uint8_t *w, const void *sc, uint16_t *y, int M, int N, int K, bool int4, bool guard, GemmTile tile, int np,
+                           float *parts, hipStream_t st) {
+    const int rc = int4 ? guard ? launch_parts<true, true>(x, w, sc, parts, M, N, K, tile, np, st) : launch_parts<true, false>(x, w, sc, parts, M, N, K, tile, np, st)
+                        : guard ? launch_parts<false, true>(x, w, sc, parts, M, N, K, tile, np, st) : launch_parts<false, false>(x, w, sc, parts, M, N, K, tile, np, st);
+    if (rc) return rc;
+    const int64_t total = (int64_t)M * N;
+    const float *const scale = int4 ? nullptr : reinterpret_cast<const float *>(sc);
+    const bool four = N % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 7u) == 0 && (int4 || aligned16(scale));
+    if (four) hipLaunchKernelGGL(gemm_sum_parts_kernel<4>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, st, parts, scale, y, N, total, np);
+    else hipLaunchKernelGGL(gemm_sum_parts_kernel<1>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, parts, scale, y, N, total, np);
+    return hip_check(hipGetLastError(), "gemm parts launch");
 }
 
 // ---- exact weights, K % 256 == 0: the projections of a prompt, whose tokens must come out as the decode step's do.

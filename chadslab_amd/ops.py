@@ -122,14 +122,18 @@ def qgemm(x: torch.Tensor, qw: QWeight, out: Optional[torch.Tensor] = None) -> t
     x = _dev(x, "x", torch.bfloat16)
     m = x.shape[0]
     y = _out(out, (m, qw.N), torch.bfloat16, x.device)
+    # scratch for the K parts of a product of few tiles (0 bytes where one part is the quicker form): a fresh one per call, as moe_ffn's
+    need = lib.chadq_gemm_bf16_workspace_bytes(m, qw.N, qw.K, int(isinstance(qw, QWeightInt8)))
+    ws = x.new_empty(need, dtype=torch.uint8) if need else None
+    ws_ptr = ws.data_ptr() if need else None
     if isinstance(qw, QWeightInt4G32):
         p, s = _dev(qw.packed, "packed", torch.uint8), _dev(qw.scale, "scale", torch.float16)
-        _lib.check(lib.chadq_gemm_i4g32_bf16(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, qw.N, qw.K,
-                                             _stream()), "chadq_gemm_i4g32_bf16")
+        _lib.check(lib.chadq_gemm_i4g32_bf16_ws(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, qw.N, qw.K, ws_ptr, need,
+                                                _stream()), "chadq_gemm_i4g32_bf16")
     elif isinstance(qw, QWeightInt8):
         w, s = _dev(qw.w, "w", torch.int8), _dev(qw.scale, "scale", torch.float32)
-        _lib.check(lib.chadq_gemm_i8row_bf16(x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, qw.N, qw.K,
-                                             _stream()), "chadq_gemm_i8row_bf16")
+        _lib.check(lib.chadq_gemm_i8row_bf16_ws(x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, qw.N, qw.K, ws_ptr, need,
+                                                _stream()), "chadq_gemm_i8row_bf16")
     else:
         raise TypeError("unknown weight container %r" % type(qw))
     return y

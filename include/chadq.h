@@ -162,6 +162,17 @@ int chadq_gemm_i4g32_bf16(const uint16_t *x_bf16, const uint8_t *wp, const uint1
 int chadq_gemm_i8row_bf16(const uint16_t *x_bf16, const int8_t *w8, const float *scale, uint16_t *y_bf16, int M,
                           int N, int K, void *stream);
 
+/*
+ * The same products with scratch memory on the device: where few tiles and a long K would leave most of the GPU idle, K is summed in up to
+ * eight parts (fp32 [parts, M, N] in `workspace`), which a second launch adds in order.  The bytes asked for are 0 where that does not pay;
+ * with a null workspace or fewer bytes the product is that of the functions above.  workspace 16-byte aligned; calls that overlap need one each.
+ */
+size_t chadq_gemm_bf16_workspace_bytes(int M, int N, int K, int int8_weights);
+int chadq_gemm_i4g32_bf16_ws(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, uint16_t *y_bf16, int M, int N, int K,
+                             void *workspace, size_t workspace_bytes, void *stream);
+int chadq_gemm_i8row_bf16_ws(const uint16_t *x_bf16, const int8_t *w8, const float *scale, uint16_t *y_bf16, int M, int N, int K,
+                             void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---- mixture-of-experts FFN (benchmark config 3) ---------------------------------------- */
 
 /*

@@ -136,3 +136,17 @@ def test_prompt_projections_are_rotated_where_they_are_written_unless_parts_pay(
     fn = _rule("_ZN5chadq19gemm_exact_qkv_paysEiii", ctypes.c_bool)  # (tokens, (hq + 2) * dh, d)
     assert fn(256, 2560, 2048) and fn(212, 2560, 1792) and fn(4, 1280, 512)          # us a prompt 2085 / 2134, 313 / 325, 203 / 208
     assert not fn(24, 2560, 2048) and not fn(35, 640, 1024) and not fn(7, 1536, 1536)  # 1088 / 1058, 283 / 277
+
+
+def test_gemm_is_summed_in_parts_where_few_tiles_walk_a_long_k():
+    lib = _lib.load()
+
+    def parts(m, n, k, int8=0):
+        return lib.chadq_gemm_bf16_workspace_bytes(m, n, k, int8) // (4 * m * n) or 1
+
+    # us in one part / in parts with the launch that adds them
+    for m, n, k, int8 in ((81, 1280, 14080, 0), (40, 1340, 10752, 0), (62, 1536, 11264, 0), (250, 640, 9760, 1), (152, 1280, 14336, 1), (48, 4096, 14336, 0), (26, 5542, 11776, 0)):
+        assert parts(m, n, k, int8) > 1, (m, n, k)  # 29.1 / 14.2, 22.6 / 11.4, 23.2 / 12.5, 25.3 / 13.3, 30.0 / 18.0, 35 / 17, 21.6 / 15.2
+    for m, n, k in ((48, 14336, 4096), (512, 4096, 4096), (1000, 4096, 14336), (4096, 14336, 4096), (48, 1024, 512), (16, 512, 16384), (33, 64, 1056), (48, 2048, 1 << 22)):
+        assert parts(m, n, k) == 1 and parts(m, n, k, 1) == 1, (m, n, k)
+    assert lib.chadq_gemm_bf16_workspace_bytes(0, 512, 4096, 0) == 0 and lib.chadq_gemm_bf16_workspace_bytes(17, -1, 4096, 1) == 0

@@ -1301,3 +1301,62 @@ def test_moe_ffn_tiled_refuses_mixed_and_unaligned_shapes(ops):
     x2 = torch.zeros(8, 288, dtype=torch.bfloat16, device=DEV)
     z1 = torch.zeros(8, 1, device=DEV)
     assert lib.chadq_moe_ffn_i4g32_tiled(x2.data_ptr(), z1.data_ptr(), arr, y.data_ptr(), 8, 288, 256, 1, 1, 1, ws.data_ptr(), need, None) == -2
+
+
+@pytest.mark.parametrize("m,n,k,shift", [(17, 512, 4096, 0), (32, 102, 8192, 0), (40, 257, 4128, 0), (48, 1024, 14336, 0), (64, 64, 4096, 1), (70, 513, 16384, 0), (100, 1000, 8160, 0),
+                                         (128, 2048, 8192, 1), (300, 1024, 16384, 0), (200, 512, 5152, 0)])
+def test_gemm_in_parts_of_k(ops, m, n, k, shift):
+    """Products of few tiles and a long K, summed in parts: ragged rows and columns (columns that no four divide, too), K that 256 does not divide,
+    parts of uneven length, scales that are not 16-byte aligned.  Weights rounded to bf16 in the reference as in the kernel: what is left
+    is the rounding of the result, 2^-9 at most per element."""
+    from chadslab_amd import QWeightInt4G32, QWeightInt8, _lib
+
+    lib = _lib.load()
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + n)
+    x = torch.randn(m, k, device=DEV, generator=g).bfloat16()
+    p = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+    s = torch.exp(torch.randn(n * (k // 32) + shift, device=DEV, generator=g) * 0.5 - 5.0).half()[shift:].view(n, k // 32)
+    w4 = ((torch.stack((p & 15, p >> 4), -1).reshape(n, k).float() - 8) * s.float().repeat_interleave(32, 1)).bfloat16().double()
+    w = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=DEV, generator=g)
+    s8 = torch.exp(torch.randn(n, device=DEV, generator=g) * 0.5 - 8.0)
+    stream = torch.cuda.current_stream().cuda_stream
+    for qw, ref, sc, name in ((QWeightInt4G32(p, s), x.double() @ w4.t(), s, "chadq_gemm_i4g32_bf16"),
+                              (QWeightInt8(w, s8), x.double() @ (w.double() * s8.double()[:, None]).t(), s8, "chadq_gemm_i8row_bf16")):
+        need = lib.chadq_gemm_bf16_workspace_bytes(m, n, k, int(sc is s8))
+        assert need >= 2 * 4 * m * n  # in parts
+        y = ops.qgemm(x, qw)
+        err = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+        assert float(err.max()) <= 2.0 ** -8, (name, float(err.max()))
+        # scratch of any content gives the same bits; none, or too little, the product in one part
+        wp = p if sc is s else w
+        scratch = torch.full((need,), 0xFF, dtype=torch.uint8, device=DEV)
+        got = [torch.empty_like(y) for _ in range(4)]
+        for out, ptr, size in ((got[0], scratch.data_ptr(), need), (got[1], None, 0), (got[2], scratch.data_ptr(), need // 2 - 16)):
+            assert getattr(lib, name + "_ws")(x.data_ptr(), wp.data_ptr(), sc.data_ptr(), out.data_ptr(), m, n, k, ptr, size, stream) == 0
+        assert getattr(lib, name)(x.data_ptr(), wp.data_ptr(), sc.data_ptr(), got[3].data_ptr(), m, n, k, stream) == 0
+        for a, b in ((got[0], y), (got[1], got[3])):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+        assert float((got[2].double() - ref).norm() / ref.norm()) <= 2.0 ** -8
+        assert getattr(lib, name + "_ws")(x.data_ptr(), wp.data_ptr(), sc.data_ptr(), got[0].data_ptr(), m, n, k, scratch.data_ptr() + 4, need, stream) == -3
+
+
+def test_gemm_in_parts_captured_in_a_graph(ops):
+    """A captured product in parts gives the eager bits on every replay, with other products in between."""
+    from chadslab_amd import QWeightInt8
+
+    g = torch.Generator(device=DEV)
+    g.manual_seed(5)
+    x = torch.randn(40, 8192, device=DEV, generator=g).bfloat16()
+    qw = QWeightInt8(torch.randint(-127, 128, (512, 8192), dtype=torch.int8, device=DEV, generator=g), torch.rand(512, device=DEV, generator=g) * 1e-3)
+    want = ops.qlinear(x, qw)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = ops.qlinear(x, qw)
+    for _ in range(4):
+        y.zero_()
+        graph.replay()
+        other = ops.qlinear(x + 1, qw)
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16)) and not torch.equal(other, want)

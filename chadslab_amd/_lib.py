@@ -36,6 +36,9 @@ SIGNATURES = {
     "chadq_gemv_i8row_fp32": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "chadq_gemm_i4g32_bf16": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "chadq_gemm_i8row_bf16": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
+    "chadq_gemv_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "chadq_gemv_i4g32_ws": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "chadq_gemv_i8row_ws": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "chadq_gemm_bf16_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "chadq_gemm_i4g32_bf16_ws": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "chadq_gemm_i8row_bf16_ws": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
@@ -119,6 +122,7 @@ def load() -> ctypes.CDLL:
 
 _NATIVE_ENTRIES = ("chadq_gemv_i4g32", "chadq_gemv_i4g32_bf16", "chadq_gemm_i4g32_bf16", "chadq_gemv_i8row", "chadq_gemv_i8row_bf16",
                    "chadq_gemm_i8row_bf16", "chadq_gemm_bf16_workspace_bytes", "chadq_gemm_i4g32_bf16_ws", "chadq_gemm_i8row_bf16_ws",
+                   "chadq_gemv_workspace_bytes", "chadq_gemv_i4g32_ws", "chadq_gemv_i8row_ws",
                    "chadq_moe_ffn_i4g32_workspace_bytes", "chadq_moe_ffn_i4g32", "chadq_moe_ffn_i4g32_tiled")
 
 

@@ -59,6 +59,10 @@ int gemv_i8row_dispatch(const float *, const int8_t *, const float *, float *, i
 int gemm_i4g32_bf16_dispatch(const uint16_t *, const uint8_t *, const uint16_t *, uint16_t *, int, int, int,
                              hipStream_t);
 size_t gemm_parts_bytes(int, int, int, bool);
+int gemv_i8row_parts(int, int, int, int *);
+int gemv_i8row_parts_launch(const float *, const int8_t *, const float *, float *, int, int, int, bool, int, int, double *, hipStream_t);
+int gemv_i4g32_parts(int, int, int, int *);
+int gemv_i4g32_parts_launch(const uint16_t *, const uint8_t *, const uint16_t *, float *, int, int, int, bool, int, int, float *, hipStream_t);
 int gemm_ws_dispatch(const uint16_t *, const uint8_t *, const void *, uint16_t *, int, int, int, bool, float *, size_t, hipStream_t);
 int gemm_i8row_bf16_dispatch(const uint16_t *, const int8_t *, const float *, uint16_t *, int, int, int,
                              hipStream_t);
@@ -284,6 +288,37 @@ int chadq_gemm_i8row_bf16(const uint16_t *x_bf16, const int8_t *w8, const float 
     CHADQ_REQUIRE(x_bf16 && w8 && scale && y_bf16, CHADQ_ERR_NULL, "chadq_gemm_i8row_bf16: null pointer");
     CHADQ_REQUIRE(aligned16(x_bf16) && aligned16(w8), CHADQ_ERR_ALIGN, "chadq_gemm_i8row_bf16: x and w8 must be 16-byte aligned");
     return gemm_i8row_bf16_dispatch(x_bf16, w8, scale, y_bf16, M, N, K, st);
+}
+
+size_t chadq_gemv_workspace_bytes(int M, int N, int K, int int8_weights) {
+    int span;
+    const int np = int8_weights ? gemv_i8row_parts(M, N, K, &span) : gemv_i4g32_parts(M, N, K, &span);
+    return np > 1 ? (size_t)np * M * N * (int8_weights ? 8 : 4) : 0;
+}
+
+int chadq_gemv_i4g32_ws(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, void *y, int M, int N, int K, int y_bf16, void *workspace,
+                        size_t workspace_bytes, void *stream) {
+    int span;
+    const int np = gemv_i4g32_parts(M, N, K, &span);
+    const bool parts = np > 1 && workspace && workspace_bytes >= (size_t)np * M * N * 4 && x_bf16 && wp && scale_f16 && y && aligned16(x_bf16) && aligned16(wp) &&
+                       aligned16(scale_f16) && (int64_t)N * (K / 2) < ((int64_t)1 << 31);
+    if (!parts) return y_bf16 ? chadq_gemv_i4g32_bf16(x_bf16, wp, scale_f16, reinterpret_cast<uint16_t *>(y), M, N, K, stream)
+                              : chadq_gemv_i4g32(x_bf16, wp, scale_f16, reinterpret_cast<float *>(y), M, N, K, stream);
+    ENTER();
+    CHADQ_REQUIRE(aligned16(workspace), CHADQ_ERR_ALIGN, "chadq_gemv_i4g32_ws: workspace must be 16-byte aligned");
+    return gemv_i4g32_parts_launch(x_bf16, wp, scale_f16, reinterpret_cast<float *>(y), M, N, K, y_bf16 != 0, np, span, reinterpret_cast<float *>(workspace), st);
+}
+
+int chadq_gemv_i8row_ws(const float *x, const int8_t *w8, const float *scale, void *y, int M, int N, int K, int y_bf16, void *workspace,
+                        size_t workspace_bytes, void *stream) {
+    int rws = 1;
+    const int np = gemv_i8row_parts(M, N, K, &rws);
+    const bool parts = np > 1 && workspace && workspace_bytes >= (size_t)np * M * N * 8 && x && w8 && scale && y && aligned16(x) && aligned16(w8);
+    if (!parts) return y_bf16 ? chadq_gemv_i8row_bf16(x, w8, scale, reinterpret_cast<uint16_t *>(y), M, N, K, stream)
+                              : chadq_gemv_i8row(x, w8, scale, reinterpret_cast<float *>(y), M, N, K, stream);
+    ENTER();
+    CHADQ_REQUIRE(aligned16(workspace), CHADQ_ERR_ALIGN, "chadq_gemv_i8row_ws: workspace must be 16-byte aligned");
+    return gemv_i8row_parts_launch(x, w8, scale, reinterpret_cast<float *>(y), M, N, K, y_bf16 != 0, np, rws, reinterpret_cast<double *>(workspace), st);
 }
 
 size_t chadq_gemm_bf16_workspace_bytes(int M, int N, int K, int int8_weights) { return gemm_parts_bytes(M, N, K, !int8_weights); }

@@ -489,14 +489,16 @@ struct GemvPairCfg {
 template <int MT, int S, int RBW, int D, int KC>
 __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(S == 16 ? 2 : 4))) void gemv_i4g32_mfma_pair_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wp, const uint16_t *__restrict__ sc,
-    float *__restrict__ y, int N, int K, int pvf) {
+    float *__restrict__ y, int N, int K, int pvf, int kspan) {
     const int pv = pvf & 0xFF;
     const bool bf16_out = pvf & kPvBf16Out;
     typedef GemvPairCfg<S, RBW, KC> C;
+    const int kbeg = blockIdx.y * kspan, kend = (kbeg + kspan < K) ? kbeg + kspan : K;  // (as in the kernel above)
     constexpr int M = MT, P = C::P, MR = C::MR, KS = C::KS, T = C::T, XI = C::XI;
     static_assert(M >= 1 && M <= MR, "eight rows of A per scale group");
     // S = 16: one 8-wave workgroup per compute unit (its LDS), so a wave may use 256 registers
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    y += (size_t)blockIdx.y * M * N;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int unit = wave >> 2, wv = wave & 3;
     const int rbs = wv / KS, ks = wv % KS;
@@ -530,7 +532,7 @@ __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(S == 
     u32x4 xr[XI];
     u32x4 sv[C::SC_NL];
     u32x4 w[S];
-    int kc0 = 0;
+    int kc0 = kbeg;
     auto issue_w = [&](int i) {
         const int gg = (kc0 >> 5) + (S * ks + i) * 4 + j;
         w[i] = load_nt_b128(wp + (wrow + (uint32_t)(gg < G ? gg : 0) * 16u));
@@ -633,7 +635,7 @@ __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(S == 
             a_addr += a_step;
         }
         kc0 += KC;
-        if (kc0 >= K) break;
+        if (kc0 >= kend) break;
         request();
     }
 
@@ -698,12 +700,14 @@ template <int S, int RBW, int D, int KC>
 // (two waves per SIMD at most: a workgroup's operands take 68 KB or more of LDS, so a wave may use 256 registers)
 __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(2))) void gemv_i4g32_mfma_rows16_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wp, const uint16_t *__restrict__ sc,
-    float *__restrict__ y, int M, int N, int K, int pvf) {
+    float *__restrict__ y, int M, int N, int K, int pvf, int kspan) {
     const int pv = pvf & 0xFF;
     const bool bf16_out = pvf & kPvBf16Out;
     typedef GemvRows16Cfg<S, RBW, KC> C;
     constexpr int P = C::P, KS = C::KS, T = C::T, XI = C::XI;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int kbeg = blockIdx.y * kspan, kend = (kbeg + kspan < K) ? kbeg + kspan : K;  // (as in the kernels above)
+    y += (size_t)blockIdx.y * M * N;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int unit = wave >> 2, wv = wave & 3;
     const int rbs = wv / KS, ks = wv % KS;
@@ -725,7 +729,7 @@ __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(2))) 
     u32x4 xr[XI];
     u32x4 sv[C::SC_NL];
     u32x4 w[S];
-    int kc0 = 0;
+    int kc0 = kbeg;
     auto issue_w = [&](int i) {
         const int gg = (kc0 >> 5) + (S * ks + i) * 4 + j;
         w[i] = load_nt_b128(wp + (wrow + (uint32_t)(gg < G ? gg : 0) * 16u));
@@ -824,7 +828,7 @@ __global__ __launch_bounds__(256 * RBW) __attribute__((amdgpu_waves_per_eu(2))) 
             a_addr += a_step;
         }
         kc0 += KC;
-        if (kc0 >= K) break;
+        if (kc0 >= kend) break;
         request();
     }
 
@@ -886,7 +890,7 @@ static int pick_tile_rows(int N, int P, int tiles_per_wg, int ksplit) {
 
 template <int MT, int HP, int S, int RBW, int D, int KC = 4096, int XM = 0, int YM = 0, int D0 = D>
 static int launch_mfma(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int N, int K,
-                       hipStream_t st, int ksplit = 1, GemvPre pre = GemvPre{}, int *workgroups = nullptr, bool bf16_out = false) {
+                       hipStream_t st, int ksplit = 1, GemvPre pre = GemvPre{}, int *workgroups = nullptr, bool bf16_out = false, int kspan = 0) {
     typedef GemvCfg<MT, HP, S, RBW, KC> C;
     static std::atomic<bool> attr_set{false};  // setting it twice from two threads is harmless
     if (!attr_set.load(std::memory_order_acquire)) {
@@ -902,13 +906,14 @@ static int launch_mfma(const uint16_t *x, const uint8_t *wp, const uint16_t *sc,
     if (workgroups) *workgroups = (tiles + tiles_per_wg - 1) / tiles_per_wg;
     if (workgroups && !wp) return 0;  // asked for the grid only
     hipLaunchKernelGGL((gemv_i4g32_mfma_kernel<MT, HP, S, RBW, D, KC, XM, YM, D0>), dim3((tiles + tiles_per_wg - 1) / tiles_per_wg, ksplit),
-                       dim3(256 * RBW), C::TOTAL, st, wp, sc, a0, pre.delta, pre.w, N, K, pv | (pre.n << 8) | (bf16_out ? kPvBf16Out : 0), K / ksplit, y, pre.res_out,
+                       dim3(256 * RBW), C::TOTAL, st, wp, sc, a0, pre.delta, pre.w, N, K, pv | (pre.n << 8) | (bf16_out ? kPvBf16Out : 0), kspan ? kspan : K / ksplit, y, pre.res_out,
                        pre.eps);
     return hip_check(hipGetLastError(), "gemv_i4g32_mfma launch");
 }
 
 template <int MT, int S, int RBW, int D, int KC = 4096>
-static int launch_pair(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int N, int K, hipStream_t st, bool bf16_out) {
+static int launch_pair(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int N, int K, hipStream_t st, bool bf16_out, int np = 1,
+                       int kspan = 0) {
     typedef GemvPairCfg<S, RBW, KC> C;
     static std::atomic<bool> attr_set{false};
     if (!attr_set.load(std::memory_order_acquire)) {
@@ -917,16 +922,16 @@ static int launch_pair(const uint16_t *x, const uint8_t *wp, const uint16_t *sc,
         attr_set.store(true, std::memory_order_release);
     }
     const int tiles_per_wg = 4 / C::KS * RBW;
-    const int pv = pick_tile_rows(N, C::P, tiles_per_wg, 1);
+    const int pv = pick_tile_rows(N, C::P, tiles_per_wg, np);
     const int tiles = (N + pv - 1) / pv;
-    hipLaunchKernelGGL((gemv_i4g32_mfma_pair_kernel<MT, S, RBW, D, KC>), dim3((tiles + tiles_per_wg - 1) / tiles_per_wg), dim3(256 * RBW),
-                       C::TOTAL, st, x, wp, sc, y, N, K, pv | (bf16_out ? kPvBf16Out : 0));
+    hipLaunchKernelGGL((gemv_i4g32_mfma_pair_kernel<MT, S, RBW, D, KC>), dim3((tiles + tiles_per_wg - 1) / tiles_per_wg, np), dim3(256 * RBW),
+                       C::TOTAL, st, x, wp, sc, y, N, K, pv | (bf16_out ? kPvBf16Out : 0), np > 1 ? kspan : K);
     return hip_check(hipGetLastError(), "gemv_i4g32_mfma_pair launch");
 }
 
 template <int S, int RBW, int D, int KC = 2048>
 static int launch_rows16(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, hipStream_t st,
-                         bool bf16_out) {
+                         bool bf16_out, int np = 1, int kspan = 0) {
     typedef GemvRows16Cfg<S, RBW, KC> C;
     static std::atomic<bool> attr_set{false};
     if (!attr_set.load(std::memory_order_acquire)) {
@@ -935,10 +940,10 @@ static int launch_rows16(const uint16_t *x, const uint8_t *wp, const uint16_t *s
         attr_set.store(true, std::memory_order_release);
     }
     const int tiles_per_wg = 4 / C::KS * RBW;
-    const int pv = pick_tile_rows(N, C::P, tiles_per_wg, 1);
+    const int pv = pick_tile_rows(N, C::P, tiles_per_wg, np);
     const int tiles = (N + pv - 1) / pv;
-    hipLaunchKernelGGL((gemv_i4g32_mfma_rows16_kernel<S, RBW, D, KC>), dim3((tiles + tiles_per_wg - 1) / tiles_per_wg), dim3(256 * RBW),
-                       C::TOTAL, st, x, wp, sc, y, M, N, K, pv | (bf16_out ? kPvBf16Out : 0));
+    hipLaunchKernelGGL((gemv_i4g32_mfma_rows16_kernel<S, RBW, D, KC>), dim3((tiles + tiles_per_wg - 1) / tiles_per_wg, np), dim3(256 * RBW),
+                       C::TOTAL, st, x, wp, sc, y, M, N, K, pv | (bf16_out ? kPvBf16Out : 0), np > 1 ? kspan : K);
     return hip_check(hipGetLastError(), "gemv_i4g32_mfma_rows16 launch");
 }
 
@@ -994,6 +999,40 @@ int gemv_i4g32_mfma_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_
         if (rc != 0) return rc;
     }
     return 0;
+}
+
+// Parts of K, fp32 sums, for few weight rows and a long K, as gemv_i8row_parts has them for int8 weights.  us, in one part / in parts, 512 x 16384: 1 row
+// 10.6 / 7.0, 4 10.3 / 7.4, 8 17.8 / 8.3, 16 23.0 / 7.6; 2048 x 8192, 8 rows 10.1 / 8.4, 16 12.8 / 9.9; 256 x 5120, 6 rows 8.6 / 7.3.
+int gemv_i4g32_parts(int M, int N, int K, int *span) {
+    const int chunk = M <= 8 ? 4096 : 2048;  // what the kernels take between two barriers
+    *span = K;
+    if (M < 1 || M > 16 || N < 1 || N > 2048 || K < 1 || K % 256 != 0) return 1;
+    const int wgs = (N + 15) / 16, blocks = (K + chunk - 1) / chunk;
+    int s = 256 / wgs < 8 ? 256 / wgs : 8;
+    s = s < blocks ? s : blocks;
+    const int per = (blocks + s - 1) / s, np = (blocks + per - 1) / per;
+    *span = per * chunk;
+    return (float)(blocks - per) * (M <= 4 ? 2.2f : M <= 8 ? 3.9f : 2.6f) > 3.5f ? np : 1;
+}
+
+int gemv_sum_parts_launch(const float *parts, float *y, int M, int N, int np, bool bf16_out, hipStream_t st);
+
+// (K % 256 == 0 and 16-byte aligned scale rows)
+int gemv_i4g32_parts_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, bool bf16_out, int np, int span,
+                            float *parts, hipStream_t st) {
+    int rc;
+    switch (M) {
+        case 1: rc = launch_mfma<1, 4, 8, 1, 3>(x, wp, sc, parts, N, K, st, np, GemvPre{}, nullptr, false, span); break;
+        case 2: rc = launch_mfma<2, 2, 8, 1, 2>(x, wp, sc, parts, N, K, st, np, GemvPre{}, nullptr, false, span); break;
+        case 3: rc = launch_mfma<3, 1, 8, 1, 8>(x, wp, sc, parts, N, K, st, np, GemvPre{}, nullptr, false, span); break;
+        case 4: rc = launch_mfma<4, 1, 8, 1, 8>(x, wp, sc, parts, N, K, st, np, GemvPre{}, nullptr, false, span); break;
+        case 5: rc = launch_pair<5, 8, 2, 3>(x, wp, sc, parts, N, K, st, false, np, span); break;
+        case 6: rc = launch_pair<6, 8, 2, 3>(x, wp, sc, parts, N, K, st, false, np, span); break;
+        case 7: rc = launch_pair<7, 8, 2, 3>(x, wp, sc, parts, N, K, st, false, np, span); break;
+        case 8: rc = launch_pair<8, 8, 2, 3>(x, wp, sc, parts, N, K, st, false, np, span); break;
+        default: rc = launch_rows16<4, 1, 4>(x, wp, sc, parts, M, N, K, st, false, np, span); break;
+    }
+    return rc ? rc : gemv_sum_parts_launch(parts, y, M, N, np, bf16_out, st);
 }
 
 // y = W x (M = 1) with the per-workgroup argmax candidates of y written beside it (YM = 2 above).  Only the shape of a

@@ -42,6 +42,8 @@
 
 namespace chadq {
 
+constexpr int kGemvMostParts = 8;
+
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 
 // RWS: blocks of 16 weight rows per workgroup (1, 2 or 4), each shared by 8 / RWS waves
@@ -70,7 +72,7 @@ __device__ __forceinline__ int half_row_merge(uint32_t old, uint32_t src) {
 template <int SETS, int RWS>
 __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__restrict__ x, const int8_t *w8,
                                                               const float *sc, float *__restrict__ y, int M, int N,
-                                                              int K, int bf16_out) {
+                                                              int K, int bf16_out, int per, double *__restrict__ parts) {
     using C = GemvI8Cfg<SETS, RWS>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint32_t *amax = reinterpret_cast<uint32_t *>(smem + C::AMAX_OFF);
@@ -85,6 +87,7 @@ __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__res
     const unsigned char *wbase = reinterpret_cast<const unsigned char *>(w8) + 16 * ((c >> 3) + 2 * g);
     const unsigned char *wpx = wbase + (size_t)rx * K, *wpy = wbase + (size_t)ry * K;
     const int pairs = K >> 7, supers = (K + 2047) >> 11;
+    const int sr0 = blockIdx.y * per, sr1 = sr0 + per < supers ? sr0 + per : supers;  // the workgroup's blocks of 2048 k
     auto pair_off = [&](int sr, int t) {  // byte offset of pair-step t of this wave in 2048-block sr
         const int p = sr * 16 + kh * C::STEPS + t;
         return (size_t)((p < pairs) ? p : pairs - 1) * 128;
@@ -189,19 +192,19 @@ __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__res
         }
     };
 
-    request_x(0);
+    request_x(sr0);
     u32x4 ring[2 * C::STEPS];
 #pragma unroll
     for (int t = 0; t < C::STEPS; ++t) {
-        ring[2 * t] = load_nt_b128(wpx + pair_off(0, t));
-        ring[2 * t + 1] = load_nt_b128(wpy + pair_off(0, t));
+        ring[2 * t] = load_nt_b128(wpx + pair_off(sr0, t));
+        ring[2 * t + 1] = load_nt_b128(wpy + pair_off(sr0, t));
     }
     // the weight stream starts before the staging below waits for anything (w8 and sc are not declared restrict so
     // that these loads cannot be moved below this point)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    stage_x(0);
-    if (supers > 1) request_x(1);
+    stage_x(sr0);
+    if (sr0 + 1 < sr1) request_x(sr0 + 1);
     __syncthreads();
 
     double yacc[C::RES];
@@ -254,14 +257,14 @@ __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__res
             }
         }
     };
-    for (int sr = 0; sr + 1 < supers; ++sr) {
+    for (int sr = sr0; sr + 1 < sr1; ++sr) {
         multiply(sr, std::true_type{});
         __syncthreads();  // every wave is done with this block's operands and row maxima
         stage_x(sr + 1);
-        request_x(sr + 2 < supers ? sr + 2 : supers - 1);
+        request_x(sr + 2 < sr1 ? sr + 2 : sr1 - 1);
         __syncthreads();
     }
-    multiply(supers - 1, std::false_type{});
+    multiply(sr1 - 1, std::false_type{});
 
     // the other waves of the row block hand their sums over
     double *const fold = reinterpret_cast<double *>(smem + C::FOLD_OFF) + rw * C::RES * 64 + lane;
@@ -280,14 +283,18 @@ __global__ __launch_bounds__(512) void gemv_i8row_mfma_kernel(const float *__res
 #pragma unroll
     for (int r = 0; r < C::RES; ++r) {
         const int m = (SETS == 3) ? 4 * g + r : 4 * r + g;
-        if (m < M && n < N) store_sum(y, (size_t)m * N + n, (float)yacc[r] * scale, bf16_out);
+        if (m < M && n < N) {
+            if (parts) parts[((size_t)blockIdx.y * M + m) * N + n] = yacc[r];
+            else store_sum(y, (size_t)m * N + n, (float)yacc[r] * scale, bf16_out);
+        }
     }
 }
 
 bool gemv_i8row_mfma_ok(int M, int K) { return M >= 1 && M <= 16 && K % 128 == 0; }
 
 template <int SETS, int RWS>
-static int launch_i8_mfma(const float *x, const int8_t *w8, const float *sc, float *y, int M, int N, int K, bool bf16_out, hipStream_t st) {
+static int launch_i8_mfma(const float *x, const int8_t *w8, const float *sc, float *y, int M, int N, int K, bool bf16_out, hipStream_t st, int np = 1,
+                          double *parts = nullptr) {
     using C = GemvI8Cfg<SETS, RWS>;
     static std::atomic<bool> attr_set{false};  // setting it twice from two threads is harmless
     if (!attr_set.load(std::memory_order_acquire)) {
@@ -295,8 +302,8 @@ static int launch_i8_mfma(const float *x, const int8_t *w8, const float *sc, flo
                                       hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS));
         attr_set.store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL((gemv_i8row_mfma_kernel<SETS, RWS>), dim3((N + 16 * RWS - 1) / (16 * RWS)), dim3(512), C::LDS, st, x, w8, sc, y, M, N, K,
-                       (int)bf16_out);
+    hipLaunchKernelGGL((gemv_i8row_mfma_kernel<SETS, RWS>), dim3((N + 16 * RWS - 1) / (16 * RWS), np), dim3(512), C::LDS, st, x, w8, sc, y, M, N, K,
+                       (int)bf16_out, ((K + 2047) / 2048 + np - 1) / np, parts);
     return hip_check(hipGetLastError(), "gemv_i8row_mfma launch");
 }
 
@@ -313,6 +320,73 @@ int gemv_i8row_mfma_launch(const float *x, const int8_t *w8, const float *sc, fl
     if (M <= 4) return launch_i8_mfma<1>(x, w8, sc, y, M, N, K, bf16_out, st);
     if (M <= 8) return launch_i8_mfma<2>(x, w8, sc, y, M, N, K, bf16_out, st);
     return launch_i8_mfma<3>(x, w8, sc, y, M, N, K, bf16_out, st);
+}
+
+// y[m,n] = the parts of an element added in order, times its row's scale if there is one, rounded once
+template <typename T>
+__global__ __launch_bounds__(256) void gemv_sum_parts_kernel(const T *__restrict__ parts, const float *__restrict__ scale, float *__restrict__ y, int N, int total,
+                                                             int np, int bf16_out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= total) return;
+    T p[kGemvMostParts];
+#pragma unroll
+    for (int s = 0; s < kGemvMostParts; ++s)
+        if (s < np) p[s] = parts[(size_t)s * total + i];
+    T a = p[0];
+#pragma unroll
+    for (int s = 1; s < kGemvMostParts; ++s)
+        if (s < np) a += p[s];
+    store_sum(y, i, scale ? (float)a * scale[i % N] : (float)a, bf16_out);
+}
+
+int gemv_sum_parts_launch(const float *parts, float *y, int M, int N, int np, bool bf16_out, hipStream_t st) {
+    hipLaunchKernelGGL(gemv_sum_parts_kernel<float>, dim3((M * N + 255) / 256), dim3(256), 0, st, parts, nullptr, y, N, M * N, np, (int)bf16_out);
+    return hip_check(hipGetLastError(), "gemv parts launch");
+}
+
+// Parts of K (float64 sums, so the result is as precise as in one part) and the blocks of 16 weight rows of a workgroup that go with them, where
+// workgroups would walk many blocks of 2048 k.  A block takes a workgroup a share for its activations' way to LDS (by rows) and one for its weights (by
+// their rows, and less while compute units idle); few weight rows want more workgroups along K, many activation rows also fewer that stage them: 64
+// weight rows each instead of 16 or 32.  The second launch and what goes with it take 3.5 us.  us, in one part / in parts: 512 x 16384, 1 row 13.2 /
+// 6.9, 4 16.7 / 7.2, 8 25.8 / 8.3, 16 47.2 / 10.2; 2048 x 8192, 8 rows 15.4 / 9.3; 4096 x 16384, 16 48.0 / 29.1; 8192 x 8192, 16 35.3 / 28.3.
+int gemv_i8row_parts(int M, int N, int K, int *rws) {
+    if (!gemv_i8row_mfma_ok(M, K) || N < 1 || N > 8192) return 1;
+    const float stage = M <= 4 ? .8f : M <= 8 ? 1.9f : 4.2f, rows = M <= 4 ? 1.4f : M <= 8 ? 1.5f : 1.45f;
+    const int blocks = (K + 2047) / 2048;
+    auto block_us = [&](int r, int wgs) { return stage + rows * (float)r * (.4f + .6f * (float)(wgs < 256 ? wgs : 256) / 256.f); };
+    const int now = N <= 4096 ? 1 : 2;
+    float best = (float)blocks * block_us(now, (N + 16 * now - 1) / (16 * now)) - 3.5f;
+    int parts = 1;
+    for (int r = 1; r <= 4; r *= 2) {
+        const int wgs = (N + 16 * r - 1) / (16 * r);
+        for (int s = 2; s <= kGemvMostParts && s <= blocks && wgs * s <= 256; ++s) {
+            const int per = (blocks + s - 1) / s;
+            const float us = (float)per * block_us(r, wgs * s);
+            if ((blocks + per - 1) / per == s && us < best) {
+                best = us;
+                parts = s;
+                *rws = r;
+            }
+        }
+    }
+    return parts;
+}
+
+template <int SETS>
+static int launch_i8_parts(const float *x, const int8_t *w8, const float *sc, float *y, int M, int N, int K, int np, int rws, double *parts, hipStream_t st) {
+    return rws == 1   ? launch_i8_mfma<SETS, 1>(x, w8, sc, y, M, N, K, false, st, np, parts)
+           : rws == 2 ? launch_i8_mfma<SETS, 2>(x, w8, sc, y, M, N, K, false, st, np, parts)
+                      : launch_i8_mfma<SETS, 4>(x, w8, sc, y, M, N, K, false, st, np, parts);
+}
+
+int gemv_i8row_parts_launch(const float *x, const int8_t *w8, const float *sc, float *y, int M, int N, int K, bool bf16_out, int np, int rws,
+                            double *parts, hipStream_t st) {
+    const int rc = M <= 4   ? launch_i8_parts<1>(x, w8, sc, y, M, N, K, np, rws, parts, st)
+                   : M <= 8 ? launch_i8_parts<2>(x, w8, sc, y, M, N, K, np, rws, parts, st)
+                            : launch_i8_parts<3>(x, w8, sc, y, M, N, K, np, rws, parts, st);
+    if (rc) return rc;
+    hipLaunchKernelGGL(gemv_sum_parts_kernel<double>, dim3((M * N + 255) / 256), dim3(256), 0, st, parts, sc, y, N, M * N, np, (int)bf16_out);
+    return hip_check(hipGetLastError(), "gemv parts launch");
 }
 
 }  // namespace chadq

@@ -22,13 +22,14 @@ namespace {
 typedef int (*product_fn)(const void *, const void *, const void *, void *, int, int, int, void *);
 typedef size_t (*product_bytes_fn)(int, int, int, int);
 typedef int (*product_ws_fn)(const void *, const void *, const void *, void *, int, int, int, void *, size_t, void *);
+typedef int (*decode_ws_fn)(const void *, const void *, const void *, void *, int, int, int, int, void *, size_t, void *);
 typedef size_t (*moe_bytes_fn)(int, int, int, int, int);
 typedef int (*moe_fn)(const void *, const void *, const chadq_moe_expert_i4g32 *, void *, int, int, int, int, int, int, void *, size_t, void *);
 
-enum Entry { GEMV_I4, GEMV_I4_BF16, GEMM_I4, GEMV_I8, GEMV_I8_BF16, GEMM_I8, GEMM_BYTES, GEMM_I4_WS, GEMM_I8_WS, MOE_BYTES, MOE_ROWS, MOE_TILES, ENTRIES };
+enum Entry { GEMV_I4, GEMV_I4_BF16, GEMM_I4, GEMV_I8, GEMV_I8_BF16, GEMM_I8, GEMM_BYTES, GEMM_I4_WS, GEMM_I8_WS, GEMV_BYTES, GEMV_I4_WS, GEMV_I8_WS, MOE_BYTES, MOE_ROWS, MOE_TILES, ENTRIES };
 const char *const kEntryNames[ENTRIES] = {"chadq_gemv_i4g32", "chadq_gemv_i4g32_bf16", "chadq_gemm_i4g32_bf16", "chadq_gemv_i8row", "chadq_gemv_i8row_bf16",
                                           "chadq_gemm_i8row_bf16", "chadq_gemm_bf16_workspace_bytes", "chadq_gemm_i4g32_bf16", "chadq_gemm_i8row_bf16",
-                                          "chadq_moe_ffn_i4g32_workspace_bytes", "chadq_moe_ffn_i4g32",
+                                          "chadq_gemv_workspace_bytes", "chadq_gemv_i4g32", "chadq_gemv_i8row", "chadq_moe_ffn_i4g32_workspace_bytes", "chadq_moe_ffn_i4g32",
                                           "chadq_moe_ffn_i4g32_tiled"};
 void *g_entry[ENTRIES];                                // of the library in use (bind)
 PyObject *g_int4 = nullptr, *g_int8 = nullptr, *g_tiles = nullptr;  // the weight containers
@@ -103,8 +104,8 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     const Entry e = !gemv ? (int4 ? GEMM_I4 : GEMM_I8) : y_type == at::kFloat ? (int4 ? GEMV_I4 : GEMV_I8) : (int4 ? GEMV_I4_BF16 : GEMV_I8_BF16);
     const at::Tensor keep[3] = {*x, *w, *s};  // whatever another thread does with the objects
     const product_fn fn = reinterpret_cast<product_fn>(g_entry[e]);
-    // scratch for the K parts of a product of few tiles; 0: one part is the quicker form
-    const size_t need = gemv ? 0 : reinterpret_cast<product_bytes_fn>(g_entry[GEMM_BYTES])((int)m, (int)n, (int)k, !int4);
+    // scratch for the K parts of a product that would leave most of the GPU idle; 0: one part is the quicker form
+    const size_t need = reinterpret_cast<product_bytes_fn>(g_entry[gemv ? GEMV_BYTES : GEMM_BYTES])((int)m, (int)n, (int)k, !int4);
     at::Tensor y, ws;
     int rc;
     {
@@ -112,6 +113,10 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
         if (need) ws = at::empty({(int64_t)need}, keep[0].options().dtype(at::kByte).requires_grad(false));
         y = at::empty({m, n}, keep[0].options().dtype(y_type).requires_grad(false));
         if (!y.unsafeGetTensorImpl()->has_storage() || (need && !ws.unsafeGetTensorImpl()->has_storage())) rc = CHADQ_ERR_NULL;
+        else if (need && gemv)
+            rc = reinterpret_cast<decode_ws_fn>(g_entry[int4 ? GEMV_I4_WS : GEMV_I8_WS])(
+                keep[0].const_data_ptr(), keep[1].const_data_ptr(), keep[2].const_data_ptr(), y.mutable_data_ptr(), (int)m, (int)n, (int)k,
+                y_type == at::kBFloat16, ws.mutable_data_ptr(), need, c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream());
         else if (need)
             rc = reinterpret_cast<product_ws_fn>(g_entry[int4 ? GEMM_I4_WS : GEMM_I8_WS])(
                 keep[0].const_data_ptr(), keep[1].const_data_ptr(), keep[2].const_data_ptr(), y.mutable_data_ptr(), (int)m, (int)n, (int)k,

@@ -102,6 +102,12 @@ def _gemv(x: torch.Tensor, qw: QWeight, out: Optional[torch.Tensor], fp32_elemen
         p, s = _dev(qw.packed, "packed", torch.uint8), _dev(qw.scale, "scale", torch.float16)
         y = _out(out, (m, n), y_dtype, x.device)
         name = "chadq_gemv_i4g32_bf16" if bf16_out else "chadq_gemv_i4g32"
+        need = lib.chadq_gemv_workspace_bytes(m, n, k, 0)  # as in qgemm
+        if need:
+            ws = x.new_empty(need, dtype=torch.uint8)
+            _lib.check(lib.chadq_gemv_i4g32_ws(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, int(bf16_out), ws.data_ptr(), need,
+                                               _stream()), name)
+            return y
         _lib.check(getattr(lib, name)(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, _stream()), name)
         return y
     if isinstance(qw, QWeightInt8):
@@ -109,6 +115,12 @@ def _gemv(x: torch.Tensor, qw: QWeight, out: Optional[torch.Tensor], fp32_elemen
         w, s = _dev(qw.w, "w", torch.int8), _dev(qw.scale, "scale", torch.float32)
         y = _out(out, (m, n), y_dtype, x.device)
         name = "chadq_gemv_i8row_fp32" if fp32_elements else "chadq_gemv_i8row_bf16" if bf16_out else "chadq_gemv_i8row"
+        need = 0 if fp32_elements else lib.chadq_gemv_workspace_bytes(m, n, k, 1)
+        if need:
+            ws = x.new_empty(need, dtype=torch.uint8)
+            _lib.check(lib.chadq_gemv_i8row_ws(x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, int(bf16_out), ws.data_ptr(), need,
+                                               _stream()), name)
+            return y
         _lib.check(getattr(lib, name)(x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, _stream()), name)
         return y
     raise TypeError("unknown weight container %r" % type(qw))

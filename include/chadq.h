@@ -149,6 +149,17 @@ int chadq_gemv_i8row_bf16(const float *x, const int8_t *w8, const float *scale, 
 int chadq_gemv_i8row_fp32(const float *x, const int8_t *w8, const float *scale, float *y, int M, int N, int K,
                           void *stream);
 
+/*
+ * The decode products with scratch memory: few weight rows and a long K are summed in up to eight parts of K in `workspace`, which a second
+ * launch adds in order (int8: in float64, so that nothing is lost; int4: in fp32, as inside a part).  The bytes asked for are 0 where that does not
+ * pay; with a null workspace or fewer bytes these are chadq_gemv_i4g32 and chadq_gemv_i8row, or their _bf16 forms (y_bf16).
+ */
+size_t chadq_gemv_workspace_bytes(int M, int N, int K, int int8_weights);
+int chadq_gemv_i4g32_ws(const uint16_t *x_bf16, const uint8_t *wp, const uint16_t *scale_f16, void *y, int M, int N, int K, int y_bf16,
+                        void *workspace, size_t workspace_bytes, void *stream);
+int chadq_gemv_i8row_ws(const float *x, const int8_t *w8, const float *scale, void *y, int M, int N, int K, int y_bf16, void *workspace,
+                        size_t workspace_bytes, void *stream);
+
 /* ---- prefill dequant-GEMM (benchmark config 2) ---------------------------------------- */
 
 /*

@@ -146,7 +146,25 @@ def test_gemm_is_summed_in_parts_where_few_tiles_walk_a_long_k():
 
     # us in one part / in parts with the launch that adds them
     for m, n, k, int8 in ((81, 1280, 14080, 0), (40, 1340, 10752, 0), (62, 1536, 11264, 0), (250, 640, 9760, 1), (152, 1280, 14336, 1), (48, 4096, 14336, 0), (26, 5542, 11776, 0)):
-        assert parts(m, n, k, int8) > 1, (m, n, k)  # 29.1 / 14.2, 22.6 / 11.4, 23.2 / 12.5, 25.3 / 13.3, 30.0 / 18.0, 35 / 17, 21.6 / 15.2
+        assert parts(m, n, k, int8) > 1, (m, n, k)  # 29.1 / 14.2, 22.6 / 11.4, 23.2 / 12.5, 25.3 / 13.3, 30.0 / 18.0, 35 / 15.7, 21.6 / 15.2
     for m, n, k in ((48, 14336, 4096), (512, 4096, 4096), (1000, 4096, 14336), (4096, 14336, 4096), (48, 1024, 512), (16, 512, 16384), (33, 64, 1056), (48, 2048, 1 << 22)):
         assert parts(m, n, k) == 1 and parts(m, n, k, 1) == 1, (m, n, k)
     assert lib.chadq_gemm_bf16_workspace_bytes(0, 512, 4096, 0) == 0 and lib.chadq_gemm_bf16_workspace_bytes(17, -1, 4096, 1) == 0
+
+
+def test_gemv_is_summed_in_parts_where_few_rows_walk_a_long_k():
+    lib = _lib.load()
+
+    def parts(m, n, k, int8):
+        return lib.chadq_gemv_workspace_bytes(m, n, k, int8) // ((8 if int8 else 4) * m * n) or 1
+
+    for int8 in (0, 1):
+        for m in (1, 4, 8, 16):
+            assert parts(m, 512, 16384, int8) > 1 and parts(m, 2048, 2048, int8) == 1 and parts(m, 16384, 16384, int8) == 1 and parts(m, 512, 4064, int8) == 1
+            for n in (1, 16, 100, 512, 1000, 2048):
+                for k in (128, 256, 4096, 6400, 8192, 16384, 65536):
+                    assert 1 <= parts(m, n, k, int8) <= 8
+    # int8, us in one part / in parts: 6.6 / 7.8, 48.0 / 29.1, 20.3 / 22.2
+    assert parts(1, 512, 6144, 1) == 1 and parts(16, 4096, 16384, 1) == 4 and parts(12, 6144, 6144, 1) == 1
+    assert parts(1, 14336, 4096, 0) == 1 and parts(1, 16384, 2048, 1) == 1 and parts(6, 11008, 4096, 0) == 1
+    assert lib.chadq_gemv_workspace_bytes(17, 512, 16384, 0) == 0 and lib.chadq_gemv_workspace_bytes(1, 512, 16400, 1) == 0

@@ -1360,3 +1360,43 @@ def test_gemm_in_parts_captured_in_a_graph(ops):
         other = ops.qlinear(x + 1, qw)
         torch.cuda.synchronize()
         assert torch.equal(y.view(torch.int16), want.view(torch.int16)) and not torch.equal(other, want)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 512, 16384), (1, 100, 13056), (2, 77, 16384), (3, 512, 16640), (4, 33, 20480), (5, 512, 8192), (7, 256, 12544), (8, 1000, 16384), (9, 512, 8192),
+                                   (12, 77, 10496), (16, 2048, 16384), (16, 16, 7168), (6, 1000, 12544), (6, 2100, 8448), (16, 4090, 16384), (13, 5000, 10496)])
+def test_gemv_in_parts_of_k(ops, m, n, k):
+    """Decode products of few weight rows and a long K, summed in parts: every kernel family, ragged rows, a last part that is shorter.  No further
+    from float64 than in one part (int8: sums in float64 either way; int4: fp32, shorter chains), results in bf16 the same sums rounded once."""
+    from chadslab_amd import QWeightInt4G32, QWeightInt8, _lib
+
+    lib = _lib.load()
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + n)
+    p = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+    s = torch.exp(torch.randn(n, k // 32, device=DEV, generator=g) * 0.5 - 5.0).half()
+    w4 = (torch.stack((p & 15, p >> 4), -1).reshape(n, k).double() - 8) * s.double().repeat_interleave(32, 1)
+    w = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=DEV, generator=g)
+    s8 = torch.exp(torch.randn(n, device=DEV, generator=g) * 0.5 - 8.0)
+    xf = torch.randn(m, k, device=DEV, generator=g)
+    stream = torch.cuda.current_stream().cuda_stream
+    for x, qw, ref, sc, name in ((xf.bfloat16(), QWeightInt4G32(p, s), xf.bfloat16().double() @ w4.t(), s, "chadq_gemv_i4g32"),
+                                 (xf, QWeightInt8(w, s8), xf.double() @ (w.double() * s8.double()[:, None]).t(), s8, "chadq_gemv_i8row")):
+        int8 = sc is s8
+        if n > 2048 and not int8:  # in one part
+            continue
+        need = lib.chadq_gemv_workspace_bytes(m, n, k, int(int8))
+        assert need >= 2 * m * n * (8 if int8 else 4)  # in parts
+        y, yb = ops.qgemv(x, qw), ops.qlinear(x, qw, out_dtype=torch.bfloat16)
+        assert torch.equal(yb.view(torch.int16), y.bfloat16().view(torch.int16)) and torch.equal(ops.qlinear(x, qw).view(torch.int32), y.view(torch.int32))
+        wp, one, again = w if int8 else p, torch.empty_like(y), torch.empty_like(y)
+        assert getattr(lib, name)(x.data_ptr(), wp.data_ptr(), sc.data_ptr(), one.data_ptr(), m, n, k, stream) == 0
+        off, off1 = (float((v.double() - ref).norm() / ref.norm()) for v in (y, one))
+        assert off <= 1.1 * off1 + 2.0 ** -25 and off <= 1e-6, (name, off, off1)
+        scratch = torch.full((need,), 0xFF, dtype=torch.uint8, device=DEV)
+        ws = getattr(lib, name + "_ws")
+        assert ws(x.data_ptr(), wp.data_ptr(), sc.data_ptr(), again.data_ptr(), m, n, k, 0, scratch.data_ptr(), need, stream) == 0
+        assert torch.equal(again.view(torch.int32), y.view(torch.int32))
+        for ptr, size in ((None, 0), (scratch.data_ptr(), need - 1)):  # none, or too little: one part
+            assert ws(x.data_ptr(), wp.data_ptr(), sc.data_ptr(), again.data_ptr(), m, n, k, 0, ptr, size, stream) == 0
+            assert torch.equal(again.view(torch.int32), one.view(torch.int32))
+        assert ws(x.data_ptr(), wp.data_ptr(), sc.data_ptr(), again.data_ptr(), m, n, k, 0, scratch.data_ptr() + 4, need, stream) == -3

@@ -15,6 +15,9 @@
 //     experts of 4096 x 14336: gate/up 87 -> 77 us, down 50 -> 49; four blocks in flight are no faster than three.
 //   * Otherwise the registers of the activations are single: a piece is requested again for the next block as soon as its MFMAs have
 //     been issued (the caches are nearer than the memory the weights come from).
+//   * Through LDS with more than four tokens, three blocks' registers and a sum per scale group modulo 4 are some ten more than there are.  The
+//     scales of a block are therefore requested a block later than its weights (kLateScales): nothing is spilled in row order.  us, row order,
+//     scales with the weights / later: 5 tokens of 16 experts of 3072 x 5376 76.5 / 74.1, 13 of 16 of 1280 x 9984 97 / 94, 6 of 8 of 2048 x 8960 71.4 / 66.9.
 //   * At most four tokens (FEW): the 16 rows of the A operand are four tokens of four scale groups, each lane group's row non-zero only
 //     where it meets that group's words, so the weights are used in the registers they arrived in (no exchange between lanes), the
 //     sums of four groups come out in one register each and one FMA per four groups and row is left of four: 188 vector instructions per
@@ -133,8 +136,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     u32x4 xq[XL ? 1 : FEW ? 8 : 4];
     // ---- the request side
     int l_item = begin, l_i = 0, l_n = 0, l_kb = 0, l_end = 0;
-    __amdgpu_buffer_rsrc_t wr[RB], sr[RB], xr, x_rsrc;
+    __amdgpu_buffer_rsrc_t wr[RB], sr[RB], xr, x_rsrc, s_rsrc[RB];
     __amdgpu_buffer_rsrc_t x_rsrc0;
+    constexpr bool kLateScales = XL && !FEW;  // requested a block later, so that two blocks' scales are in registers and not three
+    uint32_t s_voff = kBeyond, s_kb = 0;      // where those of the last block requested are
     uint32_t x_voff = kBeyond, x_kb = 0, x_voff0 = kBeyond, x_kb0 = 0;  // where the activations of the last block requested and of the one before it are
     uint32_t woff = 0, soff = 0, xoff = 0;  // of the lane, in the first row block
     // the second row block: the same rows of the up matrix, or the next 16 rows
@@ -166,24 +171,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             soff = n * (uint32_t)(K >> 4);
         }
     };
+    auto scales_of = [&](__amdgpu_buffer_rsrc_t from, int b, uint32_t sv, uint32_t kb) {
+        if constexpr (TILED) {
+            const uint32_t sk = kb * 512u + b * sblk;
+            const u32x2 ev = __builtin_amdgcn_raw_buffer_load_b64(from, sv, sk, 0), od = __builtin_amdgcn_raw_buffer_load_b64(from, sv, sk + 256u, 0);
+            return u32x4{ev.x, ev.y, od.x, od.y};
+        } else {
+            return (u32x4)__builtin_amdgcn_raw_buffer_load_b128(from, sv, kb * 16u + b * sblk, 0);
+        }
+    };
+    auto request_scales = [&](Block &q) {  // of the last block requested
+#pragma unroll
+        for (int b = 0; b < RB; ++b) q.s[b] = scales_of(s_rsrc[b], b, s_voff, s_kb);
+    };
     auto request = [&](Block &q) {
         x_rsrc0 = x_rsrc;
         x_voff0 = x_voff;
         x_kb0 = x_kb;
         if (l_item >= total) {
             x_voff = kBeyond;
+            s_voff = kBeyond;
             return;
         }
         const uint32_t kb = l_kb, beyond = l_kb < l_end ? 0u : kBeyond, wv = woff | beyond, sv = soff | beyond, xv = xoff | beyond;
 #pragma unroll
         for (int b = 0; b < RB; ++b) {
-            if (TILED) {
-                const uint32_t sk = kb * 512u + b * sblk;
-                const u32x2 ev = __builtin_amdgcn_raw_buffer_load_b64(sr[b], sv, sk, 0), od = __builtin_amdgcn_raw_buffer_load_b64(sr[b], sv, sk + 256u, 0);
-                q.s[b] = u32x4{ev.x, ev.y, od.x, od.y};
-            } else {
-                q.s[b] = __builtin_amdgcn_raw_buffer_load_b128(sr[b], sv, kb * 16u + b * sblk, 0);
-            }
+            if constexpr (kLateScales) s_rsrc[b] = sr[b];
+            else q.s[b] = scales_of(sr[b], b, sv, kb);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const uint32_t at = kb * (TILED ? 4096u : 128u) + b * wblk + h * (TILED ? 2048u : 4u * K);
@@ -191,6 +205,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
                 else q.w[b][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[b], wv, at, 0);
             }
         }
+        s_voff = sv;
+        s_kb = kb;
         if constexpr (!XL) {
             x_rsrc = xr;
             x_voff = xv;
@@ -412,12 +428,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     if constexpr (XL) {
         Block q0, q1, q2;
         request(q0);
+        if constexpr (kLateScales) request_scales(q0);
         request(q1);
         for (;;) {
+            if constexpr (kLateScales) request_scales(q1);
             request(q2);
             if (!consume(q0)) break;
+            if constexpr (kLateScales) request_scales(q2);
             request(q0);
             if (!consume(q1)) break;
+            if constexpr (kLateScales) request_scales(q0);
             request(q1);
             if (!consume(q2)) break;
         }

@@ -838,10 +838,20 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     }
 }
 
+// K in n parts (blockIdx.y) of `span` k each, a multiple of 256, the last one possibly shorter.  Whoever chooses n chooses the span with it: parts
+// that end before K would be a wrong sum, a part behind it a sum of nothing.
+struct KParts {
+    int n = 1, span = 0;
+};
+
 template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT = false, int EPI = EPI_BF16, bool SHORT = false>
-static int launch(const uint16_t *x, const uint8_t *wq, const void *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st,
+static int launch(const uint16_t *x, const uint8_t *wq, const void *sc, void *y, int M, int N, int K, KParts kp, hipStream_t st,
                   MoreOut<EPI> qkv = {}) {
     typedef Cfg<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, SHORT> C;
+    if (kp.n == 1) kp.span = K;
+    else
+        CHADQ_REQUIRE(EPI == EPI_F32 && kp.n > 1 && kp.span > 0 && kp.span % 256 == 0 && (int64_t)kp.n * kp.span >= K && (int64_t)(kp.n - 1) * kp.span < K,
+                      CHADQ_ERR_SHAPE, "gemm: %d parts of %d k do not make up %d", kp.n, kp.span, K);
     static std::atomic<bool> attr_set{false};  // setting it twice from two threads is harmless
     if (!attr_set.load(std::memory_order_acquire)) {
         CHADQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tile_q_kernel<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, EXACT, EPI, SHORT>),
@@ -849,8 +859,8 @@ static int launch(const uint16_t *x, const uint8_t *wq, const void *sc, void *y,
         attr_set.store(true, std::memory_order_release);
     }
     const int tiles = ((N + C::BN - 1) / C::BN) * ((M + C::BM - 1) / C::BM);
-    hipLaunchKernelGGL((gemm_tile_q_kernel<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, EXACT, EPI, SHORT>), dim3((tiles + 7) / 8 * 8, ksplit), dim3(C::T), C::LDS, st,
-                       x, wq, sc, y, M, N, K, ksplit == 1 ? K : (K / 256 + ksplit - 1) / ksplit * 256, qkv);
+    hipLaunchKernelGGL((gemm_tile_q_kernel<I4, WM, WN, WK, MB, NB, KW, ST, GUARD, EXACT, EPI, SHORT>), dim3((tiles + 7) / 8 * 8, kp.n), dim3(C::T), C::LDS, st,
+                       x, wq, sc, y, M, N, K, kp.span, qkv);
     return hip_check(hipGetLastError(), "gemm_tile_q launch");
 }
 
@@ -940,22 +950,22 @@ GemmTile gemm_tile_pick(int M, int N, int K, bool int4, bool guard) {
 template <bool I4, bool GUARD>
 static int launch_tile(const uint16_t *x, const uint8_t *w, const void *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st) {
     switch (tile) {
-        case TILE_32x64: return tileq::launch<I4, 1, 2, 4, 1, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
-        case TILE_64x64: return tileq::launch<I4, 1, 2, 4, 2, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
-        case TILE_96x64: return tileq::launch<I4, 1, 2, 4, 3, 1, 32, GUARD ? 3 : 4, GUARD>(x, w, sc, y, M, N, K, 1, st);
-        case TILE_128x64: return tileq::launch<I4, 1, 2, 4, 4, 1, 32, GUARD ? 3 : 4, GUARD>(x, w, sc, y, M, N, K, 1, st);
-        case TILE_96x128: return tileq::launch<I4, 1, 2, 4, 3, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
+        case TILE_32x64: return tileq::launch<I4, 1, 2, 4, 1, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, {}, st);
+        case TILE_64x64: return tileq::launch<I4, 1, 2, 4, 2, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, {}, st);
+        case TILE_96x64: return tileq::launch<I4, 1, 2, 4, 3, 1, 32, GUARD ? 3 : 4, GUARD>(x, w, sc, y, M, N, K, {}, st);
+        case TILE_128x64: return tileq::launch<I4, 1, 2, 4, 4, 1, 32, GUARD ? 3 : 4, GUARD>(x, w, sc, y, M, N, K, {}, st);
+        case TILE_96x128: return tileq::launch<I4, 1, 2, 4, 3, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, {}, st);
         case TILE_128x128:  // (the other form: int4 36.7 us against 36.3 at 1024 x 4096 x 4096, int8 113 against 107 at 1000 x 4096 x 14336)
-            if constexpr (I4) return tileq::launch<I4, 1, 4, 2, 4, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
-            else return tileq::launch<I4, 1, 2, 4, 4, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
-        case TILE_192x128: return tileq::launch<I4, 2, 2, 2, 3, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
-        case TILE_256x128: return tileq::launch<I4, 2, 2, 2, 4, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
-        case TILE_256x256: return tileq::launch<I4, 1, 8, 1, 8, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, 1, st);
-        case SHORT_32x64: return tileq::launch<I4, 1, 2, 4, 1, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, 1, st);
-        case SHORT_64x64: return tileq::launch<I4, 1, 2, 4, 2, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, 1, st);
-        case SHORT_128x128: return tileq::launch<I4, 1, 4, 2, 4, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, 1, st);
+            if constexpr (I4) return tileq::launch<I4, 1, 4, 2, 4, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, {}, st);
+            else return tileq::launch<I4, 1, 2, 4, 4, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, {}, st);
+        case TILE_192x128: return tileq::launch<I4, 2, 2, 2, 3, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, {}, st);
+        case TILE_256x128: return tileq::launch<I4, 2, 2, 2, 4, 2, 32, 3, GUARD>(x, w, sc, y, M, N, K, {}, st);
+        case TILE_256x256: return tileq::launch<I4, 1, 8, 1, 8, 1, 64, 3, GUARD>(x, w, sc, y, M, N, K, {}, st);
+        case SHORT_32x64: return tileq::launch<I4, 1, 2, 4, 1, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, {}, st);
+        case SHORT_64x64: return tileq::launch<I4, 1, 2, 4, 2, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, {}, st);
+        case SHORT_128x128: return tileq::launch<I4, 1, 4, 2, 4, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, {}, st);
         case SHORT_256x256:
-            if constexpr (I4) return tileq::launch<I4, 1, 8, 1, 8, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, 1, st);
+            if constexpr (I4) return tileq::launch<I4, 1, 8, 1, 8, 1, 64, 3, GUARD, false, tileq::EPI_BF16, true>(x, w, sc, y, M, N, K, {}, st);
             break;
     }
     return fail(CHADQ_ERR_SHAPE, "gemm: no tile %d", (int)tile);
@@ -976,16 +986,18 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
 }
 
 // ---- few tiles and a long K: the product in parts of whole 256-k blocks, one fp32 matrix each, added by a second launch.  A workgroup's walk
-// through K is what such a product takes: 48 x 4096 x 14336 is 64 workgroups of 56 steps, 35 us.  us, in one part / in parts, the launch that adds
-// them included: int4 81 x 1280 x 14080 29.1 / 14.2 (six), 62 x 1536 x 11264 23.2 / 12.5 (eight), 26 x 5542 x 11776 21.6 / 15.2 (two), 46 x 6528 x 4928
-// 14.7 / 13.6 (two); int8 250 x 640 x 9760 25.3 / 13.3 (six), 152 x 1280 x 14336 30.0 / 18.0 (four), 235 x 768 x 4352 11.2 / 11.1 (five).  Of 120 random
-// products of 17 to 1200 rows 32 are split, none of them slower, the mean of all 9 % faster.  The model of gemm_tile_pick, with what the parts
+// through K is what such a product takes: 48 x 4096 x 14336 is 64 workgroups of 56 steps, 29 us.  us, in one part / in parts, the launch that adds
+// them included: int4 81 x 1280 x 14080 29.5 / 14.9 (six), 62 x 1536 x 11264 23.6 / 12.7 (eight), 26 x 5542 x 11776 24.6 / 16.6 (two), 46 x 6528 x 4928
+// 14.6 / 13.5 (two), 48 x 4096 x 14336 29.0 / 17.9 (four), 219 x 1440 x 10432 28.8 / 20.7 (five); int8 250 x 640 x 9760 25.5 / 13.6 (six), 152 x 1280 x
+// 14336 30.1 / 17.9 (four), 235 x 768 x 4352 11.2 / 11.2 (five).  Of 600 random products of 17 to 1200 rows 137 are split and take 0.71 of the time on
+// average (34 of them with K that 256 does not divide: 0.73); those of 7 to 8 us gain nothing.  The model of gemm_tile_pick, with what the parts
 // cost on top, has to find 7 % in it.
 static const TileCost kCost32 = {TILE_32x64, 32, 64, 256, 1.9f, 2.2f, 7.6f, 0.75f, 0.f};
 
-int gemm_split_parts(int M, int N, int K, bool int4, bool guard, GemmTile *tile) {
+int gemm_split_parts(int M, int N, int K, bool int4, bool guard, GemmTile *tile, int *span) {
     constexpr float kSum = 2.5f, kMB = .3f;  // us of the second launch, of a MB of parts
     constexpr int kMost = 8;
+    *span = K;
     if (M < 17 || K < 1024 || K >= (1 << 22) || (int64_t)((M + 63) / 64) * ((N + 63) / 64) > 200) return 1;  // (what costs no time on the host)
     float whole = 0.f, best = 0.f;
     int parts = 1;
@@ -1000,6 +1012,7 @@ int gemm_split_parts(int M, int N, int K, bool int4, bool guard, GemmTile *tile)
             if (best == 0.f || us < best) {
                 best = us;
                 parts = s;
+                *span = per * 256;
                 *tile = t.tile;
             }
         }
@@ -1015,7 +1028,9 @@ int gemm_split_parts(int M, int N, int K, bool int4, bool guard, GemmTile *tile)
             if (t.tile == TILE_64x64 || t.tile == TILE_128x64) split(t);
         }
     }
-    return best != 0.f && best < .93f * whole ? parts : 1;
+    if (best != 0.f && best < .93f * whole) return parts;
+    *span = K;
+    return 1;
 }
 
 // y[m,n] = bf16(sum of the parts, in order, times the row scale of int8 weights); V columns per thread
@@ -1039,7 +1054,8 @@ __global__ __launch_bounds__(256) void gemm_sum_parts_kernel(const float *__rest
 }
 
 template <bool I4, bool GUARD>
-static int launch_parts(const uint16_t *x, const uint8_t *w, const void *sc, float *parts, int M, int N, int K, GemmTile tile, int np, hipStream_t st) {
+static int launch_parts(const uint16_t *x, const uint8_t *w, const void *sc, float *parts, int M, int N, int K, GemmTile tile, tileq::KParts np,
+                        hipStream_t st) {
     switch (tile) {
         case TILE_32x64: return tileq::launch<I4, 1, 2, 4, 1, 1, 64, 3, GUARD, false, tileq::EPI_F32>(x, w, sc, parts, M, N, K, np, st);
         case TILE_64x64: return tileq::launch<I4, 1, 2, 4, 2, 1, 64, 3, GUARD, false, tileq::EPI_F32>(x, w, sc, parts, M, N, K, np, st);
@@ -1048,9 +1064,10 @@ static int launch_parts(const uint16_t *x, const uint8_t *w, const void *sc, flo
 }
 
 int gemm_tile_parts_launch(const uint16_t *x, const uint8_t *w, const void *sc, uint16_t *y, int M, int N, int K, bool int4, bool guard, GemmTile tile, int np,
-                           float *parts, hipStream_t st) {
-    const int rc = int4 ? guard ? launch_parts<true, true>(x, w, sc, parts, M, N, K, tile, np, st) : launch_parts<true, false>(x, w, sc, parts, M, N, K, tile, np, st)
-                        : guard ? launch_parts<false, true>(x, w, sc, parts, M, N, K, tile, np, st) : launch_parts<false, false>(x, w, sc, parts, M, N, K, tile, np, st);
+                           int span, float *parts, hipStream_t st) {
+    const tileq::KParts kp = {np, span};
+    const int rc = int4 ? guard ? launch_parts<true, true>(x, w, sc, parts, M, N, K, tile, kp, st) : launch_parts<true, false>(x, w, sc, parts, M, N, K, tile, kp, st)
+                        : guard ? launch_parts<false, true>(x, w, sc, parts, M, N, K, tile, kp, st) : launch_parts<false, false>(x, w, sc, parts, M, N, K, tile, kp, st);
     if (rc) return rc;
     const int64_t total = (int64_t)M * N;
     const float *const scale = int4 ? nullptr : reinterpret_cast<const float *>(sc);
@@ -1118,22 +1135,23 @@ template <int EPI>
 static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, void *y, int M, int N, int K, int ksplit, float factor, hipStream_t st) {
     float us;
     const tileq::MoreOut<EPI> more{{factor}};
+    const tileq::KParts kp = {ksplit, (K / 256 + ksplit - 1) / ksplit * 256};  // (K % 256 == 0)
     const ExactCost &t = exact_pick(M, N, (K / 256 + ksplit - 1) / ksplit, ksplit, EPI == tileq::EPI_GEGLU, &us);
-    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st, more);
-    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st, more);
+    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st, more);
+    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st, more);
     if constexpr (EPI == tileq::EPI_GEGLU) {
-        if (t.bm == 256) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st, more);
+        if (t.bm == 256) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st, more);
     }
-    if (t.bn == 64) return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st, more);
-    return tileq::launch<true, 1, 4, 2, 4, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, ksplit, st, more);
+    if (t.bn == 64) return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st, more);
+    return tileq::launch<true, 1, 4, 2, 4, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st, more);
 }
 
 // Decode products of at most 32 rows whose K (or scales) the GEMV of gemv_i4g32_mfma.hip does not take: y fp32 or bf16 [M,N] in one
 // pass over the weights.
 int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, bool bf16_out,
                                hipStream_t st) {
-    return bf16_out ? tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, true, true, tileq::EPI_BF16>(x, wp, sc, y, M, N, K, 1, st)
-                    : tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, true, true, tileq::EPI_F32>(x, wp, sc, y, M, N, K, 1, st);
+    return bf16_out ? tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, true, true, tileq::EPI_BF16>(x, wp, sc, y, M, N, K, {}, st)
+                    : tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, true, true, tileq::EPI_F32>(x, wp, sc, y, M, N, K, {}, st);
 }
 
 // The K splits of a product, whole 256-k blocks each, the last one possibly shorter.  (With equal parts only, a down projection of 8960 k had
@@ -1179,9 +1197,9 @@ bool gemm_exact_qkv_pays(int M, int N, int K) {
 int gemm_exact_qkv_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, const QkvOut &out, int M, int K, hipStream_t st) {
     const int N = (out.hq + 2) * out.dh;
     const ExactCost &t = qkv_pick(M, N, K);
-    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, 1, st, {out});
-    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, 1, st, {out});
-    return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, 1, st, {out});
+    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, {}, st, {out});
+    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, {}, st, {out});
+    return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, {}, st, {out});
 }
 
 int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,

@@ -1341,6 +1341,46 @@ def test_gemm_in_parts_of_k(ops, m, n, k, shift):
         assert getattr(lib, name + "_ws")(x.data_ptr(), wp.data_ptr(), sc.data_ptr(), got[0].data_ptr(), m, n, k, scratch.data_ptr() + 4, need, stream) == -3
 
 
+@pytest.mark.parametrize("weight,tile,m,n,k", [
+    ("int4", 0, 17, 2052, 7712), ("int4", 1, 66, 1776, 7232), ("int4", 1, 36, 1264, 14432), ("int4", 1, 167, 1184, 5152), ("int4", 1, 68, 2049, 3104),
+    ("int4", 1, 51, 4096, 7200), ("int4", 3, 195, 2146, 7008), ("int4", 3, 219, 1440, 10432), ("int4", 3, 487, 768, 12832),
+    ("int8", 0, 17, 2058, 7696), ("int8", 0, 19, 7040, 9888), ("int8", 1, 66, 1312, 5152), ("int8", 1, 67, 1552, 4272), ("int8", 1, 258, 1392, 7232),
+    ("int8", 3, 196, 1673, 8432), ("int8", 3, 198, 1307, 7696)])
+def test_gemm_in_parts_reaches_the_end_of_k(ops, weight, tile, m, n, k):
+    """K that 256 does not divide, in a number of parts that divides K / 256 rounded down: parts of that many k each would end before K.  All three
+    tiles that are split, remainders of 16 to 240 k (whose activations are eight times the others'), element by element against float64."""
+    import ctypes
+
+    from chadslab_amd import QWeightInt4G32, QWeightInt8, _lib
+
+    rule = _lib.load()["_ZN5chadq16gemm_split_partsEiiibbPNS_8GemmTileEPi"]
+    rule.argtypes = [ctypes.c_int] * 3 + [ctypes.c_bool] * 2 + [ctypes.POINTER(ctypes.c_int)] * 2
+    picked, span = ctypes.c_int(), ctypes.c_int()
+    parts = rule(m, n, k, weight == "int4", True, ctypes.byref(picked), ctypes.byref(span))
+    assert parts > 1 and k // 256 % parts == 0 and k % 256 and picked.value == tile
+    g = torch.Generator(device=DEV)
+    g.manual_seed(m + n + k)
+    x = torch.randn(m, k, device=DEV, generator=g)
+    x[:, k // 256 * 256:] *= 8
+    x = x.bfloat16()
+    if weight == "int4":
+        p = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g)
+        s = torch.exp(torch.randn(n, k // 32, device=DEV, generator=g) * 0.5 - 5.0).half()
+        qw = QWeightInt4G32(p, s)
+        w = ((torch.stack((p & 15, p >> 4), -1).reshape(n, k).float() - 8) * s.float().repeat_interleave(32, 1)).bfloat16().double()
+    else:
+        w = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=DEV, generator=g)
+        s = torch.exp(torch.randn(n, device=DEV, generator=g) * 0.5 - 8.0)
+        qw = QWeightInt8(w, s)
+        w = w.double() * s.double()[:, None]
+    ref, mag = x.double() @ w.t(), x.double().abs() @ w.abs().t()
+    y = ops.qgemm(x, qw)
+    # the products are exact in fp32: the fp32 sum of at most k terms, the rounding to bf16
+    err = ((y.double() - ref).abs() / (2.0 ** -8 * ref.abs() + (k / 8 + 8) * 2.0 ** -24 * mag)).max()
+    assert float(err) <= 1, float(err)
+    assert torch.equal(ops.qlinear(x, qw).view(torch.int16), y.view(torch.int16))
+
+
 def test_gemm_in_parts_captured_in_a_graph(ops):
     """A captured product in parts gives the eager bits on every replay, with other products in between."""
     from chadslab_amd import QWeightInt8

@@ -448,15 +448,13 @@ int gemm_i8row_bf16_dispatch(const uint16_t *x, const int8_t *w8, const float *s
     return launch_gemm<FmtI8Row, false>(x, w8, sc, y, M, N, K, nullptr, 0, st);
 }
 
-// The same with fp32 scratch: a product of few tiles and a long K in parts of K.  Both forms of the tiles (whole and guarded steps) count, because
-// the alignment of the scales is not known when the bytes are asked for.
+// The same with fp32 scratch: a product of few tiles and a long K in parts of K.  (The rule knows sizes only: the alignment of the scales, which decides
+// between whole and guarded steps, is not known when the bytes are asked for.)
 size_t gemm_parts_bytes(int M, int N, int K, bool int4) {
     GemmTile tile;
     int span;
     if (M < 1 || N < 1 || K < 1 || !gemm_tile_q_ok(K)) return 0;
-    const int whole = int4 && K % 256 == 0 ? gemm_split_parts(M, N, K, int4, false, &tile, &span) : 1;
-    const int guarded = gemm_split_parts(M, N, K, int4, K % 256 != 0 || int4, &tile, &span);
-    const int parts = whole > guarded ? whole : guarded;
+    const int parts = gemm_split_parts(M, N, K, int4, &tile, &span);
     return parts > 1 ? (size_t)parts * M * N * 4 : 0;
 }
 
@@ -465,7 +463,7 @@ int gemm_ws_dispatch(const uint16_t *x, const uint8_t *w, const void *sc, uint16
     GemmTile tile;
     int span = K;
     const bool guard = K % 256 != 0 || (int4 && !aligned16(sc));
-    const int np = parts && gemm_tile_q_ok(K) && activations_ok(M, K) == 0 ? gemm_split_parts(M, N, K, int4, guard, &tile, &span) : 1;
+    const int np = parts && gemm_tile_q_ok(K) && activations_ok(M, K) == 0 ? gemm_split_parts(M, N, K, int4, &tile, &span) : 1;
     if (np > 1 && (size_t)np * M * N * 4 <= bytes) return gemm_tile_parts_launch(x, w, sc, y, M, N, K, int4, guard, tile, np, span, parts, st);
     return int4 ? gemm_i4g32_bf16_dispatch(x, w, reinterpret_cast<const uint16_t *>(sc), y, M, N, K, st)
                 : gemm_i8row_bf16_dispatch(x, reinterpret_cast<const int8_t *>(w), reinterpret_cast<const float *>(sc), y, M, N, K, st);

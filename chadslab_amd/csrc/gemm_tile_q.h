@@ -18,7 +18,7 @@ int gemm_tile_i4g32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t 
 int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc, uint16_t *y, int M, int N, int K, GemmTile tile, hipStream_t st);
 // K parts (1: none) in which a product of few tiles and a long K is the quicker one, their k (np * span >= K, none is empty) and tile; the parts
 // (fp32 [np][M,N], at `parts`) added to y
-int gemm_split_parts(int M, int N, int K, bool int4, bool guard, GemmTile *tile, int *span);
+int gemm_split_parts(int M, int N, int K, bool int4, GemmTile *tile, int *span);
 int gemm_tile_parts_launch(const uint16_t *x, const uint8_t *w, const void *sc, uint16_t *y, int M, int N, int K, bool int4, bool guard, GemmTile tile, int np,
                            int span, float *parts, hipStream_t st);
 // int4 weights taken exactly (nothing rounded before the fp32 sums); K % 256 == 0, x, wp and sc 16-byte aligned unless it says otherwise

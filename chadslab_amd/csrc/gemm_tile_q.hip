@@ -989,16 +989,20 @@ int gemm_tile_i8row_launch(const uint16_t *x, const int8_t *w8, const float *sc,
 // through K is what such a product takes: 48 x 4096 x 14336 is 64 workgroups of 56 steps, 29 us.  us, in one part / in parts, the launch that adds
 // them included: int4 81 x 1280 x 14080 29.5 / 14.9 (six), 62 x 1536 x 11264 23.6 / 12.7 (eight), 26 x 5542 x 11776 24.6 / 16.6 (two), 46 x 6528 x 4928
 // 14.6 / 13.5 (two), 48 x 4096 x 14336 29.0 / 17.9 (four), 219 x 1440 x 10432 28.8 / 20.7 (five); int8 250 x 640 x 9760 25.5 / 13.6 (six), 152 x 1280 x
-// 14336 30.1 / 17.9 (four), 235 x 768 x 4352 11.2 / 11.2 (five).  Of 600 random products of 17 to 1200 rows 137 are split and take 0.71 of the time on
-// average (34 of them with K that 256 does not divide: 0.73); those of 7 to 8 us gain nothing.  The model of gemm_tile_pick, with what the parts
-// cost on top, has to find 7 % in it.
+// 14336 30.1 / 17.9 (four).  A second launch and its scratch cost a call 1.5 us that its kernels' times do not show, and the constants of gemm_tile_pick,
+// fitted to fuller grids, give int8 products of few tiles a us too much in one part: both count, so that calls of 7 to 9 us stay in one (calls of
+// qlinear in a row, int8: 17 x 512 x 4096 7.9 / 9.0, 65 x 512 x 3584 8.8 / 9.5; int4 49 x 960 x 2816 8.8 / 9.2).  Of 288 random calls in parts the mean
+// takes 0.71 of the time in one (waited for one by one: 0.83), the worst 1.04.
 static const TileCost kCost32 = {TILE_32x64, 32, 64, 256, 1.9f, 2.2f, 7.6f, 0.75f, 0.f};
 
-int gemm_split_parts(int M, int N, int K, bool int4, bool guard, GemmTile *tile, int *span) {
-    constexpr float kSum = 2.5f, kMB = .3f;  // us of the second launch, of a MB of parts
+int gemm_split_parts(int M, int N, int K, bool int4, GemmTile *tile, int *span) {
+    // us of the second launch and its scratch, as far as they are not hidden, less what the model finds too long in one part; of a MB of parts
+    const float kSum = int4 ? 4.f : 5.f, kMB = .3f;
     constexpr int kMost = 8;
     *span = K;
-    if (M < 17 || K < 1024 || K >= (1 << 22) || (int64_t)((M + 63) / 64) * ((N + 63) / 64) > 200) return 1;  // (what costs no time on the host)
+    // (below 2304 k the model never finds enough.  Beyond 200 tiles parts fill no idle compute units: of twelve products of 208 to 256 tiles, 4096 to 14336
+    // k, two parts take 0.97 to 1.6 of the time in one, 48 x 14336 x 4096 20.4 us against 13.3, 256 x 3584 x 14336 39.6 against 38.5)
+    if (M < 17 || K < 2304 || K >= (1 << 22) || (int64_t)((M + 63) / 64) * ((N + 63) / 64) > 200) return 1;
     float whole = 0.f, best = 0.f;
     int parts = 1;
     auto split = [&](const TileCost &t) {
@@ -1021,14 +1025,14 @@ int gemm_split_parts(int M, int N, int K, bool int4, bool guard, GemmTile *tile,
         whole = tile_us(kCost32, tiles_of(kCost32, M, N), K);
         split(kCost32);
     } else {
-        for (const TileCost &t : kCost[int4][guard]) {
+        for (const TileCost &t : kCost[int4][K % 256 != 0]) {
             if (M <= 64 && t.tile != TILE_64x64) continue;
             const float us = tile_us(t, tiles_of(t, M, N), K);
             if (whole == 0.f || us < whole) whole = us;
             if (t.tile == TILE_64x64 || t.tile == TILE_128x64) split(t);
         }
     }
-    if (best != 0.f && best < .93f * whole) return parts;
+    if (best != 0.f && best < .98f * whole) return parts;
     *span = K;
     return 1;
 }

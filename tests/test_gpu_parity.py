@@ -1303,7 +1303,7 @@ def test_moe_ffn_tiled_refuses_mixed_and_unaligned_shapes(ops):
     assert lib.chadq_moe_ffn_i4g32_tiled(x2.data_ptr(), z1.data_ptr(), arr, y.data_ptr(), 8, 288, 256, 1, 1, 1, ws.data_ptr(), need, None) == -2
 
 
-@pytest.mark.parametrize("m,n,k,shift", [(17, 512, 4096, 0), (32, 102, 8192, 0), (40, 257, 4128, 0), (48, 1024, 14336, 0), (64, 64, 4096, 1), (70, 513, 16384, 0), (100, 1000, 8160, 0),
+@pytest.mark.parametrize("m,n,k,shift", [(17, 512, 8192, 0), (32, 102, 8192, 0), (40, 257, 4128, 0), (48, 1024, 14336, 0), (64, 64, 4096, 1), (70, 513, 16384, 0), (100, 1000, 8160, 0),
                                          (128, 2048, 8192, 1), (300, 1024, 16384, 0), (200, 512, 5152, 0)])
 def test_gemm_in_parts_of_k(ops, m, n, k, shift):
     """Products of few tiles and a long K, summed in parts: ragged rows and columns (columns that no four divide, too), K that 256 does not divide,
@@ -1342,9 +1342,9 @@ def test_gemm_in_parts_of_k(ops, m, n, k, shift):
 
 
 @pytest.mark.parametrize("weight,tile,m,n,k", [
-    ("int4", 0, 17, 2052, 7712), ("int4", 1, 66, 1776, 7232), ("int4", 1, 36, 1264, 14432), ("int4", 1, 167, 1184, 5152), ("int4", 1, 68, 2049, 3104),
-    ("int4", 1, 51, 4096, 7200), ("int4", 3, 195, 2146, 7008), ("int4", 3, 219, 1440, 10432), ("int4", 3, 487, 768, 12832),
-    ("int8", 0, 17, 2058, 7696), ("int8", 0, 19, 7040, 9888), ("int8", 1, 66, 1312, 5152), ("int8", 1, 67, 1552, 4272), ("int8", 1, 258, 1392, 7232),
+    ("int4", 0, 17, 2052, 7712), ("int4", 1, 66, 1776, 7232), ("int4", 1, 36, 1264, 14432), ("int4", 1, 167, 1184, 5152), ("int4", 1, 67, 2067, 3936),
+    ("int4", 1, 51, 4096, 7200), ("int4", 3, 202, 2066, 7904), ("int4", 3, 219, 1440, 10432), ("int4", 3, 487, 768, 12832),
+    ("int8", 0, 17, 2058, 7696), ("int8", 0, 19, 7040, 9888), ("int8", 1, 66, 1312, 5152), ("int8", 1, 67, 1538, 5248), ("int8", 1, 258, 1392, 7232),
     ("int8", 3, 196, 1673, 8432), ("int8", 3, 198, 1307, 7696)])
 def test_gemm_in_parts_reaches_the_end_of_k(ops, weight, tile, m, n, k):
     """K that 256 does not divide, in a number of parts that divides K / 256 rounded down: parts of that many k each would end before K.  All three
@@ -1353,10 +1353,10 @@ def test_gemm_in_parts_reaches_the_end_of_k(ops, weight, tile, m, n, k):
 
     from chadslab_amd import QWeightInt4G32, QWeightInt8, _lib
 
-    rule = _lib.load()["_ZN5chadq16gemm_split_partsEiiibbPNS_8GemmTileEPi"]
-    rule.argtypes = [ctypes.c_int] * 3 + [ctypes.c_bool] * 2 + [ctypes.POINTER(ctypes.c_int)] * 2
+    rule = _lib.load()["_ZN5chadq16gemm_split_partsEiiibPNS_8GemmTileEPi"]
+    rule.argtypes = [ctypes.c_int] * 3 + [ctypes.c_bool] + [ctypes.POINTER(ctypes.c_int)] * 2
     picked, span = ctypes.c_int(), ctypes.c_int()
-    parts = rule(m, n, k, weight == "int4", True, ctypes.byref(picked), ctypes.byref(span))
+    parts = rule(m, n, k, weight == "int4", ctypes.byref(picked), ctypes.byref(span))
     assert parts > 1 and k // 256 % parts == 0 and k % 256 and picked.value == tile
     g = torch.Generator(device=DEV)
     g.manual_seed(m + n + k)

@@ -145,6 +145,14 @@ class _NoHostModule:
     def moe_ffn(x, logits, experts, top_k, renorm):
         return None
 
+    @staticmethod
+    def gemv_bytes(m, n, k, int8):
+        return load().chadq_gemv_workspace_bytes(m, n, k, int8)
+
+    @staticmethod
+    def gemm_bytes(m, n, k, int8):
+        return load().chadq_gemm_bf16_workspace_bytes(m, n, k, int8)
+
 
 def native():
     """The host module (csrc/host_call.cpp), bound to the library that load() gives.  Where it cannot be loaded the calls go without it, and a

@@ -917,8 +917,8 @@ static int short_k(GemmTile t, bool int4, bool guard) {
 
 // us of `tiles` workgroups of t, `wgs` of them counted for the fill of the last round (the same number where nothing is split), k each
 static float tile_us(const TileCost &t, int64_t wgs, int k) {
-    const int64_t rounds = (wgs + 255) / 256;
-    const float fill = (float)(wgs - (rounds - 1) * 256) / 256.f, kk = (float)((k + t.ks - 1) / t.ks) * (float)t.ks;
+    const int64_t rounds = (wgs + 255) >> 8;
+    const float fill = (float)(wgs - (rounds - 1) * 256) / 256.f, kk = (float)((k + t.ks - 1) & -t.ks);  // (a step is a power of two)
     const float a = t.s + ((float)(rounds - 1) + t.b + (1.f - t.b) * fill) * (t.c0 + t.c1 * kk / 4096.f);
     return a * (1.f + t.q * a / (a + 100.f));
 }

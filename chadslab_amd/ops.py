@@ -102,7 +102,7 @@ def _gemv(x: torch.Tensor, qw: QWeight, out: Optional[torch.Tensor], fp32_elemen
         p, s = _dev(qw.packed, "packed", torch.uint8), _dev(qw.scale, "scale", torch.float16)
         y = _out(out, (m, n), y_dtype, x.device)
         name = "chadq_gemv_i4g32_bf16" if bf16_out else "chadq_gemv_i4g32"
-        need = lib.chadq_gemv_workspace_bytes(m, n, k, 0)  # as in qgemm
+        need = _lib.native().gemv_bytes(m, n, k, 0)  # as in qgemm
         if need:
             ws = x.new_empty(need, dtype=torch.uint8)
             _lib.check(lib.chadq_gemv_i4g32_ws(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, int(bf16_out), ws.data_ptr(), need,
@@ -115,7 +115,7 @@ def _gemv(x: torch.Tensor, qw: QWeight, out: Optional[torch.Tensor], fp32_elemen
         w, s = _dev(qw.w, "w", torch.int8), _dev(qw.scale, "scale", torch.float32)
         y = _out(out, (m, n), y_dtype, x.device)
         name = "chadq_gemv_i8row_fp32" if fp32_elements else "chadq_gemv_i8row_bf16" if bf16_out else "chadq_gemv_i8row"
-        need = 0 if fp32_elements else lib.chadq_gemv_workspace_bytes(m, n, k, 1)
+        need = 0 if fp32_elements else _lib.native().gemv_bytes(m, n, k, 1)
         if need:
             ws = x.new_empty(need, dtype=torch.uint8)
             _lib.check(lib.chadq_gemv_i8row_ws(x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, int(bf16_out), ws.data_ptr(), need,
@@ -129,26 +129,34 @@ def _gemv(x: torch.Tensor, qw: QWeight, out: Optional[torch.Tensor], fp32_elemen
 def qgemm(x: torch.Tensor, qw: QWeight, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Prefill product on the matrix cores: x bf16 [M,K] -> bf16 [M,N], fp32 accumulate."""
     lib = _lib.load()
-    if x.dim() != 2 or x.shape[1] != qw.K:
-        raise ValueError("x must be [M,%d], got %s" % (qw.K, tuple(x.shape)))
+    n, k = qw.N, qw.K
+    if x.dim() != 2 or x.size(1) != k:
+        raise ValueError("x must be [M,%d], got %s" % (k, tuple(x.shape)))
     x = _dev(x, "x", torch.bfloat16)
-    m = x.shape[0]
-    y = _out(out, (m, qw.N), torch.bfloat16, x.device)
-    # scratch for the K parts of a product of few tiles (0 bytes where one part is the quicker form): a fresh one per call, as moe_ffn's
-    need = lib.chadq_gemm_bf16_workspace_bytes(m, qw.N, qw.K, int(isinstance(qw, QWeightInt8)))
-    ws = x.new_empty(need, dtype=torch.uint8) if need else None
-    ws_ptr = ws.data_ptr() if need else None
+    m = x.size(0)
+    y = _out(out, (m, n), torch.bfloat16, x.device)
+    # Scratch for the K parts of a product of few tiles (0 bytes where one part is the quicker form): a fresh one per call, as moe_ffn's.
     if isinstance(qw, QWeightInt4G32):
         p, s = _dev(qw.packed, "packed", torch.uint8), _dev(qw.scale, "scale", torch.float16)
-        _lib.check(lib.chadq_gemm_i4g32_bf16_ws(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, qw.N, qw.K, ws_ptr, need,
-                                                _stream()), "chadq_gemm_i4g32_bf16")
-    elif isinstance(qw, QWeightInt8):
+        need = _lib.native().gemm_bytes(m, n, k, 0)
+        if need:
+            ws = x.new_empty(need, dtype=torch.uint8)
+            _lib.check(lib.chadq_gemm_i4g32_bf16_ws(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, ws.data_ptr(), need, _stream()),
+                       "chadq_gemm_i4g32_bf16")
+            return y
+        _lib.check(lib.chadq_gemm_i4g32_bf16(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, _stream()), "chadq_gemm_i4g32_bf16")
+        return y
+    if isinstance(qw, QWeightInt8):
         w, s = _dev(qw.w, "w", torch.int8), _dev(qw.scale, "scale", torch.float32)
-        _lib.check(lib.chadq_gemm_i8row_bf16_ws(x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, qw.N, qw.K, ws_ptr, need,
-                                                _stream()), "chadq_gemm_i8row_bf16")
-    else:
-        raise TypeError("unknown weight container %r" % type(qw))
-    return y
+        need = _lib.native().gemm_bytes(m, n, k, 1)
+        if need:
+            ws = x.new_empty(need, dtype=torch.uint8)
+            _lib.check(lib.chadq_gemm_i8row_bf16_ws(x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, ws.data_ptr(), need, _stream()),
+                       "chadq_gemm_i8row_bf16")
+            return y
+        _lib.check(lib.chadq_gemm_i8row_bf16(x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, _stream()), "chadq_gemm_i8row_bf16")
+        return y
+    raise TypeError("unknown weight container %r" % type(qw))
 
 
 def qlinear(x: torch.Tensor, qw: QWeight, *, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:

@@ -190,3 +190,16 @@ def test_gemv_is_summed_in_parts_where_few_rows_walk_a_long_k():
     assert parts(1, 512, 6144, 1) == 1 and parts(16, 4096, 16384, 1) == 4 and parts(12, 6144, 6144, 1) == 1
     assert parts(1, 14336, 4096, 0) == 1 and parts(1, 16384, 2048, 1) == 1 and parts(6, 11008, 4096, 0) == 1
     assert lib.chadq_gemv_workspace_bytes(17, 512, 16384, 0) == 0 and lib.chadq_gemv_workspace_bytes(1, 512, 16400, 1) == 0
+
+
+def test_host_module_answers_as_the_library_does():
+    """Bytes asked through the host module, which the calls of ops.py use, and through the C ABI."""
+    lib, native, r = _lib.load(), _lib.native(), random.Random(4)
+    for _ in range(3000):
+        size = (r.randint(-1, 300), r.randint(-2, 9000), r.randint(-2, 600) * 32, r.randint(0, 1))
+        assert native.gemv_bytes(*size) == lib.chadq_gemv_workspace_bytes(*size)
+        assert native.gemm_bytes(*size) == lib.chadq_gemm_bf16_workspace_bytes(*size)
+    assert native.gemv_bytes(1, 512, 16384, 0) > 0 and native.gemm_bytes(48, 4096, 14336, 1) > 0
+    assert native.gemm_bytes(1 << 40, 512, 16384, 0) == 0  # (the product refuses it)
+    with pytest.raises(TypeError):
+        native.gemv_bytes(1, 512, 16384)

@@ -22,22 +22,21 @@ int gemm_split_parts(int M, int N, int K, bool int4, GemmTile *tile, int *span);
 int gemm_tile_parts_launch(const uint16_t *x, const uint8_t *w, const void *sc, uint16_t *y, int M, int N, int K, bool int4, bool guard, GemmTile tile, int np,
                            int span, float *parts, hipStream_t st);
 // int4 weights taken exactly (nothing rounded before the fp32 sums); K % 256 == 0, x, wp and sc 16-byte aligned unless it says otherwise
-// The `scaled` products below take activations that carry this factor (exact but for magnitudes below 2^-121), and the gated one's result
-// carries it too: the operands are (u - 8) / 2^4, and with it no group's sum overflows while the activations are finite (32 x 8 < 2^9).
-// Without it, from 2^123 on.
+// The activations of a prompt's products (not those of gemm_exact_few_rows_launch) carry this factor, and the gated one's result carries it too: the
+// operands are (u - 8) / 2^4, and with it no group's sum overflows while the activations are finite.  The factor is exact for bf16 activations of
+// 2^-121 and more; smaller ones lose up to five bits.
 constexpr float kExactX = 0x1p-5f;
 constexpr int kExactMaxSplits = 8;
-int gemm_exact_splits(int M, int N, int K);  // K splits to use for gemm_exact_f32_launch
-// rows of the tile that the two launches below take for `parts` K splits of `per` 256-k blocks; *us: what the launch takes
-int gemm_exact_tile(int M, int N, int per, int parts, bool geglu, float *us);
+int gemm_exact_splits(int M, int N, int K);  // K splits to use for gemm_exact_scaled_f32_launch
+// rows (and *columns) of the tile that the f32 and geglu launches below take for `parts` K splits of `per` 256-k blocks; *us: what the launch takes
+int gemm_exact_tile(int M, int N, int per, int parts, bool geglu, float *us, int *columns);
 // y_parts fp32 [ksplit][M,N]
-int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
-                          hipStream_t st);
-// y [M,N] fp32 or bf16, at most 32 rows, any K % 32 == 0 with gemm_tile_q_ok(K), any alignment of the scales
-int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, bool bf16_out,
-                               hipStream_t st);
+int gemm_exact_scaled_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
+                                 hipStream_t st);
+// weight rows in (gate, up) pairs: h[m,i] = bf16(gelu_tanh(y[m,2i]) * y[m,2i+1] * kExactX), [M, N/2]
+int gemm_exact_scaled_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st);
 // The product of a prompt's M tokens with [q heads | k | v] (hq + 2 heads of dh, in whole K): q and k rotated at positions pos + m (table as
-// chadq_rope_table writes it), q fp32 [M][hq*dh], k and v as bf16 rows pos + m of the caches.  x carries kExactX.
+// chadq_rope_table writes it), q fp32 [M][hq*dh], k and v as bf16 rows pos + m of the caches.
 struct QkvOut {
     const float *table;
     float *q;
@@ -45,12 +44,10 @@ struct QkvOut {
     int hq, dh, pos;
 };
 bool gemm_exact_qkv_pays(int M, int N, int K);  // against the plain product and a launch for the rest
+int gemm_exact_qkv_tile(int M, int N, int K);   // rows of its tile (64 columns)
 int gemm_exact_qkv_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, const QkvOut &out, int M, int K, hipStream_t st);
-int gemm_exact_scaled_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
-                                 hipStream_t st);
-// weight rows in (gate, up) pairs: h[m,i] = bf16(gelu_tanh(y[m,2i]) * y[m,2i+1]), [M, N/2]
-int gemm_exact_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st);
-
-int gemm_exact_scaled_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st);
+// y [M,N] fp32 or bf16, at most 32 rows, any K % 32 == 0 with gemm_tile_q_ok(K), any alignment of the scales, plain activations
+int gemm_exact_few_rows_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y, int M, int N, int K, bool bf16_out,
+                               hipStream_t st);
 
 }  // namespace chadq

@@ -43,14 +43,15 @@
 // one body for all of them with its conditions at run time (24 x 1024 x 1120 6.5 us, five bodies 5.8, SHORT 5.2), no unrolled loop, no
 // second request of the last step's weights (both nothing from two steps on).
 //
-// EXACT: no weight is rounded, for callers whose sums must be those of the decode step.  The operands are integers, (u - 8) / 2^4 for
-// activations that carry 2^-5, (u - 8) / 2^9 for others; the scale of a group of 32 k is applied to its sum, one fp32 FMA per value.
-// Unpacking takes 14 instructions per 8 weights where the activations carry the factor (signed nibbles to fp32, the upper halves paired), 19
-// where not (by way of e4m3): gate/up of a 2048 x 16384 layer, 24 / 100 / 256 tokens 16.6 -> 15 / 30.2 -> 29 / 50.4 -> 43-46 us in a stream of that
+// EXACT: no weight is rounded, for callers whose sums must be those of the decode step.  The operands are integers: (u - 8) / 2^4 in products of whole
+// steps, whose activations carry the factor 2^-5 (kExactX), (u - 8) / 2^9 in guarded ones, whose activations are plain; the scale of a group of 32 k
+// is applied to its sum, one fp32 FMA per value.
+// Unpacking takes 14 instructions per 8 weights in the former (signed nibbles to fp32, the upper halves paired), 19
+// in the latter (by way of e4m3): gate/up of a 2048 x 16384 layer, 24 / 100 / 256 tokens 16.6 -> 15 / 30.2 -> 29 / 50.4 -> 43-46 us in a stream of that
 // product alone.  What bounds it is everything together, at the clock its power leaves (1.8 GHz): of 42 us at 256 tokens the FMAs taken out
 // leave 34, the LDS reads of the activations 33, their requests 37, the unpacking 42; reading three or four row blocks ahead, other
 // orders of a pair's instructions and waves of 128 x 64 (half the LDS reads, twice the unpacking: 48) give nothing.
-// (An earlier form kept a weight as the sum of two bf16 operands: twice the matrix work, 63.7 us.)  Its sums are finite for all finite
+// (An earlier form kept a weight as the sum of two bf16 operands: twice the matrix work, 63.7 us.)  A group's sum is finite for all finite
 // activations (32 x 8 < 2^9), and a weight of 0 is the operand 0: a large activation beside it leaves the other products their low bits.
 // The MFMA k-slot of a lane is free as long as A and B agree: slot group kq of slice t holds k = (KW / 2) kq + 8 t .. +7
 // (EXACT: 16 t + 8 kq .. +7).
@@ -160,20 +161,13 @@ __device__ __forceinline__ bf16x8 signed8_i4_16th(uint32_t w) {
 
 // EPI (what becomes of the sums): EPI_BF16 y bf16 [M,N], times the row scale for int8; EPI_F32 y fp32 [gridDim.y][M,N],
 // part blockIdx.y holding the sum over its kspan k; EPI_GEGLU the weight rows come in pairs (gate, up) of a feature and
-// h = bf16(gelu_tanh(gate) * up) goes to y as bf16 [M, N/2], times the factor of the activations (ExactX).  EPI_QKV (WN = 2, WK = 4): as
+// h = bf16(gelu_tanh(gate) * up) goes to y as bf16 [M, N/2], times the factor that the activations carry (kExactX).  EPI_QKV (WN = 2, WK = 4): as
 // QkvOut says; a tile's columns are 32 of a head's first half and the 32 of its second half that they are rotated with.
 // (A type of its own per epilogue: a name formed from the unnamed enumeration would not be the same for the host's and the device's compiler.)
 template <int EPI>
 struct MoreOut {};
 template <>
 struct MoreOut<EPI_QKV> : QkvOut {};
-struct ExactX {
-    float x = 1.f;  // the factor that the activations (and a gated result) carry
-};
-template <>
-struct MoreOut<EPI_F32> : ExactX {};
-template <>
-struct MoreOut<EPI_GEGLU> : ExactX {};
 template <bool I4, int WM, int WN, int WK, int MB, int NB, int KW, int ST, bool GUARD, bool EXACT, int EPI, bool SHORT>
 __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WM * WN * WK / 4, WM * WN * WK / 4))) void gemm_tile_q_kernel(
     const uint16_t *__restrict__ x, const uint8_t *__restrict__ wq, const void *__restrict__ scv, void *__restrict__ yv, int M, int N,
@@ -356,8 +350,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
     uint32_t wv[GR][2], wnx[GR][2];  // the lane's packed words of a step [group][slice], of the next one
     uint32_t sraw[GR];               // its scales
     float sc2[GR], s_last = 0.f;     // ... as floats, that of the group whose sums are next
-    float undo = 512.f;              // what operands and activations leave out
-    if constexpr (!GUARD && EPI != EPI_QKV) undo = 16.f / qkv.x;
+    constexpr float undo = 512.f;    // what the operands leave out, or (whole steps) they and the activations
+    static_assert(16.f / kExactX == undo, "operands of (u - 8) / 2^4 for activations that carry the factor");
     auto fetch = [&](int step, const uint8_t *stage) {
 #pragma unroll
         for (int g = 0; g < GR; ++g)
@@ -814,7 +808,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_
             // even lane: row r, columns (nl, nl+1) = (own a0, neighbour's a0); odd lane: row r+1, columns (nl-1, nl)
             if constexpr (GE)
                 *reinterpret_cast<uint16_t *>(lds + row * EP + (cb + nl) / 2 * 2) =
-                    (uint16_t)pack_bf16_rne(gelu_tanh_dev(odd ? recv : a0) * (odd ? a1 : recv) * qkv.x, 0.f);
+                    (uint16_t)pack_bf16_rne(gelu_tanh_dev(odd ? recv : a0) * (odd ? a1 : recv) * kExactX, 0.f);
             else
                 *reinterpret_cast<uint32_t *>(lds + row * EP + (cb + (nl & ~1)) * 2) = odd ? pack_bf16_rne(recv, a1) : pack_bf16_rne(a0, recv);
         }
@@ -1133,21 +1127,24 @@ static const ExactCost &exact_pick(int M, int N, int per, int parts, bool geglu,
     return t[best];
 }
 
-int gemm_exact_tile(int M, int N, int per, int parts, bool geglu, float *us) { return exact_pick(M, N, per, parts, geglu, us).bm; }
+int gemm_exact_tile(int M, int N, int per, int parts, bool geglu, float *us, int *columns) {
+    const ExactCost &t = exact_pick(M, N, per, parts, geglu, us);
+    *columns = t.bn;
+    return t.bm;
+}
 
 template <int EPI>
-static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, void *y, int M, int N, int K, int ksplit, float factor, hipStream_t st) {
+static int launch_exact(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, void *y, int M, int N, int K, int ksplit, hipStream_t st) {
     float us;
-    const tileq::MoreOut<EPI> more{{factor}};
     const tileq::KParts kp = {ksplit, (K / 256 + ksplit - 1) / ksplit * 256};  // (K % 256 == 0)
     const ExactCost &t = exact_pick(M, N, (K / 256 + ksplit - 1) / ksplit, ksplit, EPI == tileq::EPI_GEGLU, &us);
-    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st, more);
-    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st, more);
+    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st);
+    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st);
     if constexpr (EPI == tileq::EPI_GEGLU) {
-        if (t.bm == 256) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st, more);
+        if (t.bm == 256) return tileq::launch<true, 1, 4, 2, 8, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st);
     }
-    if (t.bn == 64) return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st, more);
-    return tileq::launch<true, 1, 4, 2, 4, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st, more);
+    if (t.bn == 64) return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st);
+    return tileq::launch<true, 1, 4, 2, 4, 1, 64, 3, false, true, EPI>(x, wp, sc, y, M, N, K, kp, st);
 }
 
 // Decode products of at most 32 rows whose K (or scales) the GEMV of gemv_i4g32_mfma.hip does not take: y fp32 or bf16 [M,N] in one
@@ -1172,7 +1169,7 @@ int gemm_exact_splits(int M, int N, int K) {
     for (int s = 1; s <= kExactMaxSplits; ++s) {
         const int per = (blocks + s - 1) / s, parts = (blocks + per - 1) / per;
         float us;
-        gemm_exact_tile(M, N, per, parts, false, &us);
+        exact_pick(M, N, per, parts, false, &us);
         us += kRead * 4e-6f * (float)rows * (float)N * (float)parts;
         if (s == 1 || us < best_us) {
             best = parts;
@@ -1194,34 +1191,26 @@ static const ExactCost &qkv_pick(int M, int N, int K) {
 bool gemm_exact_qkv_pays(int M, int N, int K) {
     const int parts = gemm_exact_splits(M, N, K), per = (K / 256 + parts - 1) / parts;
     float us;
-    gemm_exact_tile(M, N, per, parts, false, &us);
+    exact_pick(M, N, per, parts, false, &us);
     return exact_us(qkv_pick(M, N, K), M, N, K / 256, 1) <= us + 1.f;
 }
 
-int gemm_exact_qkv_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, const QkvOut &out, int M, int K, hipStream_t st) {
-    const int N = (out.hq + 2) * out.dh;
-    const ExactCost &t = qkv_pick(M, N, K);
-    if (t.bm == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, {}, st, {out});
-    if (t.bm == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, {}, st, {out});
-    return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, {}, st, {out});
-}
+int gemm_exact_qkv_tile(int M, int N, int K) { return qkv_pick(M, N, K).bm; }
 
-int gemm_exact_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
-                          hipStream_t st) {
-    return launch_exact<tileq::EPI_F32>(x, wp, sc, y_parts, M, N, K, ksplit, 1.f, st);
+int gemm_exact_qkv_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, const QkvOut &out, int M, int K, hipStream_t st) {
+    const int N = (out.hq + 2) * out.dh, rows = gemm_exact_qkv_tile(M, N, K);
+    if (rows == 32) return tileq::launch<true, 1, 2, 4, 1, 1, 64, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, {}, st, {out});
+    if (rows == 64) return tileq::launch<true, 1, 2, 4, 2, 1, 64, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, {}, st, {out});
+    return tileq::launch<true, 1, 2, 4, 4, 1, 32, 3, false, true, tileq::EPI_QKV>(x, wp, sc, nullptr, M, N, K, {}, st, {out});
 }
 
 int gemm_exact_scaled_f32_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, float *y_parts, int M, int N, int K, int ksplit,
                                  hipStream_t st) {
-    return launch_exact<tileq::EPI_F32>(x, wp, sc, y_parts, M, N, K, ksplit, kExactX, st);
-}
-
-int gemm_exact_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st) {
-    return launch_exact<tileq::EPI_GEGLU>(x, wp, sc, h, M, N, K, 1, 1.f, st);
+    return launch_exact<tileq::EPI_F32>(x, wp, sc, y_parts, M, N, K, ksplit, st);
 }
 
 int gemm_exact_scaled_geglu_launch(const uint16_t *x, const uint8_t *wp, const uint16_t *sc, uint16_t *h, int M, int N, int K, hipStream_t st) {
-    return launch_exact<tileq::EPI_GEGLU>(x, wp, sc, h, M, N, K, 1, kExactX, st);
+    return launch_exact<tileq::EPI_GEGLU>(x, wp, sc, h, M, N, K, 1, st);
 }
 
 }  // namespace chadq

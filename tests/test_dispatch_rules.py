@@ -119,11 +119,15 @@ def test_prompt_workspace_covers_shorter_chunks(d, hq, dh, ffn):
 
 def test_exact_products_take_the_tile_that_reaches_the_compute_units():
     """us in tiles of 64 / 128 (/ 256) rows."""
-    fn = _rule("_ZN5chadq15gemm_exact_tileEiiiibPf")
-    fn.argtypes = [ctypes.c_int] * 4 + [ctypes.c_bool, ctypes.POINTER(ctypes.c_float)]
+    fn = _rule("_ZN5chadq15gemm_exact_tileEiiiibPfPi")
+    fn.argtypes = [ctypes.c_int] * 4 + [ctypes.c_bool, ctypes.POINTER(ctypes.c_float), ctypes.POINTER(ctypes.c_int)]
 
-    def rows(m, n, per, parts, gated):
-        return fn(m, n, per, parts, gated, ctypes.byref(ctypes.c_float()))
+    def tile(m, n, per, parts, gated):
+        columns = ctypes.c_int()
+        return fn(m, n, per, parts, gated, ctypes.byref(ctypes.c_float()), ctypes.byref(columns)), columns.value
+
+    def rows(*size):
+        return tile(*size)[0]
 
     assert rows(101, 128, 1, 8, False) == 64      # 4.7 / 7.6
     assert rows(158, 5120, 9, 1, False) == 64     # 12.1 / 27.9
@@ -131,6 +135,7 @@ def test_exact_products_take_the_tile_that_reaches_the_compute_units():
     assert rows(101, 8192, 8, 1, True) == 64      # 11.7 / 25.9 / 32.7
     assert rows(256, 32768, 8, 1, True) == 256
     assert rows(64, 32768, 8, 1, True) == 64 and rows(32, 32768, 8, 1, True) == 32 and rows(9, 64, 1, 1, False) == 32
+    assert tile(256, 2048, 16, 4, False) == (128, 64) and tile(385, 5120, 3, 3, False) == (128, 128) and tile(300, 32768, 1, 1, True) == (128, 128)
 
 
 def test_prompt_projections_are_rotated_where_they_are_written_unless_parts_pay():

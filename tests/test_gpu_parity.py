@@ -554,34 +554,41 @@ def test_gemm_each_tile_by_itself(ops, weight, tile):
 
 
 @pytest.mark.parametrize("tile,gated,shapes", [
-    (32, False, [(1, 64, 256, 1), (31, 192, 768, 2), (32, 64, 2560, 8)]),
-    (64, False, [(33, 64, 256, 1), (64, 192, 768, 2), (67, 192, 1280, 2), (129, 512, 2560, 4), (300, 2048, 3072, 3), (193, 1472, 2048, 4)]),
-    (128, False, [(197, 7232, 256, 1), (515, 5248, 512, 1), (130, 7168, 768, 2), (129, 8192, 2560, 4), (385, 5120, 1792, 3), (641, 8192, 1024, 1)]),
-    (32, True, [(1, 512, 256), (32, 1024, 768)]),
-    (64, True, [(33, 512, 512), (70, 2560, 2048), (257, 512, 1024)]),
-    (128, True, [(300, 32768, 256), (130, 12288, 768), (70, 16896, 512), (97, 20480, 2048)]),
-    (256, True, [(130, 20480, 256), (257, 32768, 512), (511, 16384, 768), (256, 32768, 2048)])])
+    ("32x64", False, [(1, 64, 256, 1), (31, 192, 768, 2), (32, 64, 2560, 8)]),
+    ("64x64", False, [(33, 64, 256, 1), (64, 192, 768, 2), (67, 192, 1280, 2), (129, 512, 2560, 4), (300, 2048, 3072, 3), (193, 1472, 2048, 4)]),
+    ("128x128", False, [(197, 7232, 256, 1), (515, 5248, 512, 1), (130, 7168, 768, 2), (129, 8192, 2560, 4), (385, 5120, 1792, 3)]),
+    ("128x64", False, [(641, 8192, 1024, 1), (177, 7600, 2560, 1), (153, 6000, 3072, 2), (255, 2048, 4096, 3), (256, 2048, 16384, 4), (348, 3392, 3584, 3)]),
+    ("32x64", True, [(1, 512, 256), (32, 1024, 768)]),
+    ("64x64", True, [(33, 512, 512), (70, 2560, 2048), (257, 512, 1024)]),
+    ("128x64", True, [(208, 4160, 2304), (130, 6976, 1792), (335, 2880, 2304), (257, 5376, 1280)]),
+    ("128x128", True, [(300, 32768, 256), (130, 12288, 768), (70, 16896, 512), (97, 20480, 2048)]),
+    ("256x128", True, [(130, 20480, 256), (257, 32768, 512), (511, 16384, 768), (256, 32768, 2048)])])
 def test_exact_products_of_each_tile(ops, tile, gated, shapes):
     """A prompt's products by themselves, every tile at ragged ends of its rows, one step and more than the unrolled loop takes, K splits of
-    uneven length; element by element against float64.  The rule by size is asked which tile it is, so that a list goes with its tile."""
+    uneven length; element by element against float64.  The rule by size is asked which tile it is, so that a list goes with its tile.  The
+    activations carry the factor 2^-5 that these products expect, a gated result has it too; both are exact here."""
     import ctypes
 
     from chadslab_amd import _lib
 
     lib = _lib.load()
-    rule = lib["_ZN5chadq15gemm_exact_tileEiiiibPf"]
-    rule.argtypes = [ctypes.c_int] * 4 + [ctypes.c_bool, ctypes.POINTER(ctypes.c_float)]
-    launch = lib["_ZN5chadq23gemm_exact_geglu_launchEPKtPKhS1_PtiiiP12ihipStream_t" if gated else "_ZN5chadq21gemm_exact_f32_launchEPKtPKhS1_PfiiiiP12ihipStream_t"]
+    rule = lib["_ZN5chadq15gemm_exact_tileEiiiibPfPi"]
+    rule.argtypes = [ctypes.c_int] * 4 + [ctypes.c_bool, ctypes.POINTER(ctypes.c_float), ctypes.POINTER(ctypes.c_int)]
+    launch = lib["_ZN5chadq30gemm_exact_scaled_geglu_launchEPKtPKhS1_PtiiiP12ihipStream_t" if gated else
+                 "_ZN5chadq28gemm_exact_scaled_f32_launchEPKtPKhS1_PfiiiiP12ihipStream_t"]
     launch.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * (3 if gated else 4) + [ctypes.c_void_p]
     for i, (m, n, k, *splits) in enumerate(shapes):
         per = -(-(k // 256) // (splits[0] if splits else 1))
         parts = -(-(k // 256) // per)
-        assert rule(m, n, per, parts, gated, ctypes.byref(ctypes.c_float())) == tile, (m, n, k)
+        columns = ctypes.c_int()
+        rows = rule(m, n, per, parts, gated, ctypes.byref(ctypes.c_float()), ctypes.byref(columns))
+        assert "%dx%d" % (rows, columns.value) == tile, (m, n, k)
         g = torch.Generator(device=DEV)
-        g.manual_seed(9700 + 10 * tile + i)
+        g.manual_seed(9700 + 10 * rows + columns.value + i)
         packed = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device=DEV, generator=g)
         scale = torch.exp(torch.randn(n, k // 32, device=DEV, generator=g) * 0.5 - 4.0).half()
         x = torch.randn(m, k, device=DEV, generator=g).bfloat16()
+        scaled = (x.float() * 2.0 ** -5).bfloat16()
         w = torch.stack([packed & 15, packed >> 4], 2).reshape(n, k).double().sub_(8.0).mul_(scale.double().repeat_interleave(32, 1))
         ref, mag = x.double() @ w.t(), x.double().abs() @ w.abs().t()
         # 32 products of a group, its sum among K / 32 of them, the waves' and the parts' sums; an ulp each, as the matrix cores may truncate
@@ -589,15 +596,15 @@ def test_exact_products_of_each_tile(ops, tile, gated, shapes):
         s = torch.cuda.current_stream().cuda_stream
         if gated:
             y = torch.full((m + 1, n // 2), 7.0, dtype=torch.bfloat16, device=DEV)
-            assert launch(x.data_ptr(), packed.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n, k, s) == 0
-            got = y[:m].double()
+            assert launch(scaled.data_ptr(), packed.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n, k, s) == 0
+            got = y[:m].double() * 32
             gate, up = ref[:, ::2], ref[:, 1::2]
             ref = torch.nn.functional.gelu(gate, approximate="tanh") * up
             # |gelu'| <= 1.13 and |gelu(g)| <= |g|; gelu itself to 2^-18 of its argument; the result rounded to bf16
             err = 2.0**-8 * ref.abs() + 1.2 * err[:, ::2] * up.abs() + gate.abs() * err[:, 1::2] + 2.0**-18 * (gate * up).abs()
         else:
             y = torch.full((parts * m + 1, n), 7.0, device=DEV)
-            assert launch(x.data_ptr(), packed.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n, k, parts, s) == 0
+            assert launch(scaled.data_ptr(), packed.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n, k, parts, s) == 0
             got = y[:parts * m].view(parts, m, n).double().sum(0)
         assert bool((y[-1] == 7).all()), "a row too many"
         assert bool(((got - ref).abs() <= err).all()), (m, n, k, float(((got - ref).abs() / err).max()))

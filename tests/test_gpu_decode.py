@@ -1187,7 +1187,8 @@ def test_exact_gated_products_of_every_tile(m, n, k):
 
 
 @pytest.mark.parametrize("m,pos,d,hq,dh", [(1, 0, 256, 1, 64), (7, 5, 512, 4, 64), (32, 1, 256, 3, 128), (33, 100, 768, 2, 256), (64, 0, 512, 8, 64), (65, 9, 1024, 8, 128),
-                                           (256, 33, 2048, 8, 256), (200, 0, 256, 16, 64), (129, 77, 2048, 8, 256)])
+                                           (256, 33, 2048, 8, 256), (200, 0, 256, 16, 64), (129, 77, 2048, 8, 256),
+                                           (200, 3, 256, 64, 64), (300, 0, 2048, 16, 256), (200, 7, 512, 32, 128), (449, 20, 2048, 8, 256)])
 def test_exact_qkv_product_rotates_and_fills_the_caches(m, pos, d, hq, dh):
     """q, k and v with the rotation in the product's epilogue, against float64: every tile, every head size, ragged rows; cache rows outside
     pos .. pos + m - 1 keep their bits.  q in fp32 (2^-20 as the plain products), k and v rounded to bf16 (2^-8)."""
@@ -1199,6 +1200,9 @@ def test_exact_qkv_product_rotates_and_fills_the_caches(m, pos, d, hq, dh):
         _fields_ = [("table", ctypes.c_void_p), ("q", ctypes.c_void_p), ("kc", ctypes.c_void_p), ("vc", ctypes.c_void_p), ("hq", ctypes.c_int),
                     ("dh", ctypes.c_int), ("pos", ctypes.c_int)]
 
+    rule = _lib.load()["_ZN5chadq19gemm_exact_qkv_tileEiii"]
+    rule.argtypes = [ctypes.c_int] * 3
+    assert rule(m, (hq + 2) * dh, d) == (32 if m <= 32 else 128 if (m, hq, dh) in ((200, 64, 64), (300, 16, 256), (200, 32, 128), (449, 8, 256)) else 64)
     fn = _lib.load()["_ZN5chadq21gemm_exact_qkv_launchEPKtPKhS1_RKNS_6QkvOutEiiP12ihipStream_t"]
     fn.argtypes = [ctypes.c_void_p] * 3 + [ctypes.POINTER(Out), ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
     g = torch.Generator(device=DEV)

@@ -1097,7 +1097,8 @@ static const ExactCost kGeglu[4] = {{64, 64, 1.10f, 2.61f, .860f, 2.61f, .860f, 
 // constants of 64 rows and more are fitted to 18700 random products in every number of splits (33 to 700 rows, 128 to 8192 weight rows, 256 to
 // 16000 k) and 8900 gated ones, 2 to 5 % standard deviation (two numbers of the 128-row tiles and one of the gated 256 moved by 0.1 to 0.9 us
 // where tiles are even; 128 x 64, gated, by 0.9: prompts of 70 to 128 tokens took 1 % longer with it where the
-// fit has it even with 128 x 128); the tile and splits they pick take 0.2 % more than the best of all on average.
+// fit has it even with 128 x 128); the tile and splits they pick take 0.2 % more than the best of all on average.  Of 1400 other products, 65 to 600
+// rows, half of them gated, more than half of few steps, the tile picked takes 0.06 % more than the quickest on average and 15 % in the worst case.
 static float exact_us(const ExactCost &t, int M, int N, int per, int parts) {
     const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), fullest = (tiles + 7) / 8 * parts, rounds = (fullest + 31) / 32;
     const float last = t.b + (1.f - t.b) * (float)(fullest - (rounds - 1) * 32) / 32.f, first = t.c0 + t.c1 * (float)per;
@@ -1110,14 +1111,17 @@ static float exact_us(const ExactCost &t, int M, int N, int per, int parts) {
 // 2304 in one 12.1 / 27.9, 432 x 5120 x 1536 24.4 / 21.8; gate/up, 64 / 128 / 256 rows: 101 x 8192 x 2048 11.7 / 25.9 / 32.7, 237 x 32512 x 1792 71.6 /
 // 49.7 / 38.3.  128 x 64 has the unpacking of 128 rows in as many workgroups as half the rows would make: 256 x 2048 x 16384 in four parts 27.2, in 64 x 64
 // tiles in two 31.5, in 128 x 128 in eight 30.0; without it the products of more than 64 rows would take 3 % longer on average, gated ones 4 %.
-// (Three stages; four are 2 % slower.)  (In few steps the loop of 128 rows also takes 0.6 us more than the one with all requests of a step in a row did.)  A prompt of
+// (Three stages; four are 2 % slower.)  In one to three steps it is up to 1.4 times as fast as the others too (81 x 2560 x 4352 in six parts 8.6, 64 x 64
+// 11.9; gated 78 x 13824 x 512 6.9, 9.3; prompts of 115 to 183 tokens, d = 512 or 768: 0.96 to 0.97 of the time).  Only the choice of the parts counts it
+// from four steps on (`splitting`): the parts that it would add there cost the next kernel more, prompts of 110 to 240 tokens, d = 1024 to 1536, 2 to 4 %.
+// (In few steps the loop of 128 rows also takes 0.6 us more than the one with all requests of a step in a row did.)  A prompt of
 // 256 tokens through 18 layers of 2048 x 16384 2518 -> 2320.
-static const ExactCost &exact_pick(int M, int N, int per, int parts, bool geglu, float *us) {
+static const ExactCost &exact_pick(int M, int N, int per, int parts, bool geglu, float *us, bool splitting = false) {
     const ExactCost *const t = M <= 32 ? &kExact32 : geglu ? kGeglu : kExact;
     int best = 0;
     *us = exact_us(t[0], M, N, per, parts);
     for (int i = 1; i < (M <= 64 ? 1 : geglu ? 4 : 3); ++i) {
-        if (i == 1 && per < 4) continue;  // (128 x 64: a step of it is 128 k, and 64 x 64 reach more compute units for the same unpacking)
+        if (i == 1 && per < 4 && splitting) continue;
         const float u = exact_us(t[i], M, N, per, parts);
         if (u < *us) {
             best = i;
@@ -1169,7 +1173,7 @@ int gemm_exact_splits(int M, int N, int K) {
     for (int s = 1; s <= kExactMaxSplits; ++s) {
         const int per = (blocks + s - 1) / s, parts = (blocks + per - 1) / per;
         float us;
-        exact_pick(M, N, per, parts, false, &us);
+        exact_pick(M, N, per, parts, false, &us, true);
         us += kRead * 4e-6f * (float)rows * (float)N * (float)parts;
         if (s == 1 || us < best_us) {
             best = parts;

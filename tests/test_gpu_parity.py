@@ -555,9 +555,9 @@ def test_gemm_each_tile_by_itself(ops, weight, tile):
 
 @pytest.mark.parametrize("tile,gated,shapes", [
     ("32x64", False, [(1, 64, 256, 1), (31, 192, 768, 2), (32, 64, 2560, 8)]),
-    ("64x64", False, [(33, 64, 256, 1), (64, 192, 768, 2), (67, 192, 1280, 2), (129, 512, 2560, 4), (300, 2048, 3072, 3), (193, 1472, 2048, 4)]),
-    ("128x128", False, [(197, 7232, 256, 1), (515, 5248, 512, 1), (130, 7168, 768, 2), (129, 8192, 2560, 4), (385, 5120, 1792, 3)]),
-    ("128x64", False, [(641, 8192, 1024, 1), (177, 7600, 2560, 1), (153, 6000, 3072, 2), (255, 2048, 4096, 3), (256, 2048, 16384, 4), (348, 3392, 3584, 3)]),
+    ("64x64", False, [(33, 64, 256, 1), (64, 192, 768, 2), (67, 192, 1280, 2), (129, 512, 2560, 4), (300, 2048, 3072, 3), (193, 1000, 2048, 4)]),
+    ("128x128", False, [(396, 9280, 256, 1), (515, 5248, 512, 1), (130, 7168, 768, 2), (129, 8192, 2560, 4), (385, 5120, 1792, 3)]),
+    ("128x64", False, [(641, 8192, 1024, 1), (177, 7600, 2560, 1), (153, 6000, 3072, 2), (255, 2048, 4096, 3), (256, 2048, 16384, 4), (348, 3392, 3584, 3), (197, 7232, 256, 1), (193, 1472, 2048, 4)]),
     ("32x64", True, [(1, 512, 256), (32, 1024, 768)]),
     ("64x64", True, [(33, 512, 512), (70, 2560, 2048), (257, 512, 1024)]),
     ("128x64", True, [(208, 4160, 2304), (130, 6976, 1792), (335, 2880, 2304), (257, 5376, 1280)]),

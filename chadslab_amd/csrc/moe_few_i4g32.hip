@@ -7,17 +7,17 @@
 //     K split.  Three workgroups per compute unit walk the items at a stride of the grid, and the loads of the next item
 //     are requested while the present one is summed, so a workgroup's stream has no gap between items.
 //   * The four waves of a workgroup take the item's blocks of 256 k in turn; their sums meet in LDS once per item.
-//   * Everything goes straight to registers, one block ahead: 4 KiB of weights, the scales and the activation operands
-//     (which the caches serve).  Three waves per SIMD with one block ahead measured 4-8 % faster than two with two ahead.
+//   * Weights and scales go straight to registers, a block (4 KiB of weights) ahead of the one being summed.  Three waves per SIMD with one
+//     block ahead measured 4-8 % faster than two with two ahead.
 //   * Where an expert's rows of x or h fit into LDS and a workgroup has items enough (few_launch), they are put there once per
-//     expert and K split, already in operand order, a workgroup's items are neighbours instead of a grid apart, and two blocks
-//     of weights are on their way: a block's activations are 32 registers to its weights' 24, read again for every item.  4 tokens, 8
-//     experts of 4096 x 14336: gate/up 87 -> 77 us, down 50 -> 49; four blocks in flight are no faster than three.
-//   * Otherwise the registers of the activations are single: a piece is requested again for the next block as soon as its MFMAs have
-//     been issued (the caches are nearer than the memory the weights come from).
-//   * Through LDS with more than four tokens, three blocks' registers and a sum per scale group modulo 4 are some ten more than there are.  The
-//     scales of a block are therefore requested a block later than its weights (kLateScales): nothing is spilled in row order.  us, row order,
-//     scales with the weights / later: 5 tokens of 16 experts of 3072 x 5376 76.5 / 74.1, 13 of 16 of 1280 x 9984 97 / 94, 6 of 8 of 2048 x 8960 71.4 / 66.9.
+//     expert and K split, already in operand order, a workgroup's items are neighbours instead of a grid apart, and, with at most
+//     four tokens, two blocks of weights are on their way: a block's activations are 32 registers to its weights' 24, read again for every
+//     item.  4 tokens, 8 experts of 4096 x 14336: gate/up 87 -> 77 us, down 50 -> 49; four blocks in flight are no faster than three.
+//   * Otherwise the activations come from the caches, into single registers: a piece is requested again for the next block as soon as its MFMAs
+//     have been issued (the caches are nearer than the memory the weights come from).
+//   * Through LDS with more than four tokens there is one block ahead as well: two of them and a sum per scale group modulo 4 are some ten
+//     registers more than there are.  96 whole calls of 5 to 16 tokens against one sum and two blocks ahead: 0.987 of the time on average,
+//     1.028 in the worst; with two ahead and the scales requested a block later, which spilled nothing, 1.010 and 1.048; with spills 1.06.
 //   * At most four tokens (FEW): the 16 rows of the A operand are four tokens of four scale groups, each lane group's row non-zero only
 //     where it meets that group's words, so the weights are used in the registers they arrived in (no exchange between lanes), the
 //     sums of four groups come out in one register each and one FMA per four groups and row is left of four: 188 vector instructions per
@@ -46,6 +46,8 @@
 // rounding of h and y.  Signed operands, v_cvt_off_f32_i4 and no second MFMA, would leave no error and take 4 % more time;
 // this form takes 0.3 % more than 128 + u.)  An infinite activation gives NaN, as in the GEMVs.
 // Blocks past the end and rows without a token are requested beyond the buffer's range and arrive as zeros.
+#include <type_traits>
+
 #include "chadq_common.h"
 
 namespace chadq {
@@ -76,8 +78,8 @@ __device__ __forceinline__ void order_x8(const uint32_t a[4], uint32_t o[4]) {
     o[3] = __builtin_amdgcn_perm(a[3], a[2], 0x07060302u);
 }
 
-// XL: activations through LDS (at most kXlBytes of them), two blocks of weights on their way beside the one being summed.  FEW: no expert
-// has more than four rows.  stream: weights are not kept in the caches (tile order: never).
+// XL: activations through LDS (at most kXlBytes of them); with FEW two blocks of weights on their way beside the one being summed, else one.  FEW: no expert
+// has more than four rows.  stream: weights are requested non-temporal (in tile order they always are).
 template <int MODE, bool TILED, bool XL, bool FEW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void moe_few_i4g32_kernel(
     const GemmGroup *__restrict__ groups, const int32_t *__restrict__ tiles, const int32_t *__restrict__ tok, int ntiles, int E, int N,
@@ -136,10 +138,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     u32x4 xq[XL ? 1 : FEW ? 8 : 4];
     // ---- the request side
     int l_item = begin, l_i = 0, l_n = 0, l_kb = 0, l_end = 0;
-    __amdgpu_buffer_rsrc_t wr[RB], sr[RB], xr, x_rsrc, s_rsrc[RB];
-    __amdgpu_buffer_rsrc_t x_rsrc0;
-    constexpr bool kLateScales = XL && !FEW;  // requested a block later, so that two blocks' scales are in registers and not three
-    uint32_t s_voff = kBeyond, s_kb = 0;      // where those of the last block requested are
+    __amdgpu_buffer_rsrc_t wr[RB], sr[RB], xr, x_rsrc, x_rsrc0;
     uint32_t x_voff = kBeyond, x_kb = 0, x_voff0 = kBeyond, x_kb0 = 0;  // where the activations of the last block requested and of the one before it are
     uint32_t woff = 0, soff = 0, xoff = 0;  // of the lane, in the first row block
     // the second row block: the same rows of the up matrix, or the next 16 rows
@@ -171,42 +170,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             soff = n * (uint32_t)(K >> 4);
         }
     };
-    auto scales_of = [&](__amdgpu_buffer_rsrc_t from, int b, uint32_t sv, uint32_t kb) {
-        if constexpr (TILED) {
-            const uint32_t sk = kb * 512u + b * sblk;
-            const u32x2 ev = __builtin_amdgcn_raw_buffer_load_b64(from, sv, sk, 0), od = __builtin_amdgcn_raw_buffer_load_b64(from, sv, sk + 256u, 0);
-            return u32x4{ev.x, ev.y, od.x, od.y};
-        } else {
-            return (u32x4)__builtin_amdgcn_raw_buffer_load_b128(from, sv, kb * 16u + b * sblk, 0);
-        }
-    };
-    auto request_scales = [&](Block &q) {  // of the last block requested
-#pragma unroll
-        for (int b = 0; b < RB; ++b) q.s[b] = scales_of(s_rsrc[b], b, s_voff, s_kb);
-    };
     auto request = [&](Block &q) {
         x_rsrc0 = x_rsrc;
         x_voff0 = x_voff;
         x_kb0 = x_kb;
         if (l_item >= total) {
             x_voff = kBeyond;
-            s_voff = kBeyond;
             return;
         }
         const uint32_t kb = l_kb, beyond = l_kb < l_end ? 0u : kBeyond, wv = woff | beyond, sv = soff | beyond, xv = xoff | beyond;
 #pragma unroll
         for (int b = 0; b < RB; ++b) {
-            if constexpr (kLateScales) s_rsrc[b] = sr[b];
-            else q.s[b] = scales_of(sr[b], b, sv, kb);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const uint32_t at = kb * (TILED ? 4096u : 128u) + b * wblk + h * (TILED ? 2048u : 4u * K);
-                if (TILED || stream) q.w[b][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[b], wv, at, 2);
-                else q.w[b][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[b], wv, at, 0);
+            if (TILED) {
+                const uint32_t sk = kb * 512u + b * sblk;
+                const u32x2 ev = __builtin_amdgcn_raw_buffer_load_b64(sr[b], sv, sk, 0), od = __builtin_amdgcn_raw_buffer_load_b64(sr[b], sv, sk + 256u, 0);
+                q.s[b] = u32x4{ev.x, ev.y, od.x, od.y};
+            } else {
+                q.s[b] = __builtin_amdgcn_raw_buffer_load_b128(sr[b], sv, kb * 16u + b * sblk, 0);
             }
         }
-        s_voff = sv;
-        s_kb = kb;
+        auto weights = [&](auto policy) {
+#pragma unroll
+            for (int b = 0; b < RB; ++b)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    q.w[b][h] = __builtin_amdgcn_raw_buffer_load_b128(wr[b], wv, kb * (TILED ? 4096u : 128u) + b * wblk + h * (TILED ? 2048u : 4u * K),
+                                                                      decltype(policy)::value);
+        };
+        // (one branch, not one per load: 1 % of the calls of five to 16 tokens)
+        if (TILED || stream) weights(std::integral_constant<int, 2>{});
+        else weights(std::integral_constant<int, 0>{});
         if constexpr (!XL) {
             x_rsrc = xr;
             x_voff = xv;
@@ -425,27 +418,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     if (l_item >= total) return;
     open();
     c_n = l_n;
-    if constexpr (XL) {
+    if constexpr (XL && FEW) {
         Block q0, q1, q2;
         request(q0);
-        if constexpr (kLateScales) request_scales(q0);
         request(q1);
         for (;;) {
-            if constexpr (kLateScales) request_scales(q1);
             request(q2);
             if (!consume(q0)) break;
-            if constexpr (kLateScales) request_scales(q2);
             request(q0);
             if (!consume(q1)) break;
-            if constexpr (kLateScales) request_scales(q0);
             request(q1);
             if (!consume(q2)) break;
         }
     } else {
         Block q0, q1;
         request(q0);
+        if constexpr (!XL) {
 #pragma unroll
-        for (int g = 0; g < (FEW ? 8 : 4); ++g) request_x(g, true);
+            for (int g = 0; g < (FEW ? 8 : 4); ++g) request_x(g, true);
+        }
         for (;;) {
             request(q1);
             if (!consume(q0)) break;

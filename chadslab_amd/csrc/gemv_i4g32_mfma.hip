@@ -1002,7 +1002,9 @@ int gemv_i4g32_mfma_dispatch(const uint16_t *x, const uint8_t *wp, const uint16_
 }
 
 // Parts of K, fp32 sums, for few weight rows and a long K, as gemv_i8row_parts has them for int8 weights.  us, in one part / in parts, 512 x 16384: 1 row
-// 10.6 / 7.0, 4 10.3 / 7.4, 8 17.8 / 8.3, 16 23.0 / 7.6; 2048 x 8192, 8 rows 10.1 / 8.4, 16 12.8 / 9.9; 256 x 5120, 6 rows 8.6 / 7.3.
+// 10.6 / 7.0, 4 10.3 / 7.4, 8 17.8 / 8.3, 16 23.0 / 7.6; 2048 x 8192, 8 rows 10.1 / 8.4, 16 12.8 / 9.9; 256 x 5120, 6 rows 8.6 / 7.3.  73 random calls in
+// parts: 0.79 of the time waited for one by one, none slower; in a row 0.67, three of them 3 to 6 % slower (1 x 64 x 9728 8.0 / 8.4: what the host needs
+// for two launches).
 int gemv_i4g32_parts(int M, int N, int K, int *span) {
     const int chunk = M <= 8 ? 4096 : 2048;  // what the kernels take between two barriers
     *span = K;

@@ -35,7 +35,7 @@ __global__ __launch_bounds__(256) void prompt_embed_kernel(const int32_t *__rest
 }
 
 // One row per workgroup: r = res + the np parts (part p of row t at parts + (p * rows + t) * d, added in order), kept in
-// res_out if there were any (may be res), then, if y, y = bf16(r / sqrt(mean(r^2) + eps) * w) * kExactX.  d % 4 == 0, d <= 2048.
+// res_out if there were any (may be res), then, if y, y = bf16(r / sqrt(mean(r^2) + eps) * w * kExactX).  d % 4 == 0, d <= 2048.
 // NP: the number of parts, so that every load is in flight before the first sum (one memory round trip, not np of them).
 template <int NP>
 __global__ __launch_bounds__(256) void prompt_add_norm_kernel(const float *res, float *res_out, const float *__restrict__ parts,
